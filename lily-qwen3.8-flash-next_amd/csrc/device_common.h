@@ -107,6 +107,12 @@ __device__ __forceinline__ bool last_to_arrive(uint32_t* ticket, uint32_t expect
     return last;
 }
 
+// Enters an id into a scratch's maps of listed ids (`words`: of the bitmap).
+__device__ __forceinline__ void mark_listed(uint32_t* touched, uint32_t words, uint32_t id) {
+    atomicOr(&touched[id >> 5], 1u << (id & 31u));
+    atomicOr(&touched[words + LISTED_SPARE + (id >> 8)], 1u << ((id >> 3) & 31u));
+}
+
 template <int DT>
 __device__ __forceinline__ float load_logit(const void* p, uint32_t i) {
     if (DT == LILY_BF16) {

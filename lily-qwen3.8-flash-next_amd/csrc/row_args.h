@@ -73,10 +73,18 @@ struct alignas(16) RowArgs {
 };
 static_assert(sizeof(RowArgs) == 224, "RowArgs layout");
 
+// The ids a scratch ever counted ("listed" ids), as its `touched` words hold them: a bit per id;
+// LISTED_SPARE words, the first the largest count any id has reached and the second an id that
+// reached it; then the coarse map, a bit per eight ids of which at least one is listed (the scan
+// of penalised rows reads this one beside the logits, 1 / 8 of the bitmap); and four spare words.
+constexpr uint32_t LISTED_SPARE = 4;
+constexpr uint32_t listed_words(uint32_t vocab) {
+    return (vocab + 31u) / 32u + LISTED_SPARE + (vocab + 255u) / 256u + 4u;
+}
 // A scratch's device state as the small maintenance kernels take it.
 struct ScratchView {
     uint32_t* counts;    // [vocab]
-    uint32_t* touched;   // [ceil(vocab / 32) + 4]
+    uint32_t* touched;   // [listed_words(vocab)]
     uint32_t vocab;
 };
 
@@ -154,7 +162,7 @@ constexpr uint32_t SPECIAL_LIST_CAP = 2048;  // ids of penalised / biased tokens
 constexpr uint32_t STREAM_K_MAX = 64;
 constexpr uint32_t STREAM_UNROLL = 4;      // 16-byte chunks per thread per block
 constexpr uint32_t Q_CAP = 768;            // queued chunks (those holding a value at or above the bound)
-constexpr uint32_t S_CAP = 4096;           // noted chunks (summed before their listed ids were looked at)
+constexpr uint32_t S_CAP = 4096;           // noted chunks (above the sum's cut: their terms are formed behind the scan)
 constexpr uint32_t FC_CAP = 1024;          // final candidates
 constexpr uint32_t MAX_BLOCKS = 64;        // blocks of one slice
 constexpr uint32_t STREAM_BIAS_CAP = 64;   // bias pairs kept in LDS

@@ -7,6 +7,7 @@
 #include "device_common.h"
 #include "select_bitmap.h"
 #include "select_exhaustive.h"
+#include "select_lowering.h"
 #include "select_sparse.h"
 #include "select_stream.h"
 #include "tail.h"
@@ -104,6 +105,12 @@ __device__ __forceinline__ void apply_selection(RowArgs& a) {
     }
 }
 
+// Rows of select_lowering(): under penalties that can only lower a value, nothing else in play.
+__device__ __forceinline__ bool lowering_row(const RowArgs& a) {
+    return (a.flags & F_PEN) != 0u && a.repetition >= 1.0f && a.presence >= 0.0f && a.frequency >= 0.0f &&
+           a.allow == nullptr && a.n_bias == 0u;
+}
+
 template <int DT, int KIND, bool LSE, bool CHAIN = false>
 __device__ __forceinline__ void row_body(const LILY_CONST RowArgs* src, const LaunchCfg& cfg, Shared& sh) {
     if (cfg.served != nullptr && *(const LILY_CONST uint32_t*)(cfg.served + blockIdx.y) != 0u) {
@@ -146,9 +153,23 @@ __device__ __forceinline__ void row_body(const LILY_CONST RowArgs* src, const La
         bool done = false;
         uint32_t took = 2;
         if (cfg.path == 0u && (a.flags & F_STREAM)) {
-            done = select_stream<DT, LSE, KIND != 2>(a, g, a.k, sh, cfg, sorted, found);
-            if (!done) {
-                __syncthreads();
+            if (lowering_row(a)) {
+                bool again = false;
+                done = select_lowering<DT, LSE, false>(a, g, a.k, sh, cfg, again, sorted, found);
+                if (!done) {
+                    __syncthreads();
+                }
+                if (again) {
+                    done = select_lowering<DT, LSE, true>(a, g, a.k, sh, cfg, again, sorted, found);
+                    if (!done) {
+                        __syncthreads();
+                    }
+                }
+            } else {
+                done = select_stream<DT, LSE, KIND != 2>(a, g, a.k, sh, cfg, sorted, found);
+                if (!done) {
+                    __syncthreads();
+                }
             }
             took = done ? 0u : took;
         }

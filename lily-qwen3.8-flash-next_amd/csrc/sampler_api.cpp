@@ -127,9 +127,8 @@ struct lily_scratch {
     lily_sampler* s = nullptr;
     uint32_t vocab = 0;
     uint32_t words = 0;
-    uint32_t* counts = nullptr;   // [vocab]; the one allocation, the bitmap follows it
-    uint32_t* touched = nullptr;  // [words + 4] bit per id that was ever counted, then the largest
-                                  // count any id has reached
+    uint32_t* counts = nullptr;   // [vocab]; the one allocation, the maps follow it
+    uint32_t* touched = nullptr;  // [listed_words(vocab)] the ids that were ever counted
 };
 
 struct lily_draft_dists {
@@ -1005,9 +1004,9 @@ int lily_scratch_create(lily_sampler_t* s, uint32_t vocab, lily_scratch_t** out)
     sc->s = s;
     sc->vocab = vocab;
     sc->words = (vocab + 31u) / 32u;
-    // One allocation: the counts, then the bitmap (16-byte aligned, four spare words).
+    // One allocation: the counts, then the maps of listed ids (16-byte aligned).
     const size_t dense = (((size_t)vocab * 4) + 15) & ~(size_t)15;
-    const size_t bitmap = (((size_t)(sc->words + 4) * 4) + 15) & ~(size_t)15;
+    const size_t bitmap = (((size_t)listed_words(vocab) * 4) + 15) & ~(size_t)15;
     hipError_t e = hipMalloc(reinterpret_cast<void**>(&sc->counts), dense + bitmap);
     if (e != hipSuccess) {
         delete sc;
@@ -1036,7 +1035,7 @@ int lily_scratch_reset_counts(lily_scratch_t* sc) {
     }
     ON_DEVICE(sc->s->device);
     HIP_TRY(launch_fill_u32(sc->s->stream, sc->counts, sc->vocab, 0));
-    HIP_TRY(launch_fill_u32(sc->s->stream, sc->touched, sc->words + 4, 0));
+    HIP_TRY(launch_fill_u32(sc->s->stream, sc->touched, listed_words(sc->vocab), 0));
     return LILY_OK;
 }
 
@@ -1078,8 +1077,8 @@ int lily_scratch_copy_counts_from(lily_scratch_t* dst, const lily_scratch_t* src
     ON_DEVICE(dst->s->device);
     HIP_TRY(hipMemcpyAsync(dst->counts, src->counts, (size_t)src->vocab * 4, hipMemcpyDeviceToDevice,
                            dst->s->stream));
-    // (the bitmap and the largest count behind it)
-    HIP_TRY(hipMemcpyAsync(dst->touched, src->touched, (size_t)(src->words + 2) * 4,
+    // (the maps of listed ids and the largest count between them)
+    HIP_TRY(hipMemcpyAsync(dst->touched, src->touched, (size_t)listed_words(src->vocab) * 4,
                            hipMemcpyDeviceToDevice, dst->s->stream));
     return LILY_OK;
 }

@@ -2,6 +2,7 @@
 // host-callable launchers, including the dispatch among the row kernel's variants.
 #include <hip/hip_runtime.h>
 
+#include "device_common.h"
 #include "launch.h"
 
 namespace lily {
@@ -23,8 +24,8 @@ __global__ void k_add_history(ScratchView sc, const uint32_t* ids, uint32_t n) {
         const uint32_t id = ids[i];
         if (id < sc.vocab) {
             const uint32_t before = atomicAdd(&sc.counts[id], 1u);
-            atomicOr(&sc.touched[id >> 5], 1u << (id & 31u));
             const uint32_t words = (sc.vocab + 31u) / 32u;
+            mark_listed(sc.touched, words, id);
             if (atomicMax(&sc.touched[words], before + 1u) <= before + 1u) {
                 sc.touched[words + 1u] = id;
             }
@@ -65,8 +66,9 @@ __global__ void k_uncount_after(ScratchView sc, const uint32_t* draws, uint32_t 
     }
 }
 
-// After counts were written whole: touched[w] = bits of the non-zero counts in word w, and the
-// largest count (the word behind the bitmap, cleared before the launch).
+// After counts were written whole: touched[w] = bits of the non-zero counts in word w, their four
+// bits of the coarse map and the largest count (all that lies behind the bitmap is cleared before
+// the launch).
 __global__ void k_touch_from_counts(ScratchView sc) {
     const uint32_t w = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t words = (sc.vocab + 31u) / 32u;
@@ -84,6 +86,13 @@ __global__ void k_touch_from_counts(ScratchView sc) {
             }
         }
         sc.touched[w] = bits;
+        uint32_t groups = 0;
+        for (uint32_t q = 0; q < 4u; ++q) {
+            groups |= ((bits >> (8u * q)) & 0xffu) != 0u ? 1u << q : 0u;
+        }
+        if (groups != 0u) {
+            atomicOr(&sc.touched[words + LISTED_SPARE + w / 8u], groups << (4u * (w % 8u)));
+        }
         if (most != 0u && atomicMax(&sc.touched[words], most) <= most) {
             sc.touched[words + 1u] = most_id;
         }
@@ -123,7 +132,6 @@ __global__ void k_copy_row_u32(const uint32_t* src, uint32_t* dst, uint32_t word
 }
 
 // n 16-byte pieces from src to dst (src may be pinned host memory mapped into the device).
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 __global__ void __launch_bounds__(256) k_copy_pieces(const u32x4* src, u32x4* dst, uint32_t n) {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i < n) {
@@ -239,7 +247,8 @@ hipError_t launch_uncount_after(hipStream_t stream, const ScratchView& sc, const
 
 hipError_t launch_rebuild_listed(hipStream_t stream, const ScratchView& sc) {
     const uint32_t words = (sc.vocab + 31u) / 32u;
-    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, stream, sc.touched + words, 2u, 0u);
+    hipLaunchKernelGGL(k_fill_u32, dim3((listed_words(sc.vocab) - words + 255) / 256), dim3(256), 0, stream, sc.touched + words,
+                       listed_words(sc.vocab) - words, 0u);
     hipLaunchKernelGGL(k_touch_from_counts, dim3((words + 255) / 256), dim3(256), 0, stream, sc);
     return hipGetLastError();
 }

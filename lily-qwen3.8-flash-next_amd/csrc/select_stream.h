@@ -110,8 +110,386 @@ __device__ __forceinline__ double wg_sum_d(Shared& sh, double v) {
 __device__ __forceinline__ bool stream_fail(const LaunchCfg& cfg, uint32_t why) {
     if (cfg.path_stats != nullptr && threadIdx.x == 0) {
         atomicOr(&cfg.path_stats[3], 1u << why);
+        // (waited for here, where it is rare: a pending atomic makes every later wait for a load
+        // drain all loads in flight)
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
     }
     return false;
+}
+
+// Element j of a chunk: one compare picks the 8-byte half, one 64-bit shift the element.
+template <int DT>
+__device__ __forceinline__ float chunk_elem(const u32x4& q, uint32_t j) {
+    constexpr int E = Geo<DT>::E;
+    const bool upper = (j & (uint32_t)(E / 2)) != 0u;
+    const uint64_t half = upper ? (((uint64_t)q.w << 32) | q.z) : (((uint64_t)q.y << 32) | q.x);
+    if (E == 8) {
+        return lilym_bits_f32((uint32_t)(half >> ((j & 3u) * 16u)) << 16);
+    }
+    return lilym_bits_f32((uint32_t)(half >> ((j & 1u) * 32u)));
+}
+
+// The chunk with the elements of `bits` replaced by -inf.
+template <int DT>
+__device__ __forceinline__ u32x4 chunk_without(const u32x4& q, uint32_t bits) {
+    u32x4 r = q;
+    if (DT == LILY_BF16) {
+        auto fix = [](uint32_t v, uint32_t two) -> uint32_t {
+            const uint32_t m = ((two & 1u) ? 0x0000ffffu : 0u) | ((two & 2u) ? 0xffff0000u : 0u);
+            return (v & ~m) | (0xff80ff80u & m);
+        };
+        r.x = fix(q.x, bits);
+        r.y = fix(q.y, bits >> 2);
+        r.z = fix(q.z, bits >> 4);
+        r.w = fix(q.w, bits >> 6);
+    } else {
+        r.x = (bits & 1u) ? 0xff800000u : q.x;
+        r.y = (bits & 2u) ? 0xff800000u : q.y;
+        r.z = (bits & 4u) ? 0xff800000u : q.z;
+        r.w = (bits & 8u) ? 0xff800000u : q.w;
+    }
+    return r;
+}
+
+// What a thread's scan and the work behind it left of the row's sum of exponentials.
+struct StreamSums {
+    static constexpr int UP_UNSET = INT_MIN;
+    float ref_s;       // reference of acc_t and acc_r, fixed after the first block ...
+    int up;            // ... and how far above it this thread's own lies (UP_UNSET: no such term)
+    double acc_t;      // true terms added one by one
+    double acc_r;      // raw terms to take off the running sum again
+    double ref_p;      // reference of acc_p, the same in every thread
+    double acc_p;      // terms relative to ref_p
+    bool simple_p;     // every term of acc_p fits that reference (the same in every thread)
+};
+
+// Brings the workgroup's sums together: sh.lse_mc, sh.lse_s (thread 0 writes them).
+template <int DT>
+__device__ __forceinline__ void stream_row_sum(const RowArgs& a, const Geo<DT>& g, const StreamSums& t, const WaveLse& wl,
+                                               Shared& sh, const LaunchCfg& cfg) {
+    constexpr int UP_UNSET = StreamSums::UP_UNSET;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
+    const int up = t.up;
+    const double acc_p = t.acc_p, acc_t = t.acc_t, acc_r = t.acc_r, ref_p = t.ref_p;
+    const float ref_s = t.ref_s;
+    const bool simple_p = t.simple_p;
+    // A row that noted its chunks holds nothing, as a rule, but terms relative to the one
+    // reference ref_p: the waves' sums meet in LDS behind one barrier.  A thread with a sum of
+    // another kind (terms formed during the scan, terms that reference cannot hold) sends the
+    // row the long way below.
+    const bool other_sums = up != UP_UNSET || !(wl.s == 0.0f) || !(wl.booked == 0.0f);
+    const double p_wave = wave_sum_d_dpp(acc_p);
+    if (lane == 0) {
+        sh.red_d[w] = p_wave;
+    }
+    const bool long_way = __syncthreads_or((!simple_p || other_sums) ? 1 : 0) != 0;
+    double p_all = 0.0;
+    for (int i = 0; i < NWAVE; ++i) {
+        p_all += sh.red_d[i];
+    }
+    if (!long_way) {
+        phase(cfg, 10);
+        if (tid == 0) {
+            sh.lse_mc = ref_p;
+            sh.lse_s = p_all;
+        }
+    } else {
+        // Each wave brings its sums to one reference of its own: the highest of its threads'
+        // references and of the streamed sums' (wave-uniform) reference.  The waves' partial
+        // sums and references meet in LDS and are brought together after one barrier.
+        int ref_w = up;
+        for (int o = 32; o > 0; o >>= 1) {
+            ref_w = max(ref_w, __shfl_xor(ref_w, o));
+        }
+        const double stream_at = (double)wl.ref - (double)ref_s;  // exact
+        if (__ballot(wl.s > 0.0f) != 0ull) {
+            const double e = stream_at < 1.0e9 ? (stream_at > -1.0e9 ? stream_at : -1.0e9) : 1.0e9;
+            ref_w = max(ref_w, (int)__builtin_floor(e));
+        }
+        const int down = up == UP_UNSET ? 0 : up - ref_w;  // <= 0
+        double part[4];
+        {
+            double d = stream_at - (double)ref_w;  // <= 1 where there is a sum
+            d = d < -1000.0 ? -1000.0 : d;
+            const double scale = pow2_d(d);
+            part[0] = wl.s > 0.0f ? (double)wl.s * scale : 0.0;
+            part[3] = wl.booked > 0.0f ? (double)wl.booked * scale : 0.0;
+        }
+        part[1] = __builtin_ldexp(acc_r, down);
+        part[2] = __builtin_ldexp(acc_t, down);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            part[i] = wave_sum_d(part[i]);
+            if (lane == 0) {
+                sh.red3[i][w] = part[i];
+            }
+        }
+        if (lane == 0) {
+            sh.red_i[w] = (uint32_t)ref_w;
+        }
+        // A NaN logit in a summed chunk leaves its wave's running sum a NaN: such a logit is
+        // worth -inf, and the row's sum is formed again from every value.
+        const bool poisoned = __syncthreads_or(wl.s != wl.s ? 1 : 0) != 0;
+        int ref_all = (int)sh.red_i[0];
+        for (int i = 1; i < NWAVE; ++i) {
+            ref_all = max(ref_all, (int)sh.red_i[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            part[i] = 0.0;
+            for (int ww = 0; ww < NWAVE; ++ww) {
+                const int at = (int)sh.red_i[ww];
+                part[i] += at == UP_UNSET ? 0.0 : __builtin_ldexp(sh.red3[i][ww], at - ref_all);
+            }
+        }
+        if (ref_all == UP_UNSET) {
+            ref_all = 0;  // no term anywhere: the sums are zero
+        }
+        // part[0]: the running sums, the listed ids' raw terms of part[3] already taken off (and
+        // their true terms added); part[1]: raw terms still to take off; part[2]: terms added
+        // one by one.
+        const double streamed = part[0], booked = part[1], exact = part[2], taken = part[3];
+        const double rest = streamed - booked;
+        // The streamed sums are f32: taking the listed ids' raw terms off again leaves an error of
+        // about 1e-6 of what was streamed.  Where that is more than 20 times the row's sum (listed
+        // ids held nearly everything that was streamed, and nothing larger was added exactly) the
+        // difference is too coarse.
+        const bool coarse = poisoned ||
+                            (booked + taken > 0.0 &&
+                             !((rest > 0.0 ? rest : 0.0) + exact > 0.05 * (streamed + taken)));
+        phase(cfg, 10);
+        if (coarse) {
+            phase(cfg, 11);
+            LseAcc all;
+            all.init();
+            exact_terms<DT>(a, g.id_lo, g.id_hi, a.c2, all);
+            double m_e, s_e;
+            wg_merge_lse(sh, all.mc, all.s, m_e, s_e);
+            if (tid == 0) {
+                sh.lse_mc = m_e;
+                sh.lse_s = s_e;
+            }
+        } else if (tid == 0) {
+            double mc = (double)ref_s + (double)ref_all;
+            double sum = (rest > 0.0 ? rest : 0.0) + exact;
+            if (p_all > 0.0) {
+                // The terms relative to ref_p have a reference of their own: the higher of the
+                // two serves both (what lies 2^1000 below the other adds nothing).
+                if (!(sum > 0.0)) {
+                    mc = ref_p;
+                    sum = p_all;
+                } else {
+                    const double top = mc > ref_p ? mc : ref_p;
+                    const double d0 = mc - top, d1 = ref_p - top;
+                    sum = sum * pow2_d(d0 < -1000.0 ? -1000.0 : d0) +
+                          p_all * pow2_d(d1 < -1000.0 ? -1000.0 : d1);
+                    mc = top;
+                }
+            }
+            sh.lse_mc = mc;
+            sh.lse_s = sum;
+        }
+
+    }
+}
+
+// Ranks the candidates in L.fc and decides whether they stand: everything that is not a
+// candidate lies strictly below `filt`, so the result is exact if k candidates were found and the
+// k-th lies strictly above anything the division by the temperature can map such a value to.
+__device__ __forceinline__ bool stream_accept(StreamLds& L, float filt, float temperature, uint32_t k, Shared& sh,
+                                              const LaunchCfg& cfg, bool& sorted, uint64_t*& out) {
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
+    uint32_t n = sh.n_fc;
+    phase(cfg, 3);
+    if (n > FC_CAP) {
+        return stream_fail(cfg, 5u);
+    }
+    sorted = false;
+    n = select_topk(L.fc, n, k, sh, sorted);
+    phase(cfg, 12);
+    if (filt > F32_LOWEST) {
+        uint32_t lowest = 0xffffffffu;
+        if (sorted) {
+            // Ranked candidates are in descending order: the last one is the lowest.
+            lowest = n > 0u ? (uint32_t)(L.fc[n - 1u] >> 32) : lowest;
+        } else {
+            for (uint32_t i = tid; i < n; i += NT) {
+                lowest = min(lowest, (uint32_t)(L.fc[i] >> 32));
+            }
+            lowest = wave_min_u32(lowest);
+            if (lane == 0) {
+                sh.red_i[w] = lowest;
+            }
+            __syncthreads();
+            lowest = sh.red_i[0];
+            for (int i = 1; i < NWAVE; ++i) {
+                lowest = min(lowest, sh.red_i[i]);
+            }
+            __syncthreads();
+        }
+        const float below = lilym_key_value(lilym_order_key(filt) - 1u) / temperature;
+        if (!(n >= k && lilym_order_key(below) < lowest)) {
+            return stream_fail(cfg, 6u);
+        }
+    }
+    // The candidates stay where they are (the tail's arrays and the merge's buffer lie below
+    // them in dynamic LDS).
+    out = L.fc;
+    if (tid == 0) {
+        sh.n_cand = n;
+    }
+    __syncthreads();
+    return true;
+}
+
+// A wave that has further to go asks to be issued first, so that the workgroups that share a
+// compute unit advance together instead of in the order they arrived (the arbiter otherwise
+// favours the oldest wave, and the rows dispatched last scan alone at the end).  Four levels: the
+// quarter of the way the wave has come, rows dispatched earlier counted as two blocks further on
+// per generation.  The blocks at which the level changes are worked out once: two divisions and a
+// load of the grid's size for every block of every wave were a tenth of the scan's instructions.
+struct StreamPriority {
+    int32_t at1, at2, at3;   // the first blocks of levels 2, 1 and 0
+    __device__ __forceinline__ void init(uint32_t nblocks) {
+        const uint32_t gen = min((blockIdx.y * 4u) / max(gridDim.y, 1u), 3u);
+        const int32_t n = (int32_t)nblocks + 6, ahead = 2 * (3 - (int32_t)gen);
+        at1 = __builtin_amdgcn_readfirstlane((n + 3) / 4 - ahead);
+        at2 = __builtin_amdgcn_readfirstlane((2 * n + 3) / 4 - ahead);
+        at3 = __builtin_amdgcn_readfirstlane((3 * n + 3) / 4 - ahead);
+    }
+    __device__ __forceinline__ void set(uint32_t b) const {
+        const int32_t at = (int32_t)b;
+        if (at < at1) {
+            __builtin_amdgcn_s_setprio(3);
+        } else if (at < at2) {
+            __builtin_amdgcn_s_setprio(2);
+        } else if (at < at3) {
+            __builtin_amdgcn_s_setprio(1);
+        } else {
+            __builtin_amdgcn_s_setprio(0);
+        }
+    }
+};
+
+// The waves' queue segments counted through in order: place `ch` of them all.
+struct QueueOrder {
+    uint32_t seg_end[NWAVE];
+    uint32_t total;
+    __device__ __forceinline__ void init(const uint32_t* fill) {
+        total = 0;
+#pragma unroll
+        for (int i = 0; i < NWAVE; ++i) {
+            total += fill[i];
+            seg_end[i] = total;
+        }
+    }
+    template <uint32_t SEG>
+    __device__ __forceinline__ uint32_t slot(uint32_t ch) const {
+        uint32_t ww = 0, before = 0;
+#pragma unroll
+        for (int i = 0; i + 1 < NWAVE; ++i) {
+            if (ch >= seg_end[i]) {
+                ww = (uint32_t)i + 1u;
+                before = seg_end[i];
+            }
+        }
+        return ww * SEG + (ch - before);
+    }
+};
+
+// Rows under penalties that only lower: every element of a queued chunk (of those `with` admits)
+// that matters by its raw value - at or above the bound, or above the sum's cut - is listed as an
+// (id, raw value) pair, wave by wave; then one thread per pair gathers the id's count, so that all
+// of the row's gathers are one round trip to memory.  (A listed id's true value is not above its
+// raw one: what does not matter raw does not matter.)  The pairs lie where the candidates arrive
+// once every pair is in a register.
+template <int DT, class With, class Skip>
+__device__ __forceinline__ void stream_pairs_list(const StreamLds& L, const Geo<DT>& g, const QueueOrder& order, float filt,
+                                                  float cut, Shared& sh, With&& with, Skip&& skip) {
+    constexpr int E = Geo<DT>::E;
+    uint64_t* pairs = L.fc;
+    for (uint32_t ch0 = 0; ch0 < order.total; ch0 += NT) {
+        const uint32_t ch = ch0 + threadIdx.x;
+        uint32_t todo = 0, c = 0;
+        u32x4 q = {};
+        if (ch < order.total) {
+            const uint32_t slot = order.template slot<Q_CAP / NWAVE>(ch);
+            q = L.qraw[slot];
+            c = L.qidx[slot];
+            float v[E];
+            unpack<DT>(q, v);
+#pragma unroll
+            for (int j = 0; j < E; ++j) {
+                const bool cand = v[j] >= filt && v[j] > NEG_INF;
+                todo |= (v[j] > cut || cand) ? 1u << j : 0u;
+            }
+            todo = with(c) ? todo : 0u;
+        }
+        while (__ballot(todo != 0u) != 0ull) {
+            const bool has = todo != 0u;
+            const uint32_t j = has ? (uint32_t)__builtin_ctz(todo) : 0u;
+            todo &= todo - 1u;   // (0 stays 0)
+            const uint32_t id = g.id_of(c, (int)j);
+            const bool push = has && !skip(id);
+            const uint64_t mask = __ballot(push);
+            if (mask != 0ull) {
+                const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
+                    (uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+                uint32_t first = 0;
+                if (rank == 0u && push) {
+                    first = atomicAdd(&sh.n_pairs, (uint32_t)__popcll(mask));
+                }
+                first = (uint32_t)__builtin_amdgcn_readlane((int)first, __builtin_ctzll(mask));
+                if (push && first + rank < FC_CAP) {
+                    pairs[first + rank] = ((uint64_t)lilym_f32_bits(chunk_elem<DT>(q, j)) << 32) | id;
+                }
+            }
+        }
+    }
+}
+
+// Behind a barrier, with at most FC_CAP pairs: their true values become terms and candidates.
+template <class Term>
+__device__ __forceinline__ void stream_pairs_take(const StreamLds& L, const RowArgs& a, float filt, Shared& sh, Term&& add_term) {
+    static_assert(FC_CAP <= 4 * NT, "four pairs a thread");
+    const uint32_t tid = threadIdx.x;
+    const uint32_t n_pairs = sh.n_pairs;
+    uint64_t pr[4];
+    uint32_t cnt[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t at = tid + (uint32_t)i * NT;
+        pr[i] = at < n_pairs ? L.fc[at] : 0ull;
+        cnt[i] = gload(a.counts + (uint32_t)pr[i]);   // (id 0 for an empty place)
+    }
+    __syncthreads();   // every pair is in a register: the candidates may take their place
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const bool valid = tid + (uint32_t)i * NT < n_pairs;
+        const uint32_t id = (uint32_t)pr[i];
+        float x = lilym_bits_f32((uint32_t)(pr[i] >> 32));
+        if (cnt[i] > 0u) {
+            x = x > 0.0f ? x / a.repetition : x * a.repetition;
+            x -= a.presence + a.frequency * (float)cnt[i];
+        }
+        if (valid) {
+            add_term(x);
+        }
+        const bool cand = valid && x >= filt && x > NEG_INF;
+        const uint64_t mask = __ballot(cand);
+        if (mask != 0ull) {
+            const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
+                (uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+            uint32_t first = 0;
+            if (rank == 0u && cand) {
+                first = atomicAdd(&sh.n_fc, (uint32_t)__popcll(mask));
+            }
+            first = (uint32_t)__builtin_amdgcn_readlane((int)first, __builtin_ctzll(mask));
+            if (cand && first + rank < FC_CAP) {
+                L.fc[first + rank] = composite_of(x / a.temperature, id);
+            }
+        }
+    }
 }
 
 template <int DT, bool LSE, bool MASKS>
@@ -121,7 +499,6 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
     constexpr int U = STREAM_UNROLL;
     constexpr uint32_t BLOCK = NT * U;
     constexpr uint32_t QSEG = Q_CAP / NWAVE;
-    constexpr uint32_t SSEG = S_CAP / NWAVE;
     constexpr uint32_t NONE = 0xffffffffu;
     constexpr uint32_t EMASK = (1u << E) - 1u;
     constexpr uint32_t WPP = 64u * E / 32u;   // bitmap words that hold the bits of a wave's 64 chunks
@@ -211,17 +588,8 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
     //     only, and the expansion looks their bits up itself;
     //   * with bits (mode 1): every block's bits arrive beside its values - masked rows, rows
     //     whose listed ids may rise, rows with a row sum and listed ids.  A chunk above the sum's
-    //     cut is summed as it arrives and the listed ids among its elements corrected on the spot;
-    //   * noting (mode 2), for rows with a row sum whose listed ids can only be lowered (no
-    //     mask, no bias list): scanned without bits.  A chunk above the cut is summed as it is
-    //     and its number noted in a list (16 bits an entry, a segment per wave); after the scan
-    //     one thread per entry looks the chunk's bits up and, for the few chunks that hold a
-    //     listed id, takes the raw term off and adds the true one.  Rows with a dominant value
-    //     note a few dozen chunks, or a few hundred before that value has been seen.  A flat row
-    //     fills its list within a few blocks: the refresh of the bound that finds a segment
-    //     three quarters full hands the blocks after the current one to mode 1 (chunks that a
-    //     full segment cannot note are corrected on the spot from bits fetched there and then).
-    const bool noting = pen && lowering && want_lse && !masked && n_bias == 0u;
+    //     cut is summed as it arrives and the listed ids among its elements corrected on the spot.
+    // (Rows under penalties that only lower, without a mask or a bias list, are select_lowering()'s.)
     const bool special = masked || (pen && (!lowering || want_lse));
     // The largest count any id of the scratch ever had (kept in the first spare word behind
     // the bitmap) bounds how far penalties can lower a value.
@@ -301,6 +669,8 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
     phase(cfg, 1);
 
     // ---- scan
+    StreamPriority prio;
+    prio.init(nblocks);
     const uint32_t keff = min(k + k / 8u + 2u, 64u * NWAVE);
     const uint32_t kw = (keff + NWAVE - 1) / NWAVE;
     float lane_max = NEG_INF;
@@ -310,15 +680,10 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
     float skip_b = NEG_INF;     // the block's cut: chunks whose maximum is not above it are not summed
     uint32_t wq = 0;            // this wave's queue fill
     bool give_up = false;       // a wave's queue segment overflowed (the same in every thread)
-    bool stop = false;          // mode 2 ends with block `resume` - 1 (the same in every thread)
-    uint32_t resume = 0;
-    float own_max = NEG_INF;    // mode 2: what this wave's own lanes bound the row's largest value by
-    uint32_t sfill = 0;         // this wave's noted chunks
-    uint32_t note_max = 0;      // the fullest segment of noted chunks, as of the last refresh
     WaveLse wl;
     wl.init();
     double acc_t = 0.0, acc_r = 0.0;   // true terms added one by one; raw terms to take off
-    constexpr int UP_UNSET = INT_MIN;
+    constexpr int UP_UNSET = StreamSums::UP_UNSET;
     int up = UP_UNSET;          // this thread's double sums are relative to ref_s + up
     uint32_t parity = 0;
     // One term 2^(v*c2 - ref_s - up) of a double sum.  The exponent is formed in double: a
@@ -374,7 +739,6 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
         if (lane == 0) {
             sh.bound[parity][w] = mine;
             sh.wfill[parity][w] = wq;
-            sh.wnote[parity][w] = sfill;
             if (maxima) {
                 sh.wmax[parity][w] = wm;
             }
@@ -386,10 +750,8 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
         }
         T = fmaxf(T, lower_by_slack(t));
         // A wave's queue segment is full: the row gives up at once (every thread sees it).
-        note_max = 0;
         for (int i = 0; i < NWAVE; ++i) {
             give_up = give_up || sh.wfill[parity][i] > QSEG;
-            note_max = max(note_max, sh.wnote[parity][i]);
         }
         if (maxima) {
             float m = sh.wmax[parity][0];
@@ -421,36 +783,6 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
             }
         }
         parity ^= 1u;
-    };
-
-    // Element j of a chunk: one compare picks the 8-byte half, one 64-bit shift the element.
-    auto elem_of = [&](const u32x4& q, uint32_t j) -> float {
-        const bool upper = (j & (uint32_t)(E / 2)) != 0u;
-        const uint64_t half = upper ? (((uint64_t)q.w << 32) | q.z) : (((uint64_t)q.y << 32) | q.x);
-        if (E == 8) {
-            return lilym_bits_f32((uint32_t)(half >> ((j & 3u) * 16u)) << 16);
-        }
-        return lilym_bits_f32((uint32_t)(half >> ((j & 1u) * 32u)));
-    };
-    // The chunk with the elements of `bits` replaced by -inf.
-    auto without = [&](const u32x4& q, uint32_t bits) -> u32x4 {
-        u32x4 r = q;
-        if (E == 8) {
-            auto fix = [](uint32_t v, uint32_t two) -> uint32_t {
-                const uint32_t m = ((two & 1u) ? 0x0000ffffu : 0u) | ((two & 2u) ? 0xffff0000u : 0u);
-                return (v & ~m) | (0xff80ff80u & m);
-            };
-            r.x = fix(q.x, bits);
-            r.y = fix(q.y, bits >> 2);
-            r.z = fix(q.z, bits >> 4);
-            r.w = fix(q.w, bits >> 6);
-        } else {
-            r.x = (bits & 1u) ? 0xff800000u : q.x;
-            r.y = (bits & 2u) ? 0xff800000u : q.y;
-            r.z = (bits & 4u) ? 0xff800000u : q.z;
-            r.w = (bits & 8u) ? 0xff800000u : q.w;
-        }
-        return r;
     };
 
     // ---- the bits of a block's chunks
@@ -541,7 +873,7 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
             q = u == 1u ? cur[1] : q;
             q = u == 2u ? cur[2] : q;
             q = u == 3u ? cur[3] : q;
-            const float raw = elem_of(q, j);
+            const float raw = chunk_elem<DT>(q, j);
             if (!(raw > NEG_INF)) {
                 continue;  // barred as well, or -inf to begin with: no term, no candidate
             }
@@ -564,24 +896,6 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
         }
     };
 
-    // The exact terms of one chunk of the slice, one by one in double: every element whose value
-    // (the true one for the listed ids of `dm`) lies above `cut`.
-    auto chunk_terms = [&](const u32x4& q, uint32_t c, uint32_t dm, float cut, auto&& add_term) {
-#pragma unroll 1
-        for (uint32_t j = 0; j < (uint32_t)E; ++j) {
-            float x = elem_of(q, j);
-            if (!(x > cut)) {
-                continue;   // (penalties that only lower: a listed id below the cut stays below it)
-            }
-            if ((dm >> j) & 1u) {
-                x = true_value(g.id_of(c, (int)j), x);
-            }
-            if (x > cut) {
-                add_term(x);
-            }
-        }
-    };
-
     // Blocks b + 1 and b + 2 are on their way while block b is worked on (three register
     // buffers that swap roles): one block in flight per wave leaves the memory idle whenever
     // a wave's arithmetic outlasts its load.
@@ -589,32 +903,14 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
     // The scan is compiled twice, for rows whose chunks come with bits and for rows without:
     // left as a test inside the loop, the bits' loads would be loads that may be skipped, and
     // every wait behind them would drain the blocks requested ahead.
-    auto scan = [&](auto with_bits, auto queueing, uint32_t b_first) {
+    auto scan = [&](auto with_bits) {
         constexpr bool SP = decltype(with_bits)::value;
-        constexpr bool QM = LSE && decltype(queueing)::value;   // mode 2
         Bits bits_a = {}, bits_b = {}, bits_c = {};
         auto work = [&](u32x4 (&cur)[U], const Bits& bcur, uint32_t b) {
-            if (give_up || stop || b >= nblocks) {
+            if (give_up || b >= nblocks) {
                 return;
             }
-            // A wave that has further to go asks to be issued first, so that the workgroups that
-            // share a compute unit advance together instead of in the order they arrived (the
-            // arbiter otherwise favours the oldest wave, and the rows dispatched last scan alone at
-            // the end).  Four levels: the quarter of the way the wave has come, rows dispatched
-            // earlier counted as two blocks further on per generation.
-            {
-                const uint32_t gen = min((blockIdx.y * 4u) / max(gridDim.y, 1u), 3u);
-                const uint32_t q = min(((b + 2u * (3u - gen)) * 4u) / (nblocks + 6u), 3u);
-                if (q == 0u) {
-                    __builtin_amdgcn_s_setprio(3);
-                } else if (q == 1u) {
-                    __builtin_amdgcn_s_setprio(2);
-                } else if (q == 2u) {
-                    __builtin_amdgcn_s_setprio(1);
-                } else {
-                    __builtin_amdgcn_s_setprio(0);
-                }
-            }
+            prio.set(b);
             // tb_all: a byte per chunk of the block, bit j = element j is a listed id.
             uint32_t tb_all = 0u, mb[U] = {0u, 0u, 0u, 0u};
             if (SP) {
@@ -635,7 +931,7 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
             if (MASKS && masked) {
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    cur[u] = without(cur[u], mb[u]);
+                    cur[u] = chunk_without<DT>(cur[u], mb[u]);
                 }
             }
             // The block's own maxima enter the bound before the block is filtered.  Chunks below
@@ -688,73 +984,16 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
                 }
             }
             uint32_t fix = 0u;   // a byte per chunk: its listed ids that are evaluated on the spot
-            // Mode 2: a lane whose chunk lies above the cut without being queued notes the chunk's
-            // number; its terms are formed after the scan, against the row's final cut (most of
-            // what a stale cut lets through is dropped there without a single exponential).  A
-            // lane whose wave's segment is full forms its chunk's terms on the spot instead.
-            auto note_chunk = [&](int u, bool wanted) {
-                const uint64_t mask = __ballot(wanted);
-                if (mask != 0ull) {
-                    const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
-                        (uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-                    const uint32_t at = sfill + rank;
-                    if (wanted && at < SSEG) {
-                        L.noted[w * SSEG + at] = (uint16_t)((b * U + (uint32_t)u) * NT + tid);
-                    }
-                    if (sfill + (uint32_t)__popcll(mask) > SSEG) {
-                        if (wanted && at >= SSEG) {
-                            const uint32_t c = g.cb + (b * U + (uint32_t)u) * NT + tid;
-                            if (c >= g.main_lo && c < g.main_hi) {
-                                // Every element's count, asked for whatever the element is worth
-                                // and waited for here, inside the branch: a fixed number of loads
-                                // and no loop around them, so that the waits of the scan's own
-                                // loads keep counting past this branch.
-                                uint32_t cnt[E];
-#pragma unroll
-                                for (int j = 0; j < E; ++j) {
-                                    cnt[j] = gload(a.counts + g.id_of(c, j));
-                                }
-#pragma unroll
-                                for (int j = 0; j < E; ++j) {
-                                    asm volatile("" : "+v"(cnt[j]));
-                                }
-#pragma unroll
-                                for (int j = 0; j < E; ++j) {
-                                    float x = elem_of(cur[u], (uint32_t)j);
-                                    if (cnt[j] > 0u) {
-                                        x = x > 0.0f ? x / a.repetition : x * a.repetition;
-                                        x -= a.presence + a.frequency * (float)cnt[j];
-                                    }
-                                    if (x > skip_b) {
-                                        acc_t += term_d(x);
-                                    }
-                                }
-                            }
-                        }
-                    }
-                    sfill = min(sfill + (uint32_t)__popcll(mask), SSEG);
-                }
-            };
             bool some = false;
             if (LSE && want_lse) {
                 // A term 2^(v*c2) below 2^-21 / vocab of the largest one seen cannot move the row
                 // sum by more than 2^-21 of it, even with every element of the row at that level:
                 // such chunks are left out, by a rule every thread of the block can evaluate.
-                skip_b = fmaxf(row_max, own_max) - lse_cut;
+                skip_b = row_max - lse_cut;
                 wl.skip_below = skip_b;
                 // Rows with a dominant value skip nearly every block as a whole.
                 some = __ballot(block_max > skip_b) != 0ull;
-                if (QM && some) {
-                    // Between two refreshes of the row's maxima the wave's own lanes may have seen
-                    // more than the row knew then: what they saw bounds the row's largest value
-                    // just as well, and spares a row whose largest value comes late the noting of
-                    // chunk after chunk against a cut that is out of date.
-                    own_max = lowered(wave_max_dpp(lane_max));
-                    skip_b = fmaxf(row_max, own_max) - lse_cut;
-                    wl.skip_below = skip_b;
-                    some = __ballot(block_max > skip_b) != 0ull;
-                }
-                if (!QM && some) {
+                if (some) {
                     wl.prepare(block_max < T_prev ? block_max : T_prev, c2);  // nothing above T_prev is added
 #pragma unroll
                     for (int u = 0; u < U; ++u) {
@@ -773,15 +1012,8 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
                     // chunks were held back above for want of a bound) is measured against the
                     // largest value known now.  Terms between the old cut and the new one that
                     // were summed already are as negligible as those that were not.
-                    skip_b = fmaxf(row_max, own_max) - lse_cut;
+                    skip_b = row_max - lse_cut;
                     wl.skip_below = skip_b;
-                    if (QM && some) {
-                        some = __ballot(block_max > skip_b) != 0ull;
-                    }
-                }
-                if (QM && note_max >= SSEG * 3u / 4u) {
-                    stop = true;
-                    resume = b + 1u;   // this block is still finished here
                 }
             }
             if (n_bias != 0u && tid == 0) {
@@ -789,7 +1021,7 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
                 L.blk_cut[b] = skip_b;
                 L.blk_flag[b] = nonneg ? 1u : 0u;
             }
-            const bool any_late = !QM && LSE && want_lse && T != T_prev &&
+            const bool any_late = LSE && want_lse && T != T_prev &&
                                   __ballot(block_max >= T_prev && block_max > skip_b) != 0ull;
             // When values can only be lowered, a listed id in a chunk that was neither queued nor
             // summed is below the bound and below the sum's cut with its true value too: nothing
@@ -819,9 +1051,6 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
                         wl.template add_prepared<DT>(cur[u], m8[u], c2, late);
                     }
                 }
-                if (QM && some) {
-                    note_chunk(u, !pass && m8[u] > skip_b);
-                }
                 if (SP && fix_any) {
                     const uint32_t tb = (tb_all >> (8 * u)) & 0xffu;
                     const bool matters = !lowering || (LSE && want_lse && m8[u] > skip_b);
@@ -845,15 +1074,12 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
         };
         if (nblocks == 0) {
             refresh_bound(true, true);  // the same barriers in every workgroup
-        } else if (b_first < nblocks) {
-            if (b_first != 0u) {
-                fetch(buf_a, b_first);   // (block 0 was requested at the very start)
-            }
+        } else {
             if (SP) {
-                bits_request(bits_a, b_first);
+                bits_request(bits_a, 0u);
             }
-            request(buf_b, bits_b, b_first + 1u);
-            for (uint32_t b = b_first; b < nblocks && !give_up && !stop; b += 3) {
+            request(buf_b, bits_b, 1u);
+            for (uint32_t b = 0; b < nblocks && !give_up; b += 3) {
                 request(buf_c, bits_c, b + 2);
                 work(buf_a, bits_a, b);
                 if (b + 1 < nblocks) {
@@ -867,53 +1093,19 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
             }
         }
     };
-    if (noting) {
-        scan(std::false_type{}, std::true_type{}, 0u);
-        if (stop && !give_up) {
-            stop = false;
-            scan(std::true_type{}, std::false_type{}, resume);
-        }
-    } else if (special) {
-        scan(std::true_type{}, std::false_type{}, 0u);
+    if (special) {
+        scan(std::true_type{});
     } else {
-        scan(std::false_type{}, std::false_type{}, 0u);
+        scan(std::false_type{});
     }
     phase(cfg, 2);
 
     // ---- after the scan
-    const float wave_top = (LSE && noting) ? wave_max_dpp(lane_max) : 0.0f;
     if (lane == 0) {
         sh.qfill[w] = wq;
-        sh.nfill[w] = sfill;
-        sh.wmax[parity][w] = wave_top;
     }
     __syncthreads();
     phase(cfg, 14);
-    // Mode 2 forms its terms after the scan, when the row's largest streamed value is known:
-    // they are relative to that value's exponent (none of them exceeds 1: penalties only lower)
-    // and add up in `acc_p`.
-    double ref_p = 0.0, acc_p = 0.0;
-    bool simple_p = false;   // the same in every thread
-    if (LSE && noting) {
-        // The row's cut as the whole scan leaves it: what follows forms no term below it.
-        float m = sh.wmax[parity][0];
-        for (int i = 1; i < NWAVE; ++i) {
-            m = fmaxf(m, sh.wmax[parity][i]);
-        }
-        const float true_low = fmaxf(lowered(m), row_floor);   // the largest true value is not below this
-        skip_b = fmaxf(skip_b, true_low - lse_cut);
-        // One reference serves when every term above the cut is a double relative to it: the
-        // largest raw value may lie far above what the penalties leave of it, and a temperature
-        // near 0 stretches that distance beyond a double's range (such rows keep the references
-        // that move, term_d).
-        simple_p = m > NEG_INF && (m - true_low) * c2 <= 900.0f;
-        ref_p = simple_p ? (double)m * c2d : 0.0;
-        ref_p = ref_p < 1.0e30 ? (ref_p > -1.0e30 ? ref_p : -1.0e30) : 1.0e30;
-    }
-    auto term_p = [&](float v) -> double {
-        const double d = __builtin_fma((double)v, c2d, -ref_p);
-        return d > -1000.0 ? pow2_d(d < 1000.0 ? d : 1000.0) : 0.0;   // (-inf and NaN: nothing)
-    };
     const float filt = T;
     {
         bool overflow = give_up;
@@ -944,187 +1136,28 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
         return (c - g.cb) / BLOCK;
     };
     {
-        uint32_t seg_end[NWAVE], total = 0;
-#pragma unroll
-        for (int i = 0; i < NWAVE; ++i) {
-            total += sh.qfill[i];
-            seg_end[i] = total;
-        }
-        auto queue_slot = [&](uint32_t ch) -> uint32_t {
-            uint32_t ww = 0, before = 0;
-#pragma unroll
-            for (int i = 0; i + 1 < NWAVE; ++i) {
-                if (ch >= seg_end[i]) {
-                    ww = (uint32_t)i + 1u;
-                    before = seg_end[i];
-                }
-            }
-            return ww * QSEG + (ch - before);
-        };
-        // Mode 2's noted chunks: their 16 bytes and their bits of the scratch's bitmap are asked
-        // for first, four chunks a thread, and looked at behind the queue's listing below, which
-        // touches LDS only.
-        uint32_t n_seg_end[NWAVE], n_total = 0;
-#pragma unroll
-        for (int i = 0; i < NWAVE; ++i) {
-            n_total += (LSE && noting) ? sh.nfill[i] : 0u;
-            n_seg_end[i] = n_total;
-        }
-        auto noted_at = [&](uint32_t e) -> uint32_t {
-            uint32_t ww = 0, before = 0;
-#pragma unroll
-            for (int i = 0; i + 1 < NWAVE; ++i) {
-                if (e >= n_seg_end[i]) {
-                    ww = (uint32_t)i + 1u;
-                    before = n_seg_end[i];
-                }
-            }
-            return (uint32_t)L.noted[ww * SSEG + (e - before)];
-        };
-        uint32_t n_cc[4] = {0u, 0u, 0u, 0u}, n_dm[4] = {0u, 0u, 0u, 0u};
-        u32x4 n_q[4] = {};
-        bool n_ok[4] = {false, false, false, false};
-        auto noted_request = [&](uint32_t e0) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t e = e0 + (uint32_t)i * NT;
-                const uint32_t c = g.cb + noted_at(min(e, n_total - 1u));
-                // (A chunk outside the slice was scanned as -inf throughout, and is noted where
-                // chunk maxima are the kind that reports +0 for it.)
-                n_ok[i] = e < n_total && c >= g.main_lo && c < g.main_hi;
-                n_cc[i] = min(c, c_last);
-                n_q[i] = gload(reinterpret_cast<const u32x4*>(g.base + (n_cc[i] << 4)));
-                n_dm[i] = bits32_at(a.touched, row_words, (int64_t)g.id_of(n_cc[i], 0)) & EMASK;
-            }
-        };
-        // A chunk whose largest value lies above the final cut adds its terms (listed ids with
-        // their true values); the others - all that a cut which was out of date while the row's
-        // largest values had yet to come let through - are dropped.
-        auto noted_consume = [&]() {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (n_ok[i] && chunk_max<DT>(n_q[i]) > skip_b) {
-                    chunk_terms(n_q[i], n_cc[i], n_dm[i], skip_b, [&](float x) {
-                        if (simple_p) {
-                            acc_p += term_p(x);
-                        } else {
-                            acc_t += term_d(x);
-                        }
-                    });
-                }
-            }
-        };
-        if (n_total != 0u) {
-            noted_request(tid);
-        }
-        // Rows under penalties that only lower (the common kind): every element of a queued chunk
-        // that matters by its raw value - at or above the bound, or above the sum's cut - is
-        // listed as an (id, raw value) pair, wave by wave; then one thread per pair gathers the
-        // id's count, so that all of the row's gathers are one round trip to memory.  (A listed
-        // id's true value is not above its raw one: what does not matter raw does not matter.)
-        uint64_t* pairs = L.fc;   // the candidates' place: they arrive once the pairs are in registers
-        const bool pair_path = pen && lowering;
-        if (pair_path) {
-            for (uint32_t ch0 = 0; ch0 < total; ch0 += NT) {
-                const uint32_t ch = ch0 + tid;
-                uint32_t todo = 0, c = 0;
-                u32x4 q = {};
-                if (ch < total) {
-                    const uint32_t slot = queue_slot(ch);
-                    q = L.qraw[slot];
-                    c = L.qidx[slot];
-                    float v[E];
-                    unpack<DT>(q, v);
-#pragma unroll
-                    for (int j = 0; j < E; ++j) {
-                        const bool term = want_lse && v[j] > skip_b;
-                        const bool cand = v[j] >= filt && v[j] > NEG_INF;
-                        todo |= (term || cand) ? 1u << j : 0u;
-                    }
-                }
-                while (__ballot(todo != 0u) != 0ull) {
-                    const bool has = todo != 0u;
-                    const uint32_t j = has ? (uint32_t)__builtin_ctz(todo) : 0u;
-                    todo &= todo - 1u;   // (0 stays 0)
-                    const uint32_t id = g.id_of(c, (int)j);
-                    const bool push = has && !(n_bias != 0u && biased(id));
-                    const uint64_t mask = __ballot(push);
-                    if (mask != 0ull) {
-                        const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
-                            (uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-                        uint32_t first = 0;
-                        if (rank == 0u && push) {
-                            first = atomicAdd(&sh.n_pairs, (uint32_t)__popcll(mask));
-                        }
-                        first = (uint32_t)__builtin_amdgcn_readlane((int)first, __builtin_ctzll(mask));
-                        if (push && first + rank < FC_CAP) {
-                            pairs[first + rank] = ((uint64_t)lilym_f32_bits(elem_of(q, j)) << 32) | id;
-                        }
-                    }
-                }
-            }
-        }
-        if (n_total != 0u) {
-            noted_consume();
-            for (uint32_t e0 = tid + 4u * NT; e0 < n_total + tid; e0 += 4u * NT) {   // (the same trips in every thread)
-                noted_request(e0);
-                noted_consume();
-            }
-        }
+        QueueOrder order;
+        order.init(sh.qfill);
+        const uint32_t total = order.total;
         bool paired = false;
-        if (pair_path) {
+        if (pen && lowering) {
+            stream_pairs_list<DT>(L, g, order, filt, want_lse ? skip_b : __builtin_huge_valf(), sh, [](uint32_t) { return true; },
+                                  [&](uint32_t id) { return n_bias != 0u && biased(id); });
             __syncthreads();
             paired = sh.n_pairs <= FC_CAP;
-        }
-        if (paired) {
-            const uint32_t n_pairs = sh.n_pairs;
-            uint64_t pr[4];
-            uint32_t cnt[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t at = tid + (uint32_t)i * NT;
-                pr[i] = at < n_pairs ? pairs[at] : 0ull;
-                cnt[i] = gload(a.counts + (uint32_t)pr[i]);   // (id 0 for an empty place)
-            }
-            __syncthreads();   // every pair is in a register: the candidates may take their place
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const bool valid = tid + (uint32_t)i * NT < n_pairs;
-                const uint32_t id = (uint32_t)pr[i];
-                float x = lilym_bits_f32((uint32_t)(pr[i] >> 32));
-                if (cnt[i] > 0u) {
-                    x = x > 0.0f ? x / a.repetition : x * a.repetition;
-                    x -= a.presence + a.frequency * (float)cnt[i];
-                }
-                if (valid && want_lse && x > skip_b) {
-                    if (simple_p) {
-                        acc_p += term_p(x);
-                    } else {
+            if (paired) {
+                stream_pairs_take(L, a, filt, sh, [&](float x) {
+                    if (want_lse && x > skip_b) {
                         acc_t += term_d(x);
                     }
-                }
-                const bool cand = valid && x >= filt && x > NEG_INF;
-                const uint64_t mask = __ballot(cand);
-                if (mask != 0ull) {
-                    const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
-                        (uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-                    uint32_t first = 0;
-                    if (rank == 0u && cand) {
-                        first = atomicAdd(&sh.n_fc, (uint32_t)__popcll(mask));
-                    }
-                    first = (uint32_t)__builtin_amdgcn_readlane((int)first, __builtin_ctzll(mask));
-                    if (cand && first + rank < FC_CAP) {
-                        L.fc[first + rank] = composite_of(x / a.temperature, id);
-                    }
-                }
+                });
             }
         }
-        // Every other row (and a row whose pairs outgrew their place): one thread per queued
-        // chunk (the waves' segments counted through in order): its elements add their term and
+        // Every other row (and a row whose pairs outgrew their place): one thread per queued chunk (the waves' segments counted through in order): its elements add their term and
         // are offered - listed ones with their true value, ids of the bias list not at all (the
         // pass below speaks for them).
         for (uint32_t ch = tid; !paired && ch < total; ch += NT) {
-            const uint32_t slot = queue_slot(ch);
+            const uint32_t slot = order.template slot<QSEG>(ch);
             const u32x4 q = L.qraw[slot];
             const uint32_t c = L.qidx[slot];
             // Its listed elements, from the scratch's bitmap (barred ids are -inf already).
@@ -1148,7 +1181,7 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
             while (todo != 0u) {
                 const uint32_t j = (uint32_t)__builtin_ctz(todo);
                 todo &= todo - 1u;
-                float x = elem_of(q, j);
+                float x = chunk_elem<DT>(q, j);
                 const uint32_t id = g.id_of(c, (int)j);
                 if (n_bias != 0u && biased(id)) {
                     continue;
@@ -1183,7 +1216,7 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
             const uint32_t c = (id + g.pad) / E;
             u32x4 q = gload(reinterpret_cast<const u32x4*>(g.base + (c << 4)));
             if (masked) {
-                q = without(q, ~bits32_at(a.allow, row_words, (int64_t)g.id_of(c, 0)) & EMASK);
+                q = chunk_without<DT>(q, ~bits32_at(a.allow, row_words, (int64_t)g.id_of(c, 0)) & EMASK);
             }
             float cm = L.blk_flag[b] != 0u ? chunk_max_nonneg<DT>(q) : chunk_max<DT>(q);
             if (lilym_f32_bits(cm) > 0x7f800000u && !(cm < 0.0f)) {
@@ -1197,7 +1230,7 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
                 queued = queued || (bits32_at(a.touched, row_words, (int64_t)g.id_of(c, 0)) & EMASK) != 0u;
             }
             const bool summed = !queued && cm > cut;
-            const float raw = elem_of(q, (id + g.pad) % E);
+            const float raw = chunk_elem<DT>(q, (id + g.pad) % E);
             const float t = true_value(id, raw);
             if (want_lse) {
                 if (summed) {
@@ -1224,171 +1257,18 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
     }
     phase(cfg, 9);
     if (want_lse) {
-        // Mode 2 as a rule holds nothing but its post-scan terms, all relative to one reference:
-        // the waves' sums meet in LDS behind one barrier.  A thread with a sum of another kind
-        // (terms formed during the scan, edge ids, a scan that went on with bits beside the
-        // chunks) sends the row the long way below.
-        const bool other_sums = up != UP_UNSET || !(wl.s == 0.0f) || !(wl.booked == 0.0f);
-        const double p_wave = wave_sum_d_dpp(acc_p);
-        if (lane == 0) {
-            sh.red_d[w] = p_wave;
-        }
-        const bool long_way = __syncthreads_or((!simple_p || other_sums) ? 1 : 0) != 0;
-        double p_all = 0.0;
-        for (int i = 0; i < NWAVE; ++i) {
-            p_all += sh.red_d[i];
-        }
-        if (!long_way) {
-            phase(cfg, 10);
-            if (tid == 0) {
-                sh.lse_mc = ref_p;
-                sh.lse_s = p_all;
-            }
-        } else {
-            // Each wave brings its sums to one reference of its own: the highest of its threads'
-            // references and of the streamed sums' (wave-uniform) reference.  The waves' partial
-            // sums and references meet in LDS and are brought together after one barrier.
-            int ref_w = up;
-            for (int o = 32; o > 0; o >>= 1) {
-                ref_w = max(ref_w, __shfl_xor(ref_w, o));
-            }
-            const double stream_at = (double)wl.ref - (double)ref_s;  // exact
-            if (__ballot(wl.s > 0.0f) != 0ull) {
-                const double e = stream_at < 1.0e9 ? (stream_at > -1.0e9 ? stream_at : -1.0e9) : 1.0e9;
-                ref_w = max(ref_w, (int)__builtin_floor(e));
-            }
-            const int down = up == UP_UNSET ? 0 : up - ref_w;  // <= 0
-            double part[4];
-            {
-                double d = stream_at - (double)ref_w;  // <= 1 where there is a sum
-                d = d < -1000.0 ? -1000.0 : d;
-                const double scale = pow2_d(d);
-                part[0] = wl.s > 0.0f ? (double)wl.s * scale : 0.0;
-                part[3] = wl.booked > 0.0f ? (double)wl.booked * scale : 0.0;
-            }
-            part[1] = __builtin_ldexp(acc_r, down);
-            part[2] = __builtin_ldexp(acc_t, down);
-    #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                part[i] = wave_sum_d(part[i]);
-                if (lane == 0) {
-                    sh.red3[i][w] = part[i];
-                }
-            }
-            if (lane == 0) {
-                sh.red_i[w] = (uint32_t)ref_w;
-            }
-            // A NaN logit in a summed chunk leaves its wave's running sum a NaN: such a logit is
-            // worth -inf, and the row's sum is formed again from every value.
-            const bool poisoned = __syncthreads_or(wl.s != wl.s ? 1 : 0) != 0;
-            int ref_all = (int)sh.red_i[0];
-            for (int i = 1; i < NWAVE; ++i) {
-                ref_all = max(ref_all, (int)sh.red_i[i]);
-            }
-    #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                part[i] = 0.0;
-                for (int ww = 0; ww < NWAVE; ++ww) {
-                    const int at = (int)sh.red_i[ww];
-                    part[i] += at == UP_UNSET ? 0.0 : __builtin_ldexp(sh.red3[i][ww], at - ref_all);
-                }
-            }
-            if (ref_all == UP_UNSET) {
-                ref_all = 0;  // no term anywhere: the sums are zero
-            }
-            // part[0]: the running sums, the listed ids' raw terms of part[3] already taken off (and
-            // their true terms added); part[1]: raw terms still to take off; part[2]: terms added
-            // one by one.
-            const double streamed = part[0], booked = part[1], exact = part[2], taken = part[3];
-            const double rest = streamed - booked;
-            // The streamed sums are f32: taking the listed ids' raw terms off again leaves an error of
-            // about 1e-6 of what was streamed.  Where that is more than 20 times the row's sum (listed
-            // ids held nearly everything that was streamed, and nothing larger was added exactly) the
-            // difference is too coarse.
-            const bool coarse = poisoned ||
-                                (booked + taken > 0.0 &&
-                                 !((rest > 0.0 ? rest : 0.0) + exact > 0.05 * (streamed + taken)));
-            phase(cfg, 10);
-            if (coarse) {
-                phase(cfg, 11);
-                LseAcc all;
-                all.init();
-                exact_terms<DT>(a, g.id_lo, g.id_hi, c2, all);
-                double m_e, s_e;
-                wg_merge_lse(sh, all.mc, all.s, m_e, s_e);
-                if (tid == 0) {
-                    sh.lse_mc = m_e;
-                    sh.lse_s = s_e;
-                }
-            } else if (tid == 0) {
-                double mc = (double)ref_s + (double)ref_all;
-                double sum = (rest > 0.0 ? rest : 0.0) + exact;
-                if (p_all > 0.0) {
-                    // Mode 2's post-scan terms have a reference of their own: the higher of the
-                    // two serves both (what lies 2^1000 below the other adds nothing).
-                    if (!(sum > 0.0)) {
-                        mc = ref_p;
-                        sum = p_all;
-                    } else {
-                        const double top = mc > ref_p ? mc : ref_p;
-                        const double d0 = mc - top, d1 = ref_p - top;
-                        sum = sum * pow2_d(d0 < -1000.0 ? -1000.0 : d0) +
-                              p_all * pow2_d(d1 < -1000.0 ? -1000.0 : d1);
-                        mc = top;
-                    }
-                }
-                sh.lse_mc = mc;
-                sh.lse_s = sum;
-            }
-    
-        }
+        StreamSums sums;
+        sums.ref_s = ref_s;
+        sums.up = up;
+        sums.acc_t = acc_t;
+        sums.acc_r = acc_r;
+        sums.ref_p = 0.0;
+        sums.acc_p = 0.0;
+        sums.simple_p = false;
+        stream_row_sum<DT>(a, g, sums, wl, sh, cfg);
     }
     __syncthreads();
-    uint32_t n = sh.n_fc;
-    phase(cfg, 3);
-    if (n > FC_CAP) {
-        return stream_fail(cfg, 5u);
-    }
-    sorted = false;
-    n = select_topk(L.fc, n, k, sh, sorted);
-    phase(cfg, 12);
-    // Everything that is not a candidate lies strictly below `filt`: the result is exact if
-    // k candidates were found and the k-th lies strictly above anything the division can
-    // map such a value to.
-    if (filt > F32_LOWEST) {
-        uint32_t lowest = 0xffffffffu;
-        if (sorted) {
-            // Ranked candidates are in descending order: the last one is the lowest.
-            lowest = n > 0u ? (uint32_t)(L.fc[n - 1u] >> 32) : lowest;
-        } else {
-            for (uint32_t i = tid; i < n; i += NT) {
-                lowest = min(lowest, (uint32_t)(L.fc[i] >> 32));
-            }
-            lowest = wave_min_u32(lowest);
-            if (lane == 0) {
-                sh.red_i[w] = lowest;
-            }
-            __syncthreads();
-            lowest = sh.red_i[0];
-            for (int i = 1; i < NWAVE; ++i) {
-                lowest = min(lowest, sh.red_i[i]);
-            }
-            __syncthreads();
-        }
-        const float below = lilym_key_value(lilym_order_key(filt) - 1u) / a.temperature;
-        if (!(n >= k && lilym_order_key(below) < lowest)) {
-            return stream_fail(cfg, 6u);
-        }
-    }
-    // The candidates stay where they are (the tail's arrays and the merge's buffer lie below
-    // them in dynamic LDS).
-    out = L.fc;
-    if (tid == 0) {
-        sh.n_cand = n;
-    }
-    __syncthreads();
-    return true;
+    return stream_accept(L, filt, a.temperature, k, sh, cfg, sorted, out);
 }
-
 
 }  // namespace lily

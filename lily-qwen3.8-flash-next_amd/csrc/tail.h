@@ -181,7 +181,7 @@ __device__ __forceinline__ void sort_desc(uint64_t* cand, uint32_t n) {
 
 // ------------------------------------------------------------------ tail
 
-// Counts one emission of `id` in a scratch: the dense count, the id's bit in the bitmap of the
+// Counts one emission of `id` in a scratch: the dense count, the id's bits in the maps of the
 // ids that were ever counted, the largest count any id has reached (the first spare word behind
 // the bitmap: never lowered, so an upper bound after un-counting) and an id that reached it (the
 // second spare word).  That id is a hint only - writers race, un-counting leaves it alone - and
@@ -193,7 +193,7 @@ __device__ __forceinline__ uint32_t count_token(const RowArgs& a, uint32_t id, u
     const uint32_t words = (vocab + 31u) / 32u;
     const uint32_t top = gload(&a.touched[words]);
     const uint32_t before = atomicAdd(&a.counts[id], 1u);
-    atomicOr(&a.touched[id >> 5], 1u << (id & 31u));
+    mark_listed(a.touched, words, id);
     if (top <= before + 1u) {
         atomicMax(&a.touched[words], before + 1u);
         a.touched[words + 1u] = id;
@@ -205,9 +205,9 @@ __device__ __forceinline__ uint32_t count_token(const RowArgs& a, uint32_t id, u
 // has now (null otherwise: nobody then waits for the increment to come back).
 // The increments alone, nothing waited for: for rows that draw in order within one launch, whose
 // workgroup knows the counts itself and brings the largest count up to date once at the end.
-__device__ __forceinline__ void count_token_blind(const RowArgs& a, uint32_t id) {
+__device__ __forceinline__ void count_token_blind(const RowArgs& a, uint32_t id, uint32_t vocab) {
     atomicAdd(&a.counts[id], 1u);
-    atomicOr(&a.touched[id >> 5], 1u << (id & 31u));
+    mark_listed(a.touched, (vocab + 31u) / 32u, id);
 }
 
 // `sh`: where a launch whose rows draw in order learns what this row drew (null otherwise).
@@ -215,7 +215,7 @@ __device__ __forceinline__ void emit(const RowArgs& a, uint32_t id, uint32_t voc
     *a.out_id = id;
     if ((a.flags & F_PEN) && id < vocab) {
         if (sh != nullptr) {
-            count_token_blind(a, id);
+            count_token_blind(a, id, vocab);
         } else {
             count_token(a, id, vocab);
         }
@@ -265,14 +265,14 @@ __device__ __forceinline__ void finish_token(const RowArgs& a, Shared& sh, uint3
         // Rows that draw in order: the next row learns the id; nobody waits for the increments.
         sh.emitted_id = id;
         if (pen) {
-            count_token_blind(a, id);
+            count_token_blind(a, id, vocab);
         }
     } else if (pen) {
         // (count_token(), taken apart so that nothing between here and the logarithm below
         // waits for memory)
         top = gload(&a.touched[words]);
         before = atomicAdd(&a.counts[id], 1u);
-        atomicOr(&a.touched[id >> 5], 1u << (id & 31u));
+        mark_listed(a.touched, words, id);
     }
     const double base = want ? sh.lse_mc + log2(sh.lse_s) : 0.0;
     if (pen && !in_order && top <= before + 1u) {

@@ -1,0 +1,89 @@
+"""Rows under penalties that only lower (csrc/select_lowering.h) against the oracle, where that
+select changes its form: rows whose leading ids were all drawn before (none of them may enter the
+bound), flat and peaked rows with a row sum, more listed ids above the bound than the queue holds
+(the slice is taken again), more chunks of listed ids than the notes hold (the bitmap is walked),
+rows that start inside a group of eight ids, and the map of listed ids however it was written.
+"""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+import lily_sampler as LS
+import lily_workloads as W
+import oracle as O
+from gpu_util import check_row_against_oracle, dev, o_params, run_rows
+from test_gpu_stream import make_sampler
+
+
+@pytest.fixture(scope="module", params=[1, 3], ids=lambda s: f"slices{s}")
+def sampler(request):
+    s = make_sampler(request.param)
+    yield s
+    s.close()
+
+
+def _logits(rng, rows, vocab, flat, bf16):
+    x = rng.normal(0.0, 2.0, (rows, vocab))
+    if not flat:
+        heavy = rng.random((rows, vocab)) < 0.1
+        x = np.where(heavy, rng.standard_t(3.0, (rows, vocab)) * 4.0, x)
+    x = x.astype(np.float32)
+    return W.to_bf16_bits(x) if bf16 else x
+
+
+def _scratch(sampler, rng, vocab, ids, how):
+    """A scratch that counted `ids` 1 to 6 times each, the first 40 of them many times."""
+    counts = np.zeros(vocab, dtype=np.uint32)
+    counts[ids] = rng.integers(1, 7, len(ids))
+    counts[ids[:40]] += rng.integers(0, 120, len(ids[:40])).astype(np.uint32)
+    sc = LS.SamplerScratch(sampler, vocab)
+    if how == "history":
+        hist = rng.permutation(np.repeat(np.arange(vocab), counts)).astype(np.int32)
+        sc.add_history(torch.from_numpy(hist).to(dev()))
+        return sc, counts
+    sc.write_counts(torch.from_numpy(counts.view(np.int32)))
+    if how == "copy":
+        other = LS.SamplerScratch(sampler, vocab)
+        other.add_history(torch.arange(min(vocab, 500), dtype=torch.int32, device=dev()))
+        other.copy_counts_from(sc)
+        return other, counts
+    return sc, counts
+
+
+# 8 192 bf16 / 4 096 f32 ids are a block; an odd vocabulary starts its rows anywhere in eight ids.
+@pytest.mark.parametrize("vocab", [997, 8192, 16_384 + 1, 40_005, 151_936])
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("flat", [False, True])
+def test_rows_whose_leading_ids_were_drawn_before(sampler, vocab, bf16, flat):
+    rng = np.random.default_rng(vocab * 4 + 2 * bf16 + flat)
+    cases = [(0, "history"), (40, "history"), (700, "write"), (3000, "copy"), (20_000, "write")]
+    rows = len(cases)
+    x = _logits(rng, rows, vocab, flat, bf16)
+    xf = W.bf16_bits_to_f32(x) if bf16 else x
+    scratch, counts = [], []
+    for r, (n, how) in enumerate(cases):
+        leading = np.argsort(-xf[r], kind="stable")[:min(n, vocab - 1)]
+        sc, c = _scratch(sampler, rng, vocab, leading, how)
+        scratch.append(sc)
+        counts.append(c)
+    kw = [dict(temperature=[0.7, 1.0, 0.4][r % 3], top_k=[50, 64, 3][r % 3], top_p=0.95, min_p=0.01, repetition_penalty=1.1,
+               presence_penalty=0.3, frequency_penalty=[0.2, 0.02][r % 2], seed=70 + r) for r in range(rows)]
+    stats = torch.zeros(4, dtype=torch.int32, device=dev())
+    for logprobs in (False, True):
+        sampler.set_path_stats(stats)
+        for step in range(2):
+            r = run_rows(sampler, x, kw, [step] * rows, scratch=scratch, logprobs=logprobs)
+            for i in range(rows):
+                d = O.sample(xf[i], counts[i], o_params(**kw[i]), step, want_logprob=True)
+                check_row_against_oracle(r, i, d)
+                if logprobs:
+                    assert abs(r.logprobs[i] - d.logprob) <= 1e-5 * max(1.0, abs(d.logprob)), (i, r.logprobs[i], d.logprob)
+        sampler.set_path_stats(None)
+    # Every slice by the streaming selects (the smallest row aside: its slices hold few more ids than k).
+    if vocab > 997:
+        assert stats[2].item() == 0, stats.tolist()
+    for i in range(rows):
+        assert np.array_equal(scratch[i].read_counts().numpy().view(np.uint32), counts[i])
+        scratch[i].close()
