@@ -824,6 +824,29 @@ def test_heads_of_affine_codes(sampler, bits, group, rows):
     _check_draws(logits.cpu().numpy(), ids, lps, cand, counts, params_kw, steps)
 
 
+@pytest.mark.parametrize("rows,d,vocab,bits,group", [
+    (17, 512, 700, 4, 64), (32, 128, 64, 8, 64), (33, 1024, 129, 8, 128), (64, 256, 1000, 4, 64),
+    (65, 512, 333, 8, 64), (128, 768, 257, 4, 128), (129, 1536, 1160, 4, 64)])
+def test_tiles_of_codes_at_their_edges(sampler, rows, d, vocab, bits, group):
+    """More than 16 rows over codes, either side of each tile's rows (32, 64, 128), one stage of
+    codes, an odd and an even number of them, groups a row that are and are not a multiple of
+    eight (the scales' wide loads), a last tile of one column: the logits and summaries against
+    the f64 product with the weights as dequant_q4/q8_bf16 give them."""
+    rng = np.random.default_rng(rows + d + bits)
+    hidden = rng.normal(0, 1, (rows, d)).astype(np.float32)
+    qw, dense, _, _ = _quantised(rng, vocab, d, bits, group)
+    h = _bf16(hidden)
+    temps = [0.5 + 0.1 * (r % 7) for r in range(rows)]
+    buf = torch.full((rows, vocab + 4), 7.0, dtype=torch.float32, device=dev())
+    tiles = (vocab + TILE - 1) // TILE
+    tmax = torch.zeros(rows, tiles, dtype=torch.float32, device=dev())
+    tsum = torch.zeros(rows, tiles, dtype=torch.float32, device=dev())
+    sampler.lm_head(h, qw, temps, buf[:, :vocab], tmax, tsum)
+    sampler.synchronize()
+    _check_f32_product(h, dense, buf[:, :vocab], tmax, tsum, temps)
+    assert torch.all(buf[:, vocab:] == 7.0)
+
+
 @pytest.mark.parametrize("form", ["own", "library"])
 @pytest.mark.parametrize("rows,d,vocab,slack", [(130, 512, 4096 + 77, 8), (300, 128, 2000 + 3, 3),
                                                 (1024, 256, 3000, 8), (5, 64, 700, 8)])
