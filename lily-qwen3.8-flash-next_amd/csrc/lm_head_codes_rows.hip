@@ -47,7 +47,13 @@ inline uint32_t rows_lds_bytes(int mi, uint32_t groups) {
 // Before it, tiles that brought 4 or 8 bytes of codes and two 2-byte scales a thread and load (the
 // requests, not the bytes, were their bound) and turned each code into LDS.  V = 151 936, f32
 // logits, before and now: d = 4096, 8 bits, 20 rows 256 -> 152 us, 50 rows 428 -> 185, 100 rows
-// 502 -> 262, 200 rows 795 -> 476; 4 bits 357 -> 130, 258 -> 168, 439 -> 242, 723 -> 447.
+// 502 -> 260, 200 rows 795 -> 468; 4 bits 357 -> 124, 258 -> 166, 439 -> 244, 723 -> 435.
+// What bounds it now is the vector unit (4 bits, 20 rows: 71 % of the cycles; without turning codes into
+// weights the launch takes 91 us of the 124, without its products all of them): 23 instructions
+// for eight 4-bit codes.  Tried and no faster: the conversion of two 8-bit floats an instruction
+// in place of four byte conversions (124 -> 122), codes as the denormal halves of a mixed-precision
+// FMA (124 -> 118, none for 8 bits, and it overflows for scales from 2^104 on), codes read out of
+// LDS a step ahead (none).
 template <int WBITS, int MI>
 __global__ void __launch_bounds__(256, MI == 4 ? 2 : 3)
 k_lm_head_codes_rows(const uint16_t* __restrict__ hidden, uint64_t hidden_stride, const uint32_t* __restrict__ codes,
@@ -81,12 +87,13 @@ k_lm_head_codes_rows(const uint16_t* __restrict__ hidden, uint64_t hidden_stride
     uint32_t* sz = reinterpret_cast<uint32_t*>(lds + 2u * HIDDEN_BYTES + CODE_BYTES);
 
     // ---- codes: load i of a wave is the lines of its columns 8 * i ... + 7, lane l the 16 bytes that
-    // belong at l * 16: piece (l % 8) ^ (l / 8) of column 8 * i + l / 8 (pieces change places by
-    // the column's number, so that eight columns' pieces are read out of all banks)
+    // belong at l * 16: of column 8 * i + l / 8 the piece (l % 8) ^ (column / 2) % 8 (pieces change
+    // places by the column's number: two lines fill the banks, so the 16 columns whose pieces are
+    // read at once hit 16 different groups of them)
     const char* from_c[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const uint32_t col = n0 + 32u * wave + 8u * (uint32_t)i + (lane >> 3), q = (lane & 7u) ^ (lane >> 3);
+        const uint32_t col = n0 + 32u * wave + 8u * (uint32_t)i + (lane >> 3), q = (lane & 7u) ^ ((4u * (uint32_t)i + (lane >> 4)) & 7u);
         from_c[i] = reinterpret_cast<const char*>(codes) + (uint64_t)min(col, vocab - 1u) * weight_stride * 4u + q * 16u;
     }
     auto fetch_codes = [&](w32x4 (&r)[4], uint32_t stage_no) {
@@ -97,9 +104,9 @@ k_lm_head_codes_rows(const uint16_t* __restrict__ hidden, uint64_t hidden_stride
         }
     };
     // ---- hidden values: piece i of thread t is 16 bytes (t % 8) of row 32 * i + t / 8, at the place
-    // (t % 8) ^ (row % 8) of the row's 128 bytes
+    // (t % 8) ^ (row / 2) % 8 of the row's 128 bytes
     const char* from_h[MI];
-    const uint32_t hidden_at = (tid >> 3) * 128u + ((tid & 7u) ^ ((tid >> 3) & 7u)) * 16u;
+    const uint32_t hidden_at = (tid >> 3) * 128u + ((tid & 7u) ^ ((tid >> 4) & 7u)) * 16u;
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
         const uint32_t r = m0 + 32u * (uint32_t)i + (tid >> 3);
@@ -134,36 +141,44 @@ k_lm_head_codes_rows(const uint16_t* __restrict__ hidden, uint64_t hidden_stride
     // ---- scales and biases: group g of column c at sz[c * groups + (g + c) % groups] (32 columns
     // read one group at once: turned by the column's number, they lie in different banks)
     {
-        auto put = [&](uint32_t col, uint32_t g, uint32_t scale, uint32_t bias) {
-            sz[col * groups + (g + col) % groups] = scale | (bias << 16);
+        // (eight neighbouring threads a column; no division but one a column)
+        const uint32_t col0 = tid >> 3, lane8 = tid & 7u;
+        auto put = [&](uint32_t at0, uint32_t turn, uint32_t g, uint32_t scale, uint32_t bias) {
+            const uint32_t at = g + turn;
+            sz[at0 + (at >= groups ? at - groups : at)] = scale | (bias << 16);
         };
-        const bool wide = groups % 8u == 0u &&
-                          ((reinterpret_cast<uintptr_t>(scales) | reinterpret_cast<uintptr_t>(biases)) & 15u) == 0u;
-        const uint32_t per = wide ? groups / 8u : groups, n = LILY_TILE_COLS * per;
-        if (wide) {   // 16 bytes, eight groups, a load
-            for (uint32_t base = 0; base < n; base += 4u * 256u) {
+        uint32_t turn[4];
+        uint64_t from[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            turn[u] = (col0 + 32u * (uint32_t)u) % groups;
+            from[u] = (uint64_t)min(n0 + col0 + 32u * (uint32_t)u, vocab - 1u) * groups;
+        }
+        if (groups % 8u == 0u &&
+            ((reinterpret_cast<uintptr_t>(scales) | reinterpret_cast<uintptr_t>(biases)) & 15u) == 0u) {
+            for (uint32_t g0 = 0; g0 < groups; g0 += 64u) {   // 16 bytes, eight groups, a load
+                const uint32_t g = min(g0 + lane8 * 8u, groups - 8u);   // (the last ones by several: the same values)
                 w32x4 s[4], b[4];
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
-                    const uint32_t i = min(base + (uint32_t)u * 256u + tid, n - 1u);
-                    const uint64_t at = (uint64_t)min(n0 + i / per, vocab - 1u) * groups + (i % per) * 8u;
-                    s[u] = *reinterpret_cast<const w32x4*>(scales + at);
-                    b[u] = *reinterpret_cast<const w32x4*>(biases + at);
+                    s[u] = *reinterpret_cast<const w32x4*>(scales + from[u] + g);
+                    b[u] = *reinterpret_cast<const w32x4*>(biases + from[u] + g);
                 }
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
-                    const uint32_t i = min(base + (uint32_t)u * 256u + tid, n - 1u);
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
-                        put(i / per, (i % per) * 8u + (uint32_t)e, (s[u][e >> 1] >> (16 * (e & 1))) & 0xffffu,
-                            (b[u][e >> 1] >> (16 * (e & 1))) & 0xffffu);
+                        put((col0 + 32u * (uint32_t)u) * groups, turn[u], g + (uint32_t)e,
+                            (s[u][e >> 1] >> (16 * (e & 1))) & 0xffffu, (b[u][e >> 1] >> (16 * (e & 1))) & 0xffffu);
                     }
                 }
             }
         } else {
-            for (uint32_t i = tid; i < n; i += 256u) {
-                const uint64_t at = (uint64_t)min(n0 + i / per, vocab - 1u) * groups + i % per;
-                put(i / per, i % per, scales[at], biases[at]);
+            for (uint32_t g = lane8; g < groups; g += 8u) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    put((col0 + 32u * (uint32_t)u) * groups, turn[u], g, scales[from[u] + g], biases[from[u] + g]);
+                }
             }
         }
     }
@@ -194,12 +209,23 @@ k_lm_head_codes_rows(const uint16_t* __restrict__ hidden, uint64_t hidden_stride
             hi = (raw[m] >> 4) & 0x0f0f0f0fu;
         }
         w32x4 out;
+        if constexpr (WBITS == 8) {
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            const uint32_t q0 = WBITS == 8 ? ((p < 2 ? lo : hi) >> (16 * (p & 1))) & 0xffu : (lo >> (8 * p)) & 0xffu;
-            const uint32_t q1 = WBITS == 8 ? ((p < 2 ? lo : hi) >> (16 * (p & 1) + 8)) & 0xffu : (hi >> (8 * p)) & 0xffu;
-            const f32x2 f = {__builtin_fmaf((float)q0, scale, bias), __builtin_fmaf((float)q1, scale, bias)};
-            out[p] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
+            for (int p = 0; p < 4; ++p) {
+                const uint32_t word = p < 2 ? lo : hi;
+                const f32x2 f = {__builtin_fmaf((float)((word >> (16 * (p & 1))) & 0xffu), scale, bias),
+                                 __builtin_fmaf((float)((word >> (16 * (p & 1) + 8)) & 0xffu), scale, bias)};
+                out[p] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
+            }
+        } else {
+            // (opaque here: the compiler would turn the bytes back into an extraction a code)
+            asm("" : "+v"(lo), "+v"(hi));
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const f32x2 f = {__builtin_fmaf((float)((lo >> (8 * p)) & 0xffu), scale, bias),
+                                 __builtin_fmaf((float)((hi >> (8 * p)) & 0xffu), scale, bias)};
+                out[p] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
+            }
         }
         return __builtin_bit_cast(bf16x8, out);
     };
@@ -225,7 +251,7 @@ k_lm_head_codes_rows(const uint16_t* __restrict__ hidden, uint64_t hidden_stride
 #pragma unroll
             for (int i = 0; i < PIECES; ++i) {
                 const uint32_t piece = 2u * (uint32_t)(u * PIECES + i) + h;
-                raw[i] = *reinterpret_cast<const w32x4*>(own_codes + c * 128u + (piece ^ (c & 7u)) * 16u);
+                raw[i] = *reinterpret_cast<const w32x4*>(own_codes + c * 128u + (piece ^ ((c >> 1) & 7u)) * 16u);
             }
             const uint32_t g = (first_k + (uint32_t)u * STEP_K) >> group_shift;
             const uint32_t at = g + turn;
@@ -235,7 +261,7 @@ k_lm_head_codes_rows(const uint16_t* __restrict__ hidden, uint64_t hidden_stride
 #pragma unroll
             for (int m = 0; m < 4; ++m) {
                 const uint32_t piece = WBITS == 8 ? 4u * (uint32_t)(m >> 1) + 2u * h + (uint32_t)(m & 1) : 4u * h + (uint32_t)m;
-                const char* a_at = lds + buf * HIDDEN_BYTES + c * 128u + (piece ^ (c & 7u)) * 16u;
+                const char* a_at = lds + buf * HIDDEN_BYTES + c * 128u + (piece ^ ((c >> 1) & 7u)) * 16u;
                 const bf16x8 w = weights_of(raw[WBITS == 8 ? m >> 1 : 0], m, scale, bias);
 #pragma unroll
                 for (int mi = 0; mi < MI; ++mi) {

@@ -845,6 +845,22 @@ def test_tiles_of_codes_at_their_edges(sampler, rows, d, vocab, bits, group):
     sampler.synchronize()
     _check_f32_product(h, dense, buf[:, :vocab], tmax, tsum, temps)
     assert torch.all(buf[:, vocab:] == 7.0)
+    # One column's scales of about 2^116, another's of about 2^-104: the weights are the same
+    # roundings of q * scale + bias, the sums within f32's error of the magnitudes summed.
+    columns = {vocab // 2: 2.0 ** 120, vocab // 3: 2.0 ** -100}
+    for column, by in columns.items():
+        qw.scales[column] = (qw.scales[column].float() * by).to(torch.bfloat16)
+        qw.biases[column] = (qw.biases[column].float() * by).to(torch.bfloat16)
+    sampler.lm_head(h, qw, temps, buf[:, :vocab], tmax, tsum)
+    sampler.synchronize()
+    assert torch.all(torch.isfinite(buf[:, :vocab]))
+    hid, per = h.double().cpu(), 32 // bits
+    for column in list(columns) + [0, vocab - 1]:
+        q = (qw.codes[column].cpu()[:, None] >> (bits * torch.arange(per, dtype=torch.int32))) & ((1 << bits) - 1)
+        exact = (q.reshape(d).double() * qw.scales[column].cpu().double().repeat_interleave(group) +
+                 qw.biases[column].cpu().double().repeat_interleave(group))
+        w = exact.float().to(torch.bfloat16).double()
+        assert torch.all((buf[:, column].double().cpu() - hid @ w).abs() <= hid.abs() @ w.abs() * 2.0 ** -21)
 
 
 @pytest.mark.parametrize("form", ["own", "library"])
