@@ -4,17 +4,18 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "row_args.h"
 
 namespace lily {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-// x as the lane CTRL names holds it (DPP controls: 0x120 + n = rotate right by n within each
-// row of 16 lanes).
+// x as the lane that the DPP control CTRL names holds it.
 template <int CTRL>
-__device__ __forceinline__ float rotated(float x) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, false));
+__device__ __forceinline__ float moved(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
 }
 
 // acc: the sums of a wave's MI x NI products of 32 x 32; four waves, WAVES_M x (4 / WAVES_M), this
@@ -66,34 +67,50 @@ __device__ __forceinline__ void head_epilogue(f32x16 (&acc)[MI][NI], char* lds, 
         const float x = acc[mi][ni][v];
         return (in_vocab[ni] && x == x) ? x : NEG;
     };
-    // A reduction over the 32 lanes that hold one row's columns: rotations by 8, 4, 2 and 1 within
-    // each row of 16 lanes (DPP operands of the arithmetic itself), then one exchange between the
-    // two rows.  (Five exchanges through the LDS crossbar per value, as __shfl_xor compiles, made
-    // the epilogue as long as the products at 1024 rows.)
-    auto across32 = [&](float x, auto op) -> float {
-        x = op(x, rotated<0x128>(x));
-        x = op(x, rotated<0x124>(x));
-        x = op(x, rotated<0x122>(x));
-        x = op(x, rotated<0x121>(x));
-        return op(x, __shfl_xor(x, 16));
+    // A reduction of a lane's 16 values over the 32 lanes that hold the same rows: the values are
+    // halved with the lanes.  First the two rows of 16 lanes change halves (one instruction for two
+    // values: the even row then holds value v of both, the odd row value v + 8), then lanes 8, 4, 2
+    // and 1 apart.  The lane ends with the value (lane / 2) % 16: 38 instructions for 16 values where
+    // a butterfly for each value took 96 and a place in LDS for each of 16 writes.
+    auto across32 = [&](float (&x)[16], auto op) -> float {
+#pragma unroll
+        for (int v = 0; v < 8; ++v) {
+            const auto both = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, x[v]),
+                                                               __builtin_bit_cast(uint32_t, x[v + 8]), false, false);
+            x[v] = op(__builtin_bit_cast(float, (uint32_t)both[0]), __builtin_bit_cast(float, (uint32_t)both[1]));
+        }
+        auto halve = [&](int n, bool upper, auto ctrl) {
+#pragma unroll
+            for (int v = 0; v < n; ++v) {
+                const float keep = upper ? x[v + n] : x[v], give = upper ? x[v] : x[v + n];
+                x[v] = op(keep, moved<decltype(ctrl)::value>(give));
+            }
+        };
+        halve(4, (lane & 8u) != 0u, std::integral_constant<int, 0x128>{});   // (rotated by 8)
+        halve(2, (lane & 4u) != 0u, std::integral_constant<int, 0x141>{});   // (eight lanes mirrored)
+        halve(1, (lane & 2u) != 0u, std::integral_constant<int, 0x4e>{});    // (quads: 2 3 0 1)
+        return op(x[0], moved<0xb1>(x[0]));                                  // (quads: 1 0 3 2)
     };
     auto row_of = [&](int mi, int v) -> uint32_t {
         return wm * (MI * 32u) + (uint32_t)mi * 32u + 8u * (uint32_t)(v >> 2) + 4u * (lane >> 5) +
                (uint32_t)(v & 3);
     };
+    const uint32_t own_v = (lane >> 1) & 15u;   // the value a lane ends with, and its row
+    const uint32_t own_row = wm * (MI * 32u) + 8u * (own_v >> 2) + 4u * (lane >> 5) + (own_v & 3u);
 #pragma unroll
     for (int mi = 0; mi < MI; ++mi) {
+        float m[16];
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-            float m = NEG;
+            m[v] = NEG;
 #pragma unroll
             for (int ni = 0; ni < NI; ++ni) {
-                m = fmaxf(m, worth(mi, ni, v));
+                m[v] = fmaxf(m[v], worth(mi, ni, v));
             }
-            m = across32(m, [](float p, float q) { return fmaxf(p, q); });
-            if ((lane & 31u) == 0u) {
-                red[wn * BM + row_of(mi, v)] = m;
-            }
+        }
+        const float top = across32(m, [](float p, float q) { return fmaxf(p, q); });
+        if ((lane & 1u) == 0u) {
+            red[wn * BM + own_row + (uint32_t)mi * 32u] = top;
         }
     }
     __syncthreads();
@@ -108,20 +125,21 @@ __device__ __forceinline__ void head_epilogue(f32x16 (&acc)[MI][NI], char* lds, 
     __syncthreads();
 #pragma unroll
     for (int mi = 0; mi < MI; ++mi) {
+        float e[16];
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
             const uint32_t r = row_of(mi, v);
             const float c = row_c2[r], top = row_max[r] * c;
-            float e = 0.0f;
+            e[v] = 0.0f;
 #pragma unroll
             for (int ni = 0; ni < NI; ++ni) {
                 const float x = worth(mi, ni, v);
-                e += x > NEG ? __builtin_amdgcn_exp2f(__builtin_fmaf(x, c, -top)) : 0.0f;
+                e[v] += x > NEG ? __builtin_amdgcn_exp2f(__builtin_fmaf(x, c, -top)) : 0.0f;
             }
-            e = across32(e, [](float p, float q) { return p + q; });
-            if ((lane & 31u) == 0u) {
-                red[wn * BM + r] = e;
-            }
+        }
+        const float sum = across32(e, [](float p, float q) { return p + q; });
+        if ((lane & 1u) == 0u) {
+            red[wn * BM + own_row + (uint32_t)mi * 32u] = sum;
         }
     }
     __syncthreads();
@@ -135,23 +153,26 @@ __device__ __forceinline__ void head_epilogue(f32x16 (&acc)[MI][NI], char* lds, 
         tile_max[at] = row_max[tid];
         tile_sum[at] = row_max[tid] > NEG ? e : 0.0f;
     }
-    // the logits themselves
+    // the logits themselves (a lane's place once, the rows' distances the same for all lanes)
 #pragma unroll
-    for (int mi = 0; mi < MI; ++mi) {
+    for (int ni = 0; ni < NI; ++ni) {
+        const uint32_t col = n0 + wn * (NI * 32u) + (uint32_t)ni * 32u + (lane & 31u);
+        uint64_t at = (uint64_t)(m0 + row_of(0, 0)) * logits_stride + col;
+        const uint64_t jump = 5u * logits_stride;   // (from row 3 of four to the next four)
+        if (col < vocab) {
 #pragma unroll
-        for (int ni = 0; ni < NI; ++ni) {
-            const uint32_t col = n0 + wn * (NI * 32u) + (uint32_t)ni * 32u + (lane & 31u);
+            for (int mi = 0; mi < MI; ++mi) {
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const uint32_t r = m0 + row_of(mi, v);
-                if (r < rows && col < vocab) {
-                    const float f = acc[mi][ni][v];
-                    if constexpr (OUT_F32) {
-                        static_cast<float*>(logits_out)[(uint64_t)r * logits_stride + col] = f;
-                    } else {
-                        static_cast<uint16_t*>(logits_out)[(uint64_t)r * logits_stride + col] =
-                            (uint16_t)(__builtin_bit_cast(uint32_t, f) >> 16);
+                for (int v = 0; v < 16; ++v) {
+                    if (m0 + row_of(mi, v) < rows) {
+                        const float f = acc[mi][ni][v];
+                        if constexpr (OUT_F32) {
+                            static_cast<float*>(logits_out)[at] = f;
+                        } else {
+                            static_cast<uint16_t*>(logits_out)[at] = (uint16_t)(__builtin_bit_cast(uint32_t, f) >> 16);
+                        }
                     }
+                    at += (v & 3) == 3 ? jump : logits_stride;
                 }
             }
         }
