@@ -81,12 +81,12 @@ k_lm_head_codes(const uint16_t* __restrict__ hidden, uint64_t hidden_stride, con
     constexpr uint32_t WAVE_K = STAGE_K / 4u;          // ... of which a wave multiplies these
     extern __shared__ __align__(16) char lds[];
     float* part = reinterpret_cast<float*>(lds);       // [4 shares][2 * CB][4 v x 64 lanes, padded], at the end
-    uint32_t* sz = reinterpret_cast<uint32_t*>(lds + RING_BYTES);   // scales, then biases
+    uint32_t* sz = reinterpret_cast<uint32_t*>(lds + RING_BYTES);   // scales and biases
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t share = wave & 3u, half = wave >> 2;
     const uint32_t c = lane & 15u, kq = lane >> 4;
     const uint32_t n_tile = blockIdx.x, n0 = n_tile * LILY_TILE_COLS;
-    const uint32_t nstages = d / STAGE_K, groups = d >> group_shift, pairs = groups >> 1;
+    const uint32_t nstages = d / STAGE_K, groups = d >> group_shift;
     // Each tile walks d from a place of its own and wraps round: rows lie a power of two apart
     // for the usual d, and tiles that all start at column 0 and advance in step queue up at one
     // memory channel after the other.
@@ -140,8 +140,8 @@ k_lm_head_codes(const uint16_t* __restrict__ hidden, uint64_t hidden_stride, con
     for (int cb = 0; cb < CB; ++cb) {
         const uint32_t col = 64u * half + 16u * (uint32_t)cb + c, q = 2u * share + (kq >> 1);
         code_at[cb] = (col >> 3) * 1024u + ((col & 7u) * 8u + (q ^ (col & 7u))) * 16u + (kq & 1u) * 8u;
-        scale_at[cb] = col * pairs;
-        turn[cb] = col % pairs;
+        scale_at[cb] = col * groups;
+        turn[cb] = col % groups;
     }
 
     f32x4 total[CB];
@@ -174,7 +174,7 @@ k_lm_head_codes(const uint16_t* __restrict__ hidden, uint64_t hidden_stride, con
             xs = product(a[1], ONES, xs);
         }
         // the wave's values of this stage lie in one group (64 values, or 32 of one)
-        const uint32_t g = (place(stage_no) * STAGE_K + share * WAVE_K) >> group_shift, w = g >> 1, odd = (g & 1u) * 16u;
+        const uint32_t g = (place(stage_no) * STAGE_K + share * WAVE_K) >> group_shift;
         const char* codes_in = lds + buf * STAGE_BYTES;
 #pragma unroll
         for (int cb = 0; cb < CB; ++cb) {
@@ -205,10 +205,9 @@ k_lm_head_codes(const uint16_t* __restrict__ hidden, uint64_t hidden_stride, con
             if constexpr (STEPS == 2) {
                 qx = product(a[1], b[1], qx);
             }
-            uint32_t at = w + turn[cb];
-            at = at >= pairs ? at - pairs : at;
-            const float s = bf16_bits_to_f32((sz[scale_at[cb] + at] >> odd) & 0xffffu);
-            float z = bf16_bits_to_f32((sz[LILY_TILE_COLS * pairs + scale_at[cb] + at] >> odd) & 0xffffu);
+            const uint32_t at = g + turn[cb], word = sz[scale_at[cb] + (at >= groups ? at - groups : at)];
+            const float s = bf16_bits_to_f32(word);   // (the shift drops the bias)
+            float z = __builtin_bit_cast(float, word & 0xffff0000u);
             if constexpr (WBITS == 4) {
                 z = __builtin_fmaf(-128.0f, s, z);
             }
@@ -235,26 +234,51 @@ k_lm_head_codes(const uint16_t* __restrict__ hidden, uint64_t hidden_stride, con
         __builtin_amdgcn_sched_barrier(0);   // (in this order: the loop waits for the oldest only)
     }
     // (the first stages are on their way while the scales are brought)
-    // ---- the tile's scales and biases, two groups (one word) at a time: word w of column col
-    // at sz[col * pairs + (w + col) % pairs] (turned by the column's number: the 16 columns a
-    // product reads at once then lie in different banks), the biases behind all the scales.
+    // ---- the tile's scales and biases: group g of column col as one word (scale, bias) at
+    // sz[col * groups + (g + col) % groups] (turned by the column's number: the 16 columns a
+    // product reads at once then lie in different banks).  Eight neighbouring threads a column, 16
+    // bytes - eight groups - a load where the arrays allow it.  (A form that found a word's column
+    // and place by divisions, sixteen words a thread, spent 40 % of the launch's vector
+    // instructions here, and those are 80 % of its cycles: V = 151 936, 4 rows, d = 4096 / 2560: 4 bits
+    // 101 / 78 -> 98 / 71 us, 8 bits 145 / 100 -> 141 / 96.)
     {
-        const uint32_t words = LILY_TILE_COLS * pairs;
-        // (unconditional loads, the last word again past the end: eight in flight a thread)
-        for (uint32_t base = 0; base < 2u * words; base += 8u * THREADS) {
-            uint32_t got[8];
+        const uint32_t col0 = tid >> 3, lane8 = tid & 7u;
+        auto put = [&](uint32_t col, uint32_t turn_of, uint32_t g, uint32_t scale, uint32_t bias) {
+            const uint32_t at = g + turn_of;
+            sz[col * groups + (at >= groups ? at - groups : at)] = scale | (bias << 16);
+        };
+        uint32_t turned[2];
+        uint64_t from[2];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const uint32_t i = min(base + (uint32_t)u * THREADS + tid, 2u * words - 1u);
-                const uint32_t arr = i >= words ? 1u : 0u, j = i - arr * words, col = j / pairs, w = j - col * pairs;
-                const uint16_t* src = (arr != 0u ? biases : scales) + (uint64_t)min(n0 + col, vocab - 1u) * groups + 2u * w;
-                got[u] = *reinterpret_cast<const uint32_t*>(src);
+        for (int u = 0; u < 2; ++u) {
+            turned[u] = (col0 + 64u * (uint32_t)u) % groups;
+            from[u] = (uint64_t)min(n0 + col0 + 64u * (uint32_t)u, vocab - 1u) * groups;
+        }
+        if (groups % 8u == 0u &&
+            ((reinterpret_cast<uintptr_t>(scales) | reinterpret_cast<uintptr_t>(biases)) & 15u) == 0u) {
+            for (uint32_t g0 = 0; g0 < groups; g0 += 64u) {
+                const uint32_t g = min(g0 + lane8 * 8u, groups - 8u);   // (the last ones by several: the same values)
+                w32x4 sc[2], bi[2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    sc[u] = *reinterpret_cast<const w32x4*>(scales + from[u] + g);
+                    bi[u] = *reinterpret_cast<const w32x4*>(biases + from[u] + g);
+                }
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        put(col0 + 64u * (uint32_t)u, turned[u], g + (uint32_t)e, (sc[u][e >> 1] >> (16 * (e & 1))) & 0xffffu,
+                            (bi[u][e >> 1] >> (16 * (e & 1))) & 0xffffu);
+                    }
+                }
             }
+        } else {
+            for (uint32_t g = lane8; g < groups; g += 8u) {
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const uint32_t i = min(base + (uint32_t)u * THREADS + tid, 2u * words - 1u);
-                const uint32_t arr = i >= words ? 1u : 0u, j = i - arr * words, col = j / pairs, w = j - col * pairs;
-                sz[arr * words + col * pairs + (w + col) % pairs] = got[u];   // (the last word by several: the same value)
+                for (int u = 0; u < 2; ++u) {
+                    put(col0 + 64u * (uint32_t)u, turned[u], g, scales[from[u] + g], biases[from[u] + g]);
+                }
             }
         }
     }
