@@ -471,7 +471,8 @@ uint32_t lily_lm_head_tiles(uint32_t vocab);
 int lily_lm_head_bf16(lily_sampler_t* s, const lily_lm_head* head, uint32_t rows, uint32_t vocab,
                       const float* temperatures, void* logits_dev, uint64_t row_stride);
 
-/* A batch of many rows (from 129 on; from 256 on over codes) is a plain matrix product of the
+/* A batch of many rows (from 129 on; over codes from 641 on, or from 256 on where groups are
+ * smaller than 64 or d is not a multiple of 256 (4 bits) or 128 (8 bits)) is a plain matrix product of the
  * kind the platform's GEMM library (hipBLASLt) is tuned for: where a program can open that library
  * by its name (libhipblaslt.so.1: it is opened at run time, never linked) and the library has an
  * algorithm for the shape, the producer forms the logits through it - codes are first turned
