@@ -58,6 +58,8 @@ hipError_t launch_lm_head_codes(hipStream_t stream, const void* hidden, uint64_t
 // The same for any number of rows with the weights in bf16, as dequant_q4/q8_bf16 make them of the
 // codes (groups of 64 or more, whole lines of codes).
 bool lm_head_codes_rows_serves(uint32_t d, const HeadWeights& wq);
+// Workgroups of its 128-row tile that fit a compute unit's LDS (d and groups that it serves).
+uint32_t lm_head_codes_rows_resident(uint32_t d, const HeadWeights& wq);
 hipError_t launch_lm_head_codes_rows(hipStream_t stream, const void* hidden, uint64_t hidden_stride, const void* weight,
                                      uint64_t weight_stride, uint32_t rows, uint32_t d, uint32_t vocab,
                                      const float* c2_of_row, void* logits, uint64_t logits_stride, float* tile_max,

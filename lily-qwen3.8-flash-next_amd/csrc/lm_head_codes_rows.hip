@@ -20,6 +20,7 @@ namespace {
 constexpr int STEP_K = 64;                               // values of d between two barriers
 constexpr int CODE_BYTES = LILY_TILE_COLS * 128;         // a stage of codes: one line of every column
 constexpr int AHEAD = 2;                                 // stages of codes on their way in registers
+constexpr uint32_t LDS_BYTES = 160u * 1024u;             // of a compute unit
 
 inline uint32_t rows_lds_bytes(int mi, uint32_t groups) {
     return 2u * (uint32_t)mi * 32u * STEP_K * 2u + CODE_BYTES + LILY_TILE_COLS * groups * 4u;
@@ -42,7 +43,11 @@ inline uint32_t rows_lds_bytes(int mi, uint32_t groups) {
 // effective lead is HIDDEN_AHEAD steps.
 // Scales and biases: the tile's, brought once as whole lines, a word (scale, bias) per group.
 //
-// LDS: 2 x MI * 4 KB + 16 KB + 512 bytes a group: two or three workgroups a compute unit.
+// LDS: 2 x MI * 4 KB + 16 KB + 512 bytes a group.  Of a compute unit's 160 KB, three workgroups of
+// 32 rows fit up to 58 groups, two up to 112; of 64 rows three up to 42, two up to 96; of 128 rows
+// two up to 64 groups (d = 4096 in groups of 64).  One alone has nothing to cover its barriers: 512
+// rows of 4 bits take 1.21 times as long per value of d at d = 8192 as at 4096, and larger batches
+// go another way from fewer rows on (sampler_api.cpp, HEAD_LIBRARY_ROWS_CODE_LINES_ALONE).
 //
 // Before it, tiles that brought 4 or 8 bytes of codes and two 2-byte scales a thread and load (the
 // requests, not the bytes, were their bound) and turned each code into LDS.  V = 151 936, f32
@@ -308,7 +313,7 @@ static hipError_t launch_codes_rows(hipStream_t stream, const void* hidden, uint
     // that threads on several devices keep nothing between them)
     if (lds > 64u * 1024u) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_lm_head_codes_rows<WBITS, MI>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
         if (e != hipSuccess) {
             return e;
         }
@@ -328,7 +333,11 @@ bool lm_head_codes_rows_serves(uint32_t d, const HeadWeights& wq) {
     // whole stages, and all the tile's scales in LDS beside the stages
     const uint32_t groups = d >> wq.group_shift;
     return d != 0u && d % (1024u / wq.bits) == 0u && groups >= 1u && (groups << wq.group_shift) == d &&
-           rows_lds_bytes(4, groups) <= 160u * 1024u;
+           rows_lds_bytes(4, groups) <= LDS_BYTES;
+}
+
+uint32_t lm_head_codes_rows_resident(uint32_t d, const HeadWeights& wq) {
+    return LDS_BYTES / rows_lds_bytes(4, d >> wq.group_shift);
 }
 
 hipError_t launch_lm_head_codes_rows(hipStream_t stream, const void* hidden, uint64_t hidden_stride, const void* weight,

@@ -75,11 +75,20 @@ constexpr uint32_t WS_ROWS = 4096;      // rows that may span several workgroups
 // Batches of the logits' producer from this many rows on go through the vendor's GEMM library
 // where it is present (below, this library's own tiles are as fast or faster; over codes the
 // library's way begins with a pass that turns all of them into bf16 weights).  Over codes the line
-// depends on the tiles: those of lm_head_codes_rows.hip, 128 rows at a time, are the faster way up
-// to five of them (V = 151 936, d = 4096, own against library: 4 bits 256 rows 456 / 723 us, 640
-// rows 1 015 / 1 195, 1 024 rows 1 606 / 1 554; 8 bits 473 / 755, 1 089 / 1 227, 1 748 / 1 590),
-// the others (groups of 32, d that is no whole lines of codes) up to 255 rows.
-constexpr uint32_t HEAD_LIBRARY_ROWS = 129, HEAD_LIBRARY_ROWS_CODES = 256, HEAD_LIBRARY_ROWS_CODE_LINES = 641;
+// depends on the tiles.  Those of lm_head_codes_rows.hip, 128 rows at a time, are the faster way up
+// to five of them where two workgroups share a compute unit (d = 4096 in groups of 64, 8192 in
+// groups of 128), and up to three where the tile's scales leave room for one.  Own against library,
+// us, V = 151 936, 4 bits, groups of 64 (8 bits lie within 5 % of the same ratios):
+//     rows      257          384          512            640            704
+//     d 2560    375 / 553    496 / 627     514 /   677    640 /   758    744 /   782
+//     d 4096    562 / 812    749 / 916     760 /   972    952 / 1 145  1 119 / 1 180
+//     d 5120    864 / 995    878 / 1 072  1 181 / 1 186  1 477 / 1 411
+//     d 8192  1 327 / 1 519  1 367 / 1 619  1 834 / 1 791  2 416 / 2 160
+//     d 12288 1 954 / 2 208  2 046 / 2 354  2 754 / 2 601
+// (d = 4352 to 14336 at 385 rows: 1.02 to 1.08 times the library's time).  The other tiles (groups of
+// 32, d that is no whole lines of codes) are up to 255 rows.
+constexpr uint32_t HEAD_LIBRARY_ROWS = 129, HEAD_LIBRARY_ROWS_CODES = 256, HEAD_LIBRARY_ROWS_CODE_LINES = 641,
+                   HEAD_LIBRARY_ROWS_CODE_LINES_ALONE = 385;
 constexpr uint32_t WS_SLOTS = 1u << 22; // candidate slots of the workspace (rows x slices x k)
 constexpr uint32_t STAGE_SLOTS = 4;
 constexpr size_t STAGE_ROW_BYTES = sizeof(RowArgs) + 16;   // a staged row: descriptor + three words + slack
@@ -117,6 +126,7 @@ struct lily_sampler {
     // library ("own": never, "library": every batch it takes, a number: from that many rows on)
     uint32_t head_library_rows = HEAD_LIBRARY_ROWS, head_library_rows_codes = HEAD_LIBRARY_ROWS_CODES;
     uint32_t head_library_rows_code_lines = HEAD_LIBRARY_ROWS_CODE_LINES;
+    uint32_t head_library_rows_code_lines_alone = HEAD_LIBRARY_ROWS_CODE_LINES_ALONE;
     unsigned long long head_library_calls = 0;   // producer calls that went through the vendor's library
     uint32_t handover = 0;  // LILY_SAMPLER_HANDOVER: 0 = by the launch's size, 1 = strict, 2 = relaxed
     // What the last lily_lm_head_bf16 call of this sampler left: where, and with which exponent
@@ -905,7 +915,8 @@ int lily_sampler_create(int device, void* hip_stream, lily_sampler_t** out) {
     }
     if (const char* p = std::getenv("LILY_SAMPLER_HEAD")) {
         s->head_library_rows = std::strcmp(p, "own") == 0 ? 0u : std::strcmp(p, "library") == 0 ? 1u : (uint32_t)std::atoi(p);
-        s->head_library_rows_codes = s->head_library_rows_code_lines = s->head_library_rows;
+        s->head_library_rows_codes = s->head_library_rows_code_lines = s->head_library_rows_code_lines_alone =
+            s->head_library_rows;
     }
     if (const char* p = std::getenv("LILY_SAMPLER_HANDOVER")) {
         s->handover = std::strcmp(p, "strict") == 0 ? 1u : std::strcmp(p, "relaxed") == 0 ? 2u : 0u;
@@ -1793,9 +1804,10 @@ HeadWeightsOf::HeadWeightsOf(const lily_sampler* s, const lily_lm_head* h) {
         ++shift;
     }
     w.group_shift = shift;
-    w.library_rows = h->weight_bits == 0u                   ? s->head_library_rows
-                     : lm_head_codes_rows_serves(h->d, w) ? s->head_library_rows_code_lines
-                                                           : s->head_library_rows_codes;
+    w.library_rows = h->weight_bits == 0u                    ? s->head_library_rows
+                     : !lm_head_codes_rows_serves(h->d, w) ? s->head_library_rows_codes
+                     : lm_head_codes_rows_resident(h->d, w) >= 2u ? s->head_library_rows_code_lines
+                                                                  : s->head_library_rows_code_lines_alone;
 }
 
 // Rows the summaries serve: penalties only of the lowering kind, the row given as it is, and a

@@ -919,6 +919,37 @@ def test_batches_in_either_form(monkeypatch, form, rows, d, vocab, slack):
         s.close()
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("d,group,rows,library", [
+    (4096, 64, 640, False), (4096, 64, 641, True),      # 64 groups: two workgroups a compute unit
+    (4352, 64, 384, False), (4352, 64, 385, True),      # 68: one
+    (8192, 128, 640, False), (14336, 64, 640, True),    # 64 again; 224, the most the tiles take
+    (14592, 64, 256, True), (4096, 32, 255, False), (4096, 32, 256, True)])   # the other tiles
+def test_the_way_of_a_batch_over_codes(monkeypatch, bits, d, group, rows, library):
+    """Which batches over codes take the platform's GEMM library: the line lies where it is
+    measured to be the faster way, lower where the tiles' scales leave room for one workgroup a
+    compute unit."""
+    monkeypatch.delenv("LILY_SAMPLER_HEAD", raising=False)
+    vocab = 256
+    rng = np.random.default_rng(d + rows)
+    hidden = rng.normal(0, 1, (rows, d)).astype(np.float32)
+    qw, dense, _, _ = _quantised(rng, vocab, d, bits, group)
+    s = LS.Sampler(0)
+    try:
+        temps = [0.8] * rows
+        logits = torch.zeros(rows, vocab, dtype=torch.float32, device=dev())
+        tiles = (vocab + TILE - 1) // TILE
+        tmax = torch.zeros(rows, tiles, dtype=torch.float32, device=dev())
+        tsum = torch.zeros(rows, tiles, dtype=torch.float32, device=dev())
+        h = _bf16(hidden)
+        s.lm_head(h, qw, temps, logits, tmax, tsum)
+        s.synchronize()
+        assert s.lm_head_library_calls() == (1 if library else 0)
+        _check_f32_product(h, dense, logits, tmax, tsum, temps)
+    finally:
+        s.close()
+
+
 @pytest.mark.parametrize("block", range(4))
 def test_random_rows_from_summaries(sampler, block):
     """Seeded random batches through lily_sample_rows_tiled: bf16 or f32 logits of heads with few
