@@ -473,7 +473,8 @@ int lily_lm_head_bf16(lily_sampler_t* s, const lily_lm_head* head, uint32_t rows
 
 /* A batch of many rows (from 129 on; over codes from 641 on, from 385 on where a row has more than
  * 64 groups, or from 256 on where it has more than 224, groups are smaller than 64 or d is not a
- * multiple of 256 (4 bits) or 128 (8 bits)) is a plain matrix product of the kind the platform's GEMM library (hipBLASLt) is tuned for: where a program can open that library
+ * multiple of 256 (4 bits) or 128 (8 bits)) is a plain matrix product of the kind the platform's
+ * GEMM library (hipBLASLt) is tuned for: where a program can open that library
  * by its name (libhipblaslt.so.1: it is opened at run time, never linked) and the library has an
  * algorithm for the shape, the producer forms the logits through it - codes are first turned
  * into bf16 weights, all of them, in memory the call keeps (vocab x d x 2 bytes a device and

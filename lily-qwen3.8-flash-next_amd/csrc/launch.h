@@ -3,9 +3,34 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <atomic>
+
 #include "row_args.h"
 
 namespace lily {
+
+constexpr uint32_t CU_LDS_BYTES = 160u * 1024u;   // a compute unit's
+
+// A launch may have 64 KB of LDS without asking.  One of these beside a kernel asks for all of a
+// compute unit's, once per device; any number of threads launch it with any sizes meanwhile.  (A
+// table of the size each launch needed let a thread with a small one lower what another had just
+// raised.)
+struct LdsAllowed {
+    std::atomic<bool> said[64] = {};
+    hipError_t say(const void* kernel) {
+        int device = 0;
+        hipError_t e = hipGetDevice(&device);
+        const bool known = e == hipSuccess && device >= 0 && device < 64;
+        if (e != hipSuccess || (known && said[device].load(std::memory_order_acquire))) {
+            return e;
+        }
+        e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)CU_LDS_BYTES);
+        if (e == hipSuccess && known) {
+            said[device].store(true, std::memory_order_release);
+        }
+        return e;
+    }
+};
 
 // `kind`: 0 = no row has a mask, penalties or a bias list, 1 = some row has, 2 = every sampled
 // row takes the streaming select; `lse`: some row wants a log-probability.

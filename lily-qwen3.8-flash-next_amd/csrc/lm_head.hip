@@ -400,21 +400,10 @@ static hipError_t launch_head_shape(hipStream_t stream, const void* hidden, uint
                                     uint32_t vocab, const float* c2_of_row, void* logits,
                                     uint64_t logits_stride, float* tile_max, float* tile_sum,
                                     const HeadQuant& quant) {
-    static bool sized[64] = {};
-    int device = 0;
-    hipError_t e = hipGetDevice(&device);
+    static LdsAllowed allowed;
+    const hipError_t e = allowed.say(reinterpret_cast<const void*>(k_lm_head_bf16<T, OUT_F32, WBITS>));
     if (e != hipSuccess) {
         return e;
-    }
-    if (device < 0 || device >= 64 || !sized[device]) {
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_lm_head_bf16<T, OUT_F32, WBITS>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES);
-        if (e != hipSuccess) {
-            return e;
-        }
-        if (device >= 0 && device < 64) {
-            sized[device] = true;
-        }
     }
     const uint32_t tiles_per_row = (vocab + T::BN - 1u) / T::BN, m_tiles = (rows + T::BM - 1u) / T::BM;
     // slots an XCD needs at most (see the kernel's numbering)

@@ -388,22 +388,10 @@ static hipError_t launch_codes(hipStream_t stream, const void* hidden, uint64_t 
                                float* tile_sum, const HeadWeights& wq) {
     const uint32_t tiles_per_row = (vocab + LILY_TILE_COLS - 1u) / LILY_TILE_COLS;
     const size_t lds = codes_lds_bytes(d >> wq.group_shift);
-    // (more than the 64 KB a kernel may have without asking: said once per device and size)
-    static size_t sized[64] = {};
-    int device = 0;
-    hipError_t e = hipGetDevice(&device);
+    static LdsAllowed allowed;
+    const hipError_t e = allowed.say(reinterpret_cast<const void*>(k_lm_head_codes<WBITS>));
     if (e != hipSuccess) {
         return e;
-    }
-    if (device < 0 || device >= 64 || sized[device] < lds) {
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_lm_head_codes<WBITS>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) {
-            return e;
-        }
-        if (device >= 0 && device < 64) {
-            sized[device] = lds;
-        }
     }
     hipLaunchKernelGGL((k_lm_head_codes<WBITS>), dim3(tiles_per_row), dim3(THREADS), lds, stream,
                        static_cast<const uint16_t*>(hidden), hidden_stride, static_cast<const uint32_t*>(weight),
@@ -423,7 +411,7 @@ bool lm_head_codes_serves(uint32_t rows, uint32_t d, uint32_t vocab, uint64_t hi
     // read two at a time), all the tile's scales in LDS beside the stages
     const uint32_t stage_k = 128u * 8u / wq.bits, groups = d >> wq.group_shift;
     return d >= stage_k && d % stage_k == 0u && groups % 2u == 0u && (groups << wq.group_shift) == d &&
-           codes_lds_bytes(groups) <= 160u * 1024u;
+           codes_lds_bytes(groups) <= CU_LDS_BYTES;
 }
 
 hipError_t launch_lm_head_codes(hipStream_t stream, const void* hidden, uint64_t hidden_stride, const void* weight,

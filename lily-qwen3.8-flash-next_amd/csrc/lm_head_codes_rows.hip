@@ -20,7 +20,6 @@ namespace {
 constexpr int STEP_K = 64;                               // values of d between two barriers
 constexpr int CODE_BYTES = LILY_TILE_COLS * 128;         // a stage of codes: one line of every column
 constexpr int AHEAD = 2;                                 // stages of codes on their way in registers
-constexpr uint32_t LDS_BYTES = 160u * 1024u;             // of a compute unit
 
 inline uint32_t rows_lds_bytes(int mi, uint32_t groups) {
     return 2u * (uint32_t)mi * 32u * STEP_K * 2u + CODE_BYTES + LILY_TILE_COLS * groups * 4u;
@@ -309,14 +308,10 @@ static hipError_t launch_codes_rows(hipStream_t stream, const void* hidden, uint
                                     float* tile_sum, const HeadWeights& wq) {
     const uint32_t tiles_per_row = (vocab + LILY_TILE_COLS - 1u) / LILY_TILE_COLS, m_tiles = (rows + MI * 32u - 1u) / (MI * 32u);
     const uint32_t lds = rows_lds_bytes(MI, d >> wq.group_shift);
-    // (more than the 64 KB a kernel may have without asking: said on every launch that needs it, so
-    // that threads on several devices keep nothing between them)
-    if (lds > 64u * 1024u) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_lm_head_codes_rows<WBITS, MI>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
-        if (e != hipSuccess) {
-            return e;
-        }
+    static LdsAllowed allowed;
+    const hipError_t e = allowed.say(reinterpret_cast<const void*>(k_lm_head_codes_rows<WBITS, MI>));
+    if (e != hipSuccess) {
+        return e;
     }
     hipLaunchKernelGGL((k_lm_head_codes_rows<WBITS, MI>), dim3((tiles_per_row + 7u) / 8u * 8u * m_tiles), dim3(256), lds,
                        stream, static_cast<const uint16_t*>(hidden), hidden_stride, static_cast<const uint32_t*>(weight),
@@ -333,11 +328,11 @@ bool lm_head_codes_rows_serves(uint32_t d, const HeadWeights& wq) {
     // whole stages, and all the tile's scales in LDS beside the stages
     const uint32_t groups = d >> wq.group_shift;
     return d != 0u && d % (1024u / wq.bits) == 0u && groups >= 1u && (groups << wq.group_shift) == d &&
-           rows_lds_bytes(4, groups) <= LDS_BYTES;
+           rows_lds_bytes(4, groups) <= CU_LDS_BYTES;
 }
 
 uint32_t lm_head_codes_rows_resident(uint32_t d, const HeadWeights& wq) {
-    return LDS_BYTES / rows_lds_bytes(4, d >> wq.group_shift);
+    return CU_LDS_BYTES / rows_lds_bytes(4, d >> wq.group_shift);
 }
 
 hipError_t launch_lm_head_codes_rows(hipStream_t stream, const void* hidden, uint64_t hidden_stride, const void* weight,

@@ -11,6 +11,8 @@ Bar:
     log-probabilities within 1e-5 * max(1, |logprob|) - the same bar as lily_sample_rows, whose
     results the tiled draws must equal.
 """
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -917,6 +919,49 @@ def test_batches_in_either_form(monkeypatch, form, rows, d, vocab, slack):
         _check_product(h[keep], w, logits[keep], tmax[keep], tsum[keep], [temps[r] for r in keep])
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("rows", [4, 40])
+def test_two_threads_with_heads_of_different_widths(rows):
+    """Two threads, each with a sampler of its own, form heads over codes whose tiles want
+    different amounts of LDS (both above what a launch has without asking), in turn and at once:
+    every call is taken, and every result is the one a thread alone gets."""
+    vocab, calls = 300, 40
+    rng = np.random.default_rng(rows)
+
+    def job(d):
+        hidden = _bf16(rng.normal(0, 1, (rows, d)).astype(np.float32))
+        qw, dense, exact, summed = _quantised(rng, vocab, d, 4, 64)
+        return hidden, qw, (exact, summed) if rows <= 16 else (dense, None)
+
+    jobs, failed = [job(2048), job(8192)], []
+    tiles = (vocab + TILE - 1) // TILE
+    start = threading.Barrier(len(jobs))
+
+    def work(hidden, qw, ref):
+        s = LS.Sampler(0)
+        try:
+            out = [torch.zeros(rows, n, dtype=torch.float32, device=dev()) for n in (vocab, tiles, tiles)]
+            first = None
+            start.wait()
+            for i in range(calls):
+                s.lm_head(hidden, qw, [0.8] * rows, *out)
+                s.synchronize()
+                if first is None:
+                    first = [t.clone() for t in out]
+                    _check_f32_product(hidden, ref[0], *out, [0.8] * rows, summed=ref[1])
+                assert all(torch.equal(a, b) for a, b in zip(first, out)), i
+        except BaseException as e:   # noqa: BLE001 (reported by the test itself)
+            failed.append(e)
+        finally:
+            s.close()
+
+    threads = [threading.Thread(target=work, args=j) for j in jobs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed
 
 
 @pytest.mark.parametrize("bits", [4, 8])
