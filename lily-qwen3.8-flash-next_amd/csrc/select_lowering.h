@@ -431,13 +431,15 @@ __device__ __forceinline__ bool select_lowering(const RowArgs& a, const Geo<DT>&
                                 above += (uint32_t)__popcll(__ballot(v[j] > skip_b));
                             }
                         }
+                        // (red_i: what is written behind the scan could overtake a wave that still
+                        // reads here - a slice of one block has no barrier in between)
                         if (lane == 0) {
-                            sh.nfill[w] = above;
+                            sh.red_i[w] = above;
                         }
                         __syncthreads();
                         uint32_t all = 0;
                         for (int i = 0; i < NWAVE; ++i) {
-                            all += sh.nfill[i];
+                            all += sh.red_i[i];
                         }
                         if (all >= BLOCK * (uint32_t)E / 8u * 7u) {
                             // (nothing of the block has been queued or noted: it is scanned again)

@@ -87,3 +87,31 @@ def test_rows_whose_leading_ids_were_drawn_before(sampler, vocab, bf16, flat):
     for i in range(rows):
         assert np.array_equal(scratch[i].read_counts().numpy().view(np.uint32), counts[i])
         scratch[i].close()
+
+
+# One block a slice (8 192 bf16 / 4 096 f32 ids), either side of the share of elements above the
+# sum's cut - seven eighths - from which on a slice is taken as a flat one.
+@pytest.mark.parametrize("share", [0.0, 0.5, 0.86, 0.874, 0.876, 0.89, 1.0])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_slices_of_one_block_at_the_share_that_counts_as_flat(sampler, share, bf16):
+    slices = sampler.slices_for(1, 20, 1 << 20, bf16)
+    vocab = (8192 if bf16 else 4096) * slices
+    rng = np.random.default_rng(int(1000 * share) + bf16)
+    rows, temperature = 8, 0.4
+    # the cut lies (log2(V) + 21) T ln 2 below the largest value: 20 - 9.3 ... 9.9
+    x = rng.uniform(-9.0, 8.0, (rows, vocab)).astype(np.float32)
+    above = rng.permuted(np.tile(np.arange(vocab) < share * vocab, (rows, 1)), axis=1)
+    x[above] = rng.uniform(11.5, 19.0, int(above.sum())).astype(np.float32)
+    x[:, 77] = 20.0
+    x = W.to_bf16_bits(x) if bf16 else x
+    xf = W.bf16_bits_to_f32(x) if bf16 else x
+    scratch, counts = zip(*[_scratch(sampler, rng, vocab, np.argsort(-xf[r], kind="stable")[5:5 + 60 * r], "write")
+                            for r in range(rows)])
+    kw = [dict(temperature=temperature, top_k=20, top_p=0.95, repetition_penalty=1.05, presence_penalty=0.1,
+               frequency_penalty=0.01, seed=r) for r in range(rows)]
+    r = run_rows(sampler, x, kw, [3] * rows, scratch=list(scratch), logprobs=True)
+    for i in range(rows):
+        d = O.sample(xf[i], counts[i], o_params(**kw[i]), 3, want_logprob=True)
+        check_row_against_oracle(r, i, d)
+        assert abs(r.logprobs[i] - d.logprob) <= 1e-5 * max(1.0, abs(d.logprob)), (i, r.logprobs[i], d.logprob)
+        scratch[i].close()
