@@ -115,3 +115,34 @@ def test_slices_of_one_block_at_the_share_that_counts_as_flat(sampler, share, bf
         check_row_against_oracle(r, i, d)
         assert abs(r.logprobs[i] - d.logprob) <= 1e-5 * max(1.0, abs(d.logprob)), (i, r.logprobs[i], d.logprob)
         scratch[i].close()
+
+
+# Slices of 10 to 19 blocks (one of 7 with three slices) whose share of elements above the sum's cut
+# brings the notes from a tenth of their place to all of it within four blocks.
+@pytest.mark.parametrize("share", [0.02, 0.04, 0.06, 0.08, 0.1, 0.14, 0.3, 0.6, 0.86])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_notes_that_fill_up_are_handed_over_before_they_overflow(sampler, share, bf16):
+    vocab, rows, temperature = (151_936 if bf16 else 80_004), 4, 0.4
+    rng = np.random.default_rng(int(1000 * share) + bf16)
+    # the cut lies (log2(V) + 21) T ln 2 = 10.4 ... 10.6 below the largest value, which block 0 holds
+    x = rng.uniform(-9.0, 8.0, (rows, vocab)).astype(np.float32)
+    above = rng.random((rows, vocab)) < share
+    # (thinning out upwards: the queue of chunks above the k-th value is not what fills)
+    x[above] = np.minimum(11.5 + rng.exponential(0.7, int(above.sum())), 19.9).astype(np.float32)
+    x[:, 77] = 20.0
+    x = W.to_bf16_bits(x) if bf16 else x
+    xf = W.bf16_bits_to_f32(x) if bf16 else x
+    scratch, counts = zip(*[_scratch(sampler, rng, vocab, rng.permutation(vocab)[:500 * r], "write") for r in range(rows)])
+    kw = [dict(temperature=temperature, top_k=20, top_p=0.95, repetition_penalty=1.05, presence_penalty=0.1,
+               frequency_penalty=0.01, seed=r) for r in range(rows)]
+    stats = torch.zeros(4, dtype=torch.int32, device=dev())
+    sampler.set_path_stats(stats)
+    r = run_rows(sampler, x, kw, [3] * rows, scratch=list(scratch), logprobs=True)
+    sampler.set_path_stats(None)
+    for i in range(rows):
+        d = O.sample(xf[i], counts[i], o_params(**kw[i]), 3, want_logprob=True)
+        check_row_against_oracle(r, i, d)
+        assert abs(r.logprobs[i] - d.logprob) <= 1e-5 * max(1.0, abs(d.logprob)), (i, r.logprobs[i], d.logprob)
+        scratch[i].close()
+    # every slice by the streaming select, none of them twice (which would leave a reason here)
+    assert stats.tolist()[1:] == [0, 0, 0], stats.tolist()
