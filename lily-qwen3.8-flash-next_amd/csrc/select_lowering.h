@@ -104,29 +104,37 @@ __device__ __forceinline__ bool select_lowering(const RowArgs& a, const Geo<DT>&
     };
     const int32_t bit0 = (int32_t)(g.cb * (uint32_t)E) - (int32_t)g.pad;   // the slice's first chunk's first id
     const uint32_t bit_sh = (uint32_t)bit0 & 7u;
-    // The coarse map (a bit per eight ids, four words behind the bitmap): a block's chunks cover
-    // 32 of its words (16 for f32).  Lane i brings word i and the one behind it, so that whatever
-    // the slice's first bit, lane i holds the block's i-th 32 bits once shifted - and the bit
-    // before them: a chunk of a row that does not start on a multiple of eight ids lies in two
-    // groups of eight.  Words past the map's end are its last (of chunks that are not streamed).
-    constexpr uint32_t CWORDS = BLOCK * (uint32_t)E / 256u;
-    const int32_t cbit0 = (bit0 >> 3) - (DT == LILY_BF16 && g.pad == 0u ? 1 : 0);
-    const uint32_t cbit_sh = (uint32_t)cbit0 & 31u;
-    const int32_t cword_end = (int32_t)((g.vocab + 255u) / 256u);
-    const int32_t cword0 = (cbit0 >> 5) + (int32_t)min(lane, CWORDS - 1u);
+    // The coarse map (a bit per eight ids, four words behind the bitmap): the 64 chunks of a wave's
+    // load are CW consecutive words of it, read from any bit on, so the lanes of a wave bring the
+    // words of its four loads and the one behind each: lane u * CW + q (and every LANES-th from
+    // there on) word q of load u.  A chunk of a row that does not start on a multiple of eight ids
+    // lies in two groups of eight: its own bit and the next one.  Words past the map's end are its
+    // last (of chunks that are not streamed).
+    constexpr uint32_t CW = 64u * (uint32_t)E / 256u, CLANES = (uint32_t)U * CW;
+    const int32_t cbit0 = bit0 >> 3;
+    const uint32_t cbit_sh = (uint32_t)cbit0 & 31u, cbit_sh2 = cbit_sh + (DT == LILY_BF16 && g.pad != 0u ? 1u : 0u);
+    // (from the scratch's counts on, whose last words lie before the bitmap: offsets stay positive)
+    const char* maps = reinterpret_cast<const char*>(a.touched) - 16;
+    const uint32_t coarse_at = 16u + (row_words + LISTED_SPARE) * 4u;
+    const uint32_t coarse_last = coarse_at + (g.vocab + 255u) / 256u * 4u;
+    const uint32_t coarse_lane =
+        coarse_at + (uint32_t)((cbit0 >> 5) + (int32_t)((lane % CLANES / CW * NWAVE + w) * CW + lane % CW)) * 4u;
     auto fetch_coarse = [&](u32x4 (&dst)[U], Bits& d, uint32_t b) {
-        const int32_t at = min(cword0 + (int32_t)(b * CWORDS), cword_end);
-        fetch_bits(d, (int32_t)((row_words + LISTED_SPARE) * 4u) + at * 4);
+        const LILY_GLOBAL Bits8* from =
+            (const LILY_GLOBAL Bits8*)(maps + min(coarse_lane + b * (NWAVE * U * CW * 4u), coarse_last));
+        d.lo = from->lo;
+        d.hi = from->hi;
         fetch_row(dst, b);
     };
     // Whether this lane's chunk of load u may hold a listed id, from the block's coarse words.
     auto coarse_word = [&](const Bits& d) -> Bits {
-        const uint64_t v = (((uint64_t)d.hi << 32) | d.lo) >> cbit_sh;
         Bits r;
         if (DT == LILY_BF16) {
-            r.lo = (uint32_t)(v >> 1) | (g.pad != 0u ? (uint32_t)v : 0u);
+            r.lo = __builtin_amdgcn_alignbit(d.hi, d.lo, cbit_sh) |
+                   __builtin_amdgcn_alignbit(d.hi, cbit_sh2 == 32u ? d.hi : d.lo, cbit_sh2 & 31u);
             r.hi = 0u;
         } else {
+            const uint64_t v = (((uint64_t)d.hi << 32) | d.lo) >> cbit_sh;
             r.lo = (uint32_t)v;
             r.hi = (uint32_t)(v >> 32);
         }
@@ -134,14 +142,12 @@ __device__ __forceinline__ bool select_lowering(const RowArgs& a, const Geo<DT>&
     };
     auto coarse_hit = [&](const Bits& d, int u) -> bool {
         if (DT == LILY_BF16) {
-            const int at = u * 8 + (int)__builtin_amdgcn_readfirstlane((int)(w * 2u));
-            const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)d.lo, at);
-            const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)d.lo, at + 1);
+            const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)d.lo, 2 * u);
+            const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)d.lo, 2 * u + 1);
             return __builtin_amdgcn_inverse_ballot_w64(((uint64_t)hi << 32) | lo);
         }
-        const int at = u * 4 + (int)__builtin_amdgcn_readfirstlane((int)w);
-        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)d.lo, at);
-        const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)d.hi, at);
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)d.lo, u);
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)d.hi, u);
         const uint64_t v = ((uint64_t)hi << 32) | lo;
         return (((v >> ((bit_sh + 4u * lane) >> 3)) | (v >> ((bit_sh + 4u * lane + 3u) >> 3))) & 1ull) != 0ull;
     };
@@ -271,8 +277,9 @@ __device__ __forceinline__ bool select_lowering(const RowArgs& a, const Geo<DT>&
     };
     const float lse_cut = (log2f((float)g.vocab) + 21.0f) * (a.temperature * 0.6931471805599453f);
 
-    // Brings T up to date with everything the lanes have seen, the current block included.
-    auto refresh_bound = [&](bool first, bool maxima) {
+    // Brings T up to date with everything the lanes have seen, the current block included.  `count`:
+    // what the wave publishes beside it (its notes); returns the waves' sum of it.
+    auto refresh_bound = [&](bool first, bool maxima, uint32_t count) -> uint32_t {
         const uint32_t key16 = lane_max > NEG_INF ? (lilym_order_key(lane_max) >> 16) : 0u;
         const uint32_t P = wave_kth_key16(key16, kw);
         const float mine = P != 0u ? lilym_key_value(P << 16) : F32_LOWEST;
@@ -280,7 +287,7 @@ __device__ __forceinline__ bool select_lowering(const RowArgs& a, const Geo<DT>&
         if (lane == 0) {
             sh.bound[parity][w] = mine;
             sh.wfill[parity][w] = wq > QSEG || (!flat && sfill > SSEG) ? 1u : 0u;
-            sh.wnote[parity][w] = sfill;
+            sh.wnote[parity][w] = count;
             if (maxima) {
                 sh.wmax[parity][w] = wm;
             }
@@ -291,10 +298,12 @@ __device__ __forceinline__ bool select_lowering(const RowArgs& a, const Geo<DT>&
             t = fminf(t, sh.bound[parity][i]);
         }
         T = fmaxf(T, lower_by_slack(t));
+        uint32_t sum = 0;
         note_max = 0;
         for (int i = 0; i < NWAVE; ++i) {
             give_up = give_up || sh.wfill[parity][i] != 0u;
             note_max = max(note_max, sh.wnote[parity][i]);
+            sum += sh.wnote[parity][i];
         }
         if (maxima) {
             float m = sh.wmax[parity][0];
@@ -308,6 +317,7 @@ __device__ __forceinline__ bool select_lowering(const RowArgs& a, const Geo<DT>&
             }
         }
         parity ^= 1u;
+        return sum;
     };
 
     // Appends a chunk's number (within the slice) for the lanes of `mask` to the wave's notes.
@@ -383,16 +393,16 @@ __device__ __forceinline__ bool select_lowering(const RowArgs& a, const Geo<DT>&
                     block_max = max2_raw(block_max, m8[u]);
                 }
             }
-            float true_max = block_max;
-            if (!APART) {
+            if (APART) {
+                lane_max = max2_raw(lane_max, block_max);
+            } else {
                 const Bits words = coarse_word(bits);
-                true_max = NEG_INF;
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    true_max = max2_raw(true_max, coarse_hit(words, u) ? NEG_INF : m8[u]);
+                for (int u = 0; u < U; u += 2) {
+                    lane_max = max3_raw(lane_max, coarse_hit(words, u) ? NEG_INF : m8[u],
+                                        coarse_hit(words, u + 1) ? NEG_INF : m8[u + 1]);
                 }
             }
-            lane_max = max2_raw(lane_max, true_max);
             lane_raw = max2_raw(lane_raw, block_max);
             bool some = false;
             if (LSE && want_lse) {
@@ -417,16 +427,30 @@ __device__ __forceinline__ bool select_lowering(const RowArgs& a, const Geo<DT>&
             }
             if (b < 4u || (b & 3u) == 0u) {
                 const uint32_t noted = note_max;
-                refresh_bound(b == 0, b == 0 || (LSE && want_lse && (b < 4u || (b & 7u) == 0u)));
+                uint32_t count = sfill;
+                if (LSE && !APART && want_lse && b == 0u) {
+                    // (nothing is noted yet) chunks above the cut as this wave alone would place it:
+                    // no fewer than lie above the row's
+                    const float cut = wave_max_dpp(fmaxf(lane_max, lowered(lane_raw))) - lse_cut;
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        count += (uint32_t)__popcll(__ballot(m8[u] > cut));
+                    }
+                }
+                const uint32_t counted =
+                    refresh_bound(b == 0u, b == 0u || (LSE && want_lse && (b < 4u || (b & 7u) == 0u)), count);
                 if (LSE && want_lse) {
                     skip_b = fmaxf(row_max, own_max) - lse_cut;
                     wl.skip_below = skip_b;
                     some = some && __ballot(block_max > skip_b) != 0ull;
-                    if (!APART && b == 0u) {
-                        // Flat from the start?  Every wave counts its elements above the cut.  (Seven
-                        // eighths of them: a row with a heavy tail whose large values all come later
-                        // looks flat by half its elements, or by its chunks' maxima, one time in a
-                        // hundred, and then was the last of its launch by 12 us.)
+                    note_max = b == 0u ? 0u : note_max;
+                    if (!APART && b == 0u && counted >= BLOCK / 32u * 31u) {
+                        // Flat from the start?  Every wave counts its elements above the cut (where that
+                        // many chunks lie above).  31 of 32 of them: a row with a heavy tail whose large
+                        // values all come later holds seven eighths above its first block's cut one
+                        // time in two thousand, and then is the last of its launch by 12 us: one launch
+                        // in eight for 200 rows in three slices, 44.1 -> 45.7 us on average.  Flatter
+                        // rows than that (N(0, 2^2) at T 0.4: 92 %) come here by the notes' rate.
                         uint32_t above = 0;
 #pragma unroll
                         for (int u = 0; u < U; ++u) {
@@ -447,13 +471,13 @@ __device__ __forceinline__ bool select_lowering(const RowArgs& a, const Geo<DT>&
                         for (int i = 0; i < NWAVE; ++i) {
                             all += sh.red_i[i];
                         }
-                        if (all >= BLOCK * (uint32_t)E / 8u * 7u) {
+                        if (all >= BLOCK * (uint32_t)E / 32u * 31u) {
                             // (nothing of the block has been queued or noted: it is scanned again)
                             flat = true;
                             flat_from = 0u;
                             return;
                         }
-                    } else if (!APART) {
+                    } else if (!APART && b != 0u) {
                         // Would the fullest segment overflow before the next refresh, at a quarter
                         // more than the rate it grew at since the last one?  Then this block (not
                         // queued or noted yet) and those to come are scanned the other way; within
@@ -595,7 +619,7 @@ __device__ __forceinline__ bool select_lowering(const RowArgs& a, const Geo<DT>&
         }
     };
     if (nblocks == 0) {
-        refresh_bound(true, true);  // the same barriers in every workgroup
+        refresh_bound(true, true, 0u);  // the same barriers in every workgroup
     } else {
         if constexpr (FLAT) {
             // Where a slice comes here because its leading ids are listed ones by the hundred, what

@@ -90,8 +90,8 @@ def test_rows_whose_leading_ids_were_drawn_before(sampler, vocab, bf16, flat):
 
 
 # One block a slice (8 192 bf16 / 4 096 f32 ids), either side of the share of elements above the
-# sum's cut - seven eighths - from which on a slice is taken as a flat one.
-@pytest.mark.parametrize("share", [0.0, 0.5, 0.86, 0.874, 0.876, 0.89, 1.0])
+# sum's cut - 31 / 32 - from which on a slice is taken as a flat one.
+@pytest.mark.parametrize("share", [0.0, 0.5, 0.88, 0.96, 0.968, 0.97, 0.98, 1.0])
 @pytest.mark.parametrize("bf16", [False, True])
 def test_slices_of_one_block_at_the_share_that_counts_as_flat(sampler, share, bf16):
     slices = sampler.slices_for(1, 20, 1 << 20, bf16)
