@@ -105,6 +105,15 @@ __device__ __forceinline__ void apply_selection(RowArgs& a) {
     }
 }
 
+// The row's arguments once more (scalar loads, served by the scalar cache): kept in registers across
+// the scan, the fields that only the merge, the tail or a second attempt at the row uses crowd the
+// scan's own values out of the scalar registers.
+__device__ __forceinline__ void read_again(RowArgs& a, const LILY_CONST RowArgs* src) {
+    asm volatile("" : "+s"(src));
+    load_row_args(a, src);
+    apply_selection(a);
+}
+
 // Rows of select_lowering(): under penalties that can only lower a value, nothing else in play.
 __device__ __forceinline__ bool lowering_row(const RowArgs& a) {
     return (a.flags & F_PEN) != 0u && a.repetition >= 1.0f && a.presence >= 0.0f && a.frequency >= 0.0f &&
@@ -160,7 +169,13 @@ __device__ __forceinline__ void row_body(const LILY_CONST RowArgs* src, const La
                     __syncthreads();
                 }
                 if (again) {
-                    done = select_lowering<DT, LSE, true>(a, g, a.k, sh, cfg, again, sorted, found);
+                    RowArgs f = a;
+                    Geo<DT> fg = g;
+                    if constexpr (LSE) {
+                        read_again(f, src);
+                        fg.init(f.logits, vocab, s, S);
+                    }
+                    done = select_lowering<DT, LSE, true>(f, fg, f.k, sh, cfg, again, sorted, found);
                     if (!done) {
                         __syncthreads();
                     }
@@ -173,50 +188,58 @@ __device__ __forceinline__ void row_body(const LILY_CONST RowArgs* src, const La
             }
             took = done ? 0u : took;
         }
-        if (KIND == 1 && !done && cfg.path == 0u && a.allow != nullptr) {
-            done = select_sparse<DT, LSE>(a, g, a.k, cand, min(cfg.dyn_slots, MERGE_CAP), sh, sorted, cfg);
-            took = done ? 1u : took;
-        }
-        if (KIND != 2 && !done && cfg.path != 1u && cfg.bitmap_layout != 0u) {
-            const bool special = a.allow != nullptr || (a.flags & F_PEN) || a.n_bias != 0;
-            if (EXCL || !special) {
-                // A single pass whose running bound let too many candidates in is repeated
-                // as two passes (bound first, then collect) before the exhaustive select.
-#pragma nounroll
-                for (int attempt = 0; attempt < 2 && !done; ++attempt) {
-                    const bool two_pass = a.k > 64u || cfg.path == 2u || attempt == 1;
-                    if (attempt == 1) {
-                        __syncthreads();
-                    }
-                    done = select_fast<DT, EXCL, LSE>(a, g, a.k, two_pass, cand, cfg.cand_cap, excl, sh,
-                                                      cfg, sorted);
-                    if (a.k > 64u || cfg.path == 2u) {
-                        break;  // it was two passes already
-                    }
-                }
+        // The other selects.  Launches with row sums read the arguments afresh for them: kept across
+        // the streaming scan they made it spill (200 rows in three slices 46.7 -> 45.7 us).  Launches
+        // without hold fewer values and keep them; the order of the statement below is part of
+        // that (behind the exhaustive select it draws the merge's loads, and a wait for them, ahead
+        // of every row: 6.30 -> 6.50 us for one greedy row).
+        if (!LSE || !done) {
+            RowArgs f = a;
+            Geo<DT> fg = g;
+            if constexpr (LSE) {
+                read_again(f, src);
+                fg.init(f.logits, vocab, s, S);
+            }
+            if (KIND == 1 && !done && cfg.path == 0u && f.allow != nullptr) {
+                done = select_sparse<DT, LSE>(f, fg, f.k, cand, min(cfg.dyn_slots, MERGE_CAP), sh, sorted, cfg);
                 took = done ? 1u : took;
             }
+            if (KIND != 2 && !done && cfg.path != 1u && cfg.bitmap_layout != 0u) {
+                const bool special = f.allow != nullptr || (f.flags & F_PEN) || f.n_bias != 0;
+                if (EXCL || !special) {
+                    // A single pass whose running bound let too many candidates in is repeated
+                    // as two passes (bound first, then collect) before the exhaustive select.
+#pragma nounroll
+                    for (int attempt = 0; attempt < 2 && !done; ++attempt) {
+                        const bool two_pass = f.k > 64u || cfg.path == 2u || attempt == 1;
+                        if (attempt == 1) {
+                            __syncthreads();
+                        }
+                        done = select_fast<DT, EXCL, LSE>(f, fg, f.k, two_pass, cand, cfg.cand_cap, excl, sh,
+                                                          cfg, sorted);
+                        if (f.k > 64u || cfg.path == 2u) {
+                            break;  // it was two passes already
+                        }
+                    }
+                    took = done ? 1u : took;
+                }
+            }
+            if (!LSE && cfg.path_stats != nullptr && tid == 0) {
+                atomicAdd(&cfg.path_stats[took], 1u);
+            }
+            if (!done) {
+                __syncthreads();
+                sorted = false;
+                select_exhaustive<DT>(f, fg.id_lo, fg.id_hi, f.k, want_lse, cand, cfg.cand_cap, sh);
+            }
         }
-        if (cfg.path_stats != nullptr && tid == 0) {
+        if (LSE && cfg.path_stats != nullptr && tid == 0) {
             atomicAdd(&cfg.path_stats[took], 1u);
-        }
-        if (!done) {
-            __syncthreads();
-            sorted = false;
-            select_exhaustive<DT>(a, g.id_lo, g.id_hi, a.k, want_lse, cand, cfg.cand_cap, sh);
         }
     }
 
-    // What follows reads the row's arguments afresh (scalar loads, served by the scalar cache):
-    // kept in registers across the scan, the fields that only the merge and the tail use
-    // crowd the scan's own values out of the scalar registers.
     RowArgs t;
-    {
-        const LILY_CONST RowArgs* again = src;
-        asm volatile("" : "+s"(again));
-        load_row_args(t, again);
-        apply_selection(t);
-    }
+    read_again(t, src);
     const bool forced = (t.flags & F_FORCED) != 0;
     uint32_t n = (argmax || forced) ? 0u : min(sh.n_cand, cfg.cand_cap);
     phase(cfg, 4);
