@@ -407,8 +407,9 @@ bool lm_head_codes_serves(uint32_t rows, uint32_t d, uint32_t vocab, uint64_t hi
     if ((wq.bits != 4u && wq.bits != 8u) || rows < 1u || rows > 16u || wq.group_shift < 6u) {
         return false;
     }
-    // whole stages (128 bytes of codes a row), an even number of groups a row (their scales are
-    // read two at a time), all the tile's scales in LDS beside the stages
+    // whole stages (128 bytes of codes a row), all the tile's scales in LDS beside the stages, and an
+    // even number of groups a row: nothing here needs that, but heads with an odd one have always
+    // been multiplied by the weights in bf16, and their logits stay what they are
     const uint32_t stage_k = 128u * 8u / wq.bits, groups = d >> wq.group_shift;
     return d >= stage_k && d % stage_k == 0u && groups % 2u == 0u && (groups << wq.group_shift) == d &&
            codes_lds_bytes(groups) <= CU_LDS_BYTES;

@@ -1153,7 +1153,8 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
                 });
             }
         }
-        // Every other row (and a row whose pairs outgrew their place): one thread per queued chunk (the waves' segments counted through in order): its elements add their term and
+        // Every other row (and a row whose pairs outgrew their place): one thread per queued chunk
+        // (the waves' segments counted through in order): its elements add their term and
         // are offered - listed ones with their true value, ids of the bias list not at all (the
         // pass below speaks for them).
         for (uint32_t ch = tid; !paired && ch < total; ch += NT) {

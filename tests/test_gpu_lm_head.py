@@ -791,7 +791,7 @@ def _quantised(rng, vocab, d, bits, group):
             torch.from_numpy(exact).to(dev()), torch.from_numpy(summed).to(dev()))
 
 
-@pytest.mark.parametrize("bits,group", [(4, 64), (8, 64), (4, 32), (8, 128)])
+@pytest.mark.parametrize("bits,group", [(4, 64), (8, 64), (4, 32), (8, 32), (8, 128)])
 @pytest.mark.parametrize("rows", [1, 3, 16, 17, 40, 100, 300])
 def test_heads_of_affine_codes(sampler, bits, group, rows):
     """The reference's quantised head formats (QuantWeights, src/weights.rs:27-36; lm_head is 4 bits
@@ -828,12 +828,16 @@ def test_heads_of_affine_codes(sampler, bits, group, rows):
 
 @pytest.mark.parametrize("rows,d,vocab,bits,group", [
     (17, 512, 700, 4, 64), (32, 128, 64, 8, 64), (33, 1024, 129, 8, 128), (64, 256, 1000, 4, 64),
-    (65, 512, 333, 8, 64), (128, 768, 257, 4, 128), (129, 1536, 1160, 4, 64)])
+    (65, 512, 333, 8, 64), (128, 768, 257, 4, 128), (129, 1536, 1160, 4, 64),
+    (16, 768, 300, 4, 256), (20, 8192, 129, 8, 64), (64, 6144, 140, 4, 64), (65, 2560, 200, 8, 64),
+    (70, 4096, 300, 4, 64), (100, 14336, 130, 8, 64)])
 def test_tiles_of_codes_at_their_edges(sampler, rows, d, vocab, bits, group):
-    """More than 16 rows over codes, either side of each tile's rows (32, 64, 128), one stage of
-    codes, an odd and an even number of them, groups a row that are and are not a multiple of
-    eight (the scales' wide loads), a last tile of one column: the logits and summaries against
-    the f64 product with the weights as dequant_q4/q8_bf16 give them."""
+    """More than 16 rows over codes (fewer where a row has an odd number of groups), either side of
+    each tile's rows (32, 64, 128), one stage of codes, an odd and an even number of them, groups a
+    row that are and are not a multiple of eight (the scales' wide loads), scales that take a
+    launch past 64 KB of LDS and to all of a compute unit's (224 groups), a last tile of one
+    column: the logits and summaries against the f64 product with the weights as
+    dequant_q4/q8_bf16 give them."""
     rng = np.random.default_rng(rows + d + bits)
     hidden = rng.normal(0, 1, (rows, d)).astype(np.float32)
     qw, dense, _, _ = _quantised(rng, vocab, d, bits, group)
@@ -919,6 +923,54 @@ def test_batches_in_either_form(monkeypatch, form, rows, d, vocab, slack):
         _check_product(h[keep], w, logits[keep], tmax[keep], tsum[keep], [temps[r] for r in keep])
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("rows", [2, 17, 40, 100])
+def test_codes_that_are_no_whole_lines(sampler, bits, rows):
+    """d of 320, five groups of 64: no whole lines of codes at either width, so every number of rows
+    takes the tiles that bring codes through LDS."""
+    d, vocab = 320, 700
+    rng = np.random.default_rng(10 * rows + bits)
+    hidden = rng.normal(0, 1, (rows, d)).astype(np.float32)
+    qw, dense, _, _ = _quantised(rng, vocab, d, bits, 64)
+    temps = [0.5 + 0.1 * (r % 7) for r in range(rows)]
+    logits = torch.zeros(rows, vocab, dtype=torch.float32, device=dev())
+    tiles = (vocab + TILE - 1) // TILE
+    tmax = torch.zeros(rows, tiles, dtype=torch.float32, device=dev())
+    tsum = torch.zeros(rows, tiles, dtype=torch.float32, device=dev())
+    h = _bf16(hidden)
+    sampler.lm_head(h, qw, temps, logits, tmax, tsum)
+    sampler.synchronize()
+    _check_f32_product(h, dense, logits, tmax, tsum, temps)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("rows", [4, 20, 100])
+def test_scales_at_an_odd_address(sampler, bits, rows):
+    """Scales and biases two bytes past a multiple of 16, with a multiple of eight groups a row (what
+    the wide loads ask of the number alone): the same logits, bit for bit, as from aligned ones."""
+    d, vocab = 1024, 400
+    rng = np.random.default_rng(rows + bits)
+    h = _bf16(rng.normal(0, 1, (rows, d)).astype(np.float32))
+    qw, _, _, _ = _quantised(rng, vocab, d, bits, 64)
+
+    def odd(t):
+        buf = torch.zeros(t.numel() + 8, dtype=t.dtype, device=t.device)
+        view = buf[1:1 + t.numel()].view(t.shape)
+        view.copy_(t)
+        assert view.data_ptr() % 16 == 2 and view.is_contiguous()
+        return view
+
+    moved = LS.QuantWeights(qw.codes, odd(qw.scales), odd(qw.biases), 64, bits)
+    tiles = (vocab + TILE - 1) // TILE
+    got = []
+    for w in (qw, moved):
+        out = [torch.zeros(rows, n, dtype=torch.float32, device=dev()) for n in (vocab, tiles, tiles)]
+        sampler.lm_head(h, w, [0.8] * rows, *out)
+        sampler.synchronize()
+        got.append(out)
+    assert all(torch.equal(a, b) for a, b in zip(*got))
 
 
 @pytest.mark.parametrize("rows", [4, 40])
