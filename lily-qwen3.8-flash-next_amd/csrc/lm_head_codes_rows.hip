@@ -50,11 +50,13 @@ inline uint32_t rows_lds_bytes(int mi, uint32_t groups) {
 //
 // Before it, tiles that brought 4 or 8 bytes of codes and two 2-byte scales a thread and load (the
 // requests, not the bytes, were their bound) and turned each code into LDS.  V = 151 936, f32
-// logits, before and now: d = 4096, 8 bits, 20 rows 256 -> 152 us, 50 rows 428 -> 185, 100 rows
-// 502 -> 260, 200 rows 795 -> 468; 4 bits 357 -> 124, 258 -> 166, 439 -> 244, 723 -> 435.
-// What bounds it now is the vector unit (4 bits, 20 rows: 71 % of the cycles; without turning codes into
-// weights the launch takes 91 us of the 124, without its products all of them): 23 instructions
-// for eight 4-bit codes.  Tried and no faster: the conversion of two 8-bit floats an instruction
+// logits, before and now: d = 4096, 8 bits, 20 rows 256 -> 146 us, 50 rows 428 -> 169, 100 rows
+// 502 -> 237, 200 rows 795 -> 422; 4 bits 357 -> 123, 258 -> 165, 439 -> 224, 723 -> 398.
+// With 4 bits and few rows the vector unit bounds it (20 rows: 67 % of the cycles; in a first form
+// that took 124 us the launch without turning codes into weights took 91, without its products
+// 124): 23 instructions for eight 4-bit codes.  With 8 bits and 50 rows at d = 2560 nothing is
+// saturated (vector unit 47 %, products 23 %): 1 187 workgroups over 768 places are 1.55
+// generations, and each step of 64 has a barrier.  Tried on the first form and no faster: the conversion of two 8-bit floats an instruction
 // in place of four byte conversions (124 -> 122), codes as the denormal halves of a mixed-precision
 // FMA (124 -> 118, none for 8 bits, and it overflows for scales from 2^104 on), codes read out of
 // LDS a step ahead (none).

@@ -18,17 +18,16 @@ namespace lily {
 //     however many of the raw maxima the penalties take down.  (A bound of raw values with a slack
 //     of k / 8 + 2 was good until a row had drawn more than that many of its leading ids; every
 //     such row then went through the exhaustive select: 1 306 us a step instead of 140 for 200 rows
-//     of 248 320 bf16 logits over a decode of 4 000 steps; now 88.)
+//     of 248 320 bf16 logits over a decode of 4 000 steps; now 79 on a fresh history and 88 then.)
 //     Which chunks those are comes from a bit per eight ids that the scratch keeps beside its
-//     bitmap: 0.8 % of a bf16 row's bytes, one load a lane and block, and the 64 chunks of a wave's
+//     bitmap: 0.8 % of a bf16 row's bytes, eight lanes' load a block, and the 64 chunks of a wave's
 //     load are one 64-bit lane mask.  (With the bitmap itself beside the chunks - 6 % more bytes,
-//     a byte moved to every lane - the scan of 1 024 rows took 58.6 us instead of 53.3.)
+//     a byte moved to every lane - the scan of 1 024 rows took 58.6 us instead of 53.3; now 52.)
 //   * The largest of those maxima bounds the row's largest true value from below, and with it the
 //     cut below which nothing is summed.  The largest raw value under the penalty of the largest
 //     count, which used to bound it alone, is worthless once some id was drawn a hundred times
-//     (1 024 rows of 151 936 bf16 logits went
-//     from 75 to 190 us over 2 000 steps; now 75 to 80).  It still counts where it is the better
-//     one, as does the true value of the id counted most often.
+//     (1 024 rows of 151 936 bf16 logits went from 75 to 180 us over 2 000 steps; now 74 and 74).
+//     It still counts where it is the better one, as does the true value of the id counted most often.
 //   * Chunks are queued by their raw maxima and evaluated exactly behind the scan, chunks above
 //     the cut alone are noted (a number in LDS) and their terms formed behind the scan.
 //   * A flat row - most of its chunks lie above the cut - is not noted: from the first block on
