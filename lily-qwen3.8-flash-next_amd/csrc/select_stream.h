@@ -48,7 +48,7 @@ namespace lily {
 struct StreamLds {
     u32x4* qraw;
     uint32_t* qidx;
-    uint16_t* noted;    // [NWAVE][S_CAP / NWAVE] numbers (within the slice) of summed chunks
+    uint16_t* noted;    // [NWAVE][S_CAP / NWAVE] numbers (within the slice) of noted chunks
     uint32_t* win;      // [NWAVE][2][WIN_WORDS]
     float* blk_bound;   // [MAX_BLOCKS] the bound block b was filtered with
     float* blk_cut;     // [MAX_BLOCKS] the sum's cut of block b
