@@ -177,6 +177,14 @@ __device__ __forceinline__ bool select_lowering(const RowArgs& a, const Geo<DT>&
         }
         return all;
     };
+    // The chunks of block 0 that are streamed.  (Opaque: formed where it is asked for, not ahead of the
+    // scan, whose scalar registers it would hold.)
+    auto first_chunks = [&]() -> uint32_t {
+        uint32_t cb = g.cb;
+        asm volatile("" : "+s"(cb));
+        const uint32_t lo = max(g.main_lo, cb), hi = min(g.main_hi, cb + BLOCK);
+        return hi > lo ? hi - lo : 0u;
+    };
     auto full_block = [&](uint32_t b) -> bool {
         const uint32_t c0 = g.cb + b * BLOCK;
         return c0 >= g.main_lo && c0 + BLOCK <= g.main_hi;
@@ -443,26 +451,32 @@ __device__ __forceinline__ bool select_lowering(const RowArgs& a, const Geo<DT>&
                     wl.skip_below = skip_b;
                     some = some && __ballot(block_max > skip_b) != 0ull;
                     note_max = b == 0u ? 0u : note_max;
-                    if (!APART && b == 0u && counted >= BLOCK / 32u * 31u) {
-                        // Flat from the start?  Every wave counts its elements above the cut (where that
-                        // many chunks lie above).  31 of 32 of them: a row with a heavy tail whose large
-                        // values all come later holds seven eighths above its first block's cut one
-                        // time in two thousand, and then is the last of its launch by 12 us: one launch
-                        // in eight for 200 rows in three slices, 44.1 -> 45.7 us on average.  Flatter
-                        // rows than that (N(0, 2^2) at T 0.4: 92 %) come here by the notes' rate.
-                        uint32_t above = 0;
+                    if (!APART && b == 0u && counted * 8u >= first_chunks() * 7u) {
+                        // Flat from the start?  Every wave counts its elements above the cut (where
+                        // seven eighths of the block's chunks lie above): 31 of 32 of them, or seven
+                        // eighths and, for every 256, a chunk with a value in the upper quarter of the
+                        // way from the cut to the largest value.  A row with a heavy tail whose large values
+                        // all come later holds seven eighths above its first block's cut one time in
+                        // two thousand, but a dozen values in that quarter where a flat row holds
+                        // more than forty; taken for a flat one it is the last of its launch by 12 us
+                        // (one launch in eight for 200 rows in three slices, 44.1 -> 45.7 us on average).
+                        const float high = skip_b + 0.75f * lse_cut;
+                        // (Counted by the lanes: sums of ballots took scalar registers from the scan.)
+                        uint32_t above = 0;   // (and the chunks of the upper quarter in the upper half)
 #pragma unroll
                         for (int u = 0; u < U; ++u) {
                             float v[E];
                             unpack<DT>(cur[u], v);
 #pragma unroll
                             for (int j = 0; j < E; ++j) {
-                                above += (uint32_t)__popcll(__ballot(v[j] > skip_b));
+                                above += v[j] > skip_b ? 1u : 0u;
                             }
+                            above += m8[u] > high ? 0x10000u : 0u;
                         }
                         // (red_i: what is written behind the scan could overtake a wave that still
                         // reads here - a slice of one block has no barrier in between)
-                        if (lane == 0) {
+                        above = wave_scan_u32(above);
+                        if (lane == 63u) {
                             sh.red_i[w] = above;
                         }
                         __syncthreads();
@@ -470,7 +484,8 @@ __device__ __forceinline__ bool select_lowering(const RowArgs& a, const Geo<DT>&
                         for (int i = 0; i < NWAVE; ++i) {
                             all += sh.red_i[i];
                         }
-                        if (all >= BLOCK * (uint32_t)E / 32u * 31u) {
+                        const uint32_t held = first_chunks() * (uint32_t)E, low = all & 0xffffu;
+                        if (low * 32u >= held * 31u || (low * 8u >= held * 7u && (all >> 16) * 256u >= held)) {
                             // (nothing of the block has been queued or noted: it is scanned again)
                             flat = true;
                             flat_from = 0u;

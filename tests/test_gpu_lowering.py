@@ -89,19 +89,23 @@ def test_rows_whose_leading_ids_were_drawn_before(sampler, vocab, bf16, flat):
         scratch[i].close()
 
 
-# One block a slice (8 192 bf16 / 4 096 f32 ids), either side of the share of elements above the
-# sum's cut - 31 / 32 - from which on a slice is taken as a flat one.
-@pytest.mark.parametrize("share", [0.0, 0.5, 0.88, 0.96, 0.968, 0.97, 0.98, 1.0])
+# One block a slice (8 192 bf16 / 4 096 f32 ids, and less than a whole one), either side of the shares
+# of elements above the sum's cut - seven eighths with enough of them far up, 31 / 32 - from which on
+# a slice is taken as a flat one.
+@pytest.mark.parametrize("share", [0.0, 0.5, 0.87, 0.88, 0.96, 0.968, 0.97, 0.98, 1.0])
+@pytest.mark.parametrize("short,far_up", [(0, 1.0), (0, 0.002), (517, 1.0)])
 @pytest.mark.parametrize("bf16", [False, True])
-def test_slices_of_one_block_at_the_share_that_counts_as_flat(sampler, share, bf16):
+def test_slices_of_one_block_at_the_share_that_counts_as_flat(sampler, share, short, far_up, bf16):
     slices = sampler.slices_for(1, 20, 1 << 20, bf16)
-    vocab = (8192 if bf16 else 4096) * slices
+    vocab = (8192 if bf16 else 4096) * slices - short
     rng = np.random.default_rng(int(1000 * share) + bf16)
     rows, temperature = 8, 0.4
     # the cut lies (log2(V) + 21) T ln 2 below the largest value: 20 - 9.3 ... 9.9
     x = rng.uniform(-9.0, 8.0, (rows, vocab)).astype(np.float32)
     above = rng.permuted(np.tile(np.arange(vocab) < share * vocab, (rows, 1)), axis=1)
-    x[above] = rng.uniform(11.5, 19.0, int(above.sum())).astype(np.float32)
+    # (the upper quarter of the way to 20 begins at 17.5)
+    up = rng.random((rows, vocab)) < far_up
+    x[above] = np.where(up, rng.uniform(11.5, 19.0, (rows, vocab)), rng.uniform(11.5, 17.0, (rows, vocab)))[above]
     x[:, 77] = 20.0
     x = W.to_bf16_bits(x) if bf16 else x
     xf = W.bf16_bits_to_f32(x) if bf16 else x
