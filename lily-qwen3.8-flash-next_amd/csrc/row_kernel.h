@@ -314,37 +314,50 @@ __device__ __forceinline__ void row_body(const LILY_CONST RowArgs* src, const La
                     sh.lse_s = sum;
                 }
             }
-            // A bound of the k-th largest from the lanes' best entries (as in the streaming
-            // select: each wave's ceil(k / NWAVE)-th largest lane maximum, the minimum over the
-            // waves), then only entries at or above it are ranked.
-            uint64_t best_mine = 0;
-#pragma unroll
-            for (int q = 0; q < PER; ++q) {
-                best_mine = mine[q] > best_mine ? mine[q] : best_mine;
-            }
-            const uint32_t kw = (t.k + NWAVE - 1) / NWAVE;
-            const uint32_t P = kw <= 64u ? wave_kth_key16((uint32_t)(best_mine >> 48), kw) : 0u;
-            if ((tid & 63u) == 0) {
-                sh.red_i[tid >> 6] = P;
-            }
-            if (tid == 0) {
-                sh.n_cand = 0;
-            }
-            __syncthreads();
-            uint32_t bound = sh.red_i[0];
-            for (int i = 1; i < NWAVE; ++i) {
-                bound = min(bound, sh.red_i[i]);
-            }
-#pragma unroll
-            for (int q = 0; q < PER; ++q) {
-                if (mine[q] != 0ull && (uint32_t)(mine[q] >> 48) >= bound) {
-                    cand[atomicAdd(&sh.n_cand, 1u)] = mine[q];
+            bool ranked = false;
+            if constexpr (KIND != 2) {
+                // (many candidates: every entry goes into the sort as it is)
+                if (t.k > 64u && cfg.dyn_slots >= max(slots, SORT_SLOTS)) {
+                    sorted = wg_sort_topk(cand, mine, slots, t.k, sh, n);
+                    if (!sorted) {
+                        n = wg_select_topk(cand, slots, t.k, sh);
+                    }
+                    ranked = true;
                 }
             }
-            __syncthreads();
-            n = sh.n_cand;
-            sorted = false;
-            n = select_topk(cand, n, t.k, sh, sorted);
+            if (!ranked) {
+                // A bound of the k-th largest from the lanes' best entries (as in the streaming
+                // select: each wave's ceil(k / NWAVE)-th largest lane maximum, the minimum over the
+                // waves), then only entries at or above it are ranked.
+                uint64_t best_mine = 0;
+#pragma unroll
+                for (int q = 0; q < PER; ++q) {
+                    best_mine = mine[q] > best_mine ? mine[q] : best_mine;
+                }
+                const uint32_t kw = (t.k + NWAVE - 1) / NWAVE;
+                const uint32_t P = kw <= 64u ? wave_kth_key16((uint32_t)(best_mine >> 48), kw) : 0u;
+                if ((tid & 63u) == 0) {
+                    sh.red_i[tid >> 6] = P;
+                }
+                if (tid == 0) {
+                    sh.n_cand = 0;
+                }
+                __syncthreads();
+                uint32_t bound = sh.red_i[0];
+                for (int i = 1; i < NWAVE; ++i) {
+                    bound = min(bound, sh.red_i[i]);
+                }
+#pragma unroll
+                for (int q = 0; q < PER; ++q) {
+                    if (mine[q] != 0ull && (uint32_t)(mine[q] >> 48) >= bound) {
+                        cand[atomicAdd(&sh.n_cand, 1u)] = mine[q];
+                    }
+                }
+                __syncthreads();
+                n = sh.n_cand;
+                sorted = false;
+                n = select_topk<KIND != 2>(cand, n, t.k, sh, sorted, cfg.dyn_slots);
+            }
             found = cand;
         }
     }

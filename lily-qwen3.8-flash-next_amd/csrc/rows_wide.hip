@@ -377,12 +377,19 @@ __global__ __launch_bounds__(NT, 4) void k_wide_draw(InlineRows rows_arg, Launch
         return;
     }
     WIDE_MARK(7);
+    // The list's first entries are asked for together with its length: what lies behind its end is
+    // dropped (the slots are the workspace's whatever they hold).
+    constexpr int PER = MERGE_CAP / NT, FIRST = 8;
+    uint64_t mine_c[PER];
+#pragma unroll
+    for (int j = 0; j < FIRST; ++j) {
+        mine_c[j] = handed_load(cfg.ws_cand, (size_t)row * MERGE_CAP + tid + (uint32_t)j * NT);
+    }
+    const uint32_t total = load_through(&w.count[row]);
+    __syncthreads();   // (everybody has read it)
     if (tid == 0) {
-        sh.need = load_through(&w.count[row]);
         store_through(&w.count[row], 0u);
     }
-    __syncthreads();
-    const uint32_t total = sh.need;
     uint32_t n;
     bool sorted = false;
     if (total > MERGE_CAP) {
@@ -395,23 +402,16 @@ __global__ __launch_bounds__(NT, 4) void k_wide_draw(InlineRows rows_arg, Launch
             atomicAdd(&cfg.path_stats[2], 1u);
         }
     } else {
-        constexpr int PER = MERGE_CAP / NT;
-        for (int j0 = 0; j0 < PER; j0 += 8) {   // eight loads in flight
-            if ((uint32_t)j0 * NT >= total) {
-                break;
-            }
-            uint64_t got[8];
+        if (total > (uint32_t)FIRST * NT) {   // (the same in every thread)
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const uint32_t i = min((uint32_t)(j0 + u) * NT + tid, total - 1u);
-                got[u] = handed_load(cfg.ws_cand, (size_t)row * MERGE_CAP + i);
+            for (int j = FIRST; j < PER; ++j) {
+                mine_c[j] = handed_load(cfg.ws_cand, (size_t)row * MERGE_CAP + tid + (uint32_t)j * NT);
             }
+        }
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const uint32_t i = (uint32_t)(j0 + u) * NT + tid;
-                if (i < total) {
-                    cand[i] = got[u];
-                }
+        for (int j = 0; j < PER; ++j) {
+            if (tid + (uint32_t)j * NT >= total) {
+                mine_c[j] = 0ull;
             }
         }
         if (want_lse && tid < 64u) {
@@ -435,7 +435,10 @@ __global__ __launch_bounds__(NT, 4) void k_wide_draw(InlineRows rows_arg, Launch
         }
         __syncthreads();
         WIDE_MARK(13);
-        n = select_topk(cand, total, a.k, sh, sorted);
+        sorted = wg_sort_topk(cand, mine_c, total, a.k, sh, n);
+        if (!sorted) {
+            n = wg_select_topk(cand, total, a.k, sh);
+        }
         WIDE_MARK(14);
         if (cfg.path_stats != nullptr && tid == 0) {
             atomicAdd(&cfg.path_stats[1], 1u);

@@ -463,6 +463,9 @@ LaunchShape shape_of(const lily_sampler* s, const RowArgs* rows, uint32_t n, int
         sh.excl_words = masked ? (per * e + 31) / 32 + 2 : 0;
         const size_t extra = sh.excl ? ((size_t)sh.excl_words + SPECIAL_LIST_CAP) * 4 : 0;
         sh.dyn_bytes = (size_t)CAND_CAP * 8 + extra;
+        if (kmax > STREAM_K_MAX && sh.dyn_bytes < (size_t)SORT_SLOTS * 8) {
+            sh.dyn_bytes = (size_t)SORT_SLOTS * 8;   // what the sort of many candidates works in
+        }
     }
     if (any_stream && STREAM_LDS_BYTES > sh.dyn_bytes) {
         sh.dyn_bytes = STREAM_LDS_BYTES;

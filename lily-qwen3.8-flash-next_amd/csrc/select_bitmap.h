@@ -488,7 +488,7 @@ __device__ __forceinline__ bool select_fast(const RowArgs& a, const Geo<DT>& g, 
             return false;
         }
         sorted = false;
-        n = select_topk(cand, n, k, sh, sorted);  // also drops the zeros
+        n = select_topk<true>(cand, n, k, sh, sorted, cfg.dyn_slots);  // also drops the zeros
         // Every element that was not collected lies strictly below `filt`.  The result is
         // exact if k candidates were found and the k-th lies strictly above anything the
         // division could map an uncollected value to.

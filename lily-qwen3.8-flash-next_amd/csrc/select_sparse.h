@@ -137,6 +137,18 @@ __device__ __forceinline__ bool select_sparse(const RowArgs& a, const Geo<DT>& g
             ls[q] = load_logit<DT>(a.logits, ids[q]);
             cs[q] = pen ? gload(a.counts + ids[q]) : 0u;
         }
+        if (bias_lds) {
+            // (a pair is read once for the four ids; the additions keep the list's order)
+#pragma unroll 4
+            for (uint32_t j = 0; j < n_bias; ++j) {
+                const uint64_t e = cand[cap + j];
+                const float delta = lilym_bits_f32((uint32_t)(e >> 32));
+#pragma unroll
+                for (int q = 0; q < EB; ++q) {
+                    ls[q] = (uint32_t)e == ids[q] ? ls[q] + delta : ls[q];
+                }
+            }
+        }
 #pragma unroll
         for (int q = 0; q < EB; ++q) {
             const uint32_t i = i0 + (uint32_t)q * NT + tid;
@@ -144,22 +156,12 @@ __device__ __forceinline__ bool select_sparse(const RowArgs& a, const Geo<DT>& g
                 continue;
             }
             const uint32_t id = ids[q], c = cs[q];
-            float l = ls[q];
-            float u;
-            if (bias_lds) {
-                for (uint32_t j = 0; j < n_bias; ++j) {
-                    const uint64_t e = cand[cap + j];
-                    if ((uint32_t)e == id) {
-                        l += lilym_bits_f32((uint32_t)(e >> 32));
-                    }
-                }
-                if (c > 0u) {
-                    l = l > 0.0f ? l / a.repetition : l * a.repetition;
-                    l -= a.presence + a.frequency * (float)c;
-                }
-                u = l;
-            } else {
-                u = finish_pre_temperature(a, id, l, c, true);
+            float u = ls[q];
+            if (!bias_lds) {
+                u = finish_pre_temperature(a, id, u, c, true);
+            } else if (c > 0u) {
+                u = u > 0.0f ? u / a.repetition : u * a.repetition;
+                u -= a.presence + a.frequency * (float)c;
             }
             if (want_lse) {
                 lse.add_one(u, a.c2);
@@ -175,7 +177,15 @@ __device__ __forceinline__ bool select_sparse(const RowArgs& a, const Geo<DT>& g
     }
     SPARSE_MARK(13);
     sorted = false;
-    const uint32_t n = select_topk(cand, total, k, sh, sorted);
+    if (cfg.slices > 1u && total <= k) {
+        // (all of them go to the workgroup that merges the slices, which drops the zeros)
+        if (tid == 0) {
+            sh.n_cand = total;
+        }
+        __syncthreads();
+        return true;
+    }
+    const uint32_t n = select_topk<true>(cand, total, k, sh, sorted, cfg.dyn_slots);
     if (tid == 0) {
         sh.n_cand = n;
     }

@@ -305,7 +305,7 @@ __device__ __forceinline__ bool stream_accept(StreamLds& L, float filt, float te
         return stream_fail(cfg, 5u);
     }
     sorted = false;
-    n = select_topk(L.fc, n, k, sh, sorted);
+    n = select_topk<false>(L.fc, n, k, sh, sorted, 0u);
     phase(cfg, 12);
     if (filt > F32_LOWEST) {
         uint32_t lowest = 0xffffffffu;

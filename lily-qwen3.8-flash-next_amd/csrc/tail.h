@@ -463,41 +463,28 @@ __device__ __forceinline__ void tail(const RowArgs& a, uint32_t vocab, uint32_t 
     // place u, and adding p <= S rounds to m + floor(p / u) + (frac(p / u) > 1/2): integer
     // additions, which a wave sums in six data-parallel moves, exactly.  (p / u, its integer
     // part and its fraction are exact in f32: u is a power of two and p has no more bits than
-    // S.)  A block of 64 in which some fraction is exactly 1/2 (the rounding then depends on
-    // m's parity) or the sum leaves its binade - and the first block, whose sum starts at 0 -
-    // is added the slow way: a chain of 63 additions, each step adding the lane's value to the
-    // running sum of the lane below (a shift by one lane across the whole wave; lane 0 has no
-    // lane below and keeps what it has), after which every lane holds its final prefix.  The
-    // candidates' weights are at most 1 and the first is 1, so the sum crosses at most ten
-    // binades and a peaked row none.  (Restarting inside a block at the lane that leaves the
-    // binade, instead of giving the block to the chain, was slower: a round of the exact form
-    // costs a third of a chain, and a flat row then takes 25 rounds.)
+    // S.)  A fraction of exactly 1/2 rounds to the even neighbour, which depends on m: such lanes
+    // (one in 2^8 where p is eight binades below S) are settled one after the other behind the
+    // scan, each adding one or nothing to the lanes from its own on.  The scans do not need the sum
+    // ahead of them, only its binade: four blocks of 64 are scanned side by side, and what is left
+    // between one block and the next is an integer addition.  Where the sum leaves its binade, the
+    // entries before that one stand, the addition that crosses is made as it is, and the next group
+    // starts behind it.  The first block, whose sum starts at 0 and crosses binade after binade, is
+    // a chain of 63 additions, each step adding the lane's value to the running sum of the lane
+    // below (a shift by one lane across the whole wave; lane 0 has no lane below and keeps what it
+    // has), after which every lane holds its final prefix.  The candidates' weights are at most 1
+    // and the first is 1, so the sum crosses at most ten binades and a peaked row none.  (A block
+    // at a time, the chain for every block with a tie or a crossing: 4 to 6 us for 1 024 candidates.)
     if (tid < 64u) {
+        constexpr int G = 4;
         float carry = 0.0f;
-        for (uint32_t r0 = 0; r0 < k; r0 += 64u) {
-            const uint32_t i = r0 + tid;
-            const float p = i < k ? sh.prob[i] : 0.0f;
-            float run;
-            bool done = false;
+        for (uint32_t r0 = 0; r0 < k;) {
             const uint32_t sbits = lilym_f32_bits(carry), sexp = (sbits >> 23) & 0xffu;
-            // (a normal, positive sum whose last place and its inverse are normal numbers too)
-            if ((int32_t)sbits > 0 && sexp >= 24u && sexp <= 253u) {
-                const float inv_u = lilym_bits_f32((277u - sexp) << 23);   // 2^(23 - e)
-                const float u = lilym_bits_f32((sexp - 23u) << 23);        // 2^(e - 23)
-                const uint32_t m0 = (sbits & 0x7fffffu) | 0x800000u;
-                const float q = p * inv_u;
-                const uint32_t n = (uint32_t)q;
-                const float frac = q - (float)n;
-                const bool fits = p >= 0.0f && p <= carry;
-                const uint32_t m = m0 + wave_scan_u32(n + (frac > 0.5f ? 1u : 0u));
-                const uint32_t last = (uint32_t)__builtin_amdgcn_readlane((int)m, 63);
-                if (__ballot(frac == 0.5f || !fits) == 0ull && last < 0x1000000u) {
-                    run = (float)m * u;
-                    done = true;
-                }
-            }
-            if (!done) {
-                run = carry + p;  // final in lane 0
+            // (the first weight is 1, so the sum behind the first block is a normal number from 1 to
+            // 1 024 - or a NaN, of a row whose largest value is infinite, which the chain takes on)
+            if (r0 == 0u || sexp > 253u) {
+                const float p = r0 + tid < k ? sh.prob[r0 + tid] : 0.0f;
+                float run = carry + p;  // final in lane 0
 #pragma unroll
                 for (int j = 1; j < 64; ++j) {
                     // Two idle cycles between a lane's write and the neighbour's read of it.
@@ -505,11 +492,89 @@ __device__ __forceinline__ void tail(const RowArgs& a, uint32_t vocab, uint32_t 
                                  : "+v"(run)
                                  : "v"(p));
                 }
+                if (r0 + tid < k) {
+                    sh.cum[r0 + tid] = run;
+                }
+                carry = lilym_bits_f32((uint32_t)__builtin_amdgcn_readlane((int)lilym_f32_bits(run), 63));
+                r0 += 64u;
+                continue;
             }
-            if (i < k) {
-                sh.cum[i] = run;
+            const float inv_u = lilym_bits_f32((277u - sexp) << 23);   // 2^(23 - e)
+            const float u = lilym_bits_f32((sexp - 23u) << 23);        // 2^(e - 23)
+            uint32_t m0 = (sbits & 0x7fffffu) | 0x800000u;
+            float p[G];
+            uint32_t inc[G], sum[G];
+            uint64_t ties[G];
+            uint64_t any = 0;
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+                const uint32_t i = r0 + 64u * (uint32_t)q + tid;
+                const float got = sh.prob[min(i, k - 1u)];
+                p[q] = i < k ? got : 0.0f;
             }
-            carry = lilym_bits_f32((uint32_t)__builtin_amdgcn_readlane((int)lilym_f32_bits(run), 63));
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+                const float f = p[q] * inv_u;
+                const uint32_t n = (uint32_t)f;
+                const float frac = f - (float)n;
+                inc[q] = n + (frac > 0.5f ? 1u : 0u);
+                ties[q] = __ballot(frac == 0.5f);
+                any |= ties[q];
+            }
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+                inc[q] = wave_scan_u32(inc[q]);
+            }
+            uint32_t all = m0;
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+                sum[q] = (uint32_t)__builtin_amdgcn_readlane((int)inc[q], 63);
+                all += sum[q];
+            }
+            if (any == 0ull && all < 0x1000000u) {
+#pragma unroll
+                for (int q = 0; q < G; ++q) {
+                    const uint32_t i = r0 + 64u * (uint32_t)q + tid;
+                    if (i < k) {
+                        sh.cum[i] = (float)(m0 + inc[q]) * u;
+                    }
+                    m0 += sum[q];
+                }
+                carry = (float)m0 * u;
+                r0 += 64u * G;
+                continue;
+            }
+            bool going = true;   // the same in every lane
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+                if (going) {
+                    uint32_t m = m0 + inc[q];
+                    for (uint64_t t = ties[q]; t != 0ull; t &= t - 1ull) {
+                        const uint32_t l = (uint32_t)__builtin_ctzll(t);
+                        const uint32_t at = (uint32_t)__builtin_amdgcn_readlane((int)m, (int)l);
+                        m += tid >= l ? at & 1u : 0u;
+                    }
+                    const uint64_t over = __ballot(m >= 0x1000000u);   // (from the lane that crosses on)
+                    const uint32_t l = over != 0ull ? (uint32_t)__builtin_ctzll(over) : 64u;
+                    const uint32_t i = r0 + tid;
+                    if (tid < l && i < k) {
+                        sh.cum[i] = (float)m * u;
+                    }
+                    if (l != 0u) {
+                        m0 = (uint32_t)__builtin_amdgcn_readlane((int)m, (int)l - 1);
+                        carry = (float)m0 * u;
+                    }
+                    r0 += l;
+                    if (l < 64u) {
+                        carry += lilym_bits_f32((uint32_t)__builtin_amdgcn_readlane((int)lilym_f32_bits(p[q]), (int)l));
+                        if (tid == 0u && r0 < k) {
+                            sh.cum[r0] = carry;
+                        }
+                        r0 += 1u;
+                        going = false;
+                    }
+                }
+            }
         }
     }
     __syncthreads();

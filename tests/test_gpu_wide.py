@@ -249,3 +249,41 @@ def test_random_launches_of_rows_of_many_candidates(sampler):
                 assert np.array_equal(scratch[i].read_counts().numpy().view(np.uint32), counts[i]), (case, i)
                 scratch[i].close()
     assert went >= 30, went   # (a launch of one or two rows has too few slices for some k)
+
+
+@pytest.mark.parametrize("masked", [False, True], ids=["two-launches", "merged-slices"])
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+def test_sort_of_many_candidates(sampler, bf16, masked):
+    """The sort by counted bins where it can go wrong: candidates on both sides of zero, all below
+    it, an outlier that puts all others into one bin and a range past the
+    largest float (the radix select takes over), a bin of
+    just as many equal values as a bin may hold and one more, fewer than k candidates, and k just
+    above 64.  `masked`: about 3 000 allowed ids a row, whose four slices are merged."""
+    rng = np.random.default_rng(77 + bf16)
+    vocab = 151_936
+    x = np.full((8, vocab), -np.inf, dtype=np.float32)
+    some = rng.choice(vocab, 3000, replace=False)
+    x[0, some] = rng.normal(0, 1, 3000)
+    x[1, some] = -rng.random(3000) - 0.25
+    x[2, some] = rng.normal(3, 1, 3000)
+    x[2, some[0]] = 1.0e30
+    x[3, some] = rng.normal(0, 1, 3000)
+    x[3, some[1]] = 2.2e38
+    x[3, some[2]] = -2.2e38
+    x[4, some] = 1.0 + np.arange(3000) / 4096.0
+    x[4, some[500:628]] = 1.5
+    x[5] = x[4]
+    x[5, some[628]] = 1.5
+    x[6, some[:400]] = rng.normal(2, 3, 400)
+    x[7, some] = rng.standard_t(3, 3000) * 4
+    if bf16:
+        x = W.to_bf16_bits(x)
+    allow = np.zeros((8, (vocab + 31) // 32), dtype=np.uint32)
+    np.bitwise_or.at(allow, (slice(None), some >> 5), (1 << (some & 31)).astype(np.uint32))
+    for trial, k in enumerate((0, 65, 700)):
+        kw = [dict(temperature=1.0, top_k=k, top_p=0.98, seed=500 + r) for r in range(8)]
+        r = run_rows(sampler, x, kw, [trial] * 8, allow=allow if masked else None, logprobs=True)
+        for i in range(8):
+            d = O.sample(x[i], None, o_params(**kw[i]), trial, allow=allow[i] if masked else None, want_logprob=True)
+            check_row_against_oracle(r, i, d)
+            _check_logprob(r.logprobs[i], d.logprob, (k, i))
