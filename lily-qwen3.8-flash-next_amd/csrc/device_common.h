@@ -107,6 +107,42 @@ __device__ __forceinline__ bool last_to_arrive(uint32_t* ticket, uint32_t expect
     return last;
 }
 
+// The same for a wave that hands over by itself (all its stores its own, all 64 lanes at work): no
+// barrier, and the ticket's answer goes from lane to lane instead of through LDS.
+__device__ __forceinline__ bool wave_last_to_arrive(uint32_t* ticket, uint32_t expected, bool relaxed) {
+#ifdef LILY_STRICT_HANDOVER
+    relaxed = false;
+#endif
+    const bool first = (threadIdx.x & 63u) == 0u;
+    uint32_t t = 0;
+    if (relaxed) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_s_waitcnt(0);   // every counter at 0: the wave's stores have completed
+        if (first) {
+            t = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    } else {
+        // (the other lanes' stores happen before lane 0's release: one wave, one counter of stores,
+        // which the release waits for)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        if (first) {
+            t = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    const bool last = (uint32_t)__builtin_amdgcn_readfirstlane((int)t) == expected - 1u;
+    if (last) {
+        if (relaxed) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        } else {
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        }
+        if (first) {
+            store_through(ticket, 0u);
+        }
+    }
+    return last;
+}
+
 // Enters an id into a scratch's maps of listed ids (`words`: of the bitmap).
 __device__ __forceinline__ void mark_listed(uint32_t* touched, uint32_t words, uint32_t id) {
     atomicOr(&touched[id >> 5], 1u << (id & 31u));
@@ -209,12 +245,9 @@ __device__ __forceinline__ void exact_terms(const RowArgs& a, uint32_t lo, uint3
     }
 }
 
-__device__ __forceinline__ float wave_max_f(float v) {
-    for (int o = 32; o > 0; o >>= 1) {
-        v = fmaxf(v, __shfl_xor(v, o));
-    }
-    return v;
-}
+// Reductions over the 64 lanes of a wave, by moves inside the vector unit (DPP): through the LDS
+// crossbar (__shfl_xor) each of the six steps waits out an LDS access, twice for 64-bit values,
+// and nothing else in these small workgroups hides it (a row sum's merge 2.4 -> 1.7 us).
 // The wave's maximum in every lane, without LDS traffic: an inclusive running maximum inside
 // each row of 16 lanes by DPP row shifts (a lane whose source lies outside the row keeps its
 // own value), then the four row results read from lanes 15, 31, 47 and 63.
@@ -234,16 +267,10 @@ __device__ __forceinline__ float wave_max_dpp(float v) {
     const float r3 = lilym_bits_f32((uint32_t)__builtin_amdgcn_readlane(b, 63));
     return fmaxf(fmaxf(r0, r1), fmaxf(r2, r3));
 }
-__device__ __forceinline__ double wave_sum_d(double v) {
-    for (int o = 32; o > 0; o >>= 1) {
-        v += __shfl_xor(v, o);
-    }
-    return v;
-}
 // The wave's sum in every lane without LDS traffic: inclusive sums inside each row of 16 lanes
 // by DPP row shifts (a lane without such a neighbour adds 0), then the four rows' totals read
 // from lanes 15, 31, 47 and 63.
-__device__ __forceinline__ double wave_sum_d_dpp(double v) {
+__device__ __forceinline__ double wave_sum_d(double v) {
 #define LILY_ROW_SHR_ADD(n)                                                                      \
     {                                                                                            \
         const uint64_t b = __builtin_bit_cast(uint64_t, v);                                      \
@@ -266,25 +293,53 @@ __device__ __forceinline__ double wave_sum_d_dpp(double v) {
     }
     return t;
 }
-__device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int o) {
-    const uint32_t lo = __shfl_xor((uint32_t)v, o);
-    const uint32_t hi = __shfl_xor((uint32_t)(v >> 32), o);
-    return ((uint64_t)hi << 32) | lo;
+// The largest 64-bit value (BETTER(a, b): a is the one to keep) in every lane: running maxima inside
+// each row of 16 lanes, the last lane of row 0 into row 1 and of row 2 into row 3, lane 31 into
+// rows 2 and 3 (a lane without such a neighbour meets its own value), then lane 63's.
+template <class BETTER>
+__device__ __forceinline__ uint64_t wave_best_u64(uint64_t v, BETTER&& better) {
+#define LILY_BEST_FROM(ctrl, rows)                                                                                     \
+    {                                                                                                                  \
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp((int)(uint32_t)v, (int)(uint32_t)v, ctrl, rows, 0xf, false); \
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp((int)(uint32_t)(v >> 32), (int)(uint32_t)(v >> 32), ctrl,    \
+                                                                  rows, 0xf, false);                                   \
+        const uint64_t o = ((uint64_t)hi << 32) | lo;                                                                  \
+        v = better(o, v) ? o : v;                                                                                      \
+    }
+    LILY_BEST_FROM(0x111, 0xf)
+    LILY_BEST_FROM(0x112, 0xf)
+    LILY_BEST_FROM(0x114, 0xf)
+    LILY_BEST_FROM(0x118, 0xf)
+    LILY_BEST_FROM(0x142, 0xa)
+    LILY_BEST_FROM(0x143, 0xc)
+#undef LILY_BEST_FROM
+    return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), 63) << 32) |
+           (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, 63);
 }
 __device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) {
-    for (int o = 32; o > 0; o >>= 1) {
-        const uint64_t w = shfl_xor_u64(v, o);
-        v = w > v ? w : v;
-    }
-    return v;
+    return wave_best_u64(v, [](uint64_t x, uint64_t y) { return x > y; });
 }
-__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
-    for (int o = 32; o > 0; o >>= 1) {
-        const uint32_t w = __shfl_xor(v, o);
-        v = w < v ? w : v;
-    }
-    return v;
+__device__ __forceinline__ double wave_max_d(double v) {
+    return __builtin_bit_cast(double, wave_best_u64(__builtin_bit_cast(uint64_t, v), [](uint64_t x, uint64_t y) {
+                                  return __builtin_bit_cast(double, x) > __builtin_bit_cast(double, y) ||
+                                         __builtin_bit_cast(double, y) != __builtin_bit_cast(double, y);
+                              }));
 }
+// The same for 32-bit values.
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t x) {
+    int v = (int)x;
+#define LILY_MAX_FROM(ctrl, rows) v = (int)max((uint32_t)v, (uint32_t)__builtin_amdgcn_update_dpp(v, v, ctrl, rows, 0xf, false))
+    LILY_MAX_FROM(0x111, 0xf);
+    LILY_MAX_FROM(0x112, 0xf);
+    LILY_MAX_FROM(0x114, 0xf);
+    LILY_MAX_FROM(0x118, 0xf);
+    LILY_MAX_FROM(0x142, 0xa);
+    LILY_MAX_FROM(0x143, 0xc);
+#undef LILY_MAX_FROM
+    return (uint32_t)__builtin_amdgcn_readlane(v, 63);
+}
+__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) { return ~wave_max_u32(~v); }
+__device__ __forceinline__ int wave_max_i32(int v) { return (int)(wave_max_u32((uint32_t)v ^ 0x80000000u) ^ 0x80000000u); }
 
 // The value 4 order-key steps below t, not below the lowest finite float.
 __device__ __forceinline__ float lower_by_slack(float t) {
@@ -374,7 +429,7 @@ struct LseAcc {
 // Workgroup-wide merge of the threads' accumulators into sh.lse_mc / sh.lse_s.
 __device__ __forceinline__ void lse_reduce(Shared& sh, const LseAcc& l) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    float m = wave_max_f(l.mc);
+    float m = wave_max_dpp(l.mc);
     if (lane == 0) {
         sh.red_f[w] = m;
     }
@@ -418,20 +473,6 @@ __device__ __forceinline__ uint32_t wave_scan_u32(uint32_t x) {
     v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1, 3
     v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2, 3
     return (uint32_t)v;
-}
-
-// The wave's largest value in every lane: the running maximum by the same moves as the sums above.
-__device__ __forceinline__ uint32_t wave_max_u32_dpp(uint32_t x) {
-    int v = (int)x;
-#define LILY_MAX_FROM(ctrl, rows) v = (int)max((uint32_t)v, (uint32_t)__builtin_amdgcn_update_dpp(0, v, ctrl, rows, 0xf, false))
-    LILY_MAX_FROM(0x111, 0xf);
-    LILY_MAX_FROM(0x112, 0xf);
-    LILY_MAX_FROM(0x114, 0xf);
-    LILY_MAX_FROM(0x118, 0xf);
-    LILY_MAX_FROM(0x142, 0xa);
-    LILY_MAX_FROM(0x143, 0xc);
-#undef LILY_MAX_FROM
-    return (uint32_t)__builtin_amdgcn_readlane(v, 63);
 }
 
 // With sh.hist complete: finds the bin in which the count from bin 255 downwards
@@ -622,12 +663,13 @@ __device__ __forceinline__ uint32_t wg_rank_select(uint64_t* cand, uint32_t n, u
 // descending order at the front of cand, for k in the hundreds: a counting sort.  The entries' keys
 // (or values, where they lie on both sides of zero) are cut into BINS equal steps from the largest
 // down, the bins are counted and summed, every entry takes a place in its bin's stretch, and the
-// few that share a bin are ranked against each other.  Six barriers in all, none of the steps longer
-// than the longest bin.  (A radix select of 8-bit digits and a bitonic sort, 13 barriers of one and
-// 55 exchanges of the other, took 12.8 us for 1 024 of 1 200 f32 entries; this takes 4.)  False
-// where a bin that matters holds more than BIN_MAX entries (ties by the
-// hundred, an outlier that stretches the steps): the select that does not mind takes over; the entries
-// are then in cand[0..n), thread t's j-th at t + j * NT.  cand: at least SORT_SLOTS slots.
+// few that share a bin are ranked against each other.  Seven barriers, each step a chain of one or
+// two LDS accesses: latency bounds it (largest key and count 2.1 us, sums 0.9, places 1.1, ranks
+// 1.4).  A radix select of 8-bit digits and a bitonic sort, 13 barriers of one and 55 exchanges of
+// the other, took 12.8 us for 1 024 of 1 200 f32 entries where this takes 5.4.  False where a bin
+// that matters holds more than SORT_BIN_MAX entries (ties by the hundred, an outlier that stretches
+// the steps): the select that does not mind takes over; the entries are then in cand[0..n), thread
+// t's j-th at t + j * NT.  cand: at least SORT_SLOTS slots.
 constexpr uint32_t SORT_BIN_MAX = 128;
 __device__ __forceinline__ bool wg_sort_topk(uint64_t* cand, const uint64_t (&mine)[MERGE_CAP / NT], uint32_t n,
                                              uint32_t k, Shared& sh, uint32_t& n_out) {
@@ -644,8 +686,8 @@ __device__ __forceinline__ bool wg_sort_topk(uint64_t* cand, const uint64_t (&mi
         hi = max(hi, key);
         lo = mine[j] != 0ull ? min(lo, key) : lo;
     }
-    hi = wave_max_u32_dpp(hi);
-    lo = ~wave_max_u32_dpp(~lo);
+    hi = wave_max_u32(hi);
+    lo = ~wave_max_u32(~lo);
     __syncthreads();   // (cand and red_u may still be read)
     if (lane == 0) {
         sh.red_u[w] = ((uint64_t)hi << 32) | lo;
@@ -730,7 +772,7 @@ __device__ __forceinline__ bool wg_sort_topk(uint64_t* cand, const uint64_t (&mi
         at += h[i];
         h[i] = here;
     }
-    longest = wave_max_u32_dpp(longest);
+    longest = wave_max_u32(longest);
     if (lane == 0) {
         sh.red_u[w] = longest;
     }
@@ -1039,7 +1081,7 @@ struct WaveLse {
     __device__ __forceinline__ void add(const float (&v)[E], float m, float c) {
         if (__ballot(__builtin_fmaf(m, c, -ref) > LSE_RAISE) != 0ull) {
             // A term would dwarf the reference: raise it to the wave's maximum (rare).
-            const float nref = fmaxf(ref, wave_max_f(m * c));
+            const float nref = fmaxf(ref, wave_max_dpp(m * c));
             const float down = __builtin_amdgcn_exp2f(ref - nref);
             s *= down;
             booked *= down;
@@ -1057,7 +1099,7 @@ struct WaveLse {
     __device__ __forceinline__ void add_if(const float (&v)[E], float m, float c, bool active) {
         const float d = __builtin_fmaf(active ? m : NEG_INF, c, -ref);
         if (__ballot(d > LSE_RAISE) != 0ull) {
-            const float nref = fmaxf(ref, wave_max_f(active ? m * c : NEG_INF));
+            const float nref = fmaxf(ref, wave_max_dpp(active ? m * c : NEG_INF));
             const float down = __builtin_amdgcn_exp2f(ref - nref);
             s *= down;
             booked *= down;
@@ -1098,7 +1140,7 @@ struct WaveLse {
 // -inf, and the caller forms the row's sum again by the path that looks at every value).
 __device__ __forceinline__ bool wg_merge_lse(Shared& sh, float mc, float s_in, double& m_out, double& sum_out) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    float m = wave_max_f(s_in > 0.0f ? mc : NEG_INF);
+    float m = wave_max_dpp(s_in > 0.0f ? mc : NEG_INF);
     if (lane == 0) {
         sh.red_f[w] = m;
     }

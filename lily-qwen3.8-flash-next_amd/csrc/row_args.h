@@ -141,7 +141,9 @@ struct LaunchCfg {
     const uint32_t* served;
     // 1 = the slices' hand-over in its relaxed form (last_to_arrive() in device_common.h)
     uint32_t relaxed_handover;
-    uint32_t pad_cfg;
+    // 1 = the launch of a verify pass whose rows are independent: the kernel that holds the one-wave
+    // form of the speculative draw, and the acceptance behind the last row (accept_*, chain_ticket)
+    uint32_t verify;
 };
 
 constexpr uint32_t CHAIN_CAP = LILY_SAMPLE_K_CAP;   // candidates a chained row publishes

@@ -17,10 +17,10 @@ namespace lily {
 // ------------------------------------------------------------------ argmax
 
 // First maximum under float comparison (NaN never wins, -0 == +0), lowest id on
-// ties: elementwise.metal:145-150.  Result: the best (value, id) of the slice as a
-// composite; id bits all zero when no element qualified.
+// ties: elementwise.metal:145-150.  Result: the thread's best (value, id) of its share of the
+// slice as a composite; id bits all zero when no element qualified.
 template <int DT>
-__device__ __forceinline__ uint64_t slice_argmax(const RowArgs& a, const Geo<DT>& g, Shared& sh) {
+__device__ __forceinline__ uint64_t thread_argmax(const void* logits, const Geo<DT>& g) {
     constexpr int E = Geo<DT>::E;
     const uint32_t tid = threadIdx.x;
     float bv = NEG_INF;
@@ -40,9 +40,8 @@ __device__ __forceinline__ uint64_t slice_argmax(const RowArgs& a, const Geo<DT>
             for (int j = 0; j < E; ++j) {
                 const uint32_t id = g.id_of(c, j);
                 const bool inside = c >= g.main_lo && c < g.main_hi;
-                const float x = v[j];
-                if (inside && (x > bv || (x == bv && id < bi))) {
-                    bv = x;
+                if (inside && (v[j] > bv || (v[j] == bv && id < bi))) {   // (-inf counts: == on a first one)
+                    bv = v[j];
                     bi = id;
                 }
             }
@@ -52,17 +51,22 @@ __device__ __forceinline__ uint64_t slice_argmax(const RowArgs& a, const Geo<DT>
         const uint32_t lo = side == 0 ? g.id_lo : g.edge_hi_begin;
         const uint32_t hi = side == 0 ? g.edge_lo_end : g.id_hi;
         for (uint32_t id = lo + tid; id < hi; id += NT) {
-            const float x = load_logit<DT>(a.logits, id);
+            const float x = load_logit<DT>(logits, id);
             if (x > bv || (x == bv && id < bi)) {
                 bv = x;
                 bi = id;
             }
         }
     }
-    uint64_t best = ((uint64_t)lilym_order_key(bv + 0.0f) << 32) | (uint32_t)(~bi);
-    best = wave_max_u64(best);
-    if ((tid & 63u) == 0) {
-        sh.red_u[tid >> 6] = best;
+    return ((uint64_t)lilym_order_key(bv + 0.0f) << 32) | (uint32_t)(~bi);
+}
+
+// The workgroup's.
+template <int DT>
+__device__ __forceinline__ uint64_t slice_argmax(const RowArgs& a, const Geo<DT>& g, Shared& sh) {
+    uint64_t best = wave_max_u64(thread_argmax<DT>(a.logits, g));
+    if ((threadIdx.x & 63u) == 0) {
+        sh.red_u[threadIdx.x >> 6] = best;
     }
     __syncthreads();
     best = sh.red_u[0];
@@ -114,16 +118,197 @@ __device__ __forceinline__ void read_again(RowArgs& a, const LILY_CONST RowArgs*
     apply_selection(a);
 }
 
+// The control block behind an acceptance of `acc` proposals (spec.metal:14-38).
+__device__ __forceinline__ void write_accepted(const LaunchCfg& cfg, uint32_t acc) {
+    uint32_t* ctrl = cfg.accept_ctrl;
+    ctrl[0] = acc;
+    ctrl[LILY_CTRL_STRIDE] = acc + 1;
+    for (uint32_t i = 0; i < cfg.accept_chain; ++i) {
+        const uint32_t p = cfg.accept_pos0 + acc + 1 + i;
+        ctrl[(2 + 3 * i) * LILY_CTRL_STRIDE] = p;
+        ctrl[(3 + 3 * i) * LILY_CTRL_STRIDE] = p / cfg.accept_ratio;
+        ctrl[(4 + 3 * i) * LILY_CTRL_STRIDE] = ((p + 1) % cfg.accept_ratio == 0) ? 1u : 0u;
+    }
+}
+
+// One thread of the workgroup that finished a row of a verify pass (it stored the row's draw; out_of(j):
+// where row j's is): behind the last of them, the acceptance.
+template <class F>
+__device__ __forceinline__ void accept_behind_last_row(const LaunchCfg& cfg, F&& out_of) {
+    const uint32_t m = gridDim.y;
+    // (the release covers the draw, the acquire the other rows')
+    if (__hip_atomic_fetch_add(cfg.chain_ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) != m - 1u) {
+        return;
+    }
+    store_through(cfg.chain_ticket, 0u);
+    uint32_t drew[LILY_MAX_VERIFY_ROWS], given[LILY_MAX_VERIFY_ROWS];
+#pragma unroll
+    for (uint32_t j = 0; j < LILY_MAX_VERIFY_ROWS; ++j) {
+        drew[j] = load_through(out_of(min(j, m - 1u)));
+        given[j] = gload(cfg.accept_ids + min(j, m - 1u));
+    }
+    uint32_t acc = 0;
+    bool same = true;
+#pragma unroll
+    for (uint32_t j = 0; j + 1u < LILY_MAX_VERIFY_ROWS; ++j) {
+        same = same && j + 1u < m && drew[j] == given[j + 1u];
+        acc += same ? 1u : 0u;
+    }
+    write_accepted(cfg, acc);
+}
+
 // Rows of select_lowering(): under penalties that can only lower a value, nothing else in play.
 __device__ __forceinline__ bool lowering_row(const RowArgs& a) {
     return (a.flags & F_PEN) != 0u && a.repetition >= 1.0f && a.presence >= 0.0f && a.frequency >= 0.0f &&
            a.allow == nullptr && a.n_bias == 0u;
 }
 
-template <int DT, int KIND, bool LSE, bool CHAIN = false>
-__device__ __forceinline__ void row_body(const LILY_CONST RowArgs* src, const LaunchCfg& cfg, Shared& sh) {
+// What a row of few candidates (k <= 64) that several workgroups scanned has left to do once each of
+// them knows its own best: the workgroup's first wave does it all, without a barrier - the others have
+// nothing left to do and are gone.  It stores its candidates, takes the row's ticket and, if it is the
+// last, gathers every slice's, keeps the row's best (a candidate per lane, in order) and draws.
+// (With the workgroup's four waves meeting at eight barriers from here to the draw: 7.6 us of the 13.2
+// that one sampled row of 151 936 f32 logits takes in 38 slices; now 6 of 12.1.)
+constexpr uint32_t WAVE_MERGE_SLOTS = 2048;   // entries the wave gathers at most, 32 a lane
+constexpr uint32_t WAVE_MERGE_LISTS = 8;      // up to this many slices their lists are merged one by one
+
+__device__ __forceinline__ bool descending(uint64_t c) {   // lane by lane, equal only where both are 0
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)(uint32_t)c, 0x138, 0xf, 0xf, false);   // wave_shr:1
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)(uint32_t)(c >> 32), 0x138, 0xf, 0xf, false);
+    return __ballot((((uint64_t)hi << 32) | lo) < c) == 0ull;
+}
+
+template <int DT, bool LSE, bool SPEC>
+__device__ __forceinline__ bool finish_by_wave(const RowArgs& t, const LaunchCfg& cfg, uint32_t row, uint32_t s, uint32_t n,
+                                               const uint64_t* found, uint32_t step, bool want_lse, Shared& sh) {
+    const uint32_t lane = threadIdx.x, S = cfg.slices, vocab = cfg.vocab;
+    const bool forced = (t.flags & F_FORCED) != 0u;
+    const size_t slot = (size_t)row * S + s;
+    // Every place is written (0 = no candidate), so the merge needs no counts.
+    for (uint32_t i = lane; !forced && i < cfg.ws_k; i += 64u) {
+        handed_store(cfg.ws_cand, slot * cfg.ws_k + i, i < n ? found[i] : (uint64_t)0);
+    }
+    if (LSE && lane == 0u) {
+        handed_store(cfg.ws_lse, 2 * slot, want_lse ? sh.lse_mc : 0.0);
+        handed_store(cfg.ws_lse, 2 * slot + 1, want_lse ? sh.lse_s : 0.0);
+    }
+    const bool last = wave_last_to_arrive(&cfg.ws_ticket[row], S, cfg.relaxed_handover != 0u);
+    phase(cfg, 5);
+    if (!last) {
+        return false;
+    }
+    uint32_t spec_d = 0, spec_qn = 0;
+    if (SPEC && t.mode == MODE_SPEC) {
+        spec_d = *t.draft;
+        spec_qn = *t.q_n;
+    }
+    const size_t base = (size_t)row * S;
+    double mt = -__builtin_huge_val(), st = 0.0;
+    if (LSE && want_lse && lane < S) {
+        mt = handed_load(cfg.ws_lse, 2 * (base + lane));
+        st = handed_load(cfg.ws_lse, 2 * (base + lane) + 1);
+    }
+    uint64_t best = 0ull;   // the row's best, a lane each, in order
+    if (!forced && S <= WAVE_MERGE_LISTS) {
+        // Few lists, each in order as a rule: one after the other into the best so far.
+        uint64_t list[WAVE_MERGE_LISTS];
+#pragma unroll
+        for (uint32_t q = 0; q < WAVE_MERGE_LISTS; ++q) {
+            const uint32_t from = min(q, S - 1u), at = min(lane, cfg.ws_k - 1u);
+            list[q] = handed_load(cfg.ws_cand, (base + from) * cfg.ws_k + at);
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < WAVE_MERGE_LISTS; ++q) {
+            if (q < S) {
+                uint64_t c = lane < cfg.ws_k ? list[q] : 0ull;
+                if (!descending(c)) {
+                    c = wave_sort_desc(c);
+                }
+                best = q == 0u ? c : wave_merge_desc(best, c);
+            }
+        }
+    } else if (!forced) {
+        constexpr int PER = WAVE_MERGE_SLOTS / 64, GROUP = 8;
+        const uint32_t slots = S * cfg.ws_k;
+        uint64_t mine[PER];
+#pragma unroll
+        for (int q0 = 0; q0 < PER; q0 += GROUP) {
+            if ((uint32_t)q0 * 64u < slots) {
+#pragma unroll
+                for (int q = q0; q < q0 + GROUP; ++q) {
+                    mine[q] = handed_load(cfg.ws_cand, base * cfg.ws_k + min(lane + (uint32_t)q * 64u, slots - 1u));
+                }
+            }
+        }
+        uint64_t lane_best = 0ull;
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            mine[q] = lane + (uint32_t)q * 64u < slots ? mine[q] : 0ull;
+            lane_best = mine[q] > lane_best ? mine[q] : lane_best;
+        }
+        // k lanes' best reach the bound, so k entries do; what does not is dropped, the rest is
+        // listed, and the list's entries are taken in 64 at a time.
+        const uint32_t bound = wave_kth_key16((uint32_t)(lane_best >> 48), t.k);
+        uint64_t* cand = dyn_lds;
+        uint32_t kept = 0;
+#pragma unroll
+        for (int q0 = 0; q0 < PER; q0 += GROUP) {
+            if ((uint32_t)q0 * 64u < slots) {
+#pragma unroll
+                for (int q = q0; q < q0 + GROUP; ++q) {
+                    const bool in = mine[q] != 0ull && (uint32_t)(mine[q] >> 48) >= bound;
+                    const uint64_t mask = __ballot(in);
+                    if (mask != 0ull) {
+                        const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
+                            (uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+                        if (in) {
+                            cand[kept + rank] = mine[q];
+                        }
+                        kept += (uint32_t)__popcll(mask);
+                    }
+                }
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // (LDS of this wave: in order already)
+        __builtin_amdgcn_wave_barrier();
+        for (uint32_t i = 0; i < kept; i += 64u) {
+            const uint64_t c = wave_sort_desc(i + lane < kept ? cand[i + lane] : 0ull);
+            best = i == 0u ? c : wave_merge_desc(best, c);
+        }
+    }
+    if (LSE && want_lse) {
+        const bool some = st > 0.0;
+        const double m = wave_max_d(some ? mt : -__builtin_huge_val());
+        const double sum = wave_sum_d(some ? st * exp2(mt - m) : 0.0);
+        if (lane == 0u) {
+            sh.lse_mc = m;
+            sh.lse_s = sum;
+        }
+    }
+    phase(cfg, 6);
+    if (forced) {
+        if (lane == 0u) {
+            finish_token<DT>(t, sh, t.forced, vocab);
+        }
+        return true;
+    }
+    best = lane < t.k ? best : 0ull;
+    const uint32_t have = (uint32_t)__popcll(__ballot(best != 0ull));
+    if (have == 0u) {
+        if (lane == 0u) {
+            finish_empty(t, vocab, sh, cfg);
+        }
+        return true;
+    }
+    tail_wave<DT, SPEC>(t, vocab, step, best, have, sh, cfg, spec_d, spec_qn);
+    return true;
+}
+
+// True in the workgroup that finishes the row (the last of its slices to arrive).
+template <int DT, int KIND, bool LSE, bool CHAIN = false, bool SPEC = false>
+__device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const LaunchCfg& cfg, Shared& sh) {
     if (cfg.served != nullptr && *(const LILY_CONST uint32_t*)(cfg.served + blockIdx.y) != 0u) {
-        return;
+        return false;
     }
     RowArgs a;
     load_row_args(a, src);
@@ -144,7 +329,7 @@ __device__ __forceinline__ void row_body(const LILY_CONST RowArgs* src, const La
         if (s == 0 && tid == 0) {
             emit(a, a.forced, vocab);
         }
-        return;
+        return s == 0;
     }
 
     Geo<DT> g;
@@ -243,6 +428,18 @@ __device__ __forceinline__ void row_body(const LILY_CONST RowArgs* src, const La
     const bool forced = (t.flags & F_FORCED) != 0;
     uint32_t n = (argmax || forced) ? 0u : min(sh.n_cand, cfg.cand_cap);
     phase(cfg, 4);
+    if (!CHAIN && S > 1 && !argmax && t.k <= 64u && cfg.ws_k <= 64u &&
+        (S <= WAVE_MERGE_LISTS || S * cfg.ws_k <= WAVE_MERGE_SLOTS) &&
+        (t.mode != MODE_SPEC || (SPEC && *t.q_n <= 64u))) {
+        if (tid >= 64u) {
+            return false;
+        }
+        const bool finished = finish_by_wave<DT, LSE, SPEC>(t, cfg, row, s, n, found, step, want_lse, sh);
+        if (finished) {
+            phase(cfg, 7);
+        }
+        return finished;
+    }
     if (S > 1) {
         const size_t slot = (size_t)row * S + s;
         // Partials go through to memory (no dirty L2 lines to write back), the wave waits
@@ -266,7 +463,7 @@ __device__ __forceinline__ void row_body(const LILY_CONST RowArgs* src, const La
         const bool last = last_to_arrive(&cfg.ws_ticket[row], S, sh.last, cfg.relaxed_handover != 0u);
         phase(cfg, 5);
         if (!last) {
-            return;
+            return false;
         }
         const size_t base = (size_t)row * S;
         if (argmax) {
@@ -304,10 +501,7 @@ __device__ __forceinline__ void row_body(const LILY_CONST RowArgs* src, const La
                         mt = -__builtin_huge_val();
                     }
                 }
-                double m = mt;
-                for (int o = 32; o > 0; o >>= 1) {
-                    m = fmax(m, __shfl_xor(m, o));
-                }
+                const double m = wave_max_d(mt);
                 const double sum = wave_sum_d(st > 0.0 ? st * exp2(mt - m) : 0.0);
                 if (tid == 0) {
                     sh.lse_mc = m;
@@ -368,13 +562,13 @@ __device__ __forceinline__ void row_body(const LILY_CONST RowArgs* src, const La
             const uint32_t id = composite_id(best);
             *t.out_id = id == 0xffffffffu ? 0u : id;
         }
-        return;
+        return true;
     }
     if (t.flags & F_FORCED) {
         if (tid == 0) {
             finish_token<DT>(t, sh, t.forced, vocab);
         }
-        return;
+        return true;
     }
     if (CHAIN && cfg.chain_rows != 0u) {
         // Rows that draw in order.  This row's candidates - the best t.k under the counts as they
@@ -391,7 +585,7 @@ __device__ __forceinline__ void row_body(const LILY_CONST RowArgs* src, const La
             handed_store(cfg.chain_n, row, n);
         }
         if (!last_to_arrive(cfg.chain_ticket, rows, sh.last, cfg.relaxed_handover != 0u)) {
-            return;
+            return false;
         }
         const LILY_CONST RowArgs* first = src - row;
         if (cfg.accept_ctrl != nullptr && tid < rows) {
@@ -549,21 +743,14 @@ __device__ __forceinline__ void row_body(const LILY_CONST RowArgs* src, const La
             while (acc + 1 < rows && sh.drawn[acc] == sh.proposal[acc + 1]) {
                 ++acc;
             }
-            uint32_t* ctrl = cfg.accept_ctrl;
-            ctrl[0] = acc;
-            ctrl[LILY_CTRL_STRIDE] = acc + 1;
-            for (uint32_t i = 0; i < cfg.accept_chain; ++i) {
-                const uint32_t p = cfg.accept_pos0 + acc + 1 + i;
-                ctrl[(2 + 3 * i) * LILY_CTRL_STRIDE] = p;
-                ctrl[(3 + 3 * i) * LILY_CTRL_STRIDE] = p / cfg.accept_ratio;
-                ctrl[(4 + 3 * i) * LILY_CTRL_STRIDE] = ((p + 1) % cfg.accept_ratio == 0) ? 1u : 0u;
-            }
+            write_accepted(cfg, acc);
         }
         phase(cfg, 7);
-        return;
+        return true;
     }
-    tail<DT, KIND != 2>(t, vocab, step, n, sorted, found, sh, cfg);
+    tail<DT, KIND != 2, SPEC>(t, vocab, step, n, sorted, found, sh, cfg);
     phase(cfg, 7);
+    return true;
 }
 
 // Dynamic LDS: [0, cand_cap) candidates while scanning, then the bitmap.  In the tail the
@@ -603,6 +790,25 @@ __global__ __launch_bounds__(NT, KIND == 1 ? 3 : 4) void k_rows_chain(InlineRows
     row_body<DT, KIND, false, true>(table + blockIdx.y, cfg, sh);
 }
 
+// A verify pass whose rows are independent: the one-wave form of the speculative draw is compiled in,
+// and the workgroup that finishes the last row runs spec_accept (spec.metal:14-38) on the draws - a
+// launch of its own behind this one took 3.9 us of a step of three rows.
+template <int DT, int KIND>
+__global__ __launch_bounds__(NT, KIND == 1 ? 3 : 4) void k_rows_verify(InlineRows rows, LaunchCfg cfg) {
+    __shared__ Shared sh;
+    const LILY_CONST RowArgs* table =
+        (const LILY_CONST RowArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    if (threadIdx.x == 0) {
+        tail_arrays(sh);
+    }
+    __syncthreads();
+    const bool finished = row_body<DT, KIND, false, false, true>(table + blockIdx.y, cfg, sh);
+    if (!finished || threadIdx.x != 0 || cfg.accept_ctrl == nullptr) {
+        return;
+    }
+    accept_behind_last_row(cfg, [&](uint32_t j) { return (table + j)->out_id; });
+}
+
 template <int DT, int KIND, bool LSE>
 __global__ __launch_bounds__(NT, KIND == 1 ? 3 : 4) void k_rows_table(LaunchCfg cfg) {
     __shared__ Shared sh;
@@ -626,6 +832,15 @@ static hipError_t launch_variant(hipStream_t stream, uint32_t rows, const Launch
             }
         }
         return hipErrorInvalidValue;   // rows that draw in order travel inline and want no row sum
+    }
+    if (cfg.verify != 0u) {
+        if constexpr (!LSE) {
+            if (inline_rows != nullptr) {
+                hipLaunchKernelGGL((k_rows_verify<DT, KIND>), grid, block, dyn_bytes, stream, *inline_rows, cfg);
+                return hipGetLastError();
+            }
+        }
+        return hipErrorInvalidValue;   // (the same of a verify pass)
     }
     if (inline_rows != nullptr) {
         hipLaunchKernelGGL((k_rows_inline<DT, KIND, LSE>), grid, block, dyn_bytes, stream,

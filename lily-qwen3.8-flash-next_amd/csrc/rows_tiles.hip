@@ -134,7 +134,7 @@ __global__ __launch_bounds__(NT, 4) void k_rows_tiles(LaunchCfg cfg, const float
         }
         best = fmaxf(best, ms[j]);
     }
-    best = wave_max_f(best);
+    best = wave_max_dpp(best);
     if (lane == 0) {
         sh.red_f[w] = best;
     }

@@ -423,10 +423,7 @@ __global__ __launch_bounds__(NT, 4) void k_wide_draw(InlineRows rows_arg, Launch
                     mt = -__builtin_huge_val();
                 }
             }
-            double m = mt;
-            for (int o = 32; o > 0; o >>= 1) {
-                m = fmax(m, __shfl_xor(m, o));
-            }
+            const double m = wave_max_d(mt);
             const double sum = wave_sum_d(st > 0.0 ? st * exp2(mt - m) : 0.0);
             if (tid == 0) {
                 sh.lse_mc = m;

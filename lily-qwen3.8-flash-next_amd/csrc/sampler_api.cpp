@@ -561,7 +561,7 @@ int launch_part(lily_sampler* s, const LaunchPart& part, const RowArgs* table_de
     return LILY_OK;
 }
 
-// What spec_accept needs when the launch that draws the rows in order also runs it.
+// What spec_accept needs when the launch that draws a verify pass's rows also runs it.
 struct AcceptArgs {
     uint32_t* ctrl = nullptr;
     const uint32_t* ids = nullptr;
@@ -569,11 +569,11 @@ struct AcceptArgs {
 };
 
 int launch_inline(lily_sampler* s, int dtype, uint32_t vocab, const InlineRows& rows, uint32_t n,
-                  bool chained = false, const AcceptArgs& accept = AcceptArgs()) {
+                  bool chained = false, const AcceptArgs& accept = AcceptArgs(), bool verify = false) {
     ON_DEVICE(s->device);
     const uint32_t kmax = max_k(rows.r, n);
     LaunchCfg cfg;
-    if (!chained) {
+    if (!chained && !verify) {
         if (const uint32_t ws = wide_slices(s, rows.r, n, dtype, vocab)) {
             fill_cfg(s, &cfg, n, vocab, ws, kmax, 0, nullptr);
             bool lse = false;
@@ -599,6 +599,9 @@ int launch_inline(lily_sampler* s, int dtype, uint32_t vocab, const InlineRows& 
         cfg.chain_rows = n;
         cfg.chain_cand = Handed<uint64_t>{s->chain_cand};
         cfg.chain_n = Handed<uint32_t>{s->chain_n};
+    }
+    if (chained || verify) {
+        cfg.verify = verify ? 1u : 0u;
         cfg.chain_ticket = s->chain_ticket;
         cfg.accept_ctrl = accept.ctrl;
         cfg.accept_ids = accept.ids;
@@ -1548,15 +1551,17 @@ int lily_spec_verify(lily_sampler_t* s, const void* logits_dev, lily_dtype dtype
         }
     }
     if (!chained) {
+        // (one row alone may be one of many candidates, which has launches of its own)
         AcceptArgs accept;
-        if (in_order && ctrl_dev != nullptr) {
+        const bool verify = !in_order && m > 1;
+        if ((in_order || verify) && ctrl_dev != nullptr) {
             accept.ctrl = ctrl_dev;
             accept.ids = ids_dev;
             accept.pos0 = pos0;
             accept.ratio = ratio;
             accept.chain = chain;
         }
-        if (int rc = launch_inline(s, dtype, vocab, rows, m, in_order, accept)) {
+        if (int rc = launch_inline(s, dtype, vocab, rows, m, in_order, accept, verify)) {
             return rc;
         }
         if (accept.ctrl != nullptr) {

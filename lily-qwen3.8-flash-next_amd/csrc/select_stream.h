@@ -4,6 +4,7 @@
 #include <type_traits>
 
 #include "device_common.h"
+#include "wave_sort.h"
 
 namespace lily {
 
@@ -178,7 +179,7 @@ __device__ __forceinline__ void stream_row_sum(const RowArgs& a, const Geo<DT>& 
     // another kind (terms formed during the scan, terms that reference cannot hold) sends the
     // row the long way below.
     const bool other_sums = up != UP_UNSET || !(wl.s == 0.0f) || !(wl.booked == 0.0f);
-    const double p_wave = wave_sum_d_dpp(acc_p);
+    const double p_wave = wave_sum_d(acc_p);
     if (lane == 0) {
         sh.red_d[w] = p_wave;
     }
@@ -197,10 +198,7 @@ __device__ __forceinline__ void stream_row_sum(const RowArgs& a, const Geo<DT>& 
         // Each wave brings its sums to one reference of its own: the highest of its threads'
         // references and of the streamed sums' (wave-uniform) reference.  The waves' partial
         // sums and references meet in LDS and are brought together after one barrier.
-        int ref_w = up;
-        for (int o = 32; o > 0; o >>= 1) {
-            ref_w = max(ref_w, __shfl_xor(ref_w, o));
-        }
+        int ref_w = wave_max_i32(up);
         const double stream_at = (double)wl.ref - (double)ref_s;  // exact
         if (__ballot(wl.s > 0.0f) != 0ull) {
             const double e = stream_at < 1.0e9 ? (stream_at > -1.0e9 ? stream_at : -1.0e9) : 1.0e9;
@@ -303,6 +301,34 @@ __device__ __forceinline__ bool stream_accept(StreamLds& L, float filt, float te
     phase(cfg, 3);
     if (n > FC_CAP) {
         return stream_fail(cfg, 5u);
+    }
+    if (n <= 64u) {
+        // The first wave sorts them, an entry a lane, and has the answer; one barrier in all (ranked by
+        // the workgroup and looked at again behind that, three: 0.6 us more).
+        if (w == 0u) {
+            const uint64_t c = wave_sort_desc(lane < n ? L.fc[lane] : 0ull);
+            L.fc[lane] = c;
+            const uint32_t have = min((uint32_t)__popcll(__ballot(c != 0ull)), k);
+            bool good = true;
+            if (filt > F32_LOWEST) {
+                const float below = lilym_key_value(lilym_order_key(filt) - 1u) / temperature;
+                const uint32_t lowest =
+                    have != 0u ? (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(c >> 32), (int)have - 1) : 0xffffffffu;
+                good = have >= k && lilym_order_key(below) < lowest;
+            }
+            if (lane == 0u) {
+                sh.n_cand = have;
+                sh.fail = good ? 0u : 1u;
+            }
+        }
+        __syncthreads();
+        phase(cfg, 12);
+        if (sh.fail != 0u) {
+            return stream_fail(cfg, 6u);
+        }
+        sorted = true;
+        out = L.fc;
+        return true;
     }
     sorted = false;
     n = select_topk<false>(L.fc, n, k, sh, sorted, 0u);
@@ -562,10 +588,8 @@ __device__ __forceinline__ bool select_stream(const RowArgs& a, const Geo<DT>& g
         for (uint32_t i = w_lo + tid; i < w_hi; i += NT) {
             mine += (uint32_t)__popc(gload(a.allow + i) & range32_at(g.id_lo, g.id_hi, (int64_t)i * 32));
         }
-        for (int o = 32; o > 0; o >>= 1) {
-            mine += __shfl_xor(mine, o);
-        }
-        if (lane == 0) {
+        mine = wave_scan_u32(mine);
+        if (lane == 63u) {
             sh.red_i[w] = mine;
         }
         __syncthreads();

@@ -4,49 +4,11 @@
 #pragma once
 
 #include "device_common.h"
+#include "wave_sort.h"
 
 namespace lily {
 
 // ------------------------------------------------------------------ sort
-
-// The value lane ^ M holds, every lane of the wave at work - by moves inside the vector unit for
-// every M, never through the LDS crossbar, whose latency a sort of dependent exchanges would wait
-// out stage by stage.  1 and 2: a permutation inside each group of four lanes.  4: the lanes of
-// the even groups of four read four lanes up, those of the odd groups four lanes down (two moves,
-// each written to its groups only).  8: a rotation by eight within each row of 16.  16 and 32:
-// the swaps of whole rows and of the wave's halves (v_permlane16_swap / v_permlane32_swap with
-// the value as both operands leave one copy with rows 0 0 2 2 / the lower half twice and the
-// other with rows 1 1 3 3 / the upper half twice).
-template <uint32_t M>
-__device__ __forceinline__ uint32_t from_lane_xor32(uint32_t x) {
-    static_assert(M == 1u || M == 2u || M == 4u || M == 8u || M == 16u || M == 32u, "a power of two inside the wave");
-    const int v = (int)x;
-    if (M == 1u) {
-        return (uint32_t)__builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, true);   // quad_perm [1, 0, 3, 2]
-    }
-    if (M == 2u) {
-        return (uint32_t)__builtin_amdgcn_update_dpp(0, v, 0x4e, 0xf, 0xf, true);   // quad_perm [2, 3, 0, 1]
-    }
-    if (M == 4u) {
-        const int up = __builtin_amdgcn_update_dpp(0, v, 0x104, 0xf, 0x5, false);    // row_shl:4 into groups 0 and 2
-        return (uint32_t)__builtin_amdgcn_update_dpp(up, v, 0x114, 0xf, 0xa, false); // row_shr:4 into groups 1 and 3
-    }
-    if (M == 8u) {
-        return (uint32_t)__builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, false);  // row_ror:8
-    }
-    const uint32_t lane = threadIdx.x & 63u;
-    if (M == 16u) {
-        const auto two = __builtin_amdgcn_permlane16_swap(x, x, false, false);
-        return (lane & 16u) != 0u ? two[0] : two[1];
-    }
-    const auto two = __builtin_amdgcn_permlane32_swap(x, x, false, false);
-    return (lane & 32u) != 0u ? two[0] : two[1];
-}
-
-template <uint32_t M>
-__device__ __forceinline__ uint64_t from_lane_xor(uint64_t v) {
-    return ((uint64_t)from_lane_xor32<M>((uint32_t)(v >> 32)) << 32) | from_lane_xor32<M>((uint32_t)v);
-}
 
 // Descending bitonic sort of cand[0..n), n <= 4 * NT, four entries per thread (entry
 // 4 * tid + r in register r; absent entries are 0, the smallest).  Exchanges at distance
@@ -131,20 +93,7 @@ __device__ __forceinline__ void sort_desc(uint64_t* cand, uint32_t n) {
     if (n <= 64) {
         if (threadIdx.x < 64) {
             const uint32_t lane = threadIdx.x;
-            uint64_t c = lane < n ? cand[lane] : 0ull;
-#pragma unroll
-            for (uint32_t size = 2; size <= 64; size <<= 1) {
-#pragma unroll
-                for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
-                    const uint64_t o = stride == 1u ? from_lane_xor<1>(c) : stride == 2u ? from_lane_xor<2>(c)
-                                     : stride == 4u ? from_lane_xor<4>(c) : stride == 8u ? from_lane_xor<8>(c)
-                                     : stride == 16u ? from_lane_xor<16>(c) : from_lane_xor<32>(c);
-                    const bool desc = (lane & size) == 0;
-                    const bool lower = (lane & stride) == 0;
-                    const bool take_max = lower == desc;
-                    c = take_max ? (o > c ? o : c) : (o < c ? o : c);
-                }
-            }
+            const uint64_t c = wave_sort_desc(lane < n ? cand[lane] : 0ull);
             cand[lane] = c;
         }
         __syncthreads();
@@ -290,6 +239,150 @@ __device__ __forceinline__ void finish_token(const RowArgs& a, Shared& sh, uint3
     }
 }
 
+// A row without a finite value anywhere: the oracle's order then starts at id 0.  (One thread.)
+__device__ __forceinline__ void finish_empty(const RowArgs& a, uint32_t vocab, Shared& sh, const LaunchCfg& cfg) {
+    if (a.out_logprob) {
+        *a.out_logprob = NEG_INF;
+    }
+    emit(a, 0, vocab, cfg.chain_rows != 0u ? &sh : nullptr);
+    if (a.dbg_counts) {
+        a.dbg_counts[0] = 0;
+        a.dbg_counts[1] = 1;  // the reference keeps rank 0 whatever its value
+    }
+    if (a.mode == MODE_DRAFT) {
+        *a.q_n = 0;
+    }
+}
+
+// The sums p_0, p_0 + p_1, ... of the lanes' values in that order, each rounded as it is formed (the
+// reference's left-to-right f32 sums), lane by lane: each step adds a lane's value to the sum of the
+// lane below (a shift by one across the wave; lane 0 keeps what it has), so lane l holds its final
+// sum after l steps.  k: lanes from there on hold 0, and as many steps are made as that needs.
+// (Reading every lane's value into all 64 and keeping each prefix by a select was five
+// instructions a step and always 64 steps: 0.8 us of a draw.)
+__device__ __forceinline__ float wave_prefix_in_order(float p, uint32_t k) {
+    float run = p;
+    const int steps = __builtin_amdgcn_readfirstlane((int)k);
+    for (int j = 1; j < steps; j += 8) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            // Two idle cycles between a lane's write and the neighbour's read of it.
+            asm volatile("s_nop 1\n\tv_add_f32_dpp %0, %0, %1 wave_shr:1 row_mask:0xf bank_mask:0xf"
+                         : "+v"(run)
+                         : "v"(p));
+        }
+    }
+    // lanes past the steps made: the last prefix, which adding their zeros leaves as it is
+    const float last = lilym_bits_f32((uint32_t)__builtin_amdgcn_readlane((int)lilym_f32_bits(run), steps - 1));
+    return (int)(threadIdx.x & 63u) >= steps ? last : run;
+}
+
+// Lane l's value, l the same in every lane.
+__device__ __forceinline__ float lane_f32(float v, uint32_t l) {
+    return lilym_bits_f32((uint32_t)__builtin_amdgcn_readlane((int)lilym_f32_bits(v), (int)l));
+}
+
+// The tail of a draw among at most 64 candidates, by one wave (all of it at work), a candidate per
+// lane: `c` in descending order, 0 from lane k on (k >= 1 of them valid).
+// SPEC_WAVE: compile the speculative draw too (spec_d: the proposal, spec_qn: the length of the draft's
+// distribution, at most 64).
+template <int DT, bool SPEC_WAVE>
+__device__ __forceinline__ void tail_wave(const RowArgs& a, uint32_t vocab, uint32_t step, uint64_t c, uint32_t k_in, Shared& sh,
+                                          const LaunchCfg& cfg, uint32_t spec_d, uint32_t spec_qn) {
+    const uint32_t k = (uint32_t)__builtin_amdgcn_readfirstlane((int)k_in);   // (the same in every lane)
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t top_key = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(c >> 32));
+    const float top = lilym_key_value(top_key);
+    const float p = lane < k ? lilym_expf(composite_value(c) - top) : 0.0f;
+    if (lane < k) {
+        if (a.dbg_ids) {
+            a.dbg_ids[lane] = composite_id(c);
+        }
+        if (a.dbg_probs) {
+            a.dbg_probs[lane] = p;
+        }
+    }
+    const float mine = wave_prefix_in_order(p, k);
+    const float before = lilym_bits_f32((uint32_t)__builtin_amdgcn_update_dpp(
+        0, (int)lilym_f32_bits(mine), 0x138, 0xf, 0xf, false));   // wave_shr:1, 0 into lane 0
+    // (the last prefix is the row total: the same additions in the same order)
+    const float limit = a.top_p * lane_f32(mine, 63u);
+    const bool stop = lane >= 1u && lane < k && !(before < limit && p >= a.min_p);
+    const uint64_t stops = __ballot(stop);
+    const uint32_t kept = stops != 0ull ? (uint32_t)__builtin_ctzll(stops) : k;
+    const float mass = lane_f32(mine, kept - 1u);
+    if (lane == 0 && a.dbg_counts) {
+        a.dbg_counts[0] = k;
+        a.dbg_counts[1] = kept;
+    }
+    if (a.mode == MODE_DRAFT) {
+        if (lane < kept) {
+            a.q_ids[lane] = composite_id(c);
+            a.q_probs[lane] = p / mass;
+        }
+        if (lane == 0) {
+            *a.q_n = kept;
+        }
+    }
+    const float u1 = (a.flags & F_UNIFORM) ? a.uniform : lilym_uniform_for(a.seed, step);
+    if (SPEC_WAVE && a.mode == MODE_SPEC) {
+        // Speculative draw (sample.metal:596-658, cpu_spec at tests/unit/kernels/sample.rs:264-283)
+        // in the same wave: the draft's distribution (at most 64 entries here) sits an entry
+        // per lane, lookups are ballots and lane reads, and the residual's sums run the same
+        // left-to-right chains as above.
+        const uint32_t d = spec_d, qn = spec_qn;
+        const uint32_t my_id = composite_id(c);
+        const uint32_t q_id = lane < qn ? a.q_ids[lane] : 0xffffffffu;
+        const float q_p = lane < qn ? a.q_probs[lane] : 0.0f;
+        const float p_norm = p / mass;
+        const uint64_t at_p = __ballot(lane < kept && my_id == d);
+        const uint64_t at_q = __ballot(lane < qn && q_id == d);
+        const float p_d = at_p != 0ull ? lane_f32(p_norm, (uint32_t)__builtin_ctzll(at_p)) : 0.0f;
+        const float q_d = at_q != 0ull ? lane_f32(q_p, (uint32_t)__builtin_ctzll(at_q)) : 0.0f;
+        if (u1 * q_d < p_d) {
+            if (lane == 0) {
+                finish_token<DT>(a, sh, d, vocab, cfg.chain_rows != 0u);
+            }
+            return;
+        }
+        // The draft's probability of each candidate, then the residual max(0, p - q).
+        int match = -1;   // the lane that holds this candidate's id in the draft's list
+        const int qid_bits = (int)q_id;
+        const int q_end = __builtin_amdgcn_readfirstlane((int)qn);   // (at most 64)
+#pragma unroll 8
+        for (int j = 0; j < q_end; ++j) {
+            const uint32_t idj = (uint32_t)__builtin_amdgcn_readlane(qid_bits, j);
+            match = idj == my_id ? j : match;
+        }
+        const float q_there = __shfl(q_p, match < 0 ? 0 : match);
+        const float q_mine = match < 0 ? 0.0f : q_there;
+        const float res = lane < kept ? fmaxf(p_norm - q_mine, 0.0f) : 0.0f;
+        const float u2 = (a.flags & F_UNIFORM) ? a.uniform2
+                                               : lilym_uniform_for(a.seed, lilym_residual_step(step));
+        const float r_mine = wave_prefix_in_order(res, k);
+        const float r_total = lane_f32(r_mine, 63u);   // (lanes past `kept` added 0)
+        uint64_t picks;
+        if (r_total > 0.0f) {
+            picks = __ballot(lane < kept && u2 * r_total < r_mine);
+        } else {
+            // Only rounding gives a rejected proposal a massless residual: draw from p.
+            picks = __ballot(lane < kept && u2 * mass < mine);
+        }
+        const uint32_t slot = picks != 0ull ? (uint32_t)__builtin_ctzll(picks) : kept - 1u;
+        const uint32_t id = ~(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)c, (int)slot);
+        if (lane == 0) {
+            finish_token<DT>(a, sh, id, vocab, cfg.chain_rows != 0u);
+        }
+        return;
+    }
+    const uint64_t hits = __ballot(lane < kept && u1 * mass < mine);
+    const uint32_t slot = hits != 0ull ? (uint32_t)__builtin_ctzll(hits) : kept - 1u;
+    const uint32_t id = ~(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)c, (int)slot);
+    if (lane == 0) {
+        finish_token<DT>(a, sh, id, vocab, cfg.chain_rows != 0u);
+    }
+}
+
 // cand[0..n) holds the row's candidates (at least its top-k); finishes the row.
 // SPEC_WAVE: compile the speculative draw of at most 64 candidates as one wave too (the kernel
 // of rows that draw in order, where every row's tail is a step of a chain; elsewhere its scalar
@@ -304,19 +397,8 @@ __device__ __forceinline__ void tail(const RowArgs& a, uint32_t vocab, uint32_t 
 #endif
     const uint32_t tid = threadIdx.x;
     if (n == 0) {
-        // No finite value anywhere: the oracle's order then starts at id 0.
         if (tid == 0) {
-            if (a.out_logprob) {
-                *a.out_logprob = NEG_INF;
-            }
-            emit(a, 0, vocab, cfg.chain_rows != 0u ? &sh : nullptr);
-            if (a.dbg_counts) {
-                a.dbg_counts[0] = 0;
-                a.dbg_counts[1] = 1;  // the reference keeps rank 0 whatever its value
-            }
-            if (a.mode == MODE_DRAFT) {
-                *a.q_n = 0;
-            }
+            finish_empty(a, vocab, sh, cfg);
         }
         return;
     }
@@ -334,111 +416,8 @@ __device__ __forceinline__ void tail(const RowArgs& a, uint32_t vocab, uint32_t 
     const uint32_t k = min(a.k, n);
     const float top = composite_value(cand[0]);
     if (k <= 64u && (a.mode != MODE_SPEC || (SPEC_WAVE && spec_qn <= 64u))) {
-        // One wave, a candidate per lane.  The sums keep the reference's left-to-right f32
-        // order: every lane runs the same chain of 64 additions on values read lane by lane
-        // (lanes past k hold 0, which changes nothing), so nothing waits on LDS.
-        if (tid >= 64u) {
-            return;
-        }
-        const uint32_t lane = tid;
-        const uint64_t c = lane < k ? cand[lane] : 0ull;
-        const float p = lane < k ? lilym_expf(composite_value(c) - top) : 0.0f;
-        if (lane < k) {
-            if (a.dbg_ids) {
-                a.dbg_ids[lane] = composite_id(c);
-            }
-            if (a.dbg_probs) {
-                a.dbg_probs[lane] = p;
-            }
-        }
-        const int pbits = (int)lilym_f32_bits(p);
-        float cum = 0.0f, before = 0.0f, mine = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 64; ++i) {
-            before = lane == (uint32_t)i ? cum : before;
-            cum += lilym_bits_f32((uint32_t)__builtin_amdgcn_readlane(pbits, i));
-            mine = lane == (uint32_t)i ? cum : mine;
-        }
-        // (the chain's last value is the row total: the same additions in the same order)
-        const float limit = a.top_p * cum;
-        const bool stop = lane >= 1u && lane < k && !(before < limit && p >= a.min_p);
-        const uint64_t stops = __ballot(stop);
-        const uint32_t kept = stops != 0ull ? (uint32_t)__builtin_ctzll(stops) : k;
-        const float mass = __shfl(mine, (int)kept - 1);
-        if (lane == 0 && a.dbg_counts) {
-            a.dbg_counts[0] = k;
-            a.dbg_counts[1] = kept;
-        }
-        if (a.mode == MODE_DRAFT) {
-            if (lane < kept) {
-                a.q_ids[lane] = composite_id(c);
-                a.q_probs[lane] = p / mass;
-            }
-            if (lane == 0) {
-                *a.q_n = kept;
-            }
-        }
-        const float u1 = (a.flags & F_UNIFORM) ? a.uniform : lilym_uniform_for(a.seed, step);
-        if (SPEC_WAVE && a.mode == MODE_SPEC) {
-            // Speculative draw (sample.metal:596-658, cpu_spec at tests/unit/kernels/sample.rs:264-283)
-            // in the same wave: the draft's distribution (at most 64 entries here) sits an entry
-            // per lane, lookups are ballots and lane reads, and the residual's sums run the same
-            // left-to-right chains as above.
-            const uint32_t d = spec_d, qn = spec_qn;
-            const uint32_t my_id = composite_id(c);
-            const uint32_t q_id = lane < qn ? a.q_ids[lane] : 0xffffffffu;
-            const float q_p = lane < qn ? a.q_probs[lane] : 0.0f;
-            const float p_norm = p / mass;
-            const uint64_t at_p = __ballot(lane < kept && my_id == d);
-            const uint64_t at_q = __ballot(lane < qn && q_id == d);
-            const float p_d = at_p != 0ull ? __shfl(p_norm, (int)__builtin_ctzll(at_p)) : 0.0f;
-            const float q_d = at_q != 0ull ? __shfl(q_p, (int)__builtin_ctzll(at_q)) : 0.0f;
-            if (u1 * q_d < p_d) {
-                if (lane == 0) {
-                    finish_token<DT>(a, sh, d, vocab, cfg.chain_rows != 0u);
-                }
-                return;
-            }
-            // The draft's probability of each candidate, then the residual max(0, p - q).
-            int match = -1;   // the lane that holds this candidate's id in the draft's list
-            const int qid_bits = (int)q_id;
-#pragma unroll
-            for (int j = 0; j < 64; ++j) {
-                const uint32_t idj = (uint32_t)__builtin_amdgcn_readlane(qid_bits, j);
-                match = ((uint32_t)j < qn && idj == my_id) ? j : match;
-            }
-            const float q_there = __shfl(q_p, match < 0 ? 0 : match);
-            const float q_mine = match < 0 ? 0.0f : q_there;
-            const float res = lane < kept ? fmaxf(p_norm - q_mine, 0.0f) : 0.0f;
-            const int rbits = (int)lilym_f32_bits(res);
-            const float u2 = (a.flags & F_UNIFORM) ? a.uniform2
-                                                   : lilym_uniform_for(a.seed, lilym_residual_step(step));
-            float r_cum = 0.0f, r_mine = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 64; ++i) {
-                r_cum += lilym_bits_f32((uint32_t)__builtin_amdgcn_readlane(rbits, i));
-                r_mine = lane == (uint32_t)i ? r_cum : r_mine;
-            }
-            const float r_total = r_cum;   // lanes past `kept` added 0
-            uint64_t picks;
-            if (r_total > 0.0f) {
-                picks = __ballot(lane < kept && u2 * r_total < r_mine);
-            } else {
-                // Only rounding gives a rejected proposal a massless residual: draw from p.
-                picks = __ballot(lane < kept && u2 * mass < mine);
-            }
-            const uint32_t slot = picks != 0ull ? (uint32_t)__builtin_ctzll(picks) : kept - 1u;
-            const uint32_t id = ~(uint32_t)__shfl((int)(uint32_t)c, (int)slot);
-            if (lane == 0) {
-                finish_token<DT>(a, sh, id, vocab, cfg.chain_rows != 0u);
-            }
-            return;
-        }
-        const uint64_t hits = __ballot(lane < kept && u1 * mass < mine);
-        const uint32_t slot = hits != 0ull ? (uint32_t)__builtin_ctzll(hits) : kept - 1u;
-        const uint32_t id = ~(uint32_t)__shfl((int)(uint32_t)c, (int)slot);
-        if (lane == 0) {
-            finish_token<DT>(a, sh, id, vocab, cfg.chain_rows != 0u);
+        if (tid < 64u) {
+            tail_wave<DT, SPEC_WAVE>(a, vocab, step, tid < k ? cand[tid] : 0ull, k, sh, cfg, spec_d, spec_qn);
         }
         return;
     }

@@ -1,0 +1,55 @@
+"""Rows cut into slices: the one-wave merge and draw of rows of few candidates (k <= 64), on both
+sides of the limits at which it lists the slices' candidates, merges them list by list or leaves
+them to the whole workgroup; and launches of greedy rows.  Bit-exact against the oracle."""
+import os
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+import lily_sampler as LS
+import lily_workloads as W
+import oracle as O
+from gpu_util import check_row_against_oracle, dev, ls_params, o_params, run_rows, upload_logits
+
+
+def _sampler(slices):
+    old = os.environ.get("LILY_SAMPLER_SLICES")
+    os.environ["LILY_SAMPLER_SLICES"] = str(slices)
+    try:
+        return LS.Sampler(0)
+    finally:
+        if old is None:
+            os.environ.pop("LILY_SAMPLER_SLICES", None)
+        else:
+            os.environ["LILY_SAMPLER_SLICES"] = old
+
+
+def _rows(rng, rows, vocab, bf16):
+    x = rng.normal(0, 3, (rows, vocab)).astype(np.float32)
+    x[1] = np.round(x[1])                                 # ties by the hundred at every value
+    x[2, rng.random(vocab) < 0.9995] = -np.inf            # fewer finite values than k, slices without one
+    x[3, :] = -np.inf
+    x[4, vocab // 2:vocab // 2 + 300] = np.linspace(20, 21, 300, dtype=np.float32)   # one slice holds them all
+    return W.to_bf16_bits(x) if bf16 else x
+
+
+@pytest.mark.parametrize("slices", [2, 8, 9, 32, 33, 64])
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+def test_rows_of_few_candidates_over_slices(slices, bf16):
+    s = _sampler(slices)
+    rng = np.random.default_rng(slices + 100 * bf16)
+    vocab = 131_075
+    x = _rows(rng, 5, vocab, bf16)
+    for trial, k in enumerate((2, 20, 33, 63, 64)):
+        kw = [dict(temperature=0.7, top_k=k, top_p=0.97, seed=60 + r) for r in range(5)]
+        for lp in (False, True):
+            r = run_rows(s, x, kw, [trial] * 5, logprobs=lp)
+            for i in range(5):
+                d = O.sample(x[i], None, o_params(**kw[i]), trial, want_logprob=lp)
+                check_row_against_oracle(r, i, d)
+                if lp and np.isfinite(d.logprob):
+                    assert abs(r.logprobs[i] - d.logprob) <= 1e-5 * max(1.0, abs(d.logprob)), (k, i)
+    s.close()
