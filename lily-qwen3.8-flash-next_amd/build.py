@@ -44,6 +44,7 @@ def units():
     out.append(("head_library.hip", "head_library.o", []))
     out.append(("rows_tiles.hip", "rows_tiles.o", []))
     out.append(("rows_wide.hip", "rows_wide.o", []))
+    out.append(("rows_argmax.hip", "rows_argmax.o", []))
     out.append(("sampler_api.cpp", "sampler_api.o", []))
     return out
 

@@ -108,6 +108,10 @@ hipError_t launch_head_summaries(hipStream_t stream, const void* logits, uint64_
 hipError_t launch_rows_tiles(hipStream_t stream, int dtype, bool lse, bool extra, uint32_t rows,
                              const LaunchCfg& cfg, const float* tile_max, const float* tile_sum,
                              uint32_t tiles, const uint32_t* tile_row, uint32_t* served);
+// Rows that are all greedy (MODE_ARGMAX), given inline or as cfg.table; cfg.accept_ctrl (inline rows): a
+// verify pass, whose acceptance runs behind the last row.
+hipError_t launch_rows_argmax(hipStream_t stream, int dtype, uint32_t rows, const LaunchCfg& cfg,
+                              const InlineRows* inline_rows);
 // Rows that draw among many candidates (k > 64), spread over cfg.slices workgroups a row: two
 // launches (the row's bound, then the values that reach it, merge, select, tail).
 // lane_max [rows][slices][256], bound [rows], count [rows][slices].

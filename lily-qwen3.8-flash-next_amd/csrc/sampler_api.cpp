@@ -175,6 +175,7 @@ struct LaunchPart {
     uint32_t excl_words = 0;
     bool bitmap_layout = false;
     uint32_t cand_cap = 0;
+    bool argmax = false;   // every row is greedy: the kernel that holds nothing else
     bool wide = false;   // every row draws among many candidates: the two launches of rows_wide.hip
 };
 
@@ -501,6 +502,15 @@ bool heavy_row(const lily_sampler* s, const RowArgs& r) {
     return s->force_path != 0 || !(r.flags & F_STREAM) || r.allow != nullptr;
 }
 
+bool all_greedy(const RowArgs* rows, uint32_t n) {
+    for (uint32_t i = 0; i < n; ++i) {
+        if (rows[i].mode != MODE_ARGMAX) {
+            return false;
+        }
+    }
+    return true;
+}
+
 constexpr uint32_t SPLIT_MIN_LIGHT = 64;  // streamable rows worth a launch of their own
 
 // Describes the launch(es) of a packed table.  A few rows that need the kernel with every
@@ -524,6 +534,7 @@ uint32_t plan_parts(const lily_sampler* s, RowArgs* table, uint32_t rows, int dt
         part.first = q == 0 ? 0u : rows - heavy;
         part.rows = !split ? rows : (q == 0 ? rows - heavy : heavy);
         const RowArgs* sub = table + part.first;
+        part.argmax = all_greedy(sub, part.rows);
         part.ws_k = max_k(sub, part.rows);
         part.slices = choose_slices(s, part.rows, part.ws_k, vocab, dtype);
         if (const uint32_t ws = wide_slices(s, sub, part.rows, dtype, vocab)) {
@@ -552,6 +563,10 @@ int launch_part(lily_sampler* s, const LaunchPart& part, const RowArgs* table_de
     cfg.excl_words = part.excl_words;
     cfg.bitmap_layout = part.bitmap_layout ? 1u : 0u;
     cfg.cand_cap = part.cand_cap;
+    if (part.argmax) {
+        HIP_TRY(launch_rows_argmax(s->stream, dtype, part.rows, cfg, nullptr));
+        return LILY_OK;
+    }
     if (part.wide) {
         HIP_TRY(launch_rows_wide(s->stream, dtype, part.lse, part.rows, cfg, nullptr, s->wide_max,
                                  s->wide_count));
@@ -610,6 +625,10 @@ int launch_inline(lily_sampler* s, int dtype, uint32_t vocab, const InlineRows& 
         cfg.accept_chain = accept.chain;
     }
     attach_trace(s, &cfg, n);
+    if (!chained && all_greedy(rows.r, n)) {
+        HIP_TRY(launch_rows_argmax(s->stream, dtype, n, cfg, &rows));
+        return LILY_OK;
+    }
     const LaunchShape shp = shape_of(s, rows.r, n, dtype, vocab, slices, kmax);
     cfg.excl_words = shp.excl_words;
     cfg.bitmap_layout = shp.bitmap_layout ? 1u : 0u;

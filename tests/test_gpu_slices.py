@@ -53,3 +53,49 @@ def test_rows_of_few_candidates_over_slices(slices, bf16):
                 if lp and np.isfinite(d.logprob):
                     assert abs(r.logprobs[i] - d.logprob) <= 1e-5 * max(1.0, abs(d.logprob)), (k, i)
     s.close()
+
+
+@pytest.mark.parametrize("rows", [1, 8, 9, 600])
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+def test_launches_of_greedy_rows(rows, bf16):
+    """Inline and from a table, in slices and whole; the first of equal maxima, rows of -inf and of
+    NaN, rows that start inside a 16-byte piece."""
+    s = LS.Sampler(0)
+    rng = np.random.default_rng(rows)
+    vocab = 20_011
+    x = np.round(rng.normal(0, 2, (rows, vocab))).astype(np.float32)
+    x[0, ::3] = np.nan
+    if rows > 3:
+        x[1, :] = -np.inf
+        x[2, :] = np.nan
+        x[3, :vocab - 1] = -np.inf
+    if bf16:
+        x = W.to_bf16_bits(x)
+    logits = upload_logits(x)
+    out = torch.full((rows,), -1, dtype=torch.int32, device=dev())
+    p = [ls_params()] * rows
+    torch.cuda.synchronize()
+    plan = s.plan(logits, p, [0] * rows, out)
+    got = []
+    for _ in range(2):
+        plan.run(0)
+        s.synchronize()
+        got.append(out.cpu().numpy().copy())
+        out.fill_(-1)
+        torch.cuda.synchronize()
+    keep = s.sample_rows(logits, p, [0] * rows, out)
+    s.synchronize()
+    got.append(out.cpu().numpy())
+    del keep
+    f = W.bf16_bits_to_f32(x) if bf16 else x
+    f = np.where(np.isnan(f), -np.inf, f)
+    want = np.array([np.argmax(f[r]) for r in range(rows)])
+    for ids in got:
+        for r in range(rows):
+            if not np.isfinite(f[r]).any():
+                # (nothing to choose: the first id that is no NaN, or id 0)
+                assert ids[r] == 0, (r, ids[r])
+            else:
+                assert ids[r] == want[r], (r, ids[r], want[r])
+    plan.close()
+    s.close()
