@@ -117,7 +117,14 @@ hipError_t launch_rows_argmax(hipStream_t stream, int dtype, uint32_t rows, cons
 // lane_max [rows][slices][256], bound [rows], count [rows][slices].
 hipError_t launch_rows_wide(hipStream_t stream, int dtype, bool lse, uint32_t rows, const LaunchCfg& cfg,
                             const InlineRows* inline_rows, float* lane_max, uint32_t* count);
+// `bytes` (a multiple of 16) from pinned host memory, mapped into the device at src, to dst.
 hipError_t launch_copy_pieces(hipStream_t stream, const void* src, void* dst, size_t bytes);
+// The same of up to sizeof(PlacedPieces) bytes from any host memory, through the launch's arguments.
+constexpr unsigned PLACED_PIECES = 128;
+struct alignas(16) PlacedPieces {
+    char b[PLACED_PIECES * 16];
+};
+hipError_t launch_place_pieces(hipStream_t stream, const void* src, void* dst, size_t bytes);
 hipError_t launch_probe_read(hipStream_t stream, const void* base, uint32_t rows, uint64_t row_bytes,
                              uint64_t stride_bytes, uint32_t* out);
 hipError_t launch_copy_row(hipStream_t stream, const uint32_t* src, uint32_t* dst, uint32_t words,

@@ -783,6 +783,39 @@ int ensure_table(lily_sampler* s, uint32_t rows) {
     return LILY_OK;
 }
 
+// Takes the next staging buffer (waiting, if need be, for the call that used it four calls back).
+int stage_acquire(lily_sampler* s, uint32_t rows, uint32_t* slot_out) {
+    if (int rc = ensure_table(s, rows)) {
+        return rc;
+    }
+    const uint32_t slot = s->stage_next;
+    s->stage_next = (slot + 1) % STAGE_SLOTS;
+    if (s->stage_used[slot]) {
+        HIP_TRY(hipEventSynchronize(s->stage_done[slot]));
+        s->stage_used[slot] = false;
+    }
+    *slot_out = slot;
+    return LILY_OK;
+}
+
+size_t round16(size_t n) { return (n + 15u) & ~(size_t)15u; }
+
+// Carries the first `bytes` of the staging buffer to the device (same offsets in table_dev): through the
+// launch's own arguments where they fit, else by a kernel that reads the buffer.
+int stage_commit(lily_sampler* s, uint32_t slot, size_t bytes) {
+    bytes = round16(bytes);
+    if (bytes <= sizeof(PlacedPieces)) {
+        HIP_TRY(launch_place_pieces(s->stream, s->stage[slot], s->table_dev, bytes));
+        return LILY_OK;
+    }
+    void* mapped = nullptr;
+    HIP_TRY(hipHostGetDevicePointer(&mapped, s->stage[slot], 0));
+    HIP_TRY(launch_copy_pieces(s->stream, mapped, s->table_dev, bytes));
+    HIP_TRY(hipEventRecord(s->stage_done[slot], s->stream));
+    s->stage_used[slot] = true;
+    return LILY_OK;
+}
+
 }  // namespace
 
 namespace lily {
@@ -1611,13 +1644,9 @@ int lily_sample_rows(lily_sampler_t* s, const lily_rows* b) {
         return fail(LILY_ERR_INVALID_ARG, "empty batch");
     }
     ON_DEVICE(s->device);
-    if (int rc = ensure_table(s, b->rows)) {
+    uint32_t slot = 0;
+    if (int rc = stage_acquire(s, b->rows, &slot)) {
         return rc;
-    }
-    const uint32_t slot = s->stage_next;
-    s->stage_next = (slot + 1) % STAGE_SLOTS;
-    if (s->stage_used[slot]) {
-        HIP_TRY(hipEventSynchronize(s->stage_done[slot]));
     }
     if (int rc = pack_batch(b, s->stage[slot])) {
         return rc;
@@ -1629,11 +1658,9 @@ int lily_sample_rows(lily_sampler_t* s, const lily_rows* b) {
     // stream.  (The copy engine's start-up costs about 100 us a call on this system; row kernels
     // that read the descriptors in place pay a trip across the bus for every field the compiler
     // chooses to load again, about 55 us on a launch of a thousand rows.)
-    RowArgs* table_mapped = nullptr;
-    HIP_TRY(hipHostGetDevicePointer(reinterpret_cast<void**>(&table_mapped), s->stage[slot], 0));
-    HIP_TRY(launch_copy_pieces(s->stream, table_mapped, s->table_dev, (size_t)b->rows * sizeof(RowArgs)));
-    HIP_TRY(hipEventRecord(s->stage_done[slot], s->stream));
-    s->stage_used[slot] = true;
+    if (int rc = stage_commit(s, slot, (size_t)b->rows * sizeof(RowArgs))) {
+        return rc;
+    }
     for (uint32_t q = 0; q < n_parts; ++q) {
         if (int rc = launch_part(s, parts[q], s->table_dev, (int)b->dtype, b->vocab, 0, q == 0)) {
             return rc;
@@ -1734,32 +1761,6 @@ void lily_insertions_clear(lily_insertions_t* q, uint32_t row) {
 // ---- the logits' producer and the draws from its summaries
 
 namespace {
-
-size_t round16(size_t n) { return (n + 15u) & ~(size_t)15u; }
-
-// Takes the next staging buffer (waiting, if need be, for the call that used it four calls back).
-int stage_acquire(lily_sampler* s, uint32_t rows, uint32_t* slot_out) {
-    if (int rc = ensure_table(s, rows)) {
-        return rc;
-    }
-    const uint32_t slot = s->stage_next;
-    s->stage_next = (slot + 1) % STAGE_SLOTS;
-    if (s->stage_used[slot]) {
-        HIP_TRY(hipEventSynchronize(s->stage_done[slot]));
-    }
-    *slot_out = slot;
-    return LILY_OK;
-}
-
-// Carries the first `bytes` of the staging buffer to the device (same offsets in table_dev).
-int stage_commit(lily_sampler* s, uint32_t slot, size_t bytes) {
-    void* mapped = nullptr;
-    HIP_TRY(hipHostGetDevicePointer(&mapped, s->stage[slot], 0));
-    HIP_TRY(launch_copy_pieces(s->stream, mapped, s->table_dev, round16(bytes)));
-    HIP_TRY(hipEventRecord(s->stage_done[slot], s->stream));
-    s->stage_used[slot] = true;
-    return LILY_OK;
-}
 
 float c2_of_temperature(float t) {
     const float c = (float)(1.4426950408889634 / (double)t);
