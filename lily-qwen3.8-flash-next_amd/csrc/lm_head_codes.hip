@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include "launch.h"
+#include "lm_head_epilogue.h"
 
 namespace lily {
 
@@ -39,8 +40,18 @@ __device__ __forceinline__ f32x4 product(const w32x4& a, const w32x4& b, const f
                                                    c, 0, 0, 0);
 }
 
+// Words from one column's scales and biases to the next's: one more than there are groups (an even
+// number: an odd distance spreads the 16 columns a product reads at once over the banks without a
+// computed turn), unless just that word costs a workgroup its place (92 groups: two a compute unit;
+// 252: one; 16 columns then lie 28 or 60 banks apart, which are different ones too).
+__host__ __device__ constexpr uint32_t scale_pitch(uint32_t groups) {
+    const uint32_t bare = (uint32_t)RING_BYTES + (uint32_t)LILY_TILE_COLS * 4u * groups, word = (uint32_t)LILY_TILE_COLS * 4u;
+    return CU_LDS_BYTES / (bare + word) == CU_LDS_BYTES / bare ? groups + 1u : groups;
+}
 // Bytes of LDS a launch needs: the stages, then every scale and bias of the tile's 128 columns.
-inline size_t codes_lds_bytes(uint32_t groups) { return (size_t)RING_BYTES + (size_t)LILY_TILE_COLS * groups * 4u; }
+inline size_t codes_lds_bytes(uint32_t groups) {
+    return (size_t)RING_BYTES + (size_t)LILY_TILE_COLS * scale_pitch(groups) * 4u;
+}
 
 }  // namespace
 
@@ -86,7 +97,7 @@ k_lm_head_codes(const uint16_t* __restrict__ hidden, uint64_t hidden_stride, con
     const uint32_t share = wave & 3u, half = wave >> 2;
     const uint32_t c = lane & 15u, kq = lane >> 4;
     const uint32_t n_tile = blockIdx.x, n0 = n_tile * LILY_TILE_COLS;
-    const uint32_t nstages = d / STAGE_K, groups = d >> group_shift;
+    const uint32_t nstages = d / STAGE_K, groups = d >> group_shift, pitch = scale_pitch(groups);
     // Each tile walks d from a place of its own and wraps round: rows lie a power of two apart
     // for the usual d, and tiles that all start at column 0 and advance in step queue up at one
     // memory channel after the other.
@@ -135,13 +146,12 @@ k_lm_head_codes(const uint16_t* __restrict__ hidden, uint64_t hidden_stride, con
     };
     // where a lane's codes lie in a stage (block cb: column 64 * half + 16 * cb + c; the wave's
     // share of the line is its pieces 2 * share and the next, 8 bytes a lane) and its scales in sz
-    uint32_t code_at[CB], scale_at[CB], turn[CB];
+    uint32_t code_at[CB], scale_at[CB];
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb) {
         const uint32_t col = 64u * half + 16u * (uint32_t)cb + c, q = 2u * share + (kq >> 1);
         code_at[cb] = (col >> 3) * 1024u + ((col & 7u) * 8u + (q ^ (col & 7u))) * 16u + (kq & 1u) * 8u;
-        scale_at[cb] = col * groups;
-        turn[cb] = col % groups;
+        scale_at[cb] = col * pitch;
     }
 
     f32x4 total[CB];
@@ -205,7 +215,7 @@ k_lm_head_codes(const uint16_t* __restrict__ hidden, uint64_t hidden_stride, con
             if constexpr (STEPS == 2) {
                 qx = product(a[1], b[1], qx);
             }
-            const uint32_t at = g + turn[cb], word = sz[scale_at[cb] + (at >= groups ? at - groups : at)];
+            const uint32_t word = sz[scale_at[cb] + g];
             const float s = bf16_bits_to_f32(word);   // (the shift drops the bias)
             float z = __builtin_bit_cast(float, word & 0xffff0000u);
             if constexpr (WBITS == 4) {
@@ -224,9 +234,9 @@ k_lm_head_codes(const uint16_t* __restrict__ hidden, uint64_t hidden_stride, con
     // into the other half (nobody reads it: the barrier that closed the pass before saw to
     // that), asks for the codes and the hidden values AHEAD further on into the registers just
     // freed, and meets the other waves.
-    w32x4 codes_ring[AHEAD][2], hid[AHEAD][STEPS];
-    fetch_codes(codes_ring[0], 0u);
-    stage(codes_ring[0], 0u);
+    w32x4 codes_ring[AHEAD][2], hid[AHEAD][STEPS], first[2];
+    fetch_codes(first, 0u);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < AHEAD; ++j) {
         fetch_hidden(hid[j], (uint32_t)j);
@@ -235,23 +245,20 @@ k_lm_head_codes(const uint16_t* __restrict__ hidden, uint64_t hidden_stride, con
     }
     // (the first stages are on their way while the scales are brought)
     // ---- the tile's scales and biases: group g of column col as one word (scale, bias) at
-    // sz[col * groups + (g + col) % groups] (turned by the column's number: the 16 columns a
-    // product reads at once then lie in different banks).  Eight neighbouring threads a column, 16
-    // bytes - eight groups - a load where the arrays allow it.  (A form that found a word's column
-    // and place by divisions, sixteen words a thread, spent 40 % of the launch's vector
-    // instructions here, and those are 80 % of its cycles: V = 151 936, 4 rows, d = 4096 / 2560: 4 bits
-    // 101 / 78 -> 98 / 71 us, 8 bits 145 / 100 -> 141 / 96.)
+    // sz[col * pitch + g].  Eight neighbouring threads a column, 16 bytes - eight groups - a load
+    // where the arrays allow it.  What a workgroup does outside its loop bounds it as much as the loop
+    // does (each of 1 187 has some 16 stages): no division, no place turned by the column's number,
+    // the first stage's wait behind the requests for the rest, no load between the last barriers, and
+    // the maxima and sums at the end without the LDS crossbar.  (V = 151 936, 4 rows, d = 4096, 4 bits,
+    // head and draws in one call: 123.8 -> 119.1 us; this kernel is 81 of them, 4.4 TB/s.)
     {
         const uint32_t col0 = tid >> 3, lane8 = tid & 7u;
-        auto put = [&](uint32_t col, uint32_t turn_of, uint32_t g, uint32_t scale, uint32_t bias) {
-            const uint32_t at = g + turn_of;
-            sz[col * groups + (at >= groups ? at - groups : at)] = scale | (bias << 16);
+        auto put = [&](uint32_t col, uint32_t g, uint32_t scale, uint32_t bias) {
+            sz[col * pitch + g] = scale | (bias << 16);
         };
-        uint32_t turned[2];
         uint64_t from[2];
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-            turned[u] = (col0 + 64u * (uint32_t)u) % groups;
             from[u] = (uint64_t)min(n0 + col0 + 64u * (uint32_t)u, vocab - 1u) * groups;
         }
         if (groups % 8u == 0u &&
@@ -268,7 +275,7 @@ k_lm_head_codes(const uint16_t* __restrict__ hidden, uint64_t hidden_stride, con
                 for (int u = 0; u < 2; ++u) {
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
-                        put(col0 + 64u * (uint32_t)u, turned[u], g + (uint32_t)e, (sc[u][e >> 1] >> (16 * (e & 1))) & 0xffffu,
+                        put(col0 + 64u * (uint32_t)u, g + (uint32_t)e, (sc[u][e >> 1] >> (16 * (e & 1))) & 0xffffu,
                             (bi[u][e >> 1] >> (16 * (e & 1))) & 0xffffu);
                     }
                 }
@@ -277,14 +284,23 @@ k_lm_head_codes(const uint16_t* __restrict__ hidden, uint64_t hidden_stride, con
             for (uint32_t g = lane8; g < groups; g += 8u) {
 #pragma unroll
                 for (int u = 0; u < 2; ++u) {
-                    put(col0 + 64u * (uint32_t)u, turned[u], g, scales[from[u] + g], biases[from[u] + g]);
+                    put(col0 + 64u * (uint32_t)u, g, scales[from[u] + g], biases[from[u] + g]);
                 }
             }
         }
     }
+    stage(first, 0u);   // (written here, not where it was asked for: nothing waits on it alone)
     HEAD_MARK(1);
     __syncthreads();   // (the scales and stage 0 are written)
     HEAD_MARK(2);
+    // (what the exponentials at the end multiply by: the same for a wave's lanes, asked for here -
+    // each row's factor used to be a load, and a wait, of its own between the last barriers)
+    const uint32_t rq = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 7));
+    float c2[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        c2[j] = c2_of_row[min(4u * rq + (uint32_t)j, rows - 1u)];
+    }
     const uint32_t padded = (nstages + AHEAD - 1u) / AHEAD * AHEAD;
     static_assert(AHEAD % 2 == 0, "the halves of LDS alternate within a trip");
     for (uint32_t s0 = 0; s0 < padded; s0 += AHEAD) {
@@ -314,7 +330,7 @@ k_lm_head_codes(const uint16_t* __restrict__ hidden, uint64_t hidden_stride, con
         }
     }
     __syncthreads();
-    const uint32_t col_in = tid & 127u, rq = tid >> 7;   // (a wave's threads share rq)
+    const uint32_t col_in = tid & 127u;
     const uint32_t col = n0 + col_in;
     const float NEG = -__builtin_huge_valf();
     float x[4];
@@ -333,19 +349,28 @@ k_lm_head_codes(const uint16_t* __restrict__ hidden, uint64_t hidden_stride, con
     // each row's largest value and sum of exponentials over the 128 columns (two waves a row)
     float* red = part;            // [8 waves][4]
     float* row_max = part + 32;   // [16]
-    auto across = [&](float v, auto op) -> float {
+    // Four values over the 64 lanes, halved with them: the two halves of the wave, then the two rows
+    // of 16 lanes of a half, change places for two values at a time; then lanes 8, 4, 2 and 1 apart.
+    // Lane 16 * j ends with value j.  (A butterfly for each value took 24 moves through the LDS
+    // crossbar.)
+    auto across = [&](const float (&v)[4], auto op) -> float {
+        auto bits = [](float f) { return __builtin_bit_cast(uint32_t, f); };
+        float y[2];
 #pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) {
-            v = op(v, __shfl_xor(v, o));
+        for (int i = 0; i < 2; ++i) {
+            const auto both = __builtin_amdgcn_permlane32_swap(bits(v[i]), bits(v[i + 2]), false, false);
+            y[i] = op(__builtin_bit_cast(float, (uint32_t)both[0]), __builtin_bit_cast(float, (uint32_t)both[1]));
         }
-        return v;
+        const auto both = __builtin_amdgcn_permlane16_swap(bits(y[0]), bits(y[1]), false, false);
+        float z = op(__builtin_bit_cast(float, (uint32_t)both[0]), __builtin_bit_cast(float, (uint32_t)both[1]));
+        z = op(z, moved<0x128>(z));      // (rotated by 8)
+        z = op(z, moved<0x141>(z));      // (eight lanes mirrored)
+        z = op(z, moved<0x4e>(z));       // (quads: 2 3 0 1)
+        return op(z, moved<0xb1>(z));    // (quads: 1 0 3 2)
     };
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const float m = across(x[j], [](float p, float q) { return fmaxf(p, q); });
-        if (lane == 0u) {
-            red[wave * 4u + (uint32_t)j] = m;
-        }
+    const float top4 = across(x, [](float p, float q) { return fmaxf(p, q); });
+    if ((lane & 15u) == 0u) {
+        red[wave * 4u + (lane >> 4)] = top4;
     }
     __syncthreads();
     // (row r: waves 2 * (r / 4) and the next, entry r % 4 of each)
@@ -358,16 +383,13 @@ k_lm_head_codes(const uint16_t* __restrict__ hidden, uint64_t hidden_stride, con
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const uint32_t r = 4u * rq + (uint32_t)j;
-        const float cc = c2_of_row[min(r, rows - 1u)], top = row_max[r] * cc;
-        e[j] = x[j] > NEG ? __builtin_amdgcn_exp2f(__builtin_fmaf(x[j], cc, -top)) : 0.0f;
+        const float top = row_max[r] * c2[j];
+        e[j] = x[j] > NEG ? __builtin_amdgcn_exp2f(__builtin_fmaf(x[j], c2[j], -top)) : 0.0f;
     }
     // (red is free again: its readers passed the barrier above)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const float sum = across(e[j], [](float p, float q) { return p + q; });
-        if (lane == 0u) {
-            red[wave * 4u + (uint32_t)j] = sum;
-        }
+    const float sum4 = across(e, [](float p, float q) { return p + q; });
+    if ((lane & 15u) == 0u) {
+        red[wave * 4u + (lane >> 4)] = sum4;
     }
     __syncthreads();
     if (tid < 16u && tid < rows) {

@@ -827,6 +827,29 @@ def test_heads_of_affine_codes(sampler, bits, group, rows):
 
 
 @pytest.mark.parametrize("rows,d,vocab,bits,group", [
+    (13, 128, 127, 8, 64), (5, 256, 129, 4, 128), (16, 5632, 130, 4, 64), (4, 5888, 130, 4, 64),
+    (3, 6144, 257, 8, 64), (1, 15872, 129, 4, 64), (2, 16128, 130, 4, 64)])
+def test_few_rows_of_codes_over_their_scales(sampler, rows, d, vocab, bits, group):
+    """Up to 16 rows over codes at both distances of the columns' scales in LDS: two groups, the last
+    that is padded with two workgroups a compute unit (90 is as 88) and the one that is not (92), the
+    same with one (248 and 252, all that is served); one stage and many, last tiles of one, two and
+    127 columns: logits and summaries against the f64 product with the affine weights."""
+    rng = np.random.default_rng(rows + d + bits)
+    hidden = rng.normal(0, 1, (rows, d)).astype(np.float32)
+    qw, _, exact, summed = _quantised(rng, vocab, d, bits, group)
+    h = _bf16(hidden)
+    temps = [0.5 + 0.1 * (r % 7) for r in range(rows)]
+    buf = torch.full((rows, vocab + 4), 7.0, dtype=torch.float32, device=dev())
+    tiles = (vocab + TILE - 1) // TILE
+    tmax = torch.zeros(rows, tiles, dtype=torch.float32, device=dev())
+    tsum = torch.zeros(rows, tiles, dtype=torch.float32, device=dev())
+    sampler.lm_head(h, qw, temps, buf[:, :vocab], tmax, tsum)
+    sampler.synchronize()
+    _check_f32_product(h, exact, buf[:, :vocab], tmax, tsum, temps, summed=summed)
+    assert torch.all(buf[:, vocab:] == 7.0)
+
+
+@pytest.mark.parametrize("rows,d,vocab,bits,group", [
     (17, 512, 700, 4, 64), (32, 128, 64, 8, 64), (33, 1024, 129, 8, 128), (64, 256, 1000, 4, 64),
     (65, 512, 333, 8, 64), (128, 768, 257, 4, 128), (129, 1536, 1160, 4, 64),
     (16, 768, 300, 4, 256), (20, 8192, 129, 8, 64), (64, 6144, 140, 4, 64), (65, 2560, 200, 8, 64),
