@@ -170,7 +170,12 @@ __device__ __forceinline__ bool lowering_row(const RowArgs& a) {
 // (With the workgroup's four waves meeting at eight barriers from here to the draw: 7.6 us of the 13.2
 // that one sampled row of 151 936 f32 logits takes in 38 slices; now 6 of 12.1.)
 constexpr uint32_t WAVE_MERGE_SLOTS = 2048;   // entries the wave gathers at most, 32 a lane
-constexpr uint32_t WAVE_MERGE_LISTS = 8;      // up to this many slices their lists are merged one by one
+// Up to this many slices their lists are merged one by one: a merge is a chain of seven exchanges
+// and the lists follow one another, where the bound of more slices' entries, and one sort of those that
+// reach it, cost the same for six as for thirty-eight.  (Six slices, lists one by one -> this: k = 3
+// 25.6 -> 19.8 us, k = 50 28.3 -> 25.1 for 90 rows of 248 320 bf16; k = 3 17.4 -> 10.1, k = 20 17.9 -> 11.7
+// for 6 rows of 50 001 in seven.)
+constexpr uint32_t WAVE_MERGE_LISTS = 3;
 
 __device__ __forceinline__ bool descending(uint64_t c) {   // lane by lane, equal only where both are 0
     const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)(uint32_t)c, 0x138, 0xf, 0xf, false);   // wave_shr:1
@@ -227,6 +232,10 @@ __device__ __forceinline__ bool finish_by_wave(const RowArgs& t, const LaunchCfg
                 best = q == 0u ? c : wave_merge_desc(best, c);
             }
         }
+    } else if (!forced && S * cfg.ws_k <= 64u) {
+        // (no more entries than lanes: one sort)
+        const uint64_t c = handed_load(cfg.ws_cand, base * cfg.ws_k + min(lane, S * cfg.ws_k - 1u));
+        best = wave_sort_desc(lane < S * cfg.ws_k ? c : 0ull);
     } else if (!forced) {
         constexpr int PER = WAVE_MERGE_SLOTS / 64, GROUP = 8;
         const uint32_t slots = S * cfg.ws_k;

@@ -36,14 +36,14 @@ def _rows(rng, rows, vocab, bf16):
     return W.to_bf16_bits(x) if bf16 else x
 
 
-@pytest.mark.parametrize("slices", [2, 8, 9, 32, 33, 64])
+@pytest.mark.parametrize("slices", [2, 3, 4, 8, 9, 32, 33, 64])
 @pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
 def test_rows_of_few_candidates_over_slices(slices, bf16):
     s = _sampler(slices)
     rng = np.random.default_rng(slices + 100 * bf16)
     vocab = 131_075
     x = _rows(rng, 5, vocab, bf16)
-    for trial, k in enumerate((2, 20, 33, 63, 64)):
+    for trial, k in enumerate((2, 16, 20, 33, 63, 64)):
         kw = [dict(temperature=0.7, top_k=k, top_p=0.97, seed=60 + r) for r in range(5)]
         for lp in (False, True):
             r = run_rows(s, x, kw, [trial] * 5, logprobs=lp)
