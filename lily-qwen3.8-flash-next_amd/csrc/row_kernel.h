@@ -176,6 +176,10 @@ constexpr uint32_t WAVE_MERGE_SLOTS = 2048;   // entries the wave gathers at mos
 // 25.6 -> 19.8 us, k = 50 28.3 -> 25.1 for 90 rows of 248 320 bf16; k = 3 17.4 -> 10.1, k = 20 17.9 -> 11.7
 // for 6 rows of 50 001 in seven.)
 constexpr uint32_t WAVE_MERGE_LISTS = 3;
+// Above this k the bound of two values a lane lets too many entries through and the workgroup's four
+// waves merge more lists faster (15 rows of 151 936 f32 under masks, k = 50: 20.4 us by the workgroup,
+// 20.9 by the wave; 24 under penalties 33.8 and 31.7; plain rows, k = 64: 34.4 and 42.4).
+constexpr uint32_t WAVE_MERGE_K = 50;
 
 __device__ __forceinline__ bool descending(uint64_t c) {   // lane by lane, equal only where both are 0
     const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)(uint32_t)c, 0x138, 0xf, 0xf, false);   // wave_shr:1
@@ -249,15 +253,27 @@ __device__ __forceinline__ bool finish_by_wave(const RowArgs& t, const LaunchCfg
                 }
             }
         }
-        uint64_t lane_best = 0ull;
+        uint32_t lane_best = 0u, lane_next = 0u;   // the upper 16 bits of a lane's two best
 #pragma unroll
         for (int q = 0; q < PER; ++q) {
             mine[q] = lane + (uint32_t)q * 64u < slots ? mine[q] : 0ull;
-            lane_best = mine[q] > lane_best ? mine[q] : lane_best;
+            const uint32_t key = (uint32_t)(mine[q] >> 48);
+            lane_next = max(lane_next, min(lane_best, key));
+            lane_best = max(lane_best, key);
         }
-        // k lanes' best reach the bound, so k entries do; what does not is dropped, the rest is
-        // listed, and the list's entries are taken in 64 at a time.
-        const uint32_t bound = wave_kth_key16((uint32_t)(lane_best >> 48), t.k);
+        // The k-th largest of the lanes' two best bounds the k-th entry: at least k entries reach it
+        // (more than there are with fewer than k: all of them); what does not is dropped, the rest is
+        // listed, and the list's entries are taken in 64 at a time.  Of one value a lane, the bound for
+        // k = 64 was the least of 64 maxima, which most entries reached: 10 rows of 65 695 f32 in 17
+        // slices took 46 us, 33 with two, 27 with the workgroup's merge; k = 50, 24 rows under penalties
+        // 33.8 with the workgroup's merge, 31.7 with two.
+        uint32_t bound = 0u;
+#pragma unroll
+        for (int bit = 15; bit >= 0; --bit) {
+            const uint32_t at = bound | (1u << bit);
+            const uint32_t reach = (uint32_t)__popcll(__ballot(lane_best >= at)) + (uint32_t)__popcll(__ballot(lane_next >= at));
+            bound = reach >= t.k ? at : bound;
+        }
         uint64_t* cand = dyn_lds;
         uint32_t kept = 0;
 #pragma unroll
@@ -438,7 +454,7 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
     uint32_t n = (argmax || forced) ? 0u : min(sh.n_cand, cfg.cand_cap);
     phase(cfg, 4);
     if (!CHAIN && S > 1 && !argmax && t.k <= 64u && cfg.ws_k <= 64u &&
-        (S <= WAVE_MERGE_LISTS || S * cfg.ws_k <= WAVE_MERGE_SLOTS) &&
+        (S <= WAVE_MERGE_LISTS || (t.k <= WAVE_MERGE_K && S * cfg.ws_k <= WAVE_MERGE_SLOTS)) &&
         (t.mode != MODE_SPEC || (SPEC && *t.q_n <= 64u))) {
         if (tid >= 64u) {
             return false;
