@@ -157,8 +157,9 @@ constexpr uint32_t PHASE_SLOTS = 16;
 
 constexpr uint32_t CAND_CAP = 2048;   // candidates a workgroup collects while scanning
 constexpr uint32_t MERGE_CAP = 4096;  // candidates the merging workgroup gathers (slices x k)
-constexpr uint32_t SORT_BINS = 2048;  // the sort of many candidates: its bins, behind 2 048 places
-constexpr uint32_t SORT_SLOTS = 2048 + SORT_BINS / 2;   // 64-bit slots it works in
+constexpr uint32_t SORT_PLACES = 2048;   // the sort of many candidates: its places at the front of the
+constexpr uint32_t SORT_BINS = 2048;     // candidates, and its bins' 32-bit words
+constexpr uint32_t SORT_SLOTS = SORT_PLACES + SORT_BINS / 2;   // 64-bit slots it works in, the bins behind the places
 constexpr uint32_t MAX_SLICES = 64;
 constexpr uint32_t SPECIAL_LIST_CAP = 2048;  // ids of penalised / biased tokens gathered per batch
 

@@ -537,7 +537,7 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
             if constexpr (KIND != 2) {
                 // (many candidates: every entry goes into the sort as it is)
                 if (t.k > 64u && cfg.dyn_slots >= max(slots, SORT_SLOTS)) {
-                    sorted = wg_sort_topk(cand, mine, slots, t.k, sh, n);
+                    sorted = wg_sort_topk(cand, mine, slots, t.k, reinterpret_cast<uint32_t*>(cand + SORT_PLACES), sh, n);
                     if (!sorted) {
                         n = wg_select_topk(cand, slots, t.k, sh);
                     }
@@ -575,7 +575,7 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
                 __syncthreads();
                 n = sh.n_cand;
                 sorted = false;
-                n = select_topk<KIND != 2>(cand, n, t.k, sh, sorted, cfg.dyn_slots);
+                n = select_topk<KIND != 2>(cand, n, t.k, sh, sorted, reinterpret_cast<uint32_t*>(cand + SORT_PLACES));
             }
             found = cand;
         }

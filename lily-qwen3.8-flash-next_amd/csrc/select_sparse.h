@@ -185,7 +185,9 @@ __device__ __forceinline__ bool select_sparse(const RowArgs& a, const Geo<DT>& g
         __syncthreads();
         return true;
     }
-    const uint32_t n = select_topk<true>(cand, total, k, sh, sorted, cfg.dyn_slots);
+    // (the staged bias list, and where other selects keep a bitmap, may lie under the bins: neither is
+    // read again)
+    const uint32_t n = select_topk<true>(cand, total, k, sh, sorted, reinterpret_cast<uint32_t*>(cand + SORT_PLACES));
     if (tid == 0) {
         sh.n_cand = n;
     }

@@ -309,6 +309,88 @@ def test_dense_masks_are_streamed(slices):
     s.close()
 
 
+def _merging_value(rng, temperature, bf16):
+    """A value at which the bitmap select's check fails and its second collection passes: the
+    division by the temperature maps the bound of the first (4 f32 steps below the value) and the
+    value below that to the value's own quotient, and those of the second (8 below what the
+    quotient stands for) to one before it."""
+    step = np.float32(temperature)
+    less = lambda v, n: (np.float32(v).view(np.uint32) - np.uint32(n)).view(np.float32)
+    for v in rng.permutation(np.linspace(0.25, 0.48, 120, dtype=np.float32)):
+        v = W.bf16_bits_to_f32(W.to_bf16_bits(np.array([v])))[0] if bf16 else v
+        back = np.float32(v / step) * step
+        if less(v, 5) / step == v / step and less(back, 9) / step < v / step and less(back, 8) <= v:
+            return v
+    raise AssertionError("no such value")
+
+
+@pytest.mark.parametrize("logprobs", [False, True], ids=["ids", "logprobs"])
+@pytest.mark.parametrize("slices", [1, 2])
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+def test_bitmap_select_collects_a_second_time(bf16, slices, logprobs):
+    """k > 64 under dense masks (without and with penalties) and under penalties that may raise, at a
+    temperature that merges values: the check behind the first collection fails, and the second
+    reads the slice's bitmap of ids to leave out again, behind a sort of several hundred
+    candidates (by counted bins for a few equal values, by the radix select for hundreds).  The row's
+    largest raw values are barred, or lowered by their counts: none may come back."""
+    s = _sampler_with_slices(slices)
+    rng = np.random.default_rng(71 + bf16 + 2 * slices)
+    temperature, vocab = 3.0e38, 60_007
+    cases = [(220, 124, "mask"), (500, 400, "mask"), (1024, 1000, "mask"), (220, 124, "mask+pen"),
+             (1024, 1000, "mask+pen"), (220, 300, "raise"), (900, 1200, "raise")]
+    for kinds in (("mask", "mask+pen"), ("raise",)):
+        mine = [c for c in cases if c[2] in kinds]
+        rows = len(mine)
+        x = rng.uniform(-1, 0, (rows, vocab)).astype(np.float32)
+        masks = np.zeros((rows, (vocab + 31) // 32), np.uint32)
+        kw, sc, counts = [], [], []
+        for r_, (k, ties, kind) in enumerate(mine):
+            v = _merging_value(rng, temperature, bf16)
+            allowed = np.ones(vocab, bool)
+            hist = []
+            for lo, hi in ((vocab * q // slices, vocab * (q + 1) // slices) for q in range(slices)):
+                ids = lo + rng.permutation(hi - lo)
+                above, tied, high, rest = np.split(ids, np.cumsum([k - ties // 2, ties, 120]))
+                x[r_, above] = rng.uniform(v * 1.02, v * 1.9, above.size)
+                x[r_, tied] = v
+                if kind != "raise":                   # the largest raw values, one in two barred
+                    x[r_, high] = rng.uniform(3 * v, 5 * v, high.size)
+                    allowed[high[:60] if kind == "mask+pen" else high] = False
+                    allowed[rest[:rest.size // 3]] = False
+                    hist += list(high[60:]) + list(rest[-50:])
+                else:                                 # 0.8 lifts some of these above v
+                    x[r_, high] = rng.uniform(v * 0.7, v * 0.99, high.size)
+                    hist += list(high) + list(rest[-50:])
+            d = dict(temperature=temperature, top_k=k, top_p=1.0, seed=300 + r_)
+            if kind == "mask+pen":
+                d.update(presence_penalty=4.0, repetition_penalty=1.1)
+            elif kind == "raise":
+                d.update(repetition_penalty=0.8)
+            kw.append(d)
+            masks[r_] = np.packbits(np.append(allowed, np.zeros(-vocab % 32, bool)), bitorder="little").view(np.uint32)
+            hist = np.array(hist, np.int32)
+            sc.append(LS.SamplerScratch(s, vocab))
+            sc[-1].add_history(torch.from_numpy(hist).to(dev()))
+            counts.append(np.bincount(hist, minlength=vocab).astype(np.uint32))
+        xs = W.to_bf16_bits(x) if bf16 else x
+        allow = masks if kinds[0] == "mask" else None
+        stats = torch.zeros(4, dtype=torch.int32, device=dev())
+        s.set_path_stats(stats)
+        r = run_rows(s, xs, kw, [7] * rows, scratch=sc, allow=allow, logprobs=logprobs)
+        s.set_path_stats(None)
+        assert stats.cpu().tolist()[:3] == [0, rows * slices, 0], stats   # (none was left to the exhaustive select)
+        for i in range(rows):
+            pen = counts[i] if mine[i][2] != "mask" else None
+            d = O.sample(xs[i], pen, o_params(**kw[i]), 7, allow=None if allow is None else allow[i],
+                         want_logprob=logprobs)
+            check_row_against_oracle(r, i, d)
+            if logprobs:
+                _check_logprob(r, i, d, ("second collection", mine[i]))
+        for t in sc:
+            t.close()
+    s.close()
+
+
 @pytest.mark.parametrize("use_plan", [False, True], ids=["direct", "plan"])
 def test_mixed_batches_run_as_two_launches(sampler, use_plan):
     """A batch of mostly streamable rows with a few that need the other selects (k above
