@@ -730,7 +730,9 @@ __device__ __forceinline__ bool wg_sort_topk(uint64_t* cand, const uint64_t (&mi
     auto bin_of = [&](uint64_t c) -> uint32_t {   // never decreases as c does
         const uint32_t key = (uint32_t)(c >> 32);
         const float d = crosses ? top - lilym_key_value(key) : (float)(hi - key);
-        return min((uint32_t)(d * scale), SORT_BINS - 1u);
+        // (cut to the last bin before it becomes an integer: an empty entry's d * scale may be a NaN or past
+        // 2^32, of which a conversion may make anything, and a bin is where an addition goes)
+        return (uint32_t)fminf(d * scale, (float)(SORT_BINS - 1u));
     };
     // (what the count was before an entry is its place in its bin; every add is made, an empty
     // entry's of nothing, so that they are on their way together)

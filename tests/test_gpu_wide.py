@@ -287,3 +287,25 @@ def test_sort_of_many_candidates(sampler, bf16, masked):
             d = O.sample(x[i], None, o_params(**kw[i]), trial, allow=allow[i] if masked else None, want_logprob=True)
             check_row_against_oracle(r, i, d)
             _check_logprob(r.logprobs[i], d.logprob, (k, i))
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+def test_sort_with_more_empty_places_than_candidates(sampler, bf16):
+    """Masked rows whose four slices hand over some 375 candidates each in 1 024 places, so that most
+    of what the sort is given is empty: candidates so close together that an empty place's distance
+    from them, in bins, is past any integer, and on both sides of zero, where it is no number."""
+    rng = np.random.default_rng(79 + bf16)
+    vocab, n = 151_936, 1500
+    x = np.full((3, vocab), -np.inf, dtype=np.float32)
+    some = rng.choice(vocab, n, replace=False)
+    x[0, some] = 3.0 + rng.permutation(n).astype(np.float32) * 2.0 ** -22    # (one f32 step apart)
+    x[1, some] = -1.0 - rng.permutation(n).astype(np.float32) * 2.0 ** -14
+    x[2, some] = rng.normal(0, 1, n)
+    if bf16:
+        x = W.to_bf16_bits(x)
+    allow = np.zeros((3, (vocab + 31) // 32), dtype=np.uint32)
+    np.bitwise_or.at(allow, (slice(None), some >> 5), (1 << (some & 31)).astype(np.uint32))
+    kw = [dict(temperature=1.0, top_k=0, top_p=0.98, seed=600 + r) for r in range(3)]
+    r = run_rows(sampler, x, kw, [0] * 3, allow=allow)
+    for i in range(3):
+        check_row_against_oracle(r, i, O.sample(x[i], None, o_params(**kw[i]), 0, allow=allow[i]))
