@@ -669,15 +669,17 @@ __device__ __forceinline__ uint32_t wg_rank_select(uint64_t* cand, uint32_t n, u
 // the other, took 12.8 us for 1 024 of 1 200 f32 entries where this takes 5.4.  False where a bin
 // that matters holds more than SORT_BIN_MAX entries (ties by the hundred, an outlier that stretches
 // the steps): the select that does not mind takes over; the entries are then in cand[0..n), thread
-// t's j-th at t + j * NT.  cand: at least SORT_PLACES slots; bins: SORT_BINS words of LDS from a 16-byte
-// boundary on, which the caller says because it alone knows what lies behind the candidates.
+// t's j-th at t + j * NT.  cand: SORT_SLOTS slots, the bins behind the places: for a
+// caller that reads nothing of what lay there again (the bitmap select, which may go round once more
+// over a bitmap behind its candidates, keeps to the radix select).
 constexpr uint32_t SORT_BIN_MAX = 128;
 __device__ __forceinline__ bool wg_sort_topk(uint64_t* cand, const uint64_t (&mine)[MERGE_CAP / NT], uint32_t n,
-                                             uint32_t k, uint32_t* bins, Shared& sh, uint32_t& n_out) {
+                                             uint32_t k, Shared& sh, uint32_t& n_out) {
     constexpr int PER = MERGE_CAP / NT;
     constexpr uint32_t OWN = SORT_BINS / NT;                      // bins a thread sums
     constexpr int ROUNDS = (K_CAP + SORT_BIN_MAX + NT - 1) / NT;  // places a thread ranks
-    static_assert(K_CAP + SORT_BIN_MAX <= SORT_PLACES && OWN == 8u, "the bins may lie behind the places");
+    static_assert(K_CAP + SORT_BIN_MAX <= SORT_PLACES && OWN == 8u, "the bins lie behind the places");
+    uint32_t* bins = reinterpret_cast<uint32_t*>(cand + SORT_PLACES);
     const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
     uint32_t hi = 0u, lo = 0xffffffffu;
 #pragma unroll
@@ -853,28 +855,11 @@ __device__ __forceinline__ bool wg_sort_topk(uint64_t* cand, const uint64_t (&mi
     return true;
 }
 
-// Top-k of cand[0..n) to the front; `sorted` tells whether they are in descending order.  BIG: k may
-// exceed 64, and the sort has `bins` to work in (LDS that nobody reads again; else null).
-template <bool BIG>
-__device__ __forceinline__ uint32_t select_topk(uint64_t* cand, uint32_t n, uint32_t k, Shared& sh, bool& sorted,
-                                                uint32_t* bins) {
+// Top-k of cand[0..n) to the front; `sorted` tells whether they are in descending order.
+__device__ __forceinline__ uint32_t select_topk(uint64_t* cand, uint32_t n, uint32_t k, Shared& sh, bool& sorted) {
     if (n <= 256u) {
         sorted = true;
         return wg_rank_select(cand, n, k, sh);
-    }
-    if (BIG && k > 64u) {
-        constexpr int PER = MERGE_CAP / NT;
-        uint64_t mine[PER];
-#pragma unroll
-        for (int j = 0; j < PER; ++j) {
-            const uint32_t i = threadIdx.x + (uint32_t)j * NT;
-            mine[j] = i < n ? cand[i] : 0ull;
-        }
-        uint32_t got;
-        if (wg_sort_topk(cand, mine, n, k, bins, sh, got)) {
-            sorted = true;
-            return got;
-        }
     }
     sorted = false;
     return wg_select_topk(cand, n, k, sh);

@@ -451,7 +451,9 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
     RowArgs t;
     read_again(t, src);
     const bool forced = (t.flags & F_FORCED) != 0;
-    uint32_t n = (argmax || forced) ? 0u : min(sh.n_cand, cfg.cand_cap);
+    // (the sparse select of a row in one slice leaves what it evaluated, which may be more than cand_cap)
+    const uint32_t n_cap = KIND == 1 ? max(cfg.cand_cap, min(cfg.dyn_slots, MERGE_CAP)) : cfg.cand_cap;
+    uint32_t n = (argmax || forced) ? 0u : min(sh.n_cand, n_cap);
     phase(cfg, 4);
     if (!CHAIN && S > 1 && !argmax && t.k <= 64u && cfg.ws_k <= 64u &&
         (S <= WAVE_MERGE_LISTS || (t.k <= WAVE_MERGE_K && S * cfg.ws_k <= WAVE_MERGE_SLOTS)) &&
@@ -465,6 +467,58 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
         }
         return finished;
     }
+    // What is left to rank behind the slices: every slice's candidates, or those of a row of many
+    // candidates that is one slice, up to PER a thread.  (Expanded once: inside the slices' branch
+    // where only that can come to it, else behind both.)
+    constexpr int PER = MERGE_CAP / NT;
+    uint64_t mine[PER];
+    uint32_t slots = 0;
+    auto rank_them = [&]() {
+        sorted = false;
+        if (KIND != 2 && t.k > 64u) {
+            // Many candidates: every entry goes into the sort as it is.  This is the one place in a
+            // kernel that holds it: with a copy behind each select as well, the kernels that can have
+            // such rows spilled 30 to 60 vector registers more, and every row in them paid (the
+            // constrained batch of 64 rows 37.9 -> 36.6 us; 40 f32 rows without top_k, half of them forced
+            // and with log-probabilities, 70.2 -> 63.4).
+            n = slots;
+            sorted = wg_sort_topk(cand, mine, slots, t.k, sh, n);
+        } else {
+            // A bound of the k-th largest from the lanes' best entries (as in the streaming
+            // select: each wave's ceil(k / NWAVE)-th largest lane maximum, the minimum over the
+            // waves), then only entries at or above it are ranked.
+            uint64_t best_mine = 0;
+#pragma unroll
+            for (int q = 0; q < PER; ++q) {
+                best_mine = mine[q] > best_mine ? mine[q] : best_mine;
+            }
+            const uint32_t kw = (t.k + NWAVE - 1) / NWAVE;
+            const uint32_t P = kw <= 64u ? wave_kth_key16((uint32_t)(best_mine >> 48), kw) : 0u;
+            if ((tid & 63u) == 0) {
+                sh.red_i[tid >> 6] = P;
+            }
+            if (tid == 0) {
+                sh.n_cand = 0;
+            }
+            __syncthreads();
+            uint32_t bound = sh.red_i[0];
+            for (int i = 1; i < NWAVE; ++i) {
+                bound = min(bound, sh.red_i[i]);
+            }
+#pragma unroll
+            for (int q = 0; q < PER; ++q) {
+                if (mine[q] != 0ull && (uint32_t)(mine[q] >> 48) >= bound) {
+                    cand[atomicAdd(&sh.n_cand, 1u)] = mine[q];
+                }
+            }
+            __syncthreads();
+            n = sh.n_cand;
+        }
+        if (!sorted) {
+            n = select_topk(cand, n, t.k, sh, sorted);
+        }
+        found = cand;
+    };
     if (S > 1) {
         const size_t slot = (size_t)row * S + s;
         // Partials go through to memory (no dirty L2 lines to write back), the wave waits
@@ -509,9 +563,7 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
         } else {
             // Gather every slice's candidates (0 = no candidate) and the log-sum-exp partials
             // in one round trip.
-            constexpr int PER = MERGE_CAP / NT;
-            const uint32_t slots = S * cfg.ws_k;
-            uint64_t mine[PER];
+            slots = S * cfg.ws_k;
 #pragma unroll
             for (int q = 0; q < PER; ++q) {
                 const uint32_t j = tid + (uint32_t)q * NT;
@@ -533,52 +585,20 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
                     sh.lse_s = sum;
                 }
             }
-            bool ranked = false;
-            if constexpr (KIND != 2) {
-                // (many candidates: every entry goes into the sort as it is)
-                if (t.k > 64u && cfg.dyn_slots >= max(slots, SORT_SLOTS)) {
-                    sorted = wg_sort_topk(cand, mine, slots, t.k, reinterpret_cast<uint32_t*>(cand + SORT_PLACES), sh, n);
-                    if (!sorted) {
-                        n = wg_select_topk(cand, slots, t.k, sh);
-                    }
-                    ranked = true;
-                }
+            if constexpr (KIND == 2) {
+                rank_them();
             }
-            if (!ranked) {
-                // A bound of the k-th largest from the lanes' best entries (as in the streaming
-                // select: each wave's ceil(k / NWAVE)-th largest lane maximum, the minimum over the
-                // waves), then only entries at or above it are ranked.
-                uint64_t best_mine = 0;
-#pragma unroll
-                for (int q = 0; q < PER; ++q) {
-                    best_mine = mine[q] > best_mine ? mine[q] : best_mine;
-                }
-                const uint32_t kw = (t.k + NWAVE - 1) / NWAVE;
-                const uint32_t P = kw <= 64u ? wave_kth_key16((uint32_t)(best_mine >> 48), kw) : 0u;
-                if ((tid & 63u) == 0) {
-                    sh.red_i[tid >> 6] = P;
-                }
-                if (tid == 0) {
-                    sh.n_cand = 0;
-                }
-                __syncthreads();
-                uint32_t bound = sh.red_i[0];
-                for (int i = 1; i < NWAVE; ++i) {
-                    bound = min(bound, sh.red_i[i]);
-                }
-#pragma unroll
-                for (int q = 0; q < PER; ++q) {
-                    if (mine[q] != 0ull && (uint32_t)(mine[q] >> 48) >= bound) {
-                        cand[atomicAdd(&sh.n_cand, 1u)] = mine[q];
-                    }
-                }
-                __syncthreads();
-                n = sh.n_cand;
-                sorted = false;
-                n = select_topk<KIND != 2>(cand, n, t.k, sh, sorted, reinterpret_cast<uint32_t*>(cand + SORT_PLACES));
-            }
-            found = cand;
         }
+    } else if (KIND != 2 && t.k > 64u && n != 0u && !sorted) {
+        slots = n;
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            const uint32_t j = tid + (uint32_t)q * NT;
+            mine[q] = j < n ? cand[j] : 0ull;
+        }
+    }
+    if (KIND != 2 && slots != 0u) {
+        rank_them();
     }
 
     phase(cfg, 6);

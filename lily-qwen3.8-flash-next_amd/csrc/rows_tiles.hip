@@ -472,7 +472,7 @@ __global__ __launch_bounds__(NT, 4) void k_rows_tiles(LaunchCfg cfg, const float
         select_exhaustive<DT>(a, 0, vocab, k, want_lse, cand, cfg.cand_cap, sh);
         n = min(sh.n_cand, cfg.cand_cap);
     } else {
-        n = select_topk<false>(cand, n, k, sh, sorted, nullptr);
+        n = select_topk(cand, n, k, sh, sorted);
     }
     if (cfg.path_stats != nullptr && tid == 0) {
         atomicAdd(&cfg.path_stats[took], 1u);

@@ -432,7 +432,7 @@ __global__ __launch_bounds__(NT, 4) void k_wide_draw(InlineRows rows_arg, Launch
         }
         __syncthreads();
         WIDE_MARK(13);
-        sorted = wg_sort_topk(cand, mine_c, total, a.k, reinterpret_cast<uint32_t*>(cand + SORT_PLACES), sh, n);
+        sorted = wg_sort_topk(cand, mine_c, total, a.k, sh, n);
         if (!sorted) {
             n = wg_select_topk(cand, total, a.k, sh);
         }

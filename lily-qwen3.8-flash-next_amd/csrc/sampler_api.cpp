@@ -461,8 +461,7 @@ LaunchShape shape_of(const lily_sampler* s, const RowArgs* rows, uint32_t n, int
         const uint32_t e = dtype == LILY_BF16 ? 8 : 4;
         const uint32_t nch = (vocab + 2 * (e - 1)) / e + 1;
         const uint32_t per = (nch + slices - 1) / slices;
-        // (whole 16 bytes: the list behind them is also where the sort of many candidates keeps its bins)
-        sh.excl_words = masked ? ((per * e + 31) / 32 + 2 + 3) & ~3u : 0;
+        sh.excl_words = masked ? (per * e + 31) / 32 + 2 : 0;
         const size_t extra = sh.excl ? ((size_t)sh.excl_words + SPECIAL_LIST_CAP) * 4 : 0;
         sh.dyn_bytes = (size_t)CAND_CAP * 8 + extra;
         if (kmax > STREAM_K_MAX && sh.dyn_bytes < (size_t)SORT_SLOTS * 8) {

@@ -488,10 +488,9 @@ __device__ __forceinline__ bool select_fast(const RowArgs& a, const Geo<DT>& g, 
             return false;
         }
         sorted = false;
-        // (also drops the zeros; the sort's bins go where the list of specials was, which every round fills
-        // anew - the bitmap ahead of it is read again if the check below fails)
-        static_assert(SPECIAL_LIST_CAP >= SORT_BINS, "the bins take the list's place");
-        n = select_topk<true>(cand, n, k, sh, sorted, list);
+        // (also drops the zeros; within the candidates' own slots: the bitmap behind them is read again
+        // if the check below fails)
+        n = select_topk(cand, n, k, sh, sorted);
         // Every element that was not collected lies strictly below `filt`.  The result is
         // exact if k candidates were found and the k-th lies strictly above anything the
         // division could map an uncollected value to.

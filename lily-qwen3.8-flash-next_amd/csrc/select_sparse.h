@@ -177,17 +177,16 @@ __device__ __forceinline__ bool select_sparse(const RowArgs& a, const Geo<DT>& g
     }
     SPARSE_MARK(13);
     sorted = false;
-    if (cfg.slices > 1u && total <= k) {
-        // (all of them go to the workgroup that merges the slices, which drops the zeros)
+    if (cfg.slices > 1u ? total <= k : (k > 64u && total > 256u)) {
+        // (all of them go to the workgroup that merges the slices, which drops the zeros; a row that is one
+        // slice, of many candidates, to the sort that stands there)
         if (tid == 0) {
             sh.n_cand = total;
         }
         __syncthreads();
         return true;
     }
-    // (the staged bias list, and where other selects keep a bitmap, may lie under the bins: neither is
-    // read again)
-    const uint32_t n = select_topk<true>(cand, total, k, sh, sorted, reinterpret_cast<uint32_t*>(cand + SORT_PLACES));
+    const uint32_t n = select_topk(cand, total, k, sh, sorted);
     if (tid == 0) {
         sh.n_cand = n;
     }

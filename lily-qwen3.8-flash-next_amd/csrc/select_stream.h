@@ -331,7 +331,7 @@ __device__ __forceinline__ bool stream_accept(StreamLds& L, float filt, float te
         return true;
     }
     sorted = false;
-    n = select_topk<false>(L.fc, n, k, sh, sorted, nullptr);
+    n = select_topk(L.fc, n, k, sh, sorted);
     phase(cfg, 12);
     if (filt > F32_LOWEST) {
         uint32_t lowest = 0xffffffffu;
