@@ -118,6 +118,17 @@ __device__ __forceinline__ void read_again(RowArgs& a, const LILY_CONST RowArgs*
     apply_selection(a);
 }
 
+// The launch's settings once more, for the same reason.
+__device__ __forceinline__ void read_again(LaunchCfg& cfg, const LILY_CONST LaunchCfg* src) {
+    static_assert(sizeof(LaunchCfg) % 8 == 0, "LaunchCfg is copied in 8-byte pieces");
+    asm volatile("" : "+s"(src));
+    const LILY_CONST uint64_t* from = (const LILY_CONST uint64_t*)src;
+    uint64_t* to = reinterpret_cast<uint64_t*>(&cfg);
+    for (unsigned i = 0; i < sizeof(LaunchCfg) / 8; ++i) {
+        to[i] = from[i];
+    }
+}
+
 // The control block behind an acceptance of `acc` proposals (spec.metal:14-38).
 __device__ __forceinline__ void write_accepted(const LaunchCfg& cfg, uint32_t acc) {
     uint32_t* ctrl = cfg.accept_ctrl;
@@ -331,7 +342,8 @@ __device__ __forceinline__ bool finish_by_wave(const RowArgs& t, const LaunchCfg
 
 // True in the workgroup that finishes the row (the last of its slices to arrive).
 template <int DT, int KIND, bool LSE, bool CHAIN = false, bool SPEC = false>
-__device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const LaunchCfg& cfg, Shared& sh) {
+__device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const LaunchCfg& cfg, const LILY_CONST LaunchCfg* cfg_src,
+                                         Shared& sh) {
     if (cfg.served != nullptr && *(const LILY_CONST uint32_t*)(cfg.served + blockIdx.y) != 0u) {
         return false;
     }
@@ -440,7 +452,12 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
             if (!done) {
                 __syncthreads();
                 sorted = false;
-                select_exhaustive<DT>(f, fg.id_lo, fg.id_hi, f.k, want_lse, cand, cfg.cand_cap, sh);
+                // (read afresh for this select alone: of arguments that the selects above held as well,
+                // each element's evaluation reloaded up to 97 spilled lanes; 4 rows of 151 936 bf16 that
+                // come here, no top_k, 692 -> 531 us)
+                RowArgs e;
+                read_again(e, src);
+                select_exhaustive<DT>(e, fg.id_lo, fg.id_hi, e.k, want_lse, cand, cfg.cand_cap, sh);
             }
         }
         if (LSE && cfg.path_stats != nullptr && tid == 0) {
@@ -450,20 +467,28 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
 
     RowArgs t;
     read_again(t, src);
+    // The settings too, in the kernels that hold every select: what only the merge and the tail read
+    // was kept across the scan there and put the scan's own values into its loops as reloads (blocks
+    // of dense masks with row sums: 943 lane reads in a loop that has 108 now; 200 rows
+    // of them, k = 20, under penalties 140 -> 126 us).  Streaming rows' kernels have room for them.
+    LaunchCfg late = cfg;
+    if constexpr (KIND != 2 && !CHAIN) {
+        read_again(late, cfg_src);
+    }
     const bool forced = (t.flags & F_FORCED) != 0;
     // (the sparse select of a row in one slice leaves what it evaluated, which may be more than cand_cap)
-    const uint32_t n_cap = KIND == 1 ? max(cfg.cand_cap, min(cfg.dyn_slots, MERGE_CAP)) : cfg.cand_cap;
+    const uint32_t n_cap = KIND == 1 ? max(late.cand_cap, min(late.dyn_slots, MERGE_CAP)) : late.cand_cap;
     uint32_t n = (argmax || forced) ? 0u : min(sh.n_cand, n_cap);
-    phase(cfg, 4);
-    if (!CHAIN && S > 1 && !argmax && t.k <= 64u && cfg.ws_k <= 64u &&
-        (S <= WAVE_MERGE_LISTS || (t.k <= WAVE_MERGE_K && S * cfg.ws_k <= WAVE_MERGE_SLOTS)) &&
+    phase(late, 4);
+    if (!CHAIN && S > 1 && !argmax && t.k <= 64u && late.ws_k <= 64u &&
+        (S <= WAVE_MERGE_LISTS || (t.k <= WAVE_MERGE_K && S * late.ws_k <= WAVE_MERGE_SLOTS)) &&
         (t.mode != MODE_SPEC || (SPEC && *t.q_n <= 64u))) {
         if (tid >= 64u) {
             return false;
         }
-        const bool finished = finish_by_wave<DT, LSE, SPEC>(t, cfg, row, s, n, found, step, want_lse, sh);
+        const bool finished = finish_by_wave<DT, LSE, SPEC>(t, late, row, s, n, found, step, want_lse, sh);
         if (finished) {
-            phase(cfg, 7);
+            phase(late, 7);
         }
         return finished;
     }
@@ -525,22 +550,22 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
         // for its stores, the workgroup meets, and one thread takes the row's ticket.
         if (argmax) {
             if (tid == 0) {
-                handed_store(cfg.ws_cand, slot * cfg.ws_k, best);
+                handed_store(late.ws_cand, slot * late.ws_k, best);
             }
         } else {
             // Every slot is written (0 = no candidate), so the merge needs no counts.
-            for (uint32_t i = tid; !forced && i < cfg.ws_k; i += NT) {
-                handed_store(cfg.ws_cand, slot * cfg.ws_k + i, i < n ? found[i] : (uint64_t)0);
+            for (uint32_t i = tid; !forced && i < late.ws_k; i += NT) {
+                handed_store(late.ws_cand, slot * late.ws_k + i, i < n ? found[i] : (uint64_t)0);
             }
             if (tid == 0) {
-                handed_store(cfg.ws_lse, 2 * slot, want_lse ? sh.lse_mc : 0.0);
-                handed_store(cfg.ws_lse, 2 * slot + 1, want_lse ? sh.lse_s : 0.0);
+                handed_store(late.ws_lse, 2 * slot, want_lse ? sh.lse_mc : 0.0);
+                handed_store(late.ws_lse, 2 * slot + 1, want_lse ? sh.lse_s : 0.0);
             }
         }
         // The hand-over (last_to_arrive(): a release on the ticket and an acquire behind it, or
         // the relaxed form described there).
-        const bool last = last_to_arrive(&cfg.ws_ticket[row], S, sh.last, cfg.relaxed_handover != 0u);
-        phase(cfg, 5);
+        const bool last = last_to_arrive(&late.ws_ticket[row], S, sh.last, late.relaxed_handover != 0u);
+        phase(late, 5);
         if (!last) {
             return false;
         }
@@ -548,7 +573,7 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
         if (argmax) {
             best = 0;
             for (uint32_t t = tid; t < S; t += NT) {
-                const uint64_t c = handed_load(cfg.ws_cand, (base + t) * cfg.ws_k);
+                const uint64_t c = handed_load(late.ws_cand, (base + t) * late.ws_k);
                 best = c > best ? c : best;
             }
             best = wave_max_u64(best);
@@ -563,17 +588,17 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
         } else {
             // Gather every slice's candidates (0 = no candidate) and the log-sum-exp partials
             // in one round trip.
-            slots = S * cfg.ws_k;
+            slots = S * late.ws_k;
 #pragma unroll
             for (int q = 0; q < PER; ++q) {
                 const uint32_t j = tid + (uint32_t)q * NT;
-                mine[q] = (!forced && j < slots) ? handed_load(cfg.ws_cand, base * cfg.ws_k + j) : 0ull;
+                mine[q] = (!forced && j < slots) ? handed_load(late.ws_cand, base * late.ws_k + j) : 0ull;
             }
             if (want_lse && tid < 64) {
                 double mt = -__builtin_huge_val(), st = 0.0;
                 if (tid < S) {
-                    mt = handed_load(cfg.ws_lse, 2 * (base + tid));
-                    st = handed_load(cfg.ws_lse, 2 * (base + tid) + 1);
+                    mt = handed_load(late.ws_lse, 2 * (base + tid));
+                    st = handed_load(late.ws_lse, 2 * (base + tid) + 1);
                     if (!(st > 0.0)) {
                         mt = -__builtin_huge_val();
                     }
@@ -601,7 +626,7 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
         rank_them();
     }
 
-    phase(cfg, 6);
+    phase(late, 6);
     if (argmax) {
         if (tid == 0) {
             const uint32_t id = composite_id(best);
@@ -615,26 +640,26 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
         }
         return true;
     }
-    if (CHAIN && cfg.chain_rows != 0u) {
+    if (CHAIN && late.chain_rows != 0u) {
         // Rows that draw in order.  This row's candidates - the best t.k under the counts as they
         // stood when the launch began, t.k being the draw's own count plus one for every row
         // before it - are published; the workgroup that publishes last takes the rows one after
         // the other: the ids the earlier rows drew are evaluated again (penalties that can only
         // lower took them down, so the best k_draw of the row as it stands now are still among
         // the candidates), and the tail draws from the best k_draw.
-        const uint32_t rows = cfg.chain_rows;
+        const uint32_t rows = late.chain_rows;
         for (uint32_t i = tid; i < n; i += NT) {
-            handed_store(cfg.chain_cand, (size_t)row * CHAIN_CAP + i, found[i]);
+            handed_store(late.chain_cand, (size_t)row * CHAIN_CAP + i, found[i]);
         }
         if (tid == 0) {
-            handed_store(cfg.chain_n, row, n);
+            handed_store(late.chain_n, row, n);
         }
-        if (!last_to_arrive(cfg.chain_ticket, rows, sh.last, cfg.relaxed_handover != 0u)) {
+        if (!last_to_arrive(late.chain_ticket, rows, sh.last, late.relaxed_handover != 0u)) {
             return false;
         }
         const LILY_CONST RowArgs* first = src - row;
-        if (cfg.accept_ctrl != nullptr && tid < rows) {
-            sh.proposal[tid] = gload(cfg.accept_ids + tid);
+        if (late.accept_ctrl != nullptr && tid < rows) {
+            sh.proposal[tid] = gload(late.accept_ids + tid);
         }
         // Every row's first 64 candidates, their raw logits and their counts as they stand before
         // any of these rows has drawn are requested together (a wave per row, two rounds for
@@ -653,11 +678,11 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
         for (uint32_t j0 = 0; j0 < rows; j0 += NWAVE) {
             const uint32_t j = j0 + (tid >> 6), lane = tid & 63u;
             if (j < rows) {
-                const uint32_t nj = min(handed_load(cfg.chain_n, j), CHAIN_CAP);
+                const uint32_t nj = min(handed_load(late.chain_n, j), CHAIN_CAP);
                 if (lane == 0) {
                     sh.chain_n[j] = nj;
                 }
-                const uint64_t c = handed_load(cfg.chain_cand, (size_t)j * CHAIN_CAP + lane);
+                const uint64_t c = handed_load(late.chain_cand, (size_t)j * CHAIN_CAP + lane);
                 const uint32_t id = min(composite_id(c), vocab - 1u);
                 pre_c[j * PRE + lane] = c;
                 pre_l[j * PRE + lane] = load_logit<DT>((first + j)->logits, id);
@@ -676,7 +701,7 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
         __syncthreads();
         for (uint32_t j = 0; j < rows; ++j) {
 #ifdef LILY_CHAIN_TRACE
-            phase(cfg, 8 + j);
+            phase(late, 8 + j);
 #endif
             RowArgs r;
             {
@@ -709,7 +734,7 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
                 __threadfence();
                 __syncthreads();
                 for (uint32_t i = tid + PRE; i < n_now; i += NT) {
-                    const uint64_t c = handed_load(cfg.chain_cand, (size_t)j * CHAIN_CAP + i);
+                    const uint64_t c = handed_load(late.chain_cand, (size_t)j * CHAIN_CAP + i);
                     const uint32_t id = composite_id(c);
                     cand[i] = times_drawn(id) == 0u
                                   ? c
@@ -755,7 +780,7 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
                 r.q_ids = pre_qid + j * PRE;
                 r.q_probs = pre_qp + j * PRE;
             }
-            tail<DT, KIND != 2, true>(r, vocab, r.step + cfg.step_delta, n_now, ranked, cand, sh, cfg);
+            tail<DT, KIND != 2, true>(r, vocab, r.step + late.step_delta, n_now, ranked, cand, sh, late);
             // The workgroup meets over LDS only: a barrier that also waited for thread 0's stores
             // and increments to be acknowledged by memory would cost every row a round trip
             // that nothing here depends on.
@@ -782,19 +807,19 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
                 mine->touched[words + 1u] = id;
             }
         }
-        if (cfg.accept_ctrl != nullptr && tid == 0) {
+        if (late.accept_ctrl != nullptr && tid == 0) {
             // spec_accept (spec.metal:14-38) on the draws this workgroup just made.
             uint32_t acc = 0;
             while (acc + 1 < rows && sh.drawn[acc] == sh.proposal[acc + 1]) {
                 ++acc;
             }
-            write_accepted(cfg, acc);
+            write_accepted(late, acc);
         }
-        phase(cfg, 7);
+        phase(late, 7);
         return true;
     }
-    tail<DT, KIND != 2, SPEC>(t, vocab, step, n, sorted, found, sh, cfg);
-    phase(cfg, 7);
+    tail<DT, KIND != 2, SPEC>(t, vocab, step, n, sorted, found, sh, late);
+    phase(late, 7);
     return true;
 }
 
@@ -819,7 +844,7 @@ __global__ __launch_bounds__(NT, KIND == 1 ? 3 : 4) void k_rows_inline(InlineRow
         tail_arrays(sh);
     }
     __syncthreads();
-    row_body<DT, KIND, LSE>(table + blockIdx.y, cfg, sh);
+    row_body<DT, KIND, LSE>(table + blockIdx.y, cfg, (const LILY_CONST LaunchCfg*)(table + INLINE_ROWS), sh);
 }
 
 // Rows that draw in order (the verify pass under penalties): see row_body.
@@ -832,7 +857,7 @@ __global__ __launch_bounds__(NT, KIND == 1 ? 3 : 4) void k_rows_chain(InlineRows
         tail_arrays(sh);
     }
     __syncthreads();
-    row_body<DT, KIND, false, true>(table + blockIdx.y, cfg, sh);
+    row_body<DT, KIND, false, true>(table + blockIdx.y, cfg, (const LILY_CONST LaunchCfg*)(table + INLINE_ROWS), sh);
 }
 
 // A verify pass whose rows are independent: the one-wave form of the speculative draw is compiled in,
@@ -847,7 +872,7 @@ __global__ __launch_bounds__(NT, KIND == 1 ? 3 : 4) void k_rows_verify(InlineRow
         tail_arrays(sh);
     }
     __syncthreads();
-    const bool finished = row_body<DT, KIND, false, false, true>(table + blockIdx.y, cfg, sh);
+    const bool finished = row_body<DT, KIND, false, false, true>(table + blockIdx.y, cfg, (const LILY_CONST LaunchCfg*)(table + INLINE_ROWS), sh);
     if (!finished || threadIdx.x != 0 || cfg.accept_ctrl == nullptr) {
         return;
     }
@@ -862,7 +887,7 @@ __global__ __launch_bounds__(NT, KIND == 1 ? 3 : 4) void k_rows_table(LaunchCfg 
         tail_arrays(sh);
     }
     __syncthreads();
-    row_body<DT, KIND, LSE>(table + blockIdx.y, cfg, sh);
+    row_body<DT, KIND, LSE>(table + blockIdx.y, cfg, (const LILY_CONST LaunchCfg*)__builtin_amdgcn_kernarg_segment_ptr(), sh);
 }
 
 template <int DT, int KIND, bool LSE>
