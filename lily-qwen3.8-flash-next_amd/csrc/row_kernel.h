@@ -895,22 +895,22 @@ static hipError_t launch_variant(hipStream_t stream, uint32_t rows, const Launch
                                  const InlineRows* inline_rows, size_t dyn_bytes) {
     const dim3 grid(cfg.slices, rows), block(NT);
     if (cfg.chain_rows != 0u) {
-        if constexpr (!LSE) {
+        if constexpr (!LSE && KIND != 0) {
             if (inline_rows != nullptr) {
                 hipLaunchKernelGGL((k_rows_chain<DT, KIND>), grid, block, dyn_bytes, stream, *inline_rows, cfg);
                 return hipGetLastError();
             }
         }
-        return hipErrorInvalidValue;   // rows that draw in order travel inline and want no row sum
+        return hipErrorInvalidValue;   // rows that draw in order are under penalties, travel inline, want no row sum
     }
     if (cfg.verify != 0u) {
-        if constexpr (!LSE) {
+        if constexpr (!LSE && KIND != 1) {
             if (inline_rows != nullptr) {
                 hipLaunchKernelGGL((k_rows_verify<DT, KIND>), grid, block, dyn_bytes, stream, *inline_rows, cfg);
                 return hipGetLastError();
             }
         }
-        return hipErrorInvalidValue;   // (the same of a verify pass)
+        return hipErrorInvalidValue;   // (independent rows of a verify pass: no penalties, masks or bias lists)
     }
     if (inline_rows != nullptr) {
         hipLaunchKernelGGL((k_rows_inline<DT, KIND, LSE>), grid, block, dyn_bytes, stream,
