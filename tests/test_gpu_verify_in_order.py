@@ -15,7 +15,8 @@ pytestmark = pytest.mark.gpu
 
 
 def _flow(sampler, target, draft, kw, step0, uniforms=None, hist=None):
-    """Runs draft draws + lily_spec_verify and the oracle's sequence; returns (got, want, counts ok)."""
+    """Runs draft draws + lily_spec_verify and the oracle's sequence; returns (got, want, counts ok, path
+    counters and the accepted proposals)."""
     m, vocab = target.shape
     bf16 = target.dtype == np.uint16
     up = (lambda a: torch.from_numpy(a.view(np.int16)).to(dev()).view(torch.bfloat16)) if bf16 else \
@@ -71,7 +72,7 @@ def _flow(sampler, target, draft, kw, step0, uniforms=None, hist=None):
     assert np.array_equal(ctrl.cpu().numpy().view(np.uint32), wctrl)
     scratch.close()
     dists.close()
-    return list(got), want, ok, stats.cpu().tolist()
+    return list(got), want, ok, stats.cpu().tolist() + [int(wctrl[0])]
 
 
 @pytest.mark.parametrize("m", [2, 3, 5, 8])
@@ -173,4 +174,32 @@ def test_massless_residual_in_the_one_launch_form(outside):
         assert np.array_equal(scratch.read_counts().numpy().view(np.uint32), counts)
         scratch.close()
         dists.close()
+    s.close()
+
+
+@pytest.mark.parametrize("m", [2, 5, 8])
+@pytest.mark.parametrize("k", ["greedy", 64, 1024])
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+def test_acceptance_behind_independent_rows(m, k, bf16):
+    """Rows without penalties: the workgroup that finishes the last of them writes the control
+    block - behind the kernel of greedy rows, the streaming one (k 64) and the one that sorts many
+    candidates (k 1 024, draft distributions of hundreds of ids).  Row q's draft is drawn from
+    other logits, so that the acceptance ends at every row in turn (a sampled row ahead of it may end
+    it too); the last pass changes none.
+    Each pass runs behind another on the same sampler: the rows' ticket is left as it was found."""
+    s = LS.Sampler(0)
+    rng = np.random.default_rng(10 * m + bf16)
+    vocab = 60_013
+    target = rng.normal(0, 1, (m, vocab)).astype(np.float32)
+    hot = np.array([rng.choice(vocab, 6, replace=False) for _ in range(m)])
+    np.put_along_axis(target, hot, np.float32([11.0, 10.9, 10.8, 10.7, 10.6, 10.5]), 1)
+    kw = dict() if k == "greedy" else dict(temperature=1.0, top_k=0 if k == 1024 else k, top_p=0.95, seed=23)
+    for q in range(m):
+        draft = target + rng.normal(0, 0.01, target.shape).astype(np.float32)
+        if q + 1 < m:
+            draft[q] = np.roll(target[q], 1000)      # (other favourites: the proposal is rejected)
+        sides = (W.to_bf16_bits(target), W.to_bf16_bits(draft)) if bf16 else (target, draft)
+        got, want, _, st = _flow(s, *sides, kw, 30 * q)
+        assert got == want, (m, k, bf16, q, got, want)
+        assert st[4] == q if k == "greedy" else st[4] <= q, (m, k, bf16, q, st)
     s.close()
