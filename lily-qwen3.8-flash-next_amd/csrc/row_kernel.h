@@ -179,18 +179,18 @@ __device__ __forceinline__ bool lowering_row(const RowArgs& a) {
 // nothing left to do and are gone.  It stores its candidates, takes the row's ticket and, if it is the
 // last, gathers every slice's, keeps the row's best (a candidate per lane, in order) and draws.
 // (With the workgroup's four waves meeting at eight barriers from here to the draw: 7.6 us of the 13.2
-// that one sampled row of 151 936 f32 logits takes in 38 slices; now 6 of 12.1.)
-constexpr uint32_t WAVE_MERGE_SLOTS = 2048;   // entries the wave gathers at most, 32 a lane
+// that one sampled row of 151 936 f32 logits takes in 38 slices; now 6 of 11.8.)
+// Entries the wave gathers at most, 32 a lane.  Up to there it is the faster way for every k, dtype and kind of
+// row: 4 to 100 rows of 151 936 in 5 to 38 slices, k 3 to 60: 0.77 to 1.00 of the workgroup's merge (24 f32
+// rows, k = 50: 19.9 and 21.3 us), k = 64 0.79 to 0.96 (22.0 and 26.3); bf16 rows near k = 62 up to 1.03, where
+// equal values at the k-th take a second sort.
+constexpr uint32_t WAVE_MERGE_SLOTS = 2048;
 // Up to this many slices their lists are merged one by one: a merge is a chain of seven exchanges
 // and the lists follow one another, where the bound of more slices' entries, and one sort of those that
 // reach it, cost the same for six as for thirty-eight.  (Six slices, lists one by one -> this: k = 3
 // 25.6 -> 19.8 us, k = 50 28.3 -> 25.1 for 90 rows of 248 320 bf16; k = 3 17.4 -> 10.1, k = 20 17.9 -> 11.7
 // for 6 rows of 50 001 in seven.)
 constexpr uint32_t WAVE_MERGE_LISTS = 3;
-// Above this k the bound of two values a lane lets too many entries through and the workgroup's four
-// waves merge more lists faster (15 rows of 151 936 f32 under masks, k = 50: 20.4 us by the workgroup,
-// 20.9 by the wave; 24 under penalties 33.8 and 31.7; plain rows, k = 64: 34.4 and 42.4).
-constexpr uint32_t WAVE_MERGE_K = 50;
 
 __device__ __forceinline__ bool descending(uint64_t c) {   // lane by lane, equal only where both are 0
     const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)(uint32_t)c, 0x138, 0xf, 0xf, false);   // wave_shr:1
@@ -204,9 +204,21 @@ __device__ __forceinline__ bool finish_by_wave(const RowArgs& t, const LaunchCfg
     const uint32_t lane = threadIdx.x, S = cfg.slices, vocab = cfg.vocab;
     const bool forced = (t.flags & F_FORCED) != 0u;
     const size_t slot = (size_t)row * S + s;
-    // Every place is written (0 = no candidate), so the merge needs no counts.
+    // Every place is written (0 = no candidate), so the merge needs no counts.  Its lanes take every 64th
+    // place, and its bound wants the row's best spread evenly over them: the slices' best begin 64 / S lanes
+    // apart, each list turned within its places.  (Unturned, lists of k = 64 put the same rank of every slice
+    // into a lane, and the bound let 700 of 2 048 entries through; so did, less so, every k near 64 or with
+    // a large factor in common with it.  Turned, those that pass are one sort, rarely two.  Any turn is
+    // a right one, so rounded reciprocals will do.)
+    uint32_t turn = 0u;
+    if (S > WAVE_MERGE_LISTS) {
+        const float slices = (float)S, places = (float)cfg.ws_k;
+        const uint32_t at = ((uint32_t)(64.0f * (float)s * __builtin_amdgcn_rcpf(slices)) - s * cfg.ws_k) & 63u;
+        turn = min(at - (uint32_t)((float)at * __builtin_amdgcn_rcpf(places)) * cfg.ws_k, cfg.ws_k - 1u);
+    }
     for (uint32_t i = lane; !forced && i < cfg.ws_k; i += 64u) {
-        handed_store(cfg.ws_cand, slot * cfg.ws_k + i, i < n ? found[i] : (uint64_t)0);
+        const uint32_t rank = i < turn ? i + cfg.ws_k - turn : i - turn;
+        handed_store(cfg.ws_cand, slot * cfg.ws_k + i, rank < n ? found[rank] : (uint64_t)0);
     }
     if (LSE && lane == 0u) {
         handed_store(cfg.ws_lse, 2 * slot, want_lse ? sh.lse_mc : 0.0);
@@ -264,23 +276,21 @@ __device__ __forceinline__ bool finish_by_wave(const RowArgs& t, const LaunchCfg
                 }
             }
         }
-        uint32_t lane_best = 0u, lane_next = 0u;   // the upper 16 bits of a lane's two best
+        uint32_t lane_best = 0u, lane_next = 0u;   // the keys of a lane's two best
 #pragma unroll
         for (int q = 0; q < PER; ++q) {
             mine[q] = lane + (uint32_t)q * 64u < slots ? mine[q] : 0ull;
-            const uint32_t key = (uint32_t)(mine[q] >> 48);
+            const uint32_t key = (uint32_t)(mine[q] >> 32);
             lane_next = max(lane_next, min(lane_best, key));
             lane_best = max(lane_best, key);
         }
-        // The k-th largest of the lanes' two best bounds the k-th entry: at least k entries reach it
-        // (more than there are with fewer than k: all of them); what does not is dropped, the rest is
-        // listed, and the list's entries are taken in 64 at a time.  Of one value a lane, the bound for
-        // k = 64 was the least of 64 maxima, which most entries reached: 10 rows of 65 695 f32 in 17
-        // slices took 46 us, 33 with two, 27 with the workgroup's merge; k = 50, 24 rows under penalties
-        // 33.8 with the workgroup's merge, 31.7 with two.
+        // The k-th largest of the lanes' two best, to 20 bits of its key, bounds the k-th entry: at least k
+        // entries reach it (more than there are with fewer than k: all of them); what does not is dropped,
+        // the rest is listed, and the list's entries are taken in 64 at a time.  (To 16 bits some three
+        // f32 entries share the k-th's: above k = 58 a second sort, 1.0 us, for as many rows as not.)
         uint32_t bound = 0u;
 #pragma unroll
-        for (int bit = 15; bit >= 0; --bit) {
+        for (int bit = 31; bit >= 12; --bit) {
             const uint32_t at = bound | (1u << bit);
             const uint32_t reach = (uint32_t)__popcll(__ballot(lane_best >= at)) + (uint32_t)__popcll(__ballot(lane_next >= at));
             bound = reach >= t.k ? at : bound;
@@ -292,7 +302,7 @@ __device__ __forceinline__ bool finish_by_wave(const RowArgs& t, const LaunchCfg
             if ((uint32_t)q0 * 64u < slots) {
 #pragma unroll
                 for (int q = q0; q < q0 + GROUP; ++q) {
-                    const bool in = mine[q] != 0ull && (uint32_t)(mine[q] >> 48) >= bound;
+                    const bool in = mine[q] != 0ull && (uint32_t)(mine[q] >> 32) >= bound;
                     const uint64_t mask = __ballot(in);
                     if (mask != 0ull) {
                         const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
@@ -481,7 +491,7 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
     uint32_t n = (argmax || forced) ? 0u : min(sh.n_cand, n_cap);
     phase(late, 4);
     if (!CHAIN && S > 1 && !argmax && t.k <= 64u && late.ws_k <= 64u &&
-        (S <= WAVE_MERGE_LISTS || (t.k <= WAVE_MERGE_K && S * late.ws_k <= WAVE_MERGE_SLOTS)) &&
+        (S <= WAVE_MERGE_LISTS || S * late.ws_k <= WAVE_MERGE_SLOTS) &&
         (t.mode != MODE_SPEC || (SPEC && *t.q_n <= 64u))) {
         if (tid >= 64u) {
             return false;

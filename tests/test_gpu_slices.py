@@ -1,6 +1,6 @@
 """Rows cut into slices: the one-wave merge and draw of rows of few candidates (k <= 64), on both
 sides of the limits at which it lists the slices' candidates, merges them list by list or leaves
-them to the whole workgroup; and launches of greedy rows.  Bit-exact against the oracle."""
+them (more than 2 048 places) to the whole workgroup; and launches of greedy rows.  Bit-exact against the oracle."""
 import os
 
 import numpy as np
@@ -52,6 +52,21 @@ def test_rows_of_few_candidates_over_slices(slices, bf16):
                 check_row_against_oracle(r, i, d)
                 if lp and np.isfinite(d.logprob):
                     assert abs(r.logprobs[i] - d.logprob) <= 1e-5 * max(1.0, abs(d.logprob)), (k, i)
+    s.close()
+
+
+@pytest.mark.parametrize("slices", [3, 4, 31, 64])
+@pytest.mark.parametrize("ks", [(64, 2, 33, 20, 7), (63, 61, 5, 48, 32), (31, 3, 30, 2, 17)])
+def test_rows_of_different_k_over_slices(slices, ks):
+    """A slice's list has as many places as the launch's largest k asks for, and is turned within
+    them: rows whose lists fill a few of them only."""
+    s = _sampler(slices)
+    rng = np.random.default_rng(slices)
+    x = _rows(rng, 5, 131_075, False)
+    kw = [dict(temperature=0.7, top_k=k, top_p=0.97, seed=90 + r) for r, k in enumerate(ks)]
+    r = run_rows(s, x, kw, [3] * 5)
+    for i in range(5):
+        check_row_against_oracle(r, i, O.sample(x[i], None, o_params(**kw[i]), 3))
     s.close()
 
 
