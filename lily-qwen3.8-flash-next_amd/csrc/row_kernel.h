@@ -206,15 +206,14 @@ __device__ __forceinline__ bool finish_by_wave(const RowArgs& t, const LaunchCfg
     const size_t slot = (size_t)row * S + s;
     // Every place is written (0 = no candidate), so the merge needs no counts.  Its lanes take every 64th
     // place, and its bound wants the row's best spread evenly over them: the slices' best begin 64 / S lanes
-    // apart, each list turned within its places.  (Unturned, lists of k = 64 put the same rank of every slice
-    // into a lane, and the bound let 700 of 2 048 entries through; so did, less so, every k near 64 or with
-    // a large factor in common with it.  Turned, those that pass are one sort, rarely two.  Any turn is
-    // a right one, so rounded reciprocals will do.)
+    // apart, each list turned within its places.  (Unturned, lists of 64 put the same rank of every slice
+    // into a lane, and the bound let 700 of 2 048 entries through; so did, less so, every length near 64
+    // or with a large factor in common with it.  Turned, those that pass are one sort, rarely two; of
+    // lists shorter than 32 they always are.  Any turn is a right one, so a rounded reciprocal will do.)
     uint32_t turn = 0u;
-    if (S > WAVE_MERGE_LISTS) {
-        const float slices = (float)S, places = (float)cfg.ws_k;
-        const uint32_t at = ((uint32_t)(64.0f * (float)s * __builtin_amdgcn_rcpf(slices)) - s * cfg.ws_k) & 63u;
-        turn = min(at - (uint32_t)((float)at * __builtin_amdgcn_rcpf(places)) * cfg.ws_k, cfg.ws_k - 1u);
+    if (S > WAVE_MERGE_LISTS && cfg.ws_k >= 32u) {
+        turn = ((uint32_t)(64.0f * (float)s * __builtin_amdgcn_rcpf((float)S)) - s * cfg.ws_k) & 63u;
+        turn = turn >= cfg.ws_k ? turn - cfg.ws_k : turn;
     }
     for (uint32_t i = lane; !forced && i < cfg.ws_k; i += 64u) {
         const uint32_t rank = i < turn ? i + cfg.ws_k - turn : i - turn;
@@ -284,16 +283,26 @@ __device__ __forceinline__ bool finish_by_wave(const RowArgs& t, const LaunchCfg
             lane_next = max(lane_next, min(lane_best, key));
             lane_best = max(lane_best, key);
         }
-        // The k-th largest of the lanes' two best, to 20 bits of its key, bounds the k-th entry: at least k
-        // entries reach it (more than there are with fewer than k: all of them); what does not is dropped,
-        // the rest is listed, and the list's entries are taken in 64 at a time.  (To 16 bits some three
-        // f32 entries share the k-th's: above k = 58 a second sort, 1.0 us, for as many rows as not.)
+        // The k-th largest of the lanes' two best bounds the k-th entry: at least k entries reach it (more
+        // than there are with fewer than k: all of them); what does not is dropped, the rest is listed, and
+        // the list's entries are taken in 64 at a time.  Sixteen bits of the key let some three f32 entries
+        // through that share the k-th's: above k = 50 a second sort in some row of a launch, 1.0 us, which
+        // four more bits (0.2 us) save.
         uint32_t bound = 0u;
-#pragma unroll
-        for (int bit = 31; bit >= 12; --bit) {
+        auto settle = [&](int bit) {
             const uint32_t at = bound | (1u << bit);
             const uint32_t reach = (uint32_t)__popcll(__ballot(lane_best >= at)) + (uint32_t)__popcll(__ballot(lane_next >= at));
             bound = reach >= t.k ? at : bound;
+        };
+#pragma unroll
+        for (int bit = 31; bit >= 16; --bit) {
+            settle(bit);
+        }
+        if (t.k > 50u) {
+#pragma unroll
+            for (int bit = 15; bit >= 12; --bit) {
+                settle(bit);
+            }
         }
         uint64_t* cand = dyn_lds;
         uint32_t kept = 0;
