@@ -144,6 +144,10 @@ struct LaunchCfg {
     // 1 = the launch of a verify pass whose rows are independent: the kernel that holds the one-wave
     // form of the speculative draw, and the acceptance behind the last row (accept_*, chain_ticket)
     uint32_t verify;
+    // by how many places (16.16, modulo 64) a slice's list of candidates is turned more than the list of the
+    // slice before it, for the merge by one wave (merge_turn_step())
+    uint32_t turn_step;
+    uint32_t pad_cfg;
 };
 
 constexpr uint32_t CHAIN_CAP = LILY_SAMPLE_K_CAP;   // candidates a chained row publishes
@@ -161,6 +165,12 @@ constexpr uint32_t SORT_PLACES = 2048;   // the sort of many candidates: its pla
 constexpr uint32_t SORT_BINS = 2048;     // candidates, and its bins' 32-bit words
 constexpr uint32_t SORT_SLOTS = SORT_PLACES + SORT_BINS / 2;   // 64-bit slots it works in, the bins behind the places
 constexpr uint32_t MAX_SLICES = 64;
+// Up to this many slices their lists are merged one by one: a merge is a chain of seven exchanges
+// and the lists follow one another, where the bound of more slices' entries, and one sort of those that
+// reach it, cost the same for six as for thirty-eight.  (Six slices, lists one by one -> this: k = 3
+// 25.6 -> 19.8 us, k = 50 28.3 -> 25.1 for 90 rows of 248 320 bf16; k = 3 17.4 -> 10.1, k = 20 17.9 -> 11.7
+// for 6 rows of 50 001 in seven.)
+constexpr uint32_t WAVE_MERGE_LISTS = 3;
 constexpr uint32_t SPECIAL_LIST_CAP = 2048;  // ids of penalised / biased tokens gathered per batch
 
 // Streaming select (k <= STREAM_K_MAX): dynamic LDS layout in bytes.

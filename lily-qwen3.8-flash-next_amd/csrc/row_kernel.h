@@ -182,15 +182,9 @@ __device__ __forceinline__ bool lowering_row(const RowArgs& a) {
 // that one sampled row of 151 936 f32 logits takes in 38 slices; now 6 of 11.8.)
 // Entries the wave gathers at most, 32 a lane.  Up to there it is the faster way for every k, dtype and kind of
 // row: 4 to 100 rows of 151 936 in 5 to 38 slices, k 3 to 60: 0.77 to 1.00 of the workgroup's merge (24 f32
-// rows, k = 50: 19.9 and 21.3 us), k = 64 0.79 to 0.96 (22.0 and 26.3); bf16 rows near k = 62 up to 1.03, where
+// rows, k = 50: 19.8 and 21.3 us), k = 64 0.76 to 0.97 (22.1 and 26.4); bf16 rows near k = 62 up to 1.04, where
 // equal values at the k-th take a second sort.
 constexpr uint32_t WAVE_MERGE_SLOTS = 2048;
-// Up to this many slices their lists are merged one by one: a merge is a chain of seven exchanges
-// and the lists follow one another, where the bound of more slices' entries, and one sort of those that
-// reach it, cost the same for six as for thirty-eight.  (Six slices, lists one by one -> this: k = 3
-// 25.6 -> 19.8 us, k = 50 28.3 -> 25.1 for 90 rows of 248 320 bf16; k = 3 17.4 -> 10.1, k = 20 17.9 -> 11.7
-// for 6 rows of 50 001 in seven.)
-constexpr uint32_t WAVE_MERGE_LISTS = 3;
 
 __device__ __forceinline__ bool descending(uint64_t c) {   // lane by lane, equal only where both are 0
     const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)(uint32_t)c, 0x138, 0xf, 0xf, false);   // wave_shr:1
@@ -206,15 +200,12 @@ __device__ __forceinline__ bool finish_by_wave(const RowArgs& t, const LaunchCfg
     const size_t slot = (size_t)row * S + s;
     // Every place is written (0 = no candidate), so the merge needs no counts.  Its lanes take every 64th
     // place, and its bound wants the row's best spread evenly over them: the slices' best begin 64 / S lanes
-    // apart, each list turned within its places.  (Unturned, lists of 64 put the same rank of every slice
-    // into a lane, and the bound let 700 of 2 048 entries through; so did, less so, every length near 64
-    // or with a large factor in common with it.  Turned, those that pass are one sort, rarely two; of
-    // lists shorter than 32 they always are.  Any turn is a right one, so a rounded reciprocal will do.)
-    uint32_t turn = 0u;
-    if (S > WAVE_MERGE_LISTS && cfg.ws_k >= 32u) {
-        turn = ((uint32_t)(64.0f * (float)s * __builtin_amdgcn_rcpf((float)S)) - s * cfg.ws_k) & 63u;
-        turn = turn >= cfg.ws_k ? turn - cfg.ws_k : turn;
-    }
+    // apart, each list turned within its places (LaunchCfg::turn_step).  (Unturned, lists of 64 put the same
+    // rank of every slice into a lane, and the bound let 700 of 2 048 entries through; so did, less so,
+    // every length near 64 or with a large factor in common with it.  Turned, those that pass are one
+    // sort, rarely two.  Worked out here from S it took every row 0.1 us.)
+    uint32_t turn = (s * cfg.turn_step >> 16) & 63u;
+    turn = turn >= cfg.ws_k ? turn - cfg.ws_k : turn;
     for (uint32_t i = lane; !forced && i < cfg.ws_k; i += 64u) {
         const uint32_t rank = i < turn ? i + cfg.ws_k - turn : i - turn;
         handed_store(cfg.ws_cand, slot * cfg.ws_k + i, rank < n ? found[rank] : (uint64_t)0);
@@ -431,9 +422,10 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
         }
         // The other selects.  Launches with row sums read the arguments afresh for them: kept across
         // the streaming scan they made it spill (200 rows in three slices 46.7 -> 45.7 us).  Launches
-        // without hold fewer values and keep them; the order of the statement below is part of
-        // that (behind the exhaustive select it draws the merge's loads, and a wait for them, ahead
-        // of every row: 6.30 -> 6.50 us for one greedy row).
+        // without hold fewer values and keep them, and each select below asks by itself whether it is
+        // still wanted: asked once around them, the merge's loads, and a wait for them, are drawn ahead of
+        // every row (one sampled row 11.7 -> 11.9 us, a greedy one beside it 11.6 -> 11.7, four rows
+        // under penalties 14.8 -> 14.9).
         if (!LSE || !done) {
             RowArgs f = a;
             Geo<DT> fg = g;
@@ -471,11 +463,14 @@ __device__ __forceinline__ bool row_body(const LILY_CONST RowArgs* src, const La
             if (!done) {
                 __syncthreads();
                 sorted = false;
-                // (read afresh for this select alone: of arguments that the selects above held as well,
-                // each element's evaluation reloaded up to 97 spilled lanes; 4 rows of 151 936 bf16 that
-                // come here, no top_k, 692 -> 531 us)
-                RowArgs e;
-                read_again(e, src);
+                // (in the kernels that hold the others read afresh for this select alone: of arguments that
+                // those held as well, each element's evaluation reloaded up to 97 spilled lanes; 4 rows of
+                // 151 936 bf16 that come here, no top_k, 692 -> 531 us.  The streaming rows' kernels spill
+                // none of them: one sampled row 11.83 us without, 11.93 with)
+                RowArgs e = f;
+                if constexpr (KIND != 2) {
+                    read_again(e, src);
+                }
                 select_exhaustive<DT>(e, fg.id_lo, fg.id_hi, e.k, want_lse, cand, cfg.cand_cap, sh);
             }
         }

@@ -350,6 +350,12 @@ uint32_t choose_slices(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint
 // 72 that 64 rows of 1 024 candidates take over 2 x 1 024 workgroups; 1.2 us of a 4-row step).
 constexpr uint32_t RELAXED_MIN_GROUPS = 256;
 
+// LaunchCfg::turn_step: list s, whose first place lies s * k places on, shall begin at lane 64 * s / slices.
+// Lists shorter than 32 spread over the lanes by themselves, those merged one by one keep their order.
+uint32_t merge_turn_step(uint32_t slices, uint32_t k) {
+    return slices > WAVE_MERGE_LISTS && k >= 32u && k <= 64u ? (64u << 16) / slices - (k << 16) : 0u;
+}
+
 void fill_cfg(const lily_sampler* s, LaunchCfg* cfg, uint32_t rows, uint32_t vocab, uint32_t slices,
               uint32_t kmax, uint32_t step_delta, const RowArgs* table) {
     std::memset(cfg, 0, sizeof *cfg);
@@ -360,6 +366,7 @@ void fill_cfg(const lily_sampler* s, LaunchCfg* cfg, uint32_t rows, uint32_t voc
     cfg->slices = slices;
     cfg->step_delta = step_delta;
     cfg->ws_k = kmax ? kmax : 1;
+    cfg->turn_step = merge_turn_step(slices, cfg->ws_k);
     cfg->ws_cand = Handed<uint64_t>{s->ws_cand};
     cfg->ws_lse = Handed<double>{s->ws_lse};
     cfg->ws_ticket = s->ws_ticket;
