@@ -179,9 +179,10 @@ __device__ __forceinline__ bool lowering_row(const RowArgs& a) {
 // nothing left to do and are gone.  It stores its candidates, takes the row's ticket and, if it is the
 // last, gathers every slice's, keeps the row's best (a candidate per lane, in order) and draws.
 // (With the workgroup's four waves meeting at eight barriers from here to the draw: 7.6 us of the 13.2
-// that one sampled row of 151 936 f32 logits takes in 38 slices; now 6 of 11.8.)
+// that one sampled row of 151 936 f32 logits takes in 38 slices; now 6 of 11.9.)
+//
 // Entries the wave gathers at most, 32 a lane.  Up to there it is the faster way for every k, dtype and kind of
-// row: 4 to 100 rows of 151 936 in 5 to 38 slices, k 3 to 60: 0.77 to 1.00 of the workgroup's merge (24 f32
+// row: 4 to 100 rows of 151 936 in 5 to 38 slices, k 3 to 60: 0.77 to 1.01 of the workgroup's merge (24 f32
 // rows, k = 50: 19.8 and 21.3 us), k = 64 0.76 to 0.97 (22.1 and 26.4); bf16 rows near k = 62 up to 1.04, where
 // equal values at the k-th take a second sort.
 constexpr uint32_t WAVE_MERGE_SLOTS = 2048;
