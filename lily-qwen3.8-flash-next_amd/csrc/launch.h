@@ -112,6 +112,13 @@ hipError_t launch_rows_tiles(hipStream_t stream, int dtype, bool lse, bool extra
 // verify pass, whose acceptance runs behind the last row.
 hipError_t launch_rows_argmax(hipStream_t stream, int dtype, uint32_t rows, const LaunchCfg& cfg,
                               const InlineRows* inline_rows);
+// Sampled rows of the streaming kind (F_STREAM), given inline or as cfg.table, whose slices hold at most `blocks`
+// (1 or 2) times 256 x STREAM_UNROLL pieces of 16 bytes and k <= 64 candidates each, at most
+// HELD_MERGE_SLOTS a row in more than three slices.  `extra`: some row carries a mask or a bias list;
+// cfg.verify: a verify pass of independent plain rows (inline).
+constexpr uint32_t HELD_MERGE_SLOTS = 2048;
+hipError_t launch_rows_held(hipStream_t stream, int dtype, uint32_t blocks, bool lse, bool extra, uint32_t rows,
+                            const LaunchCfg& cfg, const InlineRows* inline_rows);
 // Rows that draw among many candidates (k > 64), spread over cfg.slices workgroups a row: two
 // launches (the row's bound, then the values that reach it, merge, select, tail).
 // lane_max [rows][slices][256], bound [rows], count [rows][slices].

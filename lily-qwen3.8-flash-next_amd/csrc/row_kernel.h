@@ -193,6 +193,105 @@ __device__ __forceinline__ bool descending(uint64_t c) {   // lane by lane, equa
     return __ballot((((uint64_t)hi << 32) | lo) < c) == 0ull;
 }
 
+// The row's best entries, a lane each, in order, from the lists its slices stored at `base` (by one
+// wave, all of it at work; at least the k best are among them).
+__device__ __forceinline__ uint64_t merge_slices_by_wave(const LaunchCfg& cfg, size_t base, uint32_t k) {
+    const uint32_t lane = threadIdx.x & 63u, S = cfg.slices;
+    uint64_t best = 0ull;   // the row's best, a lane each, in order
+    if (S <= WAVE_MERGE_LISTS) {
+        // Few lists, each in order as a rule: one after the other into the best so far.
+        uint64_t list[WAVE_MERGE_LISTS];
+#pragma unroll
+        for (uint32_t q = 0; q < WAVE_MERGE_LISTS; ++q) {
+            const uint32_t from = min(q, S - 1u), at = min(lane, cfg.ws_k - 1u);
+            list[q] = handed_load(cfg.ws_cand, (base + from) * cfg.ws_k + at);
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < WAVE_MERGE_LISTS; ++q) {
+            if (q < S) {
+                uint64_t c = lane < cfg.ws_k ? list[q] : 0ull;
+                if (!descending(c)) {
+                    c = wave_sort_desc(c);
+                }
+                best = q == 0u ? c : wave_merge_desc(best, c);
+            }
+        }
+    } else if (S * cfg.ws_k <= 64u) {
+        // (no more entries than lanes: one sort)
+        const uint64_t c = handed_load(cfg.ws_cand, base * cfg.ws_k + min(lane, S * cfg.ws_k - 1u));
+        best = wave_sort_desc(lane < S * cfg.ws_k ? c : 0ull);
+    } else {
+        constexpr int PER = WAVE_MERGE_SLOTS / 64, GROUP = 8;
+        const uint32_t slots = S * cfg.ws_k;
+        uint64_t mine[PER];
+#pragma unroll
+        for (int q0 = 0; q0 < PER; q0 += GROUP) {
+            if ((uint32_t)q0 * 64u < slots) {
+#pragma unroll
+                for (int q = q0; q < q0 + GROUP; ++q) {
+                    mine[q] = handed_load(cfg.ws_cand, base * cfg.ws_k + min(lane + (uint32_t)q * 64u, slots - 1u));
+                }
+            }
+        }
+        uint32_t lane_best = 0u, lane_next = 0u;   // the keys of a lane's two best
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            mine[q] = lane + (uint32_t)q * 64u < slots ? mine[q] : 0ull;
+            const uint32_t key = (uint32_t)(mine[q] >> 32);
+            lane_next = max(lane_next, min(lane_best, key));
+            lane_best = max(lane_best, key);
+        }
+        // The k-th largest of the lanes' two best bounds the k-th entry: at least k entries reach it (more
+        // than there are with fewer than k: all of them); what does not is dropped, the rest is listed, and
+        // the list's entries are taken in 64 at a time.  Sixteen bits of the key let some three f32 entries
+        // through that share the k-th's: above k = 50 a second sort in some row of a launch, 1.0 us, which
+        // four more bits (0.2 us) save.
+        uint32_t bound = 0u;
+        auto settle = [&](int bit) {
+            const uint32_t at = bound | (1u << bit);
+            const uint32_t reach = (uint32_t)__popcll(__ballot(lane_best >= at)) + (uint32_t)__popcll(__ballot(lane_next >= at));
+            bound = reach >= k ? at : bound;
+        };
+#pragma unroll
+        for (int bit = 31; bit >= 16; --bit) {
+            settle(bit);
+        }
+        if (k > 50u) {
+#pragma unroll
+            for (int bit = 15; bit >= 12; --bit) {
+                settle(bit);
+            }
+        }
+        uint64_t* cand = dyn_lds;
+        uint32_t kept = 0;
+#pragma unroll
+        for (int q0 = 0; q0 < PER; q0 += GROUP) {
+            if ((uint32_t)q0 * 64u < slots) {
+#pragma unroll
+                for (int q = q0; q < q0 + GROUP; ++q) {
+                    const bool in = mine[q] != 0ull && (uint32_t)(mine[q] >> 32) >= bound;
+                    const uint64_t mask = __ballot(in);
+                    if (mask != 0ull) {
+                        const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
+                            (uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+                        if (in) {
+                            cand[kept + rank] = mine[q];
+                        }
+                        kept += (uint32_t)__popcll(mask);
+                    }
+                }
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // (LDS of this wave: in order already)
+        __builtin_amdgcn_wave_barrier();
+        for (uint32_t i = 0; i < kept; i += 64u) {
+            const uint64_t c = wave_sort_desc(i + lane < kept ? cand[i + lane] : 0ull);
+            best = i == 0u ? c : wave_merge_desc(best, c);
+        }
+    }
+    return best;
+}
+
 template <int DT, bool LSE, bool SPEC>
 __device__ __forceinline__ bool finish_by_wave(const RowArgs& t, const LaunchCfg& cfg, uint32_t row, uint32_t s, uint32_t n,
                                                const uint64_t* found, uint32_t step, bool want_lse, Shared& sh) {
@@ -231,98 +330,7 @@ __device__ __forceinline__ bool finish_by_wave(const RowArgs& t, const LaunchCfg
         mt = handed_load(cfg.ws_lse, 2 * (base + lane));
         st = handed_load(cfg.ws_lse, 2 * (base + lane) + 1);
     }
-    uint64_t best = 0ull;   // the row's best, a lane each, in order
-    if (!forced && S <= WAVE_MERGE_LISTS) {
-        // Few lists, each in order as a rule: one after the other into the best so far.
-        uint64_t list[WAVE_MERGE_LISTS];
-#pragma unroll
-        for (uint32_t q = 0; q < WAVE_MERGE_LISTS; ++q) {
-            const uint32_t from = min(q, S - 1u), at = min(lane, cfg.ws_k - 1u);
-            list[q] = handed_load(cfg.ws_cand, (base + from) * cfg.ws_k + at);
-        }
-#pragma unroll
-        for (uint32_t q = 0; q < WAVE_MERGE_LISTS; ++q) {
-            if (q < S) {
-                uint64_t c = lane < cfg.ws_k ? list[q] : 0ull;
-                if (!descending(c)) {
-                    c = wave_sort_desc(c);
-                }
-                best = q == 0u ? c : wave_merge_desc(best, c);
-            }
-        }
-    } else if (!forced && S * cfg.ws_k <= 64u) {
-        // (no more entries than lanes: one sort)
-        const uint64_t c = handed_load(cfg.ws_cand, base * cfg.ws_k + min(lane, S * cfg.ws_k - 1u));
-        best = wave_sort_desc(lane < S * cfg.ws_k ? c : 0ull);
-    } else if (!forced) {
-        constexpr int PER = WAVE_MERGE_SLOTS / 64, GROUP = 8;
-        const uint32_t slots = S * cfg.ws_k;
-        uint64_t mine[PER];
-#pragma unroll
-        for (int q0 = 0; q0 < PER; q0 += GROUP) {
-            if ((uint32_t)q0 * 64u < slots) {
-#pragma unroll
-                for (int q = q0; q < q0 + GROUP; ++q) {
-                    mine[q] = handed_load(cfg.ws_cand, base * cfg.ws_k + min(lane + (uint32_t)q * 64u, slots - 1u));
-                }
-            }
-        }
-        uint32_t lane_best = 0u, lane_next = 0u;   // the keys of a lane's two best
-#pragma unroll
-        for (int q = 0; q < PER; ++q) {
-            mine[q] = lane + (uint32_t)q * 64u < slots ? mine[q] : 0ull;
-            const uint32_t key = (uint32_t)(mine[q] >> 32);
-            lane_next = max(lane_next, min(lane_best, key));
-            lane_best = max(lane_best, key);
-        }
-        // The k-th largest of the lanes' two best bounds the k-th entry: at least k entries reach it (more
-        // than there are with fewer than k: all of them); what does not is dropped, the rest is listed, and
-        // the list's entries are taken in 64 at a time.  Sixteen bits of the key let some three f32 entries
-        // through that share the k-th's: above k = 50 a second sort in some row of a launch, 1.0 us, which
-        // four more bits (0.2 us) save.
-        uint32_t bound = 0u;
-        auto settle = [&](int bit) {
-            const uint32_t at = bound | (1u << bit);
-            const uint32_t reach = (uint32_t)__popcll(__ballot(lane_best >= at)) + (uint32_t)__popcll(__ballot(lane_next >= at));
-            bound = reach >= t.k ? at : bound;
-        };
-#pragma unroll
-        for (int bit = 31; bit >= 16; --bit) {
-            settle(bit);
-        }
-        if (t.k > 50u) {
-#pragma unroll
-            for (int bit = 15; bit >= 12; --bit) {
-                settle(bit);
-            }
-        }
-        uint64_t* cand = dyn_lds;
-        uint32_t kept = 0;
-#pragma unroll
-        for (int q0 = 0; q0 < PER; q0 += GROUP) {
-            if ((uint32_t)q0 * 64u < slots) {
-#pragma unroll
-                for (int q = q0; q < q0 + GROUP; ++q) {
-                    const bool in = mine[q] != 0ull && (uint32_t)(mine[q] >> 32) >= bound;
-                    const uint64_t mask = __ballot(in);
-                    if (mask != 0ull) {
-                        const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
-                            (uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-                        if (in) {
-                            cand[kept + rank] = mine[q];
-                        }
-                        kept += (uint32_t)__popcll(mask);
-                    }
-                }
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // (LDS of this wave: in order already)
-        __builtin_amdgcn_wave_barrier();
-        for (uint32_t i = 0; i < kept; i += 64u) {
-            const uint64_t c = wave_sort_desc(i + lane < kept ? cand[i + lane] : 0ull);
-            best = i == 0u ? c : wave_merge_desc(best, c);
-        }
-    }
+    const uint64_t gathered = forced ? 0ull : merge_slices_by_wave(cfg, base, t.k);   // the row's best, a lane each, in order
     if (LSE && want_lse) {
         const bool some = st > 0.0;
         const double m = wave_max_d(some ? mt : -__builtin_huge_val());
@@ -339,7 +347,7 @@ __device__ __forceinline__ bool finish_by_wave(const RowArgs& t, const LaunchCfg
         }
         return true;
     }
-    best = lane < t.k ? best : 0ull;
+    const uint64_t best = lane < t.k ? gathered : 0ull;
     const uint32_t have = (uint32_t)__popcll(__ballot(best != 0ull));
     if (have == 0u) {
         if (lane == 0u) {

@@ -122,6 +122,7 @@ struct lily_sampler {
     uint32_t force_path = 0;
     uint32_t force_slices = 0;
     bool no_wide = false;   // LILY_SAMPLER_WIDE=0: rows of many candidates go the other kernels' way
+    bool no_held = false;   // LILY_SAMPLER_HELD=0: no slices held in registers (rows_held.hip)
     // LILY_SAMPLER_HEAD: batches of this many rows or more are produced through the vendor's GEMM
     // library ("own": never, "library": every batch it takes, a number: from that many rows on)
     uint32_t head_library_rows = HEAD_LIBRARY_ROWS, head_library_rows_codes = HEAD_LIBRARY_ROWS_CODES;
@@ -177,6 +178,8 @@ struct LaunchPart {
     uint32_t cand_cap = 0;
     bool argmax = false;   // every row is greedy: the kernel that holds nothing else
     bool wide = false;   // every row draws among many candidates: the two launches of rows_wide.hip
+    uint32_t held = 0;   // slices of so many blocks, held in registers (rows_held.hip)
+    bool extra = false;  // ... with a mask or a bias list on some row
 };
 
 struct lily_plan {
@@ -343,6 +346,46 @@ uint32_t choose_slices(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint
     const uint64_t by_ws = (uint64_t)s->ws_slots / ((uint64_t)rows * (kmax ? kmax : 1));
     sl = sl > by_ws ? (uint32_t)by_ws : sl;
     return sl < 1 ? 1 : sl;
+}
+
+// Rows of few candidates whose slices a workgroup can hold in registers (rows_held.hip): how many blocks
+// of 256 x STREAM_UNROLL pieces of 16 bytes a slice then has, and how many slices a row.  blocks 0: not this way.
+struct HeldShape {
+    uint32_t blocks = 0, slices = 0;
+};
+// Workgroups of a launch: as many as the chip holds at once (four a compute unit with one block, three with two).
+constexpr uint32_t HELD_MAX_GROUPS[3] = {0, 1024, 768};
+HeldShape held_shape(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint32_t vocab, int dtype) {
+    HeldShape out;
+    if (s->force_path != 0 || s->no_held || kmax > STREAM_K_MAX || rows > s->ws_rows) {
+        return out;
+    }
+    const uint32_t e = dtype == LILY_BF16 ? 8 : 4;
+    const uint32_t nch = (vocab + 2 * (e - 1)) / e + 1;   // wherever the row starts
+    for (uint32_t blocks = 1; blocks <= 2 && out.blocks == 0; ++blocks) {
+        const uint32_t per = blocks * 256u * STREAM_UNROLL, least = (nch + per - 1) / per;
+        const uint32_t sl = s->force_slices > least ? s->force_slices : least;
+        if (sl > MAX_SLICES || (s->force_slices != 0 && s->force_slices < least) ||
+            (sl > WAVE_MERGE_LISTS && sl * kmax > HELD_MERGE_SLOTS) ||
+            (uint64_t)rows * sl * kmax > s->ws_slots || (uint64_t)rows * sl > HELD_MAX_GROUPS[blocks]) {
+            continue;
+        }
+        out.blocks = blocks;
+        out.slices = sl;
+    }
+    return out;
+}
+
+// Whether every row of a launch is a draw that kernel takes; `extra`: some row has a mask or a bias list.
+bool all_held(const RowArgs* rows, uint32_t n, bool* extra) {
+    *extra = false;
+    for (uint32_t i = 0; i < n; ++i) {
+        if (rows[i].mode == MODE_ARGMAX || !(rows[i].flags & F_STREAM)) {
+            return false;
+        }
+        *extra = *extra || rows[i].allow != nullptr || rows[i].n_bias != 0;
+    }
+    return true;
 }
 
 // Launches of more than this many workgroups hand their slices over in the relaxed form (see
@@ -530,7 +573,10 @@ uint32_t plan_parts(const lily_sampler* s, RowArgs* table, uint32_t rows, int dt
     for (uint32_t i = 0; i < rows; ++i) {
         heavy += heavy_row(s, table[i]) ? 1u : 0u;
     }
-    const bool split = heavy != 0 && rows - heavy >= SPLIT_MIN_LIGHT;
+    // (a launch that holds its slices takes both kinds alike)
+    bool extra = false;
+    const bool together = all_held(table, rows, &extra) && held_shape(s, rows, max_k(table, rows), vocab, dtype).blocks != 0;
+    const bool split = !together && heavy != 0 && rows - heavy >= SPLIT_MIN_LIGHT;
     if (split) {
         std::stable_partition(table, table + rows,
                               [s](const RowArgs& r) { return !heavy_row(s, r); });
@@ -547,6 +593,11 @@ uint32_t plan_parts(const lily_sampler* s, RowArgs* table, uint32_t rows, int dt
         if (const uint32_t ws = wide_slices(s, sub, part.rows, dtype, vocab)) {
             part.wide = true;
             part.slices = ws;
+        }
+        if (all_held(sub, part.rows, &part.extra)) {
+            const HeldShape held = held_shape(s, part.rows, part.ws_k, vocab, dtype);
+            part.held = held.blocks;
+            part.slices = held.blocks != 0 ? held.slices : part.slices;
         }
         const LaunchShape shp = shape_of(s, sub, part.rows, dtype, vocab, part.slices, part.ws_k);
         part.kind = shp.kind();
@@ -579,6 +630,10 @@ int launch_part(lily_sampler* s, const LaunchPart& part, const RowArgs* table_de
                                  s->wide_count));
         return LILY_OK;
     }
+    if (part.held != 0) {
+        HIP_TRY(launch_rows_held(s->stream, dtype, part.held, part.lse, part.extra, part.rows, cfg, nullptr));
+        return LILY_OK;
+    }
     HIP_TRY(launch_rows(s->stream, dtype, part.kind, part.lse, part.rows, cfg, nullptr, part.dyn_bytes));
     return LILY_OK;
 }
@@ -606,7 +661,10 @@ int launch_inline(lily_sampler* s, int dtype, uint32_t vocab, const InlineRows& 
             return LILY_OK;
         }
     }
-    const uint32_t slices = choose_slices(s, n, kmax, vocab, dtype);
+    bool extra = false;
+    const HeldShape held =
+        !chained && all_held(rows.r, n, &extra) ? held_shape(s, n, kmax, vocab, dtype) : HeldShape();
+    const uint32_t slices = held.blocks != 0 ? held.slices : choose_slices(s, n, kmax, vocab, dtype);
     fill_cfg(s, &cfg, n, vocab, slices, kmax, 0, nullptr);
     if (chained) {
         // Rows that draw in order count what the rows before them drew into one histogram: the
@@ -637,6 +695,13 @@ int launch_inline(lily_sampler* s, int dtype, uint32_t vocab, const InlineRows& 
         return LILY_OK;
     }
     const LaunchShape shp = shape_of(s, rows.r, n, dtype, vocab, slices, kmax);
+    if (held.blocks != 0) {
+        for (uint32_t i = 0; i < n; ++i) {
+            cfg.verify = rows.r[i].mode == MODE_SPEC ? 1u : cfg.verify;   // (the kernel that holds that draw)
+        }
+        HIP_TRY(launch_rows_held(s->stream, dtype, held.blocks, shp.lse, extra, n, cfg, &rows));
+        return LILY_OK;
+    }
     cfg.excl_words = shp.excl_words;
     cfg.bitmap_layout = shp.bitmap_layout ? 1u : 0u;
     cfg.cand_cap = shp.cand_cap;
@@ -978,6 +1043,9 @@ int lily_sampler_create(int device, void* hip_stream, lily_sampler_t** out) {
     if (const char* p = std::getenv("LILY_SAMPLER_WIDE")) {
         s->no_wide = std::atoi(p) == 0;
     }
+    if (const char* p = std::getenv("LILY_SAMPLER_HELD")) {
+        s->no_held = std::atoi(p) == 0;
+    }
     if (const char* p = std::getenv("LILY_SAMPLER_HEAD")) {
         s->head_library_rows = std::strcmp(p, "own") == 0 ? 0u : std::strcmp(p, "library") == 0 ? 1u : (uint32_t)std::atoi(p);
         s->head_library_rows_codes = s->head_library_rows_code_lines = s->head_library_rows_code_lines_alone =
@@ -1059,7 +1127,8 @@ uint32_t lily_sampler_slices_for(const lily_sampler_t* s, uint32_t rows, uint32_
     if (s == nullptr || rows == 0) {
         return 0;
     }
-    return choose_slices(s, rows, k ? k : 1, vocab, (int)dtype);
+    const HeldShape held = held_shape(s, rows, k ? k : 1, vocab, (int)dtype);
+    return held.blocks != 0 ? held.slices : choose_slices(s, rows, k ? k : 1, vocab, (int)dtype);
 }
 
 int lily_sampler_synchronize(lily_sampler_t* s) {

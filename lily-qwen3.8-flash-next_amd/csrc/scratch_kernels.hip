@@ -229,6 +229,25 @@ hipError_t launch_rows(hipStream_t stream, int dtype, int kind, bool lse, uint32
     }
 }
 
+#define LILY_HELD(DT, NB)                                                                                  \
+    hipError_t launch_rows_held_dt##DT##_blocks##NB(hipStream_t stream, bool lse, bool extra, uint32_t rows, \
+                                                    const LaunchCfg& cfg, const InlineRows* inline_rows);
+LILY_HELD(0, 1)
+LILY_HELD(0, 2)
+LILY_HELD(1, 1)
+LILY_HELD(1, 2)
+#undef LILY_HELD
+
+hipError_t launch_rows_held(hipStream_t stream, int dtype, uint32_t blocks, bool lse, bool extra, uint32_t rows,
+                            const LaunchCfg& cfg, const InlineRows* inline_rows) {
+    if (dtype == LILY_BF16) {
+        return blocks == 1u ? launch_rows_held_dt1_blocks1(stream, lse, extra, rows, cfg, inline_rows)
+                            : launch_rows_held_dt1_blocks2(stream, lse, extra, rows, cfg, inline_rows);
+    }
+    return blocks == 1u ? launch_rows_held_dt0_blocks1(stream, lse, extra, rows, cfg, inline_rows)
+                        : launch_rows_held_dt0_blocks2(stream, lse, extra, rows, cfg, inline_rows);
+}
+
 hipError_t launch_fill_u32(hipStream_t stream, uint32_t* p, uint32_t n, uint32_t v) {
     if (n == 0) {
         return hipSuccess;

@@ -1,0 +1,173 @@
+"""Rows of few candidates in slices that a workgroup holds in registers (rows_held.hip), and the same
+rows through the streaming selects (LILY_SAMPLER_HELD=0): sizes around a block and two (4 096 / 8 192 f32
+ids, twice that in bf16), rows that start inside a 16-byte piece, penalties of either sign over sparse and
+dense histories, masks and bias lists, ties by the thousand, NaN and infinite logits, forced ids, drafts
+longer than a wave.  Bit-exact against the oracle; log-probabilities at the bar of the other tests."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+import lily_sampler as LS
+import lily_workloads as W
+import oracle as O
+from gpu_util import both_params, check_row_against_oracle, dev, o_params, run_rows
+
+ROWS = 8
+
+
+def _sampler(monkeypatch, held, slices=0):
+    monkeypatch.setenv("LILY_SAMPLER_HELD", "1" if held else "0")
+    monkeypatch.setenv("LILY_SAMPLER_SLICES", str(slices))
+    return LS.Sampler(0)
+
+
+def _rows(rng, vocab, bf16):
+    x = rng.normal(0, 3, (ROWS, vocab)).astype(np.float32)
+    x[1] = 1.5                                                        # one value: ties by the thousand
+    x[2] = np.round(x[2])
+    x[3, rng.random(vocab) < 0.998] = -np.inf
+    x[4, rng.random(vocab) < 0.3] = np.nan
+    x[5, vocab // 2:vocab // 2 + 300] = np.linspace(20, 21, len(x[5, vocab // 2:vocab // 2 + 300]), dtype=np.float32)
+    x[6] = -np.inf
+    return W.to_bf16_bits(x) if bf16 else x
+
+
+def _check(r, x, kw, step, lp, counts=None, **ext):
+    clean = np.where(np.isnan(x), -np.inf, x) if x.dtype == np.float32 else x.copy()
+    if x.dtype == np.uint16:
+        clean[(clean & 0x7fff) > 0x7f80] = 0xff80
+    for i in range(len(x)):
+        own = {k: v[i] for k, v in ext.items() if v[i] is not None and not (k == "bias" and not v[i])}
+        d = O.sample(clean[i], None if counts is None else counts[i], o_params(**kw[i]), step, want_logprob=lp, **own)
+        if "forced" in own:
+            assert r.ids[i] == own["forced"]
+        else:
+            check_row_against_oracle(r, i, d)
+        if lp and np.isfinite(d.logprob):
+            assert abs(r.logprobs[i] - d.logprob) <= 1e-5 * max(1.0, abs(d.logprob)), (i, r.logprobs[i], d.logprob)
+
+
+@pytest.mark.parametrize("held", [True, False], ids=["held", "streamed"])
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+@pytest.mark.parametrize("vocab", [1, 9, 4097, 8190, 16_381, 24_601, 65_543, 131_099])
+def test_plain_rows(monkeypatch, held, bf16, vocab):
+    rng = np.random.default_rng(vocab)
+    x = _rows(rng, vocab, bf16)
+    for slices in (0, max(1, vocab * (1 if bf16 else 2) // 16_384)):   # one block a slice, and about two
+        s = _sampler(monkeypatch, held, slices)
+        for trial, k in enumerate((2, 20, 64)):
+            kw = [dict(temperature=0.7, top_k=k, top_p=0.97, min_p=0.01, seed=60 + i) for i in range(ROWS)]
+            for lp in (False, True):
+                _check(run_rows(s, x, kw, [trial] * ROWS, logprobs=lp, use_plan=lp), x, kw, trial, lp)
+        s.close()
+
+
+@pytest.mark.parametrize("held", [True, False], ids=["held", "streamed"])
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+@pytest.mark.parametrize("history", [40, 3000, 60_000])
+def test_rows_under_penalties(monkeypatch, held, bf16, history):
+    vocab = 40_009
+    rng = np.random.default_rng(history)
+    x = _rows(rng, vocab, bf16)
+    for slices in (0, 3 if bf16 else 6):
+        s = _sampler(monkeypatch, held, slices)
+        hist = rng.integers(0, vocab, (ROWS, history)).astype(np.int32)
+        hist[:, :history // 2] = rng.integers(0, 50, (ROWS, history // 2))
+        for pen in (dict(repetition_penalty=1.1, presence_penalty=0.3, frequency_penalty=0.0625),
+                    dict(repetition_penalty=0.9, presence_penalty=-0.5, frequency_penalty=0.03125)):
+            for lp in (False, True):
+                sc, counts = [], []
+                for i in range(ROWS):
+                    t = LS.SamplerScratch(s, vocab)
+                    t.add_history(torch.from_numpy(hist[i]).to(dev()))
+                    sc.append(t)
+                    counts.append(np.bincount(hist[i], minlength=vocab).astype(np.uint32))
+                kw = [dict(temperature=0.8, top_k=33, top_p=0.95, seed=7 + i, **pen) for i in range(ROWS)]
+                r = run_rows(s, x, kw, [4] * ROWS, scratch=sc, logprobs=lp)
+                _check(r, x, kw, 4, lp, counts)
+                for i in range(ROWS):
+                    assert np.array_equal(sc[i].read_counts().numpy(), counts[i]), i   # (the oracle counted its draw)
+                    sc[i].close()
+        s.close()
+
+
+@pytest.mark.parametrize("held", [True, False], ids=["held", "streamed"])
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+def test_rows_with_masks_bias_lists_and_forced_ids(monkeypatch, held, bf16):
+    vocab = 50_021
+    rng = np.random.default_rng(5)
+    x = _rows(rng, vocab, bf16)
+    x[4] = x[0]
+    allow = np.stack([W.allow_mask(rng, vocab, frac=f) for f in (0.0005, 0.02, 0.02, 0.1, 0.1, 0.5, 0.02, 0.9)])
+    bias = [[(int(i), float(d)) for i, d in zip(rng.integers(0, vocab, 30), rng.choice([-5.0, 5.0, 0.5], 30))]
+            for _ in range(ROWS)]
+    bias[0] += [(0, 4.0), (vocab - 1, 4.0), (vocab - 1, 4.0)]
+    bias[7] = []
+    forced = [None] * ROWS
+    forced[3] = 77
+    for slices in (0, 4 if bf16 else 7):
+        s = _sampler(monkeypatch, held, slices)
+        hist = rng.integers(0, vocab, (ROWS, 2000)).astype(np.int32)
+        for use in (dict(allow=True), dict(bias=True), dict(allow=True, bias=True, forced=True, pen=True)):
+            pen = dict(repetition_penalty=1.2, presence_penalty=0.1, frequency_penalty=0.2) if use.get("pen") else {}
+            for lp in (False, True):
+                sc = counts = None
+                if pen:
+                    sc, counts = [], []
+                    for i in range(ROWS):
+                        t = LS.SamplerScratch(s, vocab)
+                        t.add_history(torch.from_numpy(hist[i]).to(dev()))
+                        sc.append(t)
+                        counts.append(np.bincount(hist[i], minlength=vocab).astype(np.uint32))
+                kw = [dict(temperature=0.8, top_k=50, top_p=0.95, seed=9 + i, **pen) for i in range(ROWS)]
+                ext = dict(allow=allow if use.get("allow") else None, bias=bias if use.get("bias") else None,
+                           forced=forced if use.get("forced") else None)
+                r = run_rows(s, x, kw, [1] * ROWS, scratch=sc, logprobs=lp, **ext)
+                _check(r, x, kw, 1, lp, counts, **{k: v for k, v in ext.items() if v is not None})
+        s.close()
+
+
+@pytest.mark.parametrize("held", [True, False], ids=["held", "streamed"])
+@pytest.mark.parametrize("draft_k", [20, 0], ids=["20 drafted from", "all drafted from"])
+def test_verify_pass(monkeypatch, held, draft_k):
+    """Drafts from 20 and from 1 024 candidates (the latter's distribution is longer than a wave), verified
+    among 20, three rows a pass with the acceptance behind them."""
+    s = _sampler(monkeypatch, held)
+    rng = np.random.default_rng(3)
+    v, m = 30_011, 3
+    head = rng.normal(0, 1.2, (m, v)).astype(np.float32)
+    trunk = (head + rng.normal(0, 0.4, (m, v))).astype(np.float32)
+    t_head, t_trunk = torch.from_numpy(head).to(dev()), torch.from_numpy(trunk).to(dev())
+    lp, op = both_params(temperature=1.0, top_k=20, top_p=0.95, seed=77)
+    dp = LS.SamplingParams.greedy(temperature=1.0, top_k=draft_k, top_p=1.0, seed=77)
+    dop = O.params(temperature=1.0, top_k=draft_k, top_p=1.0, seed=77)
+    scratch, dists = LS.SamplerScratch(s, v), LS.DraftDists(s, m)
+    ids = torch.zeros(m, dtype=torch.int32, device=dev())
+    out = torch.zeros(m, dtype=torch.int32, device=dev())
+    ctrl = torch.zeros(LS.ctrl_words(m - 1), dtype=torch.int32, device=dev())
+    outcomes = set()
+    for step in range(0, 60, m):
+        for j in range(m - 1):
+            s.sample_draft_f32(t_head[j], scratch, dp, LS.draft_step(step + j), ids[j + 1:j + 2], dists.slot(j))
+        s.spec_verify(t_trunk, scratch, lp, step, dists, ids, out, ctrl, pos0=10, ratio=4, chain=m - 1)
+        s.synchronize()
+        drafted, got = ids.cpu().numpy(), out.cpu().numpy()
+        for j in range(m - 1):
+            d = O.sample(head[j], None, dop, O.lib().lo_draft_step(step + j))
+            assert drafted[j + 1] == d.chosen
+            p_ids, p_pr = O.kept(trunk[j], op)
+            q_ids, q_pr = O.kept(head[j], dop)
+            want, acc, zero, gap = O.spec(p_ids, p_pr, q_ids, q_pr, int(drafted[j + 1]), op.seed, step + j)
+            assert zero or got[j] == want, (step, j)
+            outcomes.add(acc)
+        assert got[m - 1] == O.sample(trunk[m - 1], None, op, step + m - 1).chosen
+        acc = 0
+        while acc + 1 < m and got[acc] == drafted[acc + 1]:
+            acc += 1
+        assert int(ctrl.cpu()[0]) == acc
+    assert outcomes == {True, False}
+    scratch.close()
+    dists.close()
+    s.close()
