@@ -119,6 +119,8 @@ hipError_t launch_rows_argmax(hipStream_t stream, int dtype, uint32_t rows, cons
 constexpr uint32_t HELD_MERGE_SLOTS = 2048;
 hipError_t launch_rows_held(hipStream_t stream, int dtype, uint32_t blocks, bool lse, bool extra, uint32_t rows,
                             const LaunchCfg& cfg, const InlineRows* inline_rows);
+// The same rows of cfg.table (no mask, no bias list, plain draws) in slices of any length, a block at a time.
+hipError_t launch_rows_blocks(hipStream_t stream, int dtype, bool lse, bool pen, uint32_t rows, const LaunchCfg& cfg);
 // Rows that draw among many candidates (k > 64), spread over cfg.slices workgroups a row: two
 // launches (the row's bound, then the values that reach it, merge, select, tail).
 // lane_max [rows][slices][256], bound [rows], count [rows][slices].

@@ -122,7 +122,9 @@ struct lily_sampler {
     uint32_t force_path = 0;
     uint32_t force_slices = 0;
     bool no_wide = false;   // LILY_SAMPLER_WIDE=0: rows of many candidates go the other kernels' way
-    bool no_held = false;   // LILY_SAMPLER_HELD=0: no slices held in registers (rows_held.hip)
+    // LILY_SAMPLER_HELD: "0" = no slices held in registers (rows_held.hip, rows_blocks.hip), "blocks" = every
+    // row that can goes a block at a time
+    bool no_held = false, only_blocks = false;
     // LILY_SAMPLER_HEAD: batches of this many rows or more are produced through the vendor's GEMM
     // library ("own": never, "library": every batch it takes, a number: from that many rows on)
     uint32_t head_library_rows = HEAD_LIBRARY_ROWS, head_library_rows_codes = HEAD_LIBRARY_ROWS_CODES;
@@ -180,6 +182,8 @@ struct LaunchPart {
     bool wide = false;   // every row draws among many candidates: the two launches of rows_wide.hip
     uint32_t held = 0;   // slices of so many blocks, held in registers (rows_held.hip)
     bool extra = false;  // ... with a mask or a bias list on some row
+    bool blocks = false; // slices of any length, a block at a time (rows_blocks.hip)
+    bool pen = false;    // ... with penalties on some row
 };
 
 struct lily_plan {
@@ -354,10 +358,13 @@ struct HeldShape {
     uint32_t blocks = 0, slices = 0;
 };
 // Workgroups of a launch: as many as the chip holds at once (four a compute unit with one block, three with two).
+// Rows under penalties without log-probabilities stay below that (bf16, 151 936 ids, streamed -> held: 40 rows
+// in 19 slices 21.9 -> 21.9 us, 50 rows 22.3 -> 23.2, 60 rows in 10 slices of two blocks 23.8 -> 25.6).
 constexpr uint32_t HELD_MAX_GROUPS[3] = {0, 1024, 768};
-HeldShape held_shape(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint32_t vocab, int dtype) {
+constexpr uint32_t HELD_MAX_GROUPS_LISTED = 768;
+HeldShape held_shape(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint32_t vocab, int dtype, bool pen, bool lse) {
     HeldShape out;
-    if (s->force_path != 0 || s->no_held || kmax > STREAM_K_MAX || rows > s->ws_rows) {
+    if (s->force_path != 0 || s->no_held || s->only_blocks || kmax > STREAM_K_MAX || rows > s->ws_rows) {
         return out;
     }
     const uint32_t e = dtype == LILY_BF16 ? 8 : 4;
@@ -370,22 +377,64 @@ HeldShape held_shape(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint32
             (uint64_t)rows * sl * kmax > s->ws_slots || (uint64_t)rows * sl > HELD_MAX_GROUPS[blocks]) {
             continue;
         }
+        if (pen && !lse && ((uint64_t)rows * sl > HELD_MAX_GROUPS_LISTED || (blocks == 2 && dtype == LILY_BF16))) {
+            continue;
+        }
         out.blocks = blocks;
         out.slices = sl;
     }
     return out;
 }
 
-// Whether every row of a launch is a draw that kernel takes; `extra`: some row has a mask or a bias list.
-bool all_held(const RowArgs* rows, uint32_t n, bool* extra) {
-    *extra = false;
-    for (uint32_t i = 0; i < n; ++i) {
-        if (rows[i].mode == MODE_ARGMAX || !(rows[i].flags & F_STREAM)) {
-            return false;
-        }
-        *extra = *extra || rows[i].allow != nullptr || rows[i].n_bias != 0;
+constexpr uint32_t BLOCKS_GROUPS = 1024;
+// Workgroups a row where rows without masks and bias lists go a block at a time (rows_blocks.hip); 0: they do not.
+// Up to a fifth of the workgroups that the chip holds at once (four a compute unit) as many as that: workgroups that
+// are not the same number on every compute unit leave some idle (200 rows in 5 slices 53 us, in 3 66), a second
+// generation costs more than the slices save.
+//
+// Which launches: bf16 rows of 151 936, us, before -> a block at a time.  Without penalties all of them (with
+// log-probabilities 100 rows 35.0 -> 23.8, 1 024 77.5 -> 70.2; without 19.2 -> 16.6, 62.0 -> 56.6).  Under penalties
+// those with log-probabilities up to a fifth of the chip's workgroups: flat rows of 248 320 59.0 -> 39.6 at 100, 75.7 ->
+// 53.1 at 200, rows with a heavy tail 33.4 -> 31.7 and 40.3 -> 39.6, but at 280 rows 89.5 -> 72.2 and 40.5 -> 44.9.
+// Without log-probabilities the streaming kernel's coarse map is the cheaper look at listed ids (80 rows 23.5 -> 25.3).
+uint32_t blocks_slices(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint32_t vocab, int dtype, bool pen, bool lse) {
+    if (s->force_path != 0 || s->no_held || kmax > STREAM_K_MAX) {
+        return 0;
     }
-    return true;
+    if (pen && !s->only_blocks && !(lse && rows <= BLOCKS_GROUPS / 5u)) {
+        return 0;
+    }
+    if (rows > BLOCKS_GROUPS / 5u) {
+        // (the streaming launches' slices: 280 rows with log-probabilities 43 us in two, 40 in three, without 26.0
+        // and 26.5)
+        return choose_slices(s, rows, kmax, vocab, dtype);
+    }
+    uint32_t sl = s->force_slices != 0 ? s->force_slices : BLOCKS_GROUPS / rows;
+    const uint32_t e = dtype == LILY_BF16 ? 8 : 4;
+    const uint32_t nch = (vocab + 2 * (e - 1)) / e + 1;
+    const uint32_t by_block = (nch + 256u * STREAM_UNROLL - 1) / (256u * STREAM_UNROLL);   // no finer than a block a slice
+    sl = sl > by_block && s->force_slices == 0 ? by_block : sl;
+    sl = sl > MAX_SLICES ? MAX_SLICES : sl;
+    sl = sl > WAVE_MERGE_LISTS && sl * kmax > HELD_MERGE_SLOTS ? std::max(WAVE_MERGE_LISTS, HELD_MERGE_SLOTS / kmax) : sl;
+    const uint64_t by_ws = (uint64_t)s->ws_slots / ((uint64_t)rows * kmax);
+    sl = sl > by_ws ? (uint32_t)by_ws : sl;
+    return sl < 1 ? 1 : sl;
+}
+
+// Whether every row of a launch is a draw that those kernels take, and what some row has of a mask or a bias
+// list, penalties, a log-probability.
+struct HeldRows {
+    bool all = true, extra = false, pen = false, lse = false;
+};
+HeldRows held_rows(const RowArgs* rows, uint32_t n) {
+    HeldRows h;
+    for (uint32_t i = 0; i < n && h.all; ++i) {
+        h.all = rows[i].mode != MODE_ARGMAX && (rows[i].flags & F_STREAM) != 0;
+        h.extra = h.extra || rows[i].allow != nullptr || rows[i].n_bias != 0;
+        h.pen = h.pen || (rows[i].flags & F_PEN) != 0;
+        h.lse = h.lse || rows[i].out_logprob != nullptr;
+    }
+    return h;
 }
 
 // Launches of more than this many workgroups hand their slices over in the relaxed form (see
@@ -574,8 +623,9 @@ uint32_t plan_parts(const lily_sampler* s, RowArgs* table, uint32_t rows, int dt
         heavy += heavy_row(s, table[i]) ? 1u : 0u;
     }
     // (a launch that holds its slices takes both kinds alike)
-    bool extra = false;
-    const bool together = all_held(table, rows, &extra) && held_shape(s, rows, max_k(table, rows), vocab, dtype).blocks != 0;
+    const HeldRows whole = held_rows(table, rows);
+    const bool together =
+        whole.all && held_shape(s, rows, max_k(table, rows), vocab, dtype, whole.pen, whole.lse).blocks != 0;
     const bool split = !together && heavy != 0 && rows - heavy >= SPLIT_MIN_LIGHT;
     if (split) {
         std::stable_partition(table, table + rows,
@@ -594,10 +644,16 @@ uint32_t plan_parts(const lily_sampler* s, RowArgs* table, uint32_t rows, int dt
             part.wide = true;
             part.slices = ws;
         }
-        if (all_held(sub, part.rows, &part.extra)) {
-            const HeldShape held = held_shape(s, part.rows, part.ws_k, vocab, dtype);
+        const HeldRows is = held_rows(sub, part.rows);
+        part.extra = is.extra;
+        part.pen = is.pen;
+        if (is.all) {
+            const HeldShape held = held_shape(s, part.rows, part.ws_k, vocab, dtype, is.pen, is.lse);
+            const uint32_t blocks = held.blocks == 0 && !is.extra && part.rows <= s->ws_rows
+                                        ? blocks_slices(s, part.rows, part.ws_k, vocab, dtype, is.pen, is.lse) : 0u;
             part.held = held.blocks;
-            part.slices = held.blocks != 0 ? held.slices : part.slices;
+            part.blocks = blocks != 0;
+            part.slices = held.blocks != 0 ? held.slices : blocks != 0 ? blocks : part.slices;
         }
         const LaunchShape shp = shape_of(s, sub, part.rows, dtype, vocab, part.slices, part.ws_k);
         part.kind = shp.kind();
@@ -628,6 +684,10 @@ int launch_part(lily_sampler* s, const LaunchPart& part, const RowArgs* table_de
     if (part.wide) {
         HIP_TRY(launch_rows_wide(s->stream, dtype, part.lse, part.rows, cfg, nullptr, s->wide_max,
                                  s->wide_count));
+        return LILY_OK;
+    }
+    if (part.blocks) {
+        HIP_TRY(launch_rows_blocks(s->stream, dtype, part.lse, part.pen, part.rows, cfg));
         return LILY_OK;
     }
     if (part.held != 0) {
@@ -661,9 +721,9 @@ int launch_inline(lily_sampler* s, int dtype, uint32_t vocab, const InlineRows& 
             return LILY_OK;
         }
     }
-    bool extra = false;
+    const HeldRows is = held_rows(rows.r, n);
     const HeldShape held =
-        !chained && all_held(rows.r, n, &extra) ? held_shape(s, n, kmax, vocab, dtype) : HeldShape();
+        !chained && is.all ? held_shape(s, n, kmax, vocab, dtype, is.pen, is.lse) : HeldShape();
     const uint32_t slices = held.blocks != 0 ? held.slices : choose_slices(s, n, kmax, vocab, dtype);
     fill_cfg(s, &cfg, n, vocab, slices, kmax, 0, nullptr);
     if (chained) {
@@ -699,7 +759,7 @@ int launch_inline(lily_sampler* s, int dtype, uint32_t vocab, const InlineRows& 
         for (uint32_t i = 0; i < n; ++i) {
             cfg.verify = rows.r[i].mode == MODE_SPEC ? 1u : cfg.verify;   // (the kernel that holds that draw)
         }
-        HIP_TRY(launch_rows_held(s->stream, dtype, held.blocks, shp.lse, extra, n, cfg, &rows));
+        HIP_TRY(launch_rows_held(s->stream, dtype, held.blocks, shp.lse, is.extra, n, cfg, &rows));
         return LILY_OK;
     }
     cfg.excl_words = shp.excl_words;
@@ -1044,7 +1104,8 @@ int lily_sampler_create(int device, void* hip_stream, lily_sampler_t** out) {
         s->no_wide = std::atoi(p) == 0;
     }
     if (const char* p = std::getenv("LILY_SAMPLER_HELD")) {
-        s->no_held = std::atoi(p) == 0;
+        s->only_blocks = std::strcmp(p, "blocks") == 0;
+        s->no_held = std::strcmp(p, "0") == 0;
     }
     if (const char* p = std::getenv("LILY_SAMPLER_HEAD")) {
         s->head_library_rows = std::strcmp(p, "own") == 0 ? 0u : std::strcmp(p, "library") == 0 ? 1u : (uint32_t)std::atoi(p);
@@ -1127,8 +1188,9 @@ uint32_t lily_sampler_slices_for(const lily_sampler_t* s, uint32_t rows, uint32_
     if (s == nullptr || rows == 0) {
         return 0;
     }
-    const HeldShape held = held_shape(s, rows, k ? k : 1, vocab, (int)dtype);
-    return held.blocks != 0 ? held.slices : choose_slices(s, rows, k ? k : 1, vocab, (int)dtype);
+    const HeldShape held = held_shape(s, rows, k ? k : 1, vocab, (int)dtype, false, false);
+    const uint32_t blocks = blocks_slices(s, rows, k ? k : 1, vocab, (int)dtype, false, false);
+    return held.blocks != 0 ? held.slices : blocks != 0 ? blocks : choose_slices(s, rows, k ? k : 1, vocab, (int)dtype);
 }
 
 int lily_sampler_synchronize(lily_sampler_t* s) {
@@ -2008,7 +2070,7 @@ int rows_with_tiles(lily_sampler* s, const lily_lm_head* h, const lily_rows* b, 
     // Rows under penalties whose slices can be held in registers are drawn from their logits at once (masks: most
     // rows are drawn from a few tiles): the launch that would stand behind the draws from summaries anyway is no slower for drawing them
     // all (4 rows under penalties 17 us, 23 with the summaries first; 24 rows 27 and 31).
-    bool held = true;
+    bool held = true, behind_pen = false, behind_lse = false;
     uint32_t behind = 0, behind_k = 1;
     for (uint32_t r = 0; r < rows; ++r) {
         const RowArgs& row = packed[r];
@@ -2016,13 +2078,15 @@ int rows_with_tiles(lily_sampler* s, const lily_lm_head* h, const lily_rows* b, 
         const bool pen = serve && row.mode != MODE_ARGMAX && ((row.flags & F_PEN) != 0 || row.allow != nullptr);
         group_of[r] = !serve ? 2 : (pen ? 1 : 0);
         if (group_of[r] != 0) {
-            bool extra_row;
-            held = held && all_held(&row, 1, &extra_row) && (!serve || row.allow == nullptr);
+            const HeldRows is = held_rows(&row, 1);
+            held = held && is.all && (!serve || row.allow == nullptr);
+            behind_pen = behind_pen || is.pen;
+            behind_lse = behind_lse || is.lse;
             behind += 1;
             behind_k = row.k > behind_k ? row.k : behind_k;
         }
     }
-    held = held && behind != 0 && held_shape(s, behind, behind_k, b->vocab, (int)b->dtype).blocks != 0;
+    held = held && behind != 0 && held_shape(s, behind, behind_k, b->vocab, (int)b->dtype, behind_pen, behind_lse).blocks != 0;
     for (int group = 0; group < 3; ++group) {
         for (uint32_t r = 0; r < rows; ++r) {
             const RowArgs& row = packed[r];

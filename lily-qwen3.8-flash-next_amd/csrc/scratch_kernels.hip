@@ -248,6 +248,14 @@ hipError_t launch_rows_held(hipStream_t stream, int dtype, uint32_t blocks, bool
                         : launch_rows_held_dt0_blocks2(stream, lse, extra, rows, cfg, inline_rows);
 }
 
+hipError_t launch_rows_blocks_dt0(hipStream_t stream, bool lse, bool pen, uint32_t rows, const LaunchCfg& cfg);
+hipError_t launch_rows_blocks_dt1(hipStream_t stream, bool lse, bool pen, uint32_t rows, const LaunchCfg& cfg);
+
+hipError_t launch_rows_blocks(hipStream_t stream, int dtype, bool lse, bool pen, uint32_t rows, const LaunchCfg& cfg) {
+    return dtype == LILY_BF16 ? launch_rows_blocks_dt1(stream, lse, pen, rows, cfg)
+                              : launch_rows_blocks_dt0(stream, lse, pen, rows, cfg);
+}
+
 hipError_t launch_fill_u32(hipStream_t stream, uint32_t* p, uint32_t n, uint32_t v) {
     if (n == 0) {
         return hipSuccess;

@@ -1,5 +1,5 @@
-"""Rows of few candidates in slices that a workgroup holds in registers (rows_held.hip), and the same
-rows through the streaming selects (LILY_SAMPLER_HELD=0): sizes around a block and two (4 096 / 8 192 f32
+"""Rows of few candidates in slices that a workgroup holds in registers (rows_held.hip), a block at a time
+(rows_blocks.hip, LILY_SAMPLER_HELD=blocks) and through the streaming selects (LILY_SAMPLER_HELD=0): sizes around a block and two (4 096 / 8 192 f32
 ids, twice that in bf16), rows that start inside a 16-byte piece, penalties of either sign over sparse and
 dense histories, masks and bias lists, ties by the thousand, NaN and infinite logits, forced ids, drafts
 longer than a wave.  Bit-exact against the oracle; log-probabilities at the bar of the other tests."""
@@ -18,7 +18,7 @@ ROWS = 8
 
 
 def _sampler(monkeypatch, held, slices=0):
-    monkeypatch.setenv("LILY_SAMPLER_HELD", "1" if held else "0")
+    monkeypatch.setenv("LILY_SAMPLER_HELD", held)
     monkeypatch.setenv("LILY_SAMPLER_SLICES", str(slices))
     return LS.Sampler(0)
 
@@ -49,7 +49,7 @@ def _check(r, x, kw, step, lp, counts=None, **ext):
             assert abs(r.logprobs[i] - d.logprob) <= 1e-5 * max(1.0, abs(d.logprob)), (i, r.logprobs[i], d.logprob)
 
 
-@pytest.mark.parametrize("held", [True, False], ids=["held", "streamed"])
+@pytest.mark.parametrize("held", ["1", "blocks", "0"], ids=["held", "blocks", "streamed"])
 @pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
 @pytest.mark.parametrize("vocab", [1, 9, 4097, 8190, 16_381, 24_601, 65_543, 131_099])
 def test_plain_rows(monkeypatch, held, bf16, vocab):
@@ -60,18 +60,19 @@ def test_plain_rows(monkeypatch, held, bf16, vocab):
         for trial, k in enumerate((2, 20, 64)):
             kw = [dict(temperature=0.7, top_k=k, top_p=0.97, min_p=0.01, seed=60 + i) for i in range(ROWS)]
             for lp in (False, True):
-                _check(run_rows(s, x, kw, [trial] * ROWS, logprobs=lp, use_plan=lp), x, kw, trial, lp)
+                for use_plan in (False, True):   # (a plan's rows may go a block at a time)
+                    _check(run_rows(s, x, kw, [trial] * ROWS, logprobs=lp, use_plan=use_plan), x, kw, trial, lp)
         s.close()
 
 
-@pytest.mark.parametrize("held", [True, False], ids=["held", "streamed"])
+@pytest.mark.parametrize("held", ["1", "blocks", "0"], ids=["held", "blocks", "streamed"])
 @pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
 @pytest.mark.parametrize("history", [40, 3000, 60_000])
 def test_rows_under_penalties(monkeypatch, held, bf16, history):
     vocab = 40_009
     rng = np.random.default_rng(history)
     x = _rows(rng, vocab, bf16)
-    for slices in (0, 3 if bf16 else 6):
+    for slices in (0, 3 if bf16 else 6, 1):
         s = _sampler(monkeypatch, held, slices)
         hist = rng.integers(0, vocab, (ROWS, history)).astype(np.int32)
         hist[:, :history // 2] = rng.integers(0, 50, (ROWS, history // 2))
@@ -85,7 +86,7 @@ def test_rows_under_penalties(monkeypatch, held, bf16, history):
                     sc.append(t)
                     counts.append(np.bincount(hist[i], minlength=vocab).astype(np.uint32))
                 kw = [dict(temperature=0.8, top_k=33, top_p=0.95, seed=7 + i, **pen) for i in range(ROWS)]
-                r = run_rows(s, x, kw, [4] * ROWS, scratch=sc, logprobs=lp)
+                r = run_rows(s, x, kw, [4] * ROWS, scratch=sc, logprobs=lp, use_plan=True)
                 _check(r, x, kw, 4, lp, counts)
                 for i in range(ROWS):
                     assert np.array_equal(sc[i].read_counts().numpy(), counts[i]), i   # (the oracle counted its draw)
@@ -93,7 +94,7 @@ def test_rows_under_penalties(monkeypatch, held, bf16, history):
         s.close()
 
 
-@pytest.mark.parametrize("held", [True, False], ids=["held", "streamed"])
+@pytest.mark.parametrize("held", ["1", "blocks", "0"], ids=["held", "blocks", "streamed"])
 @pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
 def test_rows_with_masks_bias_lists_and_forced_ids(monkeypatch, held, bf16):
     vocab = 50_021
@@ -129,7 +130,7 @@ def test_rows_with_masks_bias_lists_and_forced_ids(monkeypatch, held, bf16):
         s.close()
 
 
-@pytest.mark.parametrize("held", [True, False], ids=["held", "streamed"])
+@pytest.mark.parametrize("held", ["1", "blocks", "0"], ids=["held", "blocks", "streamed"])
 @pytest.mark.parametrize("draft_k", [20, 0], ids=["20 drafted from", "all drafted from"])
 def test_verify_pass(monkeypatch, held, draft_k):
     """Drafts from 20 and from 1 024 candidates (the latter's distribution is longer than a wave), verified
