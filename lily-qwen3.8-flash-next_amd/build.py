@@ -39,6 +39,7 @@ def units():
     out += [("rows_held.hip", f"rows_held_dt{dt}_blocks{nb}.o", [f"-DLILY_DT={dt}", f"-DLILY_BLOCKS={nb}"])
             for dt in (0, 1) for nb in (2, 1)]
     out += [("rows_blocks.hip", f"rows_blocks_dt{dt}.o", [f"-DLILY_DT={dt}"]) for dt in (0, 1)]
+    out += [("rows_masked.hip", f"rows_masked_dt{dt}.o", [f"-DLILY_DT={dt}"]) for dt in (0, 1)]
     out.append(("scratch_kernels.hip", "scratch_kernels.o", []))
     out.append(("static_entry.hip", "static_entry.o", []))
     out.append(("lm_head.hip", "lm_head.o", []))

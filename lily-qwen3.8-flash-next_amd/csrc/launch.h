@@ -17,14 +17,15 @@ constexpr uint32_t CU_LDS_BYTES = 160u * 1024u;   // a compute unit's
 // raised.)
 struct LdsAllowed {
     std::atomic<bool> said[64] = {};
-    hipError_t say(const void* kernel) {
+    // `bytes`: always the same for one kernel (a kernel with LDS of its own cannot have all of it)
+    hipError_t say(const void* kernel, uint32_t bytes = CU_LDS_BYTES) {
         int device = 0;
         hipError_t e = hipGetDevice(&device);
         const bool known = e == hipSuccess && device >= 0 && device < 64;
         if (e != hipSuccess || (known && said[device].load(std::memory_order_acquire))) {
             return e;
         }
-        e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)CU_LDS_BYTES);
+        e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
         if (e == hipSuccess && known) {
             said[device].store(true, std::memory_order_release);
         }
@@ -121,6 +122,11 @@ hipError_t launch_rows_held(hipStream_t stream, int dtype, uint32_t blocks, bool
                             const LaunchCfg& cfg, const InlineRows* inline_rows);
 // The same rows of cfg.table (no mask, no bias list, plain draws) in slices of any length, a block at a time.
 hipError_t launch_rows_blocks(hipStream_t stream, int dtype, bool lse, bool pen, uint32_t rows, const LaunchCfg& cfg);
+// Plain draws under an allow-mask with at most STREAM_BIAS_CAP bias pairs, given inline or as cfg.table: a workgroup a
+// row whatever cfg.slices says, vocabularies up to MASKED_MAX_VOCAB.  cfg.masked_served: which rows it drew.
+constexpr uint32_t MASKED_MAX_VOCAB = 262144;
+hipError_t launch_rows_masked(hipStream_t stream, int dtype, bool lse, uint32_t rows, const LaunchCfg& cfg,
+                              const InlineRows* inline_rows);
 // Rows that draw among many candidates (k > 64), spread over cfg.slices workgroups a row: two
 // launches (the row's bound, then the values that reach it, merge, select, tail).
 // lane_max [rows][slices][256], bound [rows], count [rows][slices].

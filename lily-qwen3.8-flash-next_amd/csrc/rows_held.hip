@@ -440,10 +440,10 @@ __device__ __forceinline__ bool held_row(const LILY_CONST RowArgs* src, const La
             }
         }
     } else {
-        // More than that (masks, ties): every thread counts what its entries have ahead of them.
-        constexpr int PER = HELD_CAP / NT;
-        uint64_t mine[PER];
+        // More than that: masks that leave whole waves without a value, ties.
         if (!overflow) {
+            constexpr int PER = HELD_CAP / NT;
+            uint64_t mine[PER];
 #pragma unroll
             for (int q = 0; q < PER; ++q) {
                 const uint32_t i = tid + (uint32_t)q * NT;
@@ -454,62 +454,34 @@ __device__ __forceinline__ bool held_row(const LILY_CONST RowArgs* src, const La
                     listed_sum += term(x);
                 }
             }
-        } else {
-            // Ties by the thousand.  (From the row itself: by now the values' registers are free.)
-            select_exhaustive<DT>(a, g.id_lo, g.id_hi, a.k, want_lse, ranked, 64u, sh);
-            n = min(sh.n_cand, 64u);
-#pragma unroll
-            for (int q = 0; q < PER; ++q) {
-                const uint32_t i = tid + (uint32_t)q * NT;
-                mine[q] = i < n ? ranked[i] : 0ull;
-            }
-        }
-        __syncthreads();   // (the pairs, or the ranked ones' place, have been read)
-        const uint32_t rounds = (n + NT - 1u) / NT;
-#pragma unroll
-        for (int q = 0; q < PER; ++q) {
-            if ((uint32_t)q < rounds) {
-                pairs[tid + (uint32_t)q * NT] = mine[q];   // (0 from n on, up to a multiple of NT)
-            }
-        }
-        if (tid < 64u) {
-            ranked[tid] = 0ull;
-        }
-        if (LSE && want_lse) {
-            listed_sum = wave_sum_d(listed_sum);
-            if (lane == 0u) {
-                sh.red3[0][w] = listed_sum;
-            }
-        }
-        __syncthreads();
-        uint32_t ahead[PER] = {};
-        for (uint32_t i = 0; i < n; i += 8u) {
-            uint64_t other[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                other[q] = pairs[i + (uint32_t)q];
-            }
-#pragma unroll
-            for (int p = 0; p < PER; ++p) {
-                if ((uint32_t)p < rounds) {
-#pragma unroll
-                    for (int q = 0; q < 8; ++q) {
-                        ahead[p] += other[q] > mine[p] ? 1u : 0u;
-                    }
+            if (LSE && want_lse) {
+                listed_sum = wave_sum_d(listed_sum);
+                if (lane == 0u) {
+                    sh.red3[0][w] = listed_sum;
                 }
             }
-        }
+            __syncthreads();   // (the pairs have been read)
 #pragma unroll
-        for (int p = 0; p < PER; ++p) {
-            if (mine[p] != 0ull && ahead[p] < 64u) {
-                ranked[ahead[p]] = mine[p];
+            for (int q = 0; q < PER; ++q) {
+                if (tid + (uint32_t)q * NT < n) {
+                    pairs[tid + (uint32_t)q * NT] = mine[q];
+                }
             }
+            __syncthreads();
+        } else {
+            // Ties by the thousand.  (From the row itself: by now the values' registers are free.)
+            select_exhaustive<DT>(a, g.id_lo, g.id_hi, a.k, want_lse, pairs, 64u, sh);
+            n = min(sh.n_cand, 64u);
         }
+        bool sorted = false;
+        n = select_topk(pairs, n, a.k, sh, sorted);
         __syncthreads();
         if (w != 0u && !by_workgroup) {
             return false;
         }
-        c = w == 0u ? ranked[lane] : 0ull;
+        if (w == 0u) {
+            c = wave_sort_desc(lane < n ? pairs[lane] : 0ull);
+        }
         if (LSE && want_lse) {
             listed_sum = 0.0;
             for (int i = 0; i < NWAVE; ++i) {

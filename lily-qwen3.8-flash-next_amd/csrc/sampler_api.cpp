@@ -109,6 +109,7 @@ struct lily_sampler {
     // rows that draw among many candidates (rows_wide.hip): null in a view without them
     float* wide_max = nullptr;     // [WIDE_FLOATS] lane maxima, rows x slices x 256
     uint32_t* wide_count = nullptr;  // [WS_ROWS] candidates listed so far, 0 between launches
+    uint32_t* masked_served = nullptr;   // [WS_ROWS] rows that a launch over masks' words has drawn
     uint32_t ws_rows = WS_ROWS;    // rows that may span several workgroups
     uint32_t ws_slots = WS_SLOTS;  // candidate slots behind ws_cand
     // Row table of lily_sample_rows batches above INLINE_ROWS.
@@ -182,6 +183,7 @@ struct LaunchPart {
     bool wide = false;   // every row draws among many candidates: the two launches of rows_wide.hip
     uint32_t held = 0;   // slices of so many blocks, held in registers (rows_held.hip)
     bool extra = false;  // ... with a mask or a bias list on some row
+    bool masked = false; // every row under a mask: a workgroup a row (rows_masked.hip)
     bool blocks = false; // slices of any length, a block at a time (rows_blocks.hip)
     bool pen = false;    // ... with penalties on some row
 };
@@ -361,8 +363,9 @@ struct HeldShape {
 // Rows under penalties without log-probabilities stay below that (bf16, 151 936 ids, streamed -> held: 40 rows
 // in 19 slices 21.9 -> 21.9 us, 50 rows 22.3 -> 23.2, 60 rows in 10 slices of two blocks 23.8 -> 25.6).
 constexpr uint32_t HELD_MAX_GROUPS[3] = {0, 1024, 768};
-constexpr uint32_t HELD_MAX_GROUPS_LISTED = 768;
-HeldShape held_shape(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint32_t vocab, int dtype, bool pen, bool lse) {
+// Rows with masks too (2 % admitted, k = 50: 30 rows 21.8 -> 19.6, 64 rows in slices of two blocks 21.8 -> 27.3).
+constexpr uint32_t HELD_MAX_GROUPS_LISTED = 768, HELD_MAX_GROUPS_EXTRA = 600;
+HeldShape held_shape(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint32_t vocab, int dtype, bool pen, bool lse, bool extra) {
     HeldShape out;
     if (s->force_path != 0 || s->no_held || s->only_blocks || kmax > STREAM_K_MAX || rows > s->ws_rows) {
         return out;
@@ -375,6 +378,9 @@ HeldShape held_shape(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint32
         if (sl > MAX_SLICES || (s->force_slices != 0 && s->force_slices < least) ||
             (sl > WAVE_MERGE_LISTS && sl * kmax > HELD_MERGE_SLOTS) ||
             (uint64_t)rows * sl * kmax > s->ws_slots || (uint64_t)rows * sl > HELD_MAX_GROUPS[blocks]) {
+            continue;
+        }
+        if (extra && (uint64_t)rows * sl > HELD_MAX_GROUPS_EXTRA) {
             continue;
         }
         if (pen && !lse && ((uint64_t)rows * sl > HELD_MAX_GROUPS_LISTED || (blocks == 2 && dtype == LILY_BF16))) {
@@ -435,6 +441,25 @@ HeldRows held_rows(const RowArgs* rows, uint32_t n) {
         h.lse = h.lse || rows[i].out_logprob != nullptr;
     }
     return h;
+}
+
+constexpr uint32_t MASKED_MAX_ROWS = 256;
+// Whether a launch goes a workgroup a row over the masks' words first (rows_masked.hip): where rows draw among
+// many candidates, and a workgroup a row fills the chip no more than once.  (bf16, 151 936 ids, no top_k, us, before ->
+// now: 2 % admitted 1 row 28.1 -> 24.7, 64 rows 36.3 -> 28.3; a tenth of that 24.8 -> 18.2, 28.5 -> 19.7; ten times as much 71 ->
+// 75, 1 819 -> 86; all of them, which the launch behind takes, 74.7 -> 81.2, 89.9 -> 97.8.  For k <= 64 the
+// streaming selects make less of the difference: 64 rows 21.8 -> 19.8, all ids admitted 32 -> 39.)
+bool all_masked(const lily_sampler* s, const RowArgs* rows, uint32_t n, uint32_t vocab, uint32_t kmax) {
+    if (kmax <= STREAM_K_MAX || n > MASKED_MAX_ROWS || s->masked_served == nullptr || n > s->ws_rows || s->force_path != 0 ||
+        s->no_held || (s->force_slices != 0 && !s->only_blocks) || vocab > MASKED_MAX_VOCAB) {
+        return false;
+    }
+    for (uint32_t i = 0; i < n; ++i) {
+        if (rows[i].mode != MODE_PLAIN || rows[i].allow == nullptr || rows[i].n_bias > STREAM_BIAS_CAP) {
+            return false;
+        }
+    }
+    return true;
 }
 
 // Launches of more than this many workgroups hand their slices over in the relaxed form (see
@@ -625,7 +650,7 @@ uint32_t plan_parts(const lily_sampler* s, RowArgs* table, uint32_t rows, int dt
     // (a launch that holds its slices takes both kinds alike)
     const HeldRows whole = held_rows(table, rows);
     const bool together =
-        whole.all && held_shape(s, rows, max_k(table, rows), vocab, dtype, whole.pen, whole.lse).blocks != 0;
+        whole.all && held_shape(s, rows, max_k(table, rows), vocab, dtype, whole.pen, whole.lse, whole.extra).blocks != 0;
     const bool split = !together && heavy != 0 && rows - heavy >= SPLIT_MIN_LIGHT;
     if (split) {
         std::stable_partition(table, table + rows,
@@ -648,13 +673,14 @@ uint32_t plan_parts(const lily_sampler* s, RowArgs* table, uint32_t rows, int dt
         part.extra = is.extra;
         part.pen = is.pen;
         if (is.all) {
-            const HeldShape held = held_shape(s, part.rows, part.ws_k, vocab, dtype, is.pen, is.lse);
+            const HeldShape held = held_shape(s, part.rows, part.ws_k, vocab, dtype, is.pen, is.lse, is.extra);
             const uint32_t blocks = held.blocks == 0 && !is.extra && part.rows <= s->ws_rows
                                         ? blocks_slices(s, part.rows, part.ws_k, vocab, dtype, is.pen, is.lse) : 0u;
             part.held = held.blocks;
             part.blocks = blocks != 0;
             part.slices = held.blocks != 0 ? held.slices : blocks != 0 ? blocks : part.slices;
         }
+        part.masked = all_masked(s, sub, part.rows, vocab, part.ws_k);
         const LaunchShape shp = shape_of(s, sub, part.rows, dtype, vocab, part.slices, part.ws_k);
         part.kind = shp.kind();
         part.lse = shp.lse;
@@ -685,6 +711,13 @@ int launch_part(lily_sampler* s, const LaunchPart& part, const RowArgs* table_de
         HIP_TRY(launch_rows_wide(s->stream, dtype, part.lse, part.rows, cfg, nullptr, s->wide_max,
                                  s->wide_count));
         return LILY_OK;
+    }
+    if (part.masked && served == nullptr) {
+        LaunchCfg first = cfg;
+        first.masked_served = s->masked_served;
+        HIP_TRY(launch_rows_masked(s->stream, dtype, part.lse, part.rows, first, nullptr));
+        cfg.served = s->masked_served;
+        cfg.phase_trace = nullptr;
     }
     if (part.blocks) {
         HIP_TRY(launch_rows_blocks(s->stream, dtype, part.lse, part.pen, part.rows, cfg));
@@ -723,7 +756,8 @@ int launch_inline(lily_sampler* s, int dtype, uint32_t vocab, const InlineRows& 
     }
     const HeldRows is = held_rows(rows.r, n);
     const HeldShape held =
-        !chained && is.all ? held_shape(s, n, kmax, vocab, dtype, is.pen, is.lse) : HeldShape();
+        !chained && is.all ? held_shape(s, n, kmax, vocab, dtype, is.pen, is.lse, is.extra) : HeldShape();
+    const bool masked = !chained && !verify && all_masked(s, rows.r, n, vocab, kmax);
     const uint32_t slices = held.blocks != 0 ? held.slices : choose_slices(s, n, kmax, vocab, dtype);
     fill_cfg(s, &cfg, n, vocab, slices, kmax, 0, nullptr);
     if (chained) {
@@ -755,6 +789,12 @@ int launch_inline(lily_sampler* s, int dtype, uint32_t vocab, const InlineRows& 
         return LILY_OK;
     }
     const LaunchShape shp = shape_of(s, rows.r, n, dtype, vocab, slices, kmax);
+    if (masked) {
+        cfg.masked_served = s->masked_served;
+        HIP_TRY(launch_rows_masked(s->stream, dtype, shp.lse, n, cfg, &rows));
+        cfg.served = s->masked_served;
+        cfg.phase_trace = nullptr;
+    }
     if (held.blocks != 0) {
         for (uint32_t i = 0; i < n; ++i) {
             cfg.verify = rows.r[i].mode == MODE_SPEC ? 1u : cfg.verify;   // (the kernel that holds that draw)
@@ -1123,6 +1163,7 @@ int lily_sampler_create(int device, void* hip_stream, lily_sampler_t** out) {
     if (err == hipSuccess) err = hipMemset(s->ws_ticket, 0, WS_ROWS * 4);
     if (err == hipSuccess) err = hipMalloc(reinterpret_cast<void**>(&s->wide_max), (size_t)WIDE_FLOATS * 4);
     if (err == hipSuccess) err = hipMalloc(reinterpret_cast<void**>(&s->wide_count), WS_ROWS * 4);
+    if (err == hipSuccess) err = hipMalloc(reinterpret_cast<void**>(&s->masked_served), WS_ROWS * 4);
     if (err == hipSuccess) err = hipMemset(s->wide_count, 0, WS_ROWS * 4);
     const size_t chain_bytes = (size_t)LILY_MAX_VERIFY_ROWS * CHAIN_CAP * 8 + (LILY_MAX_VERIFY_ROWS + 1) * 4;
     if (err == hipSuccess) err = hipMalloc(reinterpret_cast<void**>(&s->chain_cand), chain_bytes);
@@ -1157,6 +1198,7 @@ void lily_sampler_destroy(lily_sampler_t* s) {
     (void)hipFree(s->ws_ticket);
     (void)hipFree(s->wide_max);
     (void)hipFree(s->wide_count);
+    (void)hipFree(s->masked_served);
     (void)hipFree(s->chain_cand);
     (void)hipFree(s->table_dev);
     for (uint32_t i = 0; i < STAGE_SLOTS; ++i) {
@@ -1188,7 +1230,7 @@ uint32_t lily_sampler_slices_for(const lily_sampler_t* s, uint32_t rows, uint32_
     if (s == nullptr || rows == 0) {
         return 0;
     }
-    const HeldShape held = held_shape(s, rows, k ? k : 1, vocab, (int)dtype, false, false);
+    const HeldShape held = held_shape(s, rows, k ? k : 1, vocab, (int)dtype, false, false, false);
     const uint32_t blocks = blocks_slices(s, rows, k ? k : 1, vocab, (int)dtype, false, false);
     return held.blocks != 0 ? held.slices : blocks != 0 ? blocks : choose_slices(s, rows, k ? k : 1, vocab, (int)dtype);
 }
@@ -2070,7 +2112,7 @@ int rows_with_tiles(lily_sampler* s, const lily_lm_head* h, const lily_rows* b, 
     // Rows under penalties whose slices can be held in registers are drawn from their logits at once (masks: most
     // rows are drawn from a few tiles): the launch that would stand behind the draws from summaries anyway is no slower for drawing them
     // all (4 rows under penalties 17 us, 23 with the summaries first; 24 rows 27 and 31).
-    bool held = true, behind_pen = false, behind_lse = false;
+    bool held = true, behind_pen = false, behind_lse = false, behind_extra = false;
     uint32_t behind = 0, behind_k = 1;
     for (uint32_t r = 0; r < rows; ++r) {
         const RowArgs& row = packed[r];
@@ -2082,11 +2124,12 @@ int rows_with_tiles(lily_sampler* s, const lily_lm_head* h, const lily_rows* b, 
             held = held && is.all && (!serve || row.allow == nullptr);
             behind_pen = behind_pen || is.pen;
             behind_lse = behind_lse || is.lse;
+            behind_extra = behind_extra || is.extra;
             behind += 1;
             behind_k = row.k > behind_k ? row.k : behind_k;
         }
     }
-    held = held && behind != 0 && held_shape(s, behind, behind_k, b->vocab, (int)b->dtype, behind_pen, behind_lse).blocks != 0;
+    held = held && behind != 0 && held_shape(s, behind, behind_k, b->vocab, (int)b->dtype, behind_pen, behind_lse, behind_extra).blocks != 0;
     for (int group = 0; group < 3; ++group) {
         for (uint32_t r = 0; r < rows; ++r) {
             const RowArgs& row = packed[r];

@@ -256,6 +256,15 @@ hipError_t launch_rows_blocks(hipStream_t stream, int dtype, bool lse, bool pen,
                               : launch_rows_blocks_dt0(stream, lse, pen, rows, cfg);
 }
 
+hipError_t launch_rows_masked_dt0(hipStream_t stream, bool lse, uint32_t rows, const LaunchCfg& cfg, const InlineRows* inline_rows);
+hipError_t launch_rows_masked_dt1(hipStream_t stream, bool lse, uint32_t rows, const LaunchCfg& cfg, const InlineRows* inline_rows);
+
+hipError_t launch_rows_masked(hipStream_t stream, int dtype, bool lse, uint32_t rows, const LaunchCfg& cfg,
+                              const InlineRows* inline_rows) {
+    return dtype == LILY_BF16 ? launch_rows_masked_dt1(stream, lse, rows, cfg, inline_rows)
+                              : launch_rows_masked_dt0(stream, lse, rows, cfg, inline_rows);
+}
+
 hipError_t launch_fill_u32(hipStream_t stream, uint32_t* p, uint32_t n, uint32_t v) {
     if (n == 0) {
         return hipSuccess;

@@ -172,3 +172,47 @@ def test_verify_pass(monkeypatch, held, draft_k):
     scratch.close()
     dists.close()
     s.close()
+
+
+@pytest.mark.parametrize("held", ["1", "0"], ids=["masked", "other"])
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+@pytest.mark.parametrize("vocab", [33, 2051, 70_001])
+def test_masked_rows_of_many_candidates(monkeypatch, held, bf16, vocab):
+    """A workgroup a row over the mask's words (rows_masked.hip), and the selects it replaces: masks that admit
+    nothing, a few ids, what the sort holds (8 192) and a little more, and nearly all (left to the
+    launch behind); equal values by the thousand; bias lists, penalties and a forced id; inline and from a table."""
+    rng = np.random.default_rng(vocab)
+    rows = 9
+    x = np.concatenate([_rows(rng, vocab, False), rng.normal(0, 2, (1, vocab)).astype(np.float32)])
+    x[4] = x[0]
+    x[6] = x[7]
+    allow = np.zeros((rows, (vocab + 31) // 32), dtype=np.uint32)
+    for i, admitted in enumerate((0.02, 0.05, 0.13, 0.6, 8192 / vocab, 8300 / vocab, 0.0, 0.97, 0.3)):
+        ids = np.flatnonzero(rng.random(vocab) < admitted)
+        if i in (4, 5):
+            ids = rng.choice(vocab, min(vocab, 8192 + 108 * (i - 4)), replace=False)
+        np.bitwise_or.at(allow[i], ids >> 5, (1 << (ids & 31)).astype(np.uint32))
+    bias = [[(int(i), float(d)) for i, d in zip(rng.integers(0, vocab, 30), rng.choice([-5.0, 5.0, 0.5], 30))]
+            for _ in range(rows)]
+    bias[2] = []
+    forced = [None] * rows
+    forced[0] = 1
+    xs = W.to_bf16_bits(x) if bf16 else x
+    s = _sampler(monkeypatch, held)
+    hist = rng.integers(0, vocab, (rows, 700)).astype(np.int32)
+    for trial, (k, lp, few) in enumerate(((0, True, False), (300, False, True), (65, True, True))):
+        sc, counts = [], []
+        for i in range(rows):
+            t = LS.SamplerScratch(s, vocab)
+            t.add_history(torch.from_numpy(hist[i]).to(dev()))
+            sc.append(t)
+            counts.append(np.bincount(hist[i], minlength=vocab).astype(np.uint32))
+        n = 8 if few else rows   # (up to eight rows travel with the launch)
+        kw = [dict(temperature=0.8, top_k=k, top_p=0.95, seed=9 + i, repetition_penalty=1.2, presence_penalty=0.1,
+                   frequency_penalty=0.2) for i in range(n)]
+        ext = dict(allow=allow[:n], bias=bias[:n], forced=(forced if lp else [None] * rows)[:n])
+        r = run_rows(s, xs[:n], kw, [trial] * n, scratch=sc[:n], logprobs=lp, **ext)
+        _check(r, xs[:n], kw, trial, lp, counts[:n], **ext)
+        for t in sc:
+            t.close()
+    s.close()
