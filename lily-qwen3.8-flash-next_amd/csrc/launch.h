@@ -55,6 +55,14 @@ hipError_t launch_spec_accept(hipStream_t stream, const uint32_t* draws, const u
 // out_f32: the logits are f32 [rows, logits_stride] instead of bf16.  wq.bits 4 / 8: `weight` points
 // at the reference's affine codes (u32 words, weight_stride words a row), wq.scales / wq.biases at
 // bf16 [vocab, d >> wq.group_shift]; f32 logits only.
+// The rows' exponent scales: in device memory, or (p null, at most SCALES_INLINE rows) with the launch itself.
+constexpr uint32_t SCALES_INLINE = 8;
+struct RowScales {
+    const float* p = nullptr;
+    float few[SCALES_INLINE] = {};
+    RowScales() = default;
+    RowScales(const float* from) : p(from) {}
+};
 struct HeadWeights {
     uint32_t bits = 0;          // 0 = bf16 weights
     const void* scales = nullptr;
@@ -69,7 +77,7 @@ struct HeadWeights {
 };
 hipError_t launch_lm_head_bf16(hipStream_t stream, const void* hidden, uint64_t hidden_stride,
                                const void* weight, uint64_t weight_stride, uint32_t rows, uint32_t d,
-                               uint32_t vocab, const float* c2_of_row, void* logits,
+                               uint32_t vocab, const RowScales& c2_of_row, void* logits,
                                uint64_t logits_stride, float* tile_max, float* tile_sum, bool out_f32,
                                const HeadWeights& wq);
 // The same over codes for up to 16 rows in the reference's form for few rows (the codes are not
@@ -79,7 +87,7 @@ bool lm_head_codes_serves(uint32_t rows, uint32_t d, uint32_t vocab, uint64_t hi
                           const HeadWeights& wq);
 hipError_t launch_lm_head_codes(hipStream_t stream, const void* hidden, uint64_t hidden_stride, const void* weight,
                                 uint64_t weight_stride, uint32_t rows, uint32_t d, uint32_t vocab,
-                                const float* c2_of_row, void* logits, uint64_t logits_stride, float* tile_max,
+                                const RowScales& c2_of_row, void* logits, uint64_t logits_stride, float* tile_max,
                                 float* tile_sum, const HeadWeights& wq);
 // The same for any number of rows with the weights in bf16, as dequant_q4/q8_bf16 make them of the
 // codes (groups of 64 or more, whole lines of codes).
@@ -88,7 +96,7 @@ bool lm_head_codes_rows_serves(uint32_t d, const HeadWeights& wq);
 uint32_t lm_head_codes_rows_resident(uint32_t d, const HeadWeights& wq);
 hipError_t launch_lm_head_codes_rows(hipStream_t stream, const void* hidden, uint64_t hidden_stride, const void* weight,
                                      uint64_t weight_stride, uint32_t rows, uint32_t d, uint32_t vocab,
-                                     const float* c2_of_row, void* logits, uint64_t logits_stride, float* tile_max,
+                                     const RowScales& c2_of_row, void* logits, uint64_t logits_stride, float* tile_max,
                                      float* tile_sum, const HeadWeights& wq);
 // The batch form through the vendor's GEMM library, opened by name at run time: the product alone
 // (codes are turned into bf16 weights first, in memory this call keeps per device and stream);
@@ -102,6 +110,11 @@ hipError_t launch_head_library(hipStream_t stream, const void* hidden, uint64_t 
 hipError_t launch_head_summaries(hipStream_t stream, const void* logits, uint64_t logits_stride, uint32_t rows,
                                  uint32_t vocab, const float* c2_of_row, float* tile_max, float* tile_sum,
                                  bool f32);
+// The same of at most INLINE_ROWS rows that travel with the launch, each with its row of the summaries in
+// RowArgs::pad; none under penalties or a mask.
+hipError_t launch_rows_tiles_inline(hipStream_t stream, int dtype, bool lse, bool extra, uint32_t rows, const LaunchCfg& cfg,
+                                    const InlineRows& inline_rows, const float* tile_max, const float* tile_sum,
+                                    uint32_t tiles);
 // The draw of `rows` rows of cfg.table from the summaries ([.., tiles] each) and the few tiles of
 // the logits (bf16 or f32) that matter; tile_row[r] = the summaries' row of table row r; served[r] is set
 // for rows under penalties or a mask (1 = drawn, 0 = declined: the row is better read whole).

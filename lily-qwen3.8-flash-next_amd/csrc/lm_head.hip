@@ -73,11 +73,11 @@ struct HeadQuant {
 
 template <class T, bool OUT_F32, int WBITS>
 __global__ void __launch_bounds__(256, T::RESIDENT)
-k_lm_head_bf16(const uint16_t* __restrict__ hidden, uint64_t hidden_stride,
+k_lm_head_bf16(const RowScales scales_arg, const uint16_t* __restrict__ hidden, uint64_t hidden_stride,
                const uint16_t* __restrict__ weight, uint64_t weight_stride, uint32_t rows,
-               uint32_t d, uint32_t vocab, const float* __restrict__ c2_of_row,
-               void* __restrict__ logits_out, uint64_t logits_stride, float* __restrict__ tile_max,
+               uint32_t d, uint32_t vocab, void* __restrict__ logits_out, uint64_t logits_stride, float* __restrict__ tile_max,
                float* __restrict__ tile_sum, uint32_t tiles_per_row, uint32_t m_tiles, HeadQuant quant) {
+    const float* __restrict__ c2_of_row = scales_of(scales_arg);
     static_assert(WBITS == 0 || !T::DIRECT, "codes pass through registers");
     constexpr int BM = T::BM, BN = T::BN, BK = T::BK, MI = T::MI, NI = T::NI, ROW_BYTES = T::ROW_BYTES;
     extern __shared__ __align__(16) char lds[];
@@ -397,7 +397,7 @@ k_lm_head_bf16(const uint16_t* __restrict__ hidden, uint64_t hidden_stride,
 template <class T, bool OUT_F32, int WBITS>
 static hipError_t launch_head_shape(hipStream_t stream, const void* hidden, uint64_t hidden_stride,
                                     const void* weight, uint64_t weight_stride, uint32_t rows, uint32_t d,
-                                    uint32_t vocab, const float* c2_of_row, void* logits,
+                                    uint32_t vocab, const RowScales& c2_of_row, void* logits,
                                     uint64_t logits_stride, float* tile_max, float* tile_sum,
                                     const HeadQuant& quant) {
     static LdsAllowed allowed;
@@ -409,16 +409,16 @@ static hipError_t launch_head_shape(hipStream_t stream, const void* hidden, uint
     // slots an XCD needs at most (see the kernel's numbering)
     const uint32_t slots = m_tiles <= 8u ? (tiles_per_row + (8u / m_tiles) - 1u) / (8u / m_tiles)
                                          : ((m_tiles + 7u) / 8u) * tiles_per_row;
-    hipLaunchKernelGGL((k_lm_head_bf16<T, OUT_F32, WBITS>), dim3(8u * slots), dim3(256), T::LDS_BYTES, stream,
+    hipLaunchKernelGGL((k_lm_head_bf16<T, OUT_F32, WBITS>), dim3(8u * slots), dim3(256), T::LDS_BYTES, stream, c2_of_row,
                        reinterpret_cast<const uint16_t*>(hidden), hidden_stride,
                        reinterpret_cast<const uint16_t*>(weight), weight_stride, rows, d, vocab,
-                       c2_of_row, logits, logits_stride, tile_max, tile_sum, tiles_per_row, m_tiles, quant);
+                       logits, logits_stride, tile_max, tile_sum, tiles_per_row, m_tiles, quant);
     return hipGetLastError();
 }
 
 hipError_t launch_lm_head_bf16(hipStream_t stream, const void* hidden, uint64_t hidden_stride,
                                const void* weight, uint64_t weight_stride, uint32_t rows, uint32_t d,
-                               uint32_t vocab, const float* c2_of_row, void* logits,
+                               uint32_t vocab, const RowScales& c2_of_row, void* logits,
                                uint64_t logits_stride, float* tile_max, float* tile_sum, bool out_f32,
                                const HeadWeights& wq) {
     HeadQuant quant;
@@ -435,7 +435,7 @@ hipError_t launch_lm_head_bf16(hipStream_t stream, const void* hidden, uint64_t 
     // (the pass over the stored logits reads 16-byte pieces: rows that start at multiples of 16 bytes)
     const bool rows_aligned = (reinterpret_cast<uintptr_t>(logits) & 15u) == 0u &&
                               (logits_stride * (out_f32 ? 4u : 2u)) % 16u == 0u;
-    if (wq.library_rows != 0u && rows >= wq.library_rows && (wq.bits == 0u || out_f32) && rows_aligned &&
+    if (c2_of_row.p != nullptr && wq.library_rows != 0u && rows >= wq.library_rows && (wq.bits == 0u || out_f32) && rows_aligned &&
         (vocab + LILY_TILE_COLS - 1u) / LILY_TILE_COLS <= HEAD_LIBRARY_MAX_TILES) {
         const hipError_t e = launch_head_library(stream, hidden, hidden_stride, weight, weight_stride, rows, d, vocab,
                                                  logits, logits_stride, out_f32, wq);
@@ -443,7 +443,7 @@ hipError_t launch_lm_head_bf16(hipStream_t stream, const void* hidden, uint64_t 
             if (wq.library_calls != nullptr) {
                 ++*wq.library_calls;
             }
-            return launch_head_summaries(stream, logits, logits_stride, rows, vocab, c2_of_row, tile_max, tile_sum,
+            return launch_head_summaries(stream, logits, logits_stride, rows, vocab, c2_of_row.p, tile_max, tile_sum,
                                          out_f32);
         }
         if (e != hipErrorNotSupported) {

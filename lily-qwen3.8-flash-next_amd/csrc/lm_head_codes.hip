@@ -73,12 +73,13 @@ inline size_t codes_lds_bytes(uint32_t groups) {
 // upper half is the bf16.
 template <int WBITS>
 __global__ void __launch_bounds__(THREADS, 4)   // (four waves a SIMD: two workgroups a compute unit)
-k_lm_head_codes(const uint16_t* __restrict__ hidden, uint64_t hidden_stride, const uint32_t* __restrict__ codes,
+k_lm_head_codes(const RowScales scales_arg, const uint16_t* __restrict__ hidden, uint64_t hidden_stride, const uint32_t* __restrict__ codes,
                 uint64_t weight_stride, uint32_t rows, uint32_t d, uint32_t vocab,
-                const float* __restrict__ c2_of_row, float* __restrict__ logits, uint64_t logits_stride,
+                float* __restrict__ logits, uint64_t logits_stride,
                 float* __restrict__ tile_max, float* __restrict__ tile_sum, uint32_t tiles_per_row,
                 const uint16_t* __restrict__ scales, const uint16_t* __restrict__ biases, uint32_t group_shift,
                 unsigned long long* trace) {
+    const float* __restrict__ c2_of_row = scales_of(scales_arg);
     // Diagnostic stamps, compiled in with -DLILY_HEAD_TRACE: [workgroup][8] device-clock values
     // (0 start, 1 scales and first stage written, 2 past the barrier, 3 loop done, 4 end).
 #ifdef LILY_HEAD_TRACE
@@ -406,7 +407,7 @@ k_lm_head_codes(const uint16_t* __restrict__ hidden, uint64_t hidden_stride, con
 template <int WBITS>
 static hipError_t launch_codes(hipStream_t stream, const void* hidden, uint64_t hidden_stride, const void* weight,
                                uint64_t weight_stride, uint32_t rows, uint32_t d, uint32_t vocab,
-                               const float* c2_of_row, void* logits, uint64_t logits_stride, float* tile_max,
+                               const RowScales& c2_of_row, void* logits, uint64_t logits_stride, float* tile_max,
                                float* tile_sum, const HeadWeights& wq) {
     const uint32_t tiles_per_row = (vocab + LILY_TILE_COLS - 1u) / LILY_TILE_COLS;
     const size_t lds = codes_lds_bytes(d >> wq.group_shift);
@@ -415,9 +416,9 @@ static hipError_t launch_codes(hipStream_t stream, const void* hidden, uint64_t 
     if (e != hipSuccess) {
         return e;
     }
-    hipLaunchKernelGGL((k_lm_head_codes<WBITS>), dim3(tiles_per_row), dim3(THREADS), lds, stream,
+    hipLaunchKernelGGL((k_lm_head_codes<WBITS>), dim3(tiles_per_row), dim3(THREADS), lds, stream, c2_of_row,
                        static_cast<const uint16_t*>(hidden), hidden_stride, static_cast<const uint32_t*>(weight),
-                       weight_stride, rows, d, vocab, c2_of_row, static_cast<float*>(logits), logits_stride,
+                       weight_stride, rows, d, vocab, static_cast<float*>(logits), logits_stride,
                        tile_max, tile_sum, tiles_per_row, static_cast<const uint16_t*>(wq.scales),
                        static_cast<const uint16_t*>(wq.biases), wq.group_shift,
                        wq.trace_words >= (unsigned long long)tiles_per_row * 8u ? wq.trace : nullptr);
@@ -439,7 +440,7 @@ bool lm_head_codes_serves(uint32_t rows, uint32_t d, uint32_t vocab, uint64_t hi
 
 hipError_t launch_lm_head_codes(hipStream_t stream, const void* hidden, uint64_t hidden_stride, const void* weight,
                                 uint64_t weight_stride, uint32_t rows, uint32_t d, uint32_t vocab,
-                                const float* c2_of_row, void* logits, uint64_t logits_stride, float* tile_max,
+                                const RowScales& c2_of_row, void* logits, uint64_t logits_stride, float* tile_max,
                                 float* tile_sum, const HeadWeights& wq) {
     if (!lm_head_codes_serves(rows, d, vocab, hidden_stride, weight_stride, wq)) {
         return hipErrorInvalidValue;

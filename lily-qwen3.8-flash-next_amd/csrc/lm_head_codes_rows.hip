@@ -62,12 +62,13 @@ inline uint32_t rows_lds_bytes(int mi, uint32_t groups) {
 // LDS a step ahead (none).
 template <int WBITS, int MI>
 __global__ void __launch_bounds__(256, MI == 4 ? 2 : 3)
-k_lm_head_codes_rows(const uint16_t* __restrict__ hidden, uint64_t hidden_stride, const uint32_t* __restrict__ codes,
+k_lm_head_codes_rows(const RowScales scales_arg, const uint16_t* __restrict__ hidden, uint64_t hidden_stride, const uint32_t* __restrict__ codes,
                      uint64_t weight_stride, uint32_t rows, uint32_t d, uint32_t vocab,
-                     const float* __restrict__ c2_of_row, float* __restrict__ logits, uint64_t logits_stride,
+                     float* __restrict__ logits, uint64_t logits_stride,
                      float* __restrict__ tile_max, float* __restrict__ tile_sum, uint32_t tiles_per_row,
                      uint32_t m_tiles, const uint16_t* __restrict__ scales, const uint16_t* __restrict__ biases,
                      uint32_t group_shift) {
+    const float* __restrict__ c2_of_row = scales_of(scales_arg);
     constexpr int BM = MI * 32;
     constexpr int STAGE_K = 1024 / WBITS, STEPS = STAGE_K / STEP_K;   // steps of 64 in a stage: 2 or 4
     constexpr int HIDDEN_AHEAD = MI == 4 ? 2 : 4;
@@ -306,7 +307,7 @@ k_lm_head_codes_rows(const uint16_t* __restrict__ hidden, uint64_t hidden_stride
 template <int WBITS, int MI>
 static hipError_t launch_codes_rows(hipStream_t stream, const void* hidden, uint64_t hidden_stride, const void* weight,
                                     uint64_t weight_stride, uint32_t rows, uint32_t d, uint32_t vocab,
-                                    const float* c2_of_row, void* logits, uint64_t logits_stride, float* tile_max,
+                                    const RowScales& c2_of_row, void* logits, uint64_t logits_stride, float* tile_max,
                                     float* tile_sum, const HeadWeights& wq) {
     const uint32_t tiles_per_row = (vocab + LILY_TILE_COLS - 1u) / LILY_TILE_COLS, m_tiles = (rows + MI * 32u - 1u) / (MI * 32u);
     const uint32_t lds = rows_lds_bytes(MI, d >> wq.group_shift);
@@ -316,8 +317,8 @@ static hipError_t launch_codes_rows(hipStream_t stream, const void* hidden, uint
         return e;
     }
     hipLaunchKernelGGL((k_lm_head_codes_rows<WBITS, MI>), dim3((tiles_per_row + 7u) / 8u * 8u * m_tiles), dim3(256), lds,
-                       stream, static_cast<const uint16_t*>(hidden), hidden_stride, static_cast<const uint32_t*>(weight),
-                       weight_stride, rows, d, vocab, c2_of_row, static_cast<float*>(logits), logits_stride, tile_max,
+                       stream, c2_of_row, static_cast<const uint16_t*>(hidden), hidden_stride, static_cast<const uint32_t*>(weight),
+                       weight_stride, rows, d, vocab, static_cast<float*>(logits), logits_stride, tile_max,
                        tile_sum, tiles_per_row, m_tiles, static_cast<const uint16_t*>(wq.scales),
                        static_cast<const uint16_t*>(wq.biases), wq.group_shift);
     return hipGetLastError();
@@ -339,7 +340,7 @@ uint32_t lm_head_codes_rows_resident(uint32_t d, const HeadWeights& wq) {
 
 hipError_t launch_lm_head_codes_rows(hipStream_t stream, const void* hidden, uint64_t hidden_stride, const void* weight,
                                      uint64_t weight_stride, uint32_t rows, uint32_t d, uint32_t vocab,
-                                     const float* c2_of_row, void* logits, uint64_t logits_stride, float* tile_max,
+                                     const RowScales& c2_of_row, void* logits, uint64_t logits_stride, float* tile_max,
                                      float* tile_sum, const HeadWeights& wq) {
     if (!lm_head_codes_rows_serves(d, wq)) {
         return hipErrorInvalidValue;

@@ -4,8 +4,10 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cstddef>
 #include <type_traits>
 
+#include "launch.h"
 #include "row_args.h"
 
 namespace lily {
@@ -16,6 +18,13 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 template <int CTRL>
 __device__ __forceinline__ float moved(float x) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+}
+
+// (For kernels whose first argument the scales are.  Those that travel with the launch are read from where the
+// arguments lie.)
+__device__ __forceinline__ const float* scales_of(const RowScales& c2) {
+    const char* args = (const char*)(const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr();
+    return c2.p != nullptr ? c2.p : reinterpret_cast<const float*>(args + offsetof(RowScales, few));
 }
 
 // acc: the sums of a wave's MI x NI products of 32 x 32; four waves, WAVES_M x (4 / WAVES_M), this

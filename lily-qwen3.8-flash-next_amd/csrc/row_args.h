@@ -62,7 +62,7 @@ struct alignas(16) RowArgs {
     uint32_t k_draw;           // rows of a chained launch: the draw's own candidate count (k is
                                // then what the select collects); 0 otherwise
     uint32_t sel_rows;         // rows behind `logits` that sel_row may pick from
-    uint32_t pad;
+    uint32_t pad;              // draws from summaries whose rows travel inline: the row of the summaries
     // A draw whose row and step a kernel before it chose (words of the speculative control
     // block, typically): the row is logits + min(*sel_row, sel_rows - 1) * sel_stride bytes and
     // the step is step + *sel_step.  Null pointers: the row and the step as given.

@@ -2,6 +2,7 @@
 // value and the sum of exponentials of every LILY_TILE_COLS columns): the row is not read,
 // only the summaries and the few tiles that can hold one of its k largest values.
 #include <algorithm>
+#include <type_traits>
 
 #include "row_kernel.h"
 
@@ -42,10 +43,11 @@ constexpr uint32_t REF_CAP = 2048;                       // pieces evaluated ele
 // written for rows under penalties or a mask: 1 = drawn here, 0 = left to the launch that follows.
 // EXTRA: rows with a bias list or a mask are among the launch's (the kernel without them keeps the
 // row's descriptor in fewer scalar registers, which the other spills).
+// tile_row null: the rows' own pad words say it.
 template <int DT, bool LSE, bool EXTRA>
-__global__ __launch_bounds__(NT, 4) void k_rows_tiles(LaunchCfg cfg, const float* tile_max,
-                                                      const float* tile_sum, uint32_t tiles,
-                                                      const uint32_t* tile_row, uint32_t* served) {
+__device__ __forceinline__ void tiles_row(const LILY_CONST RowArgs* table, const LaunchCfg& cfg, const float* tile_max,
+                                          const float* tile_sum, uint32_t tiles, const uint32_t* tile_row,
+                                          uint32_t* served) {
     __shared__ Shared sh;
     __shared__ uint16_t listed[TILES_MAX];   // tiles to read; bit 15: summed element by element
     __shared__ uint32_t refs[REF_CAP];       // pieces to evaluate: first id; bit 31: summed
@@ -55,7 +57,6 @@ __global__ __launch_bounds__(NT, 4) void k_rows_tiles(LaunchCfg cfg, const float
     __shared__ uint32_t bias_tiles[TILES_MAX / 32u];   // bit t: tile t holds a biased id
     constexpr uint32_t E = (uint32_t)Geo<DT>::E;          // values in a piece of 16 bytes
     constexpr uint32_t ELEM = DT == LILY_BF16 ? 2u : 4u;  // bytes a value
-    const LILY_CONST RowArgs* table = (const LILY_CONST RowArgs*)cfg.table;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
     if (tid == 0) {
         tail_arrays(sh);
@@ -86,7 +87,7 @@ __global__ __launch_bounds__(NT, 4) void k_rows_tiles(LaunchCfg cfg, const float
             bias_delta[tid] = gload(&a.bias[tid].delta);
         }
     }
-    const size_t srow = (size_t)gload(tile_row + blockIdx.y) * tiles;
+    const size_t srow = (size_t)(tile_row != nullptr ? gload(tile_row + blockIdx.y) : a.pad) * tiles;
     // the summaries: both arrays asked for at once (clamped, so that no load hangs on a test)
     float ms[TILES_PER_THREAD], ss[TILES_PER_THREAD];
     float best = NEG_INF;
@@ -482,9 +483,23 @@ __global__ __launch_bounds__(NT, 4) void k_rows_tiles(LaunchCfg cfg, const float
     phase(cfg, 7);
 }
 
-hipError_t launch_rows_tiles(hipStream_t stream, int dtype, bool lse, bool extra, uint32_t rows,
-                             const LaunchCfg& cfg_in, const float* tile_max, const float* tile_sum,
-                             uint32_t tiles, const uint32_t* tile_row, uint32_t* served) {
+template <int DT, bool LSE, bool EXTRA>
+__global__ __launch_bounds__(NT, 4) void k_rows_tiles(LaunchCfg cfg, const float* tile_max,
+                                                      const float* tile_sum, uint32_t tiles,
+                                                      const uint32_t* tile_row, uint32_t* served) {
+    tiles_row<DT, LSE, EXTRA>((const LILY_CONST RowArgs*)cfg.table, cfg, tile_max, tile_sum, tiles, tile_row, served);
+}
+
+template <int DT, bool LSE, bool EXTRA>
+__global__ __launch_bounds__(NT, 4) void k_rows_tiles_inline(InlineRows rows, LaunchCfg cfg, const float* tile_max,
+                                                             const float* tile_sum, uint32_t tiles) {
+    tiles_row<DT, LSE, EXTRA>((const LILY_CONST RowArgs*)__builtin_amdgcn_kernarg_segment_ptr(), cfg, tile_max, tile_sum, tiles,
+                              nullptr, nullptr);
+}
+
+static hipError_t launch_tiles(hipStream_t stream, int dtype, bool lse, bool extra, uint32_t rows, const LaunchCfg& cfg_in,
+                               const InlineRows* inline_rows, const float* tile_max, const float* tile_sum,
+                               uint32_t tiles, const uint32_t* tile_row, uint32_t* served) {
     if (tiles == 0 || tiles > TILES_MAX) {
         return hipErrorInvalidValue;
     }
@@ -495,29 +510,49 @@ hipError_t launch_rows_tiles(hipStream_t stream, int dtype, bool lse, bool extra
     const size_t dyn_bytes = std::max(tail_bytes, (size_t)TILE_CAND_CAP * 8);
     cfg.dyn_slots = (uint32_t)(dyn_bytes / 8);
     const dim3 grid(1, rows), block(NT);
-#define LILY_TILES(DT, LSE)                                                                       \
-    do {                                                                                          \
-        if (extra) {                                                                              \
-            hipLaunchKernelGGL((k_rows_tiles<DT, LSE, true>), grid, block, dyn_bytes, stream, cfg, tile_max,  \
-                               tile_sum, tiles, tile_row, served);                                \
-        } else {                                                                                  \
-            hipLaunchKernelGGL((k_rows_tiles<DT, LSE, false>), grid, block, dyn_bytes, stream, cfg, tile_max, \
-                               tile_sum, tiles, tile_row, served);                                \
-        }                                                                                         \
-    } while (0)
-    if (dtype == LILY_BF16) {
-        if (lse) {
-            LILY_TILES(LILY_BF16, true);
+    auto launch = [&](auto dt, auto with_lse, auto with_extra) {
+        constexpr int DT = decltype(dt)::value;
+        constexpr bool LSE = decltype(with_lse)::value, EXTRA = decltype(with_extra)::value;
+        if (inline_rows != nullptr) {
+            hipLaunchKernelGGL((k_rows_tiles_inline<DT, LSE, EXTRA>), grid, block, dyn_bytes, stream, *inline_rows, cfg,
+                               tile_max, tile_sum, tiles);
         } else {
-            LILY_TILES(LILY_BF16, false);
+            hipLaunchKernelGGL((k_rows_tiles<DT, LSE, EXTRA>), grid, block, dyn_bytes, stream, cfg, tile_max, tile_sum,
+                               tiles, tile_row, served);
         }
-    } else if (lse) {
-        LILY_TILES(LILY_F32, true);
+    };
+    auto by_extra = [&](auto dt, auto with_lse) {
+        if (extra) {
+            launch(dt, with_lse, std::true_type{});
+        } else {
+            launch(dt, with_lse, std::false_type{});
+        }
+    };
+    auto by_lse = [&](auto dt) {
+        if (lse) {
+            by_extra(dt, std::true_type{});
+        } else {
+            by_extra(dt, std::false_type{});
+        }
+    };
+    if (dtype == LILY_BF16) {
+        by_lse(std::integral_constant<int, LILY_BF16>{});
     } else {
-        LILY_TILES(LILY_F32, false);
+        by_lse(std::integral_constant<int, LILY_F32>{});
     }
-#undef LILY_TILES
     return hipGetLastError();
+}
+
+hipError_t launch_rows_tiles(hipStream_t stream, int dtype, bool lse, bool extra, uint32_t rows,
+                             const LaunchCfg& cfg, const float* tile_max, const float* tile_sum,
+                             uint32_t tiles, const uint32_t* tile_row, uint32_t* served) {
+    return launch_tiles(stream, dtype, lse, extra, rows, cfg, nullptr, tile_max, tile_sum, tiles, tile_row, served);
+}
+
+hipError_t launch_rows_tiles_inline(hipStream_t stream, int dtype, bool lse, bool extra, uint32_t rows, const LaunchCfg& cfg,
+                                    const InlineRows& inline_rows, const float* tile_max, const float* tile_sum,
+                                    uint32_t tiles) {
+    return launch_tiles(stream, dtype, lse, extra, rows, cfg, &inline_rows, tile_max, tile_sum, tiles, nullptr, nullptr);
 }
 
 }  // namespace lily

@@ -363,7 +363,8 @@ struct HeldShape {
 // Rows under penalties without log-probabilities stay below that (bf16, 151 936 ids, streamed -> held: 40 rows
 // in 19 slices 21.9 -> 21.9 us, 50 rows 22.3 -> 23.2, 60 rows in 10 slices of two blocks 23.8 -> 25.6).
 constexpr uint32_t HELD_MAX_GROUPS[3] = {0, 1024, 768};
-// Rows with masks too (2 % admitted, k = 50: 30 rows 21.8 -> 19.6, 64 rows in slices of two blocks 21.8 -> 27.3).
+// Rows with masks too, and in slices of one block only (2 % admitted: 30 rows, k = 50, 21.8 -> 19.6, 64 rows in
+// slices of two blocks 21.8 -> 27.3; 16 f32 rows of 248 320, k = 64, 23.6 -> 24.0 in two).
 constexpr uint32_t HELD_MAX_GROUPS_LISTED = 768, HELD_MAX_GROUPS_EXTRA = 600;
 HeldShape held_shape(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint32_t vocab, int dtype, bool pen, bool lse, bool extra) {
     HeldShape out;
@@ -380,7 +381,7 @@ HeldShape held_shape(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint32
             (uint64_t)rows * sl * kmax > s->ws_slots || (uint64_t)rows * sl > HELD_MAX_GROUPS[blocks]) {
             continue;
         }
-        if (extra && (uint64_t)rows * sl > HELD_MAX_GROUPS_EXTRA) {
+        if (extra && (blocks == 2 || (uint64_t)rows * sl > HELD_MAX_GROUPS_EXTRA)) {
             continue;
         }
         if (pen && !lse && ((uint64_t)rows * sl > HELD_MAX_GROUPS_LISTED || (blocks == 2 && dtype == LILY_BF16))) {
@@ -1999,6 +2000,7 @@ int check_head(const lily_lm_head* h, uint32_t rows, uint32_t vocab, const void*
 }
 
 struct HeadWeightsOf : HeadWeights {
+    HeadWeightsOf() = default;
     HeadWeightsOf(const lily_sampler* s, const lily_lm_head* h);
 };
 HeadWeightsOf::HeadWeightsOf(const lily_sampler* s, const lily_lm_head* h) {
@@ -2073,30 +2075,11 @@ int rows_with_tiles(lily_sampler* s, const lily_lm_head* h, const lily_rows* b, 
         }
     }
     ON_DEVICE(s->device);
-    uint32_t slot = 0;
-    if (int rc = stage_acquire(s, rows, &slot)) {
-        return rc;
-    }
     static thread_local std::vector<RowArgs> packed;
     packed.resize(rows);
     if (int rc = pack_batch(b, packed.data())) {
         return rc;
     }
-    // staged: the descriptors - rows the summaries serve for certain, then rows under penalties
-    // (served from the summaries unless the kernel declines them: the launch of the remaining
-    // rows covers them too and skips those already drawn), then the others -, each row's row of
-    // the summaries, every row's exponent scale (the producer's), a word per row that says
-    // whether the row has been drawn
-    char* stage = reinterpret_cast<char*>(s->stage[slot]);
-    RowArgs* table = reinterpret_cast<RowArgs*>(stage);
-    const size_t idx_off = (size_t)rows * sizeof(RowArgs), c2_off = idx_off + round16((size_t)rows * 4);
-    const size_t served_off = c2_off + round16((size_t)rows * 4);
-    uint32_t* tile_row = reinterpret_cast<uint32_t*>(stage + idx_off);
-    float* c2 = reinterpret_cast<float*>(stage + c2_off);
-    uint32_t* served_flags = reinterpret_cast<uint32_t*>(stage + served_off);
-    uint32_t certain = 0, maybe = 0;
-    bool lse = false, extra = false;
-    uint32_t at = 0;
     // Summaries this sampler's lily_lm_head_bf16 produced at another temperature than the row's
     // (or at none) would give the row a wrong log-probability with the right token: such a row
     // is drawn from its logits instead.  (Summaries of any other origin are taken on trust.)
@@ -2130,6 +2113,65 @@ int rows_with_tiles(lily_sampler* s, const lily_lm_head* h, const lily_rows* b, 
         }
     }
     held = held && behind != 0 && held_shape(s, behind, behind_k, b->vocab, (int)b->dtype, behind_pen, behind_lse, behind_extra).blocks != 0;
+    auto scale_of_row = [&](uint32_t r) { return std::isfinite(packed[r].c2) ? packed[r].c2 : 0.0f; };
+    // Few rows, none of which the summaries may decline: everything travels with the launches (carried to the
+    // device by a kernel of its own the descriptors cost 2.8 of the 223 us of four rows over bf16 weights).
+    const HeadWeightsOf few_weights = h != nullptr ? HeadWeightsOf(s, h) : HeadWeightsOf();
+    bool none_maybe = true;
+    for (uint32_t r = 0; r < rows; ++r) {
+        none_maybe = none_maybe && (group_of[r] != 1 || held);
+    }
+    if (rows <= (uint32_t)INLINE_ROWS && none_maybe && (few_weights.library_rows == 0u || rows < few_weights.library_rows)) {
+        InlineRows from_tiles, from_rows;
+        uint32_t n_tiles = 0, n_rows = 0;
+        bool lse = false, extra = false;
+        RowScales scales;
+        for (uint32_t r = 0; r < rows; ++r) {
+            scales.few[r] = scale_of_row(r);
+            if (group_of[r] == 0) {
+                lse = lse || packed[r].out_logprob != nullptr;
+                extra = extra || packed[r].n_bias != 0;
+                from_tiles.r[n_tiles] = packed[r];
+                from_tiles.r[n_tiles++].pad = r;
+            } else {
+                from_rows.r[n_rows++] = packed[r];
+            }
+        }
+        if (h != nullptr) {
+            s->head_sum = h->tile_sum_dev;
+            s->head_c2.assign(scales.few, scales.few + rows);
+            HIP_TRY(launch_lm_head_bf16(s->stream, h->hidden_dev, h->hidden_stride, h->weight_dev, h->weight_stride, rows,
+                                        h->d, b->vocab, scales, const_cast<void*>(b->logits_dev), b->row_stride,
+                                        h->tile_max_dev, h->tile_sum_dev, h->logits_f32 != 0u, few_weights));
+        }
+        if (n_tiles != 0) {
+            LaunchCfg cfg;
+            fill_cfg(s, &cfg, n_tiles, b->vocab, 1, 1, 0, nullptr);
+            attach_trace(s, &cfg, n_tiles);
+            HIP_TRY(launch_rows_tiles_inline(s->stream, (int)b->dtype, lse, extra, n_tiles, cfg, from_tiles, tile_max, tile_sum,
+                                             tiles));
+        }
+        return n_rows != 0 ? launch_inline(s, (int)b->dtype, b->vocab, from_rows, n_rows) : LILY_OK;
+    }
+    uint32_t slot = 0;
+    if (int rc = stage_acquire(s, rows, &slot)) {
+        return rc;
+    }
+    // staged: the descriptors - rows the summaries serve for certain, then rows under penalties
+    // (served from the summaries unless the kernel declines them: the launch of the remaining
+    // rows covers them too and skips those already drawn), then the others -, each row's row of
+    // the summaries, every row's exponent scale (the producer's), a word per row that says
+    // whether the row has been drawn
+    char* stage = reinterpret_cast<char*>(s->stage[slot]);
+    RowArgs* table = reinterpret_cast<RowArgs*>(stage);
+    const size_t idx_off = (size_t)rows * sizeof(RowArgs), c2_off = idx_off + round16((size_t)rows * 4);
+    const size_t served_off = c2_off + round16((size_t)rows * 4);
+    uint32_t* tile_row = reinterpret_cast<uint32_t*>(stage + idx_off);
+    float* c2 = reinterpret_cast<float*>(stage + c2_off);
+    uint32_t* served_flags = reinterpret_cast<uint32_t*>(stage + served_off);
+    uint32_t certain = 0, maybe = 0;
+    bool lse = false, extra = false;
+    uint32_t at = 0;
     for (int group = 0; group < 3; ++group) {
         for (uint32_t r = 0; r < rows; ++r) {
             const RowArgs& row = packed[r];
@@ -2150,7 +2192,7 @@ int rows_with_tiles(lily_sampler* s, const lily_lm_head* h, const lily_rows* b, 
         }
     }
     for (uint32_t r = 0; r < rows; ++r) {
-        c2[r] = std::isfinite(packed[r].c2) ? packed[r].c2 : 0.0f;
+        c2[r] = scale_of_row(r);
     }
     if (h != nullptr) {
         s->head_sum = h->tile_sum_dev;
@@ -2209,25 +2251,30 @@ int lily_lm_head_bf16(lily_sampler_t* s, const lily_lm_head* h, uint32_t rows, u
         return rc;
     }
     ON_DEVICE(s->device);
-    uint32_t slot = 0;
-    if (int rc = stage_acquire(s, rows, &slot)) {
-        return rc;
-    }
-    float* c2 = reinterpret_cast<float*>(s->stage[slot]);
-    s->head_sum = h->tile_sum_dev;
-    s->head_c2.resize(rows);
-    for (uint32_t r = 0; r < rows; ++r) {
-        c2[r] = temperatures != nullptr ? c2_of_temperature(temperatures[r]) : 0.0f;
-        s->head_c2[r] = c2[r];
-    }
-    if (int rc = stage_commit(s, slot, (size_t)rows * 4)) {
-        return rc;
-    }
     HeadWeightsOf hw(s, h);
     hw.trace = reinterpret_cast<unsigned long long*>(s->phase_trace);
     hw.trace_words = s->phase_words;
+    s->head_sum = h->tile_sum_dev;
+    s->head_c2.resize(rows);
+    for (uint32_t r = 0; r < rows; ++r) {
+        s->head_c2[r] = temperatures != nullptr ? c2_of_temperature(temperatures[r]) : 0.0f;
+    }
+    RowScales scales;
+    if (rows <= SCALES_INLINE && (hw.library_rows == 0u || rows < hw.library_rows)) {
+        std::copy(s->head_c2.begin(), s->head_c2.end(), scales.few);
+    } else {
+        uint32_t slot = 0;
+        if (int rc = stage_acquire(s, rows, &slot)) {
+            return rc;
+        }
+        std::copy(s->head_c2.begin(), s->head_c2.end(), reinterpret_cast<float*>(s->stage[slot]));
+        if (int rc = stage_commit(s, slot, (size_t)rows * 4)) {
+            return rc;
+        }
+        scales.p = reinterpret_cast<const float*>(s->table_dev);
+    }
     HIP_TRY(launch_lm_head_bf16(s->stream, h->hidden_dev, h->hidden_stride, h->weight_dev, h->weight_stride,
-                                rows, h->d, vocab, reinterpret_cast<const float*>(s->table_dev), logits_dev,
+                                rows, h->d, vocab, scales, logits_dev,
                                 row_stride, h->tile_max_dev, h->tile_sum_dev, h->logits_f32 != 0u, hw));
     return LILY_OK;
 }
