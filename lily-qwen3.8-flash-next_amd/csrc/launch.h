@@ -68,8 +68,6 @@ struct HeadWeights {
     const void* scales = nullptr;
     const void* biases = nullptr;
     uint32_t group_shift = 6;   // log2 of the group size
-    unsigned long long* trace = nullptr;   // diagnostic stamps, [workgroups][8] (builds with -DLILY_HEAD_TRACE)
-    unsigned long long trace_words = 0;
     // batches of at least this many rows go through the vendor's GEMM library where it is present
     // and takes the shape, followed by the pass that forms the summaries (0: never)
     uint32_t library_rows = 0;

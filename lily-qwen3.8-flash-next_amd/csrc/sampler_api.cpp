@@ -2252,8 +2252,6 @@ int lily_lm_head_bf16(lily_sampler_t* s, const lily_lm_head* h, uint32_t rows, u
     }
     ON_DEVICE(s->device);
     HeadWeightsOf hw(s, h);
-    hw.trace = reinterpret_cast<unsigned long long*>(s->phase_trace);
-    hw.trace_words = s->phase_words;
     s->head_sum = h->tile_sum_dev;
     s->head_c2.resize(rows);
     for (uint32_t r = 0; r < rows; ++r) {

@@ -850,6 +850,17 @@ def test_few_rows_of_codes_over_their_scales(sampler, rows, d, vocab, bits, grou
 
 
 @pytest.mark.parametrize("rows,d,vocab,bits,group", [
+    (8, 512, 65_541, 4, 64), (9, 512, 65_670, 4, 64), (2, 256, 131_329, 4, 64), (5, 640, 66_000, 8, 64),
+    (8, 4352, 258, 4, 64), (3, 5120, 130, 8, 64)])
+def test_workgroups_that_take_several_tiles_of_codes(sampler, rows, d, vocab, bits, group):
+    """Up to 16 rows over codes where a launch's 512 workgroups take more than one tile: two (the last
+    of them the vocabulary's ragged one) and three, one trip of stages a tile and two that are not whole, either
+    form of the hidden values (8 and 9 rows), groups a row below eight, ten (the last eight brought from an even
+    place that is no multiple of eight), and between 64 and 80 (the load beside the first 64)."""
+    test_few_rows_of_codes_over_their_scales(sampler, rows, d, vocab, bits, group)
+
+
+@pytest.mark.parametrize("rows,d,vocab,bits,group", [
     (17, 512, 700, 4, 64), (32, 128, 64, 8, 64), (33, 1024, 129, 8, 128), (64, 256, 1000, 4, 64),
     (65, 512, 333, 8, 64), (128, 768, 257, 4, 128), (129, 1536, 1160, 4, 64),
     (16, 768, 300, 4, 256), (20, 8192, 129, 8, 64), (64, 6144, 140, 4, 64), (65, 2560, 200, 8, 64),
