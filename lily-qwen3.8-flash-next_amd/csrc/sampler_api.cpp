@@ -363,9 +363,9 @@ struct HeldShape {
 // Rows under penalties without log-probabilities stay below that (bf16, 151 936 ids, streamed -> held: 40 rows
 // in 19 slices 21.9 -> 21.9 us, 50 rows 22.3 -> 23.2, 60 rows in 10 slices of two blocks 23.8 -> 25.6).
 constexpr uint32_t HELD_MAX_GROUPS[3] = {0, 1024, 768};
-// Rows with masks too, and in slices of one block only (2 % admitted: 30 rows, k = 50, 21.8 -> 19.6, 64 rows in
-// slices of two blocks 21.8 -> 27.3; 16 f32 rows of 248 320, k = 64, 23.6 -> 24.0 in two).
-constexpr uint32_t HELD_MAX_GROUPS_LISTED = 768, HELD_MAX_GROUPS_EXTRA = 600;
+// Rows with masks too, and in slices of two blocks up to a workgroup a compute unit (2 % admitted: 30 rows, k = 50,
+// 21.8 -> 19.6, 64 rows in slices of two blocks 21.8 -> 27.3; 16 f32 rows of 248 320, k = 64, 23.6 -> 24.0 in two).
+constexpr uint32_t HELD_MAX_GROUPS_LISTED = 768, HELD_MAX_GROUPS_EXTRA[3] = {0, 600, 256};
 HeldShape held_shape(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint32_t vocab, int dtype, bool pen, bool lse, bool extra) {
     HeldShape out;
     if (s->force_path != 0 || s->no_held || s->only_blocks || kmax > STREAM_K_MAX || rows > s->ws_rows) {
@@ -381,7 +381,7 @@ HeldShape held_shape(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint32
             (uint64_t)rows * sl * kmax > s->ws_slots || (uint64_t)rows * sl > HELD_MAX_GROUPS[blocks]) {
             continue;
         }
-        if (extra && (blocks == 2 || (uint64_t)rows * sl > HELD_MAX_GROUPS_EXTRA)) {
+        if (extra && (uint64_t)rows * sl > HELD_MAX_GROUPS_EXTRA[blocks]) {
             continue;
         }
         if (pen && !lse && ((uint64_t)rows * sl > HELD_MAX_GROUPS_LISTED || (blocks == 2 && dtype == LILY_BF16))) {
