@@ -2,15 +2,19 @@
 // which is what a request without top_k gets: src/kernels/sample.rs:17, :326-331), spread over
 // as many workgroups as rows of few candidates are.
 //
-// Two launches.  In the first every workgroup reads its slice of the row once and leaves its
-// lanes' largest values (penalised ids at their penalised worth).  In the second every
-// workgroup first takes the k-th largest of all the row's lane maxima: k lanes reach it, so k
-// values do - a lower bound of the row's k-th largest value that about k * (1 + a few per cent)
-// values reach -, then reads its slice again (from the L2 now) and appends the values that
-// reach the bound to the row's list; the one that finishes last reads the list - a thousand and
-// some, whatever the number of slices -, selects, and runs the common tail.  (The select of the
-// other kernels keeps k candidates per slice and can therefore spread a row with k = 1024 over
-// 4 workgroups only.)
+// One launch where a slice fits its workgroup's registers and the launch the chip (k_wide_held), two otherwise
+// (k_wide_bound, k_wide_draw).  Every slice's lanes take their largest values (penalised ids at their penalised
+// worth), its waves name one each that r lanes reach, and from what all the row's waves named comes a lower bound of the
+// row's k-th largest value that k lanes, so k values reach, and some 1.5 k in all (bound_of_keys).  The values
+// that reach it are appended to the row's list - after a second look at the slice, from the L2, where there are two
+// launches -; the workgroup that finishes last sorts the list, whatever the number of slices, and runs the common
+// tail.  (The select of the other kernels keeps k candidates per slice and can therefore spread a row with
+// k = 1024 over 4 workgroups only.)
+//
+// Bound: a chain of latencies.  us a launch, no top_k, two launches -> one: 4 f32 rows of 151 936 with log-probabilities
+// 27.3 -> 24.4, under penalties 31.1 -> 25.2, 13 rows under penalties 39.6 -> 31.9, 26 bf16 rows under penalties 52.7 ->
+// 38.8, without 37.6 -> 35.4; 40 bf16 rows in 760 workgroups 46.6 -> 41.9.  4 bf16 rows of 32 000 in 16 slices, where a block
+// a slice were 4, 41.9 -> 25.9.
 #include <algorithm>
 
 #ifdef LILY_WIDE_TRACE
@@ -33,8 +37,11 @@ namespace lily {
 // What the two launches share beyond LaunchCfg.
 struct WideArgs {
     Handed<float> lane_max;   // [rows][slices][lanes]
-    Handed<float> slice_bound;   // [rows][slices] a value that k / slices of the slice's lanes reach
+    Handed<uint64_t> slice_keys;   // [rows][slices] four waves' keys (slice_keys_of())
     uint32_t lanes;       // values a slice leaves: NT, or NT / 2 (the larger of each pair of lanes)
+    // k_wide_held: [rows][MAX_SLICES] slices' keys, then as many words for slices that have left their lanes' maxima
+    // (0 between launches); null: two launches
+    uint64_t* bounds;
     uint32_t* count;      // [rows] candidates the row's slices have left so far (0 between launches)
 };
 
@@ -112,6 +119,44 @@ __device__ __forceinline__ void wide_edges(const RowArgs& a, const Geo<DT>& g, F
 // The row's ticket: true in every thread of the workgroup that arrives last (last_to_arrive()).
 __device__ __forceinline__ bool wide_last(const LaunchCfg& cfg, uint32_t row, uint32_t S, Shared& sh) {
     return last_to_arrive(&cfg.ws_ticket[row], S, sh.last, cfg.relaxed_handover != 0u);
+}
+
+// The row's bound.  Each of the row's 4 x S waves names the r-th largest of its lanes' maxima (the leading 16 bits of
+// the order key, by a ballot search); the largest value that ceil(k / r) of the waves name or exceed is then reached
+// by k lanes, so by k values.  r lies a little above the waves' share ceil(k / 4S): where the least of all the waves'
+// share-th values was taken, one poor wave of 244 set the bound (8 f32 rows of 248 320 with k = 1 024: a list
+// beyond MERGE_CAP in every second launch, 1 500 us by the exhaustive select), and a slice of ids that nothing favours did.
+__device__ __forceinline__ uint32_t wide_rank(uint32_t k, uint32_t S) {
+    const uint32_t share = (k + 4u * S - 1u) / (4u * S);
+    return min(share + (share + 7u) / 8u + 1u, 64u);
+}
+constexpr uint32_t WIDE_LEAST_KEY = 0x0080u;   // of F32_LOWEST: what a wave with fewer finite lane maxima names
+// A slice's four keys of 16 bits as one word, never 0, in thread 0 (every thread calls).
+__device__ __forceinline__ uint64_t slice_keys_of(float lane_max, uint32_t k, uint32_t S, Shared& sh) {
+    const uint32_t tid = threadIdx.x;
+    const uint32_t P = wave_kth_key16(lane_max > NEG_INF ? (lilym_order_key(lane_max) >> 16) : 0u, wide_rank(k, S));
+    if ((tid & 63u) == 0u) {
+        sh.hist[tid >> 6] = max(P, WIDE_LEAST_KEY);
+    }
+    __syncthreads();
+    static_assert(NWAVE == 4, "a word of four keys");
+    return tid != 0u ? 0ull : ((uint64_t)(sh.hist[3] << 16 | sh.hist[2]) << 32) | (sh.hist[1] << 16 | sh.hist[0]);
+}
+// Of the keys that lane l of a wave has of slice l (0 past the last); F32_LOWEST: too many waves had none to name.
+__device__ __forceinline__ float bound_of_keys(uint64_t keys, uint32_t k, uint32_t S) {
+    const uint32_t r = wide_rank(k, S), need = (k + r - 1u) / r;
+    uint32_t T = 0;
+#pragma unroll
+    for (int bit = 15; bit >= 0; --bit) {
+        const uint32_t t = T | (1u << bit);
+        uint32_t n = 0;
+#pragma unroll
+        for (int i = 0; i < NWAVE; ++i) {
+            n += (uint32_t)__popcll(__ballot(((uint32_t)(keys >> (16 * i)) & 0xffffu) >= t));
+        }
+        T = n >= need ? t : T;
+    }
+    return T > WIDE_LEAST_KEY ? lilym_key_value(T << 16) : F32_LOWEST;
 }
 
 // ---- first launch: lane maxima, the slice's sum of exponentials
@@ -194,29 +239,10 @@ __global__ __launch_bounds__(NT, 4) void k_wide_bound(InlineRows rows_arg, Launc
             handed_store(w.lane_max, slot * (NT / 2) + tid / 2u, lane_max);
         }
     }
-    // ... and one value per slice that at least ceil(k / slices) of its lanes reach: in each wave
-    // the ceil(k / (4 * slices))-th largest of the 64 lane maxima (a 16-step ballot search on the
-    // leading 16 bits of the order key, as the streaming select takes its bound), the least of the
-    // four.  The least of a row's slices' values is then reached by k lanes of the row, so by k
-    // values: the second launch takes that as the row's bound without looking at the lanes'
-    // maxima.  F32_LOWEST from a wave with fewer finite lane maxima than that: the second launch
-    // then takes the bound from all the lanes' maxima.
-    {
-        const float whole = pair_max;   // (every lane's own maximum, whatever was stored above)
-        const uint32_t per_wave = (a.k + 4u * S - 1u) / (4u * S);
-        const uint32_t key16 = whole > NEG_INF ? (lilym_order_key(whole) >> 16) : 0u;
-        const uint32_t P = per_wave <= 64u ? wave_kth_key16(key16, per_wave) : 0u;
-        if ((tid & 63u) == 0u) {
-            sh.bound[0][tid >> 6] = P != 0u ? lilym_key_value(P << 16) : F32_LOWEST;
-        }
-        __syncthreads();
-        if (tid == 0) {
-            float least = sh.bound[0][0];
-            for (int i = 1; i < NWAVE; ++i) {
-                least = fminf(least, sh.bound[0][i]);
-            }
-            handed_store(w.slice_bound, slot, least);
-        }
+    // (every lane's own maximum, whatever was stored above)
+    const uint64_t keys = slice_keys_of(pair_max, a.k, S, sh);
+    if (tid == 0) {
+        handed_store(w.slice_keys, slot, keys);
     }
     if (want_lse) {
         lse_reduce(sh, lse);
@@ -292,77 +318,19 @@ __device__ __forceinline__ float wide_bound_of(const WideArgs& w, uint32_t row, 
     return enough ? lilym_key_value(prefix) : F32_LOWEST;
 }
 
-// ---- second launch: the values that reach the bound, then merge, select and tail
-
-template <int DT, bool LSE, bool INLINE>
-__global__ __launch_bounds__(NT, 4) void k_wide_draw(InlineRows rows_arg, LaunchCfg cfg, WideArgs w) {
-    __shared__ Shared sh;
-    __shared__ uint32_t n_mine;
-    constexpr int E = Geo<DT>::E;
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, s = blockIdx.x, row = blockIdx.y, S = cfg.slices;
-    if (cfg.served != nullptr && *(const LILY_CONST uint32_t*)(cfg.served + row) != 0u) {
-        return;
-    }
-    WIDE_MARK(5);
-    if (tid == 0) {
-        tail_arrays(sh);
-        n_mine = 0;
-    }
-    RowArgs a;
-    load_row_args(a, wide_table<INLINE>(cfg) + row);
-    apply_selection(a);
-    const uint32_t vocab = cfg.vocab;
-    const uint32_t step = a.step + cfg.step_delta;
-    const bool want_lse = LSE && a.out_logprob != nullptr;
-    const bool pen = (a.flags & F_PEN) != 0;   // (of the kind that only lowers: the host sees to it)
-    // The bound (of the values' worth under the penalties): the least of the slices' values, which
-    // k lanes of the row reach; where a wave of some slice had too few finite lane maxima to name
-    // one, the k-th largest of all the lanes' maxima.  Every wave reads the slices' values itself.
-    float bound;
-    {
-        const float mine = lane < S ? handed_load(w.slice_bound, (size_t)row * S + lane) : __builtin_huge_valf();
-        bound = -wave_max_dpp(-mine);
-    }
-    if (!(bound > F32_LOWEST)) {   // (the same in every wave)
-        bound = wide_bound_of(w, row, S, a.k, sh);
-    }
-    Geo<DT> g;
-    g.init(a.logits, vocab, s, S);
-    uint64_t* cand = dyn_lds;
-    const uint32_t cap = MERGE_CAP;   // what the slice's own list holds
-    __syncthreads();
-    auto offer = [&](float x, uint32_t id) {
-        if (!(x >= bound)) {
-            return;
-        }
-        if (pen) {
-            x = wide_worth(a, x, id);   // (never more than the raw value: the host sees to it)
-            if (!(x >= bound)) {
-                return;
-            }
-        }
-        const uint32_t at = atomicAdd(&n_mine, 1u);
-        if (at < cap) {
-            cand[at] = composite_of(x / a.temperature, id);
-        }
-    };
-    wide_scan<DT>(g, [&](const u32x4& q, uint32_t c) {
-        if (chunk_max<DT>(q) >= bound) {
-            float v[E];
-            unpack<DT>(q, v);
-#pragma unroll
-            for (int j = 0; j < E; ++j) {
-                offer(v[j], g.id_of(c, j));
-            }
-        }
-    });
-    wide_edges<DT>(a, g, [&](float x, uint32_t id) { offer(x, id); });
+// From a slice's candidates (n_mine of them in cand) to the row's draw, in the workgroup that arrives last.
+// gave_up: the slice has none because it did not learn the row's bound; the row is then taken
+// by the select that is right for any input.
+template <int DT, bool LSE>
+__device__ __forceinline__ void wide_finish(RowArgs& a, const LaunchCfg& cfg, const WideArgs& w, Shared& sh, uint32_t& n_mine,
+                                            uint64_t* cand, uint32_t row, uint32_t S, uint32_t step, bool want_lse, bool gave_up) {
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
     __syncthreads();
     WIDE_MARK(6);
     // The slice's candidates go behind those the row's other slices have left (any order: the
     // select does not care).  A row whose list would pass MERGE_CAP is counted on and not
     // written: the last workgroup sees the count and takes the exhaustive select.
-    const uint32_t mine = n_mine;
+    const uint32_t mine = gave_up ? MERGE_CAP + 1u : n_mine;
     if (tid == 0) {
         n_mine = __hip_atomic_fetch_add(&w.count[row], mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -375,6 +343,11 @@ __global__ __launch_bounds__(NT, 4) void k_wide_draw(InlineRows rows_arg, Launch
     }
     if (!wide_last(cfg, row, S, sh)) {
         return;
+    }
+    if (w.bounds != nullptr && tid < S) {
+        // (every slice has read them)
+        store_through(w.bounds + (size_t)row * MAX_SLICES + tid, (uint64_t)0);
+        store_through(w.bounds + ((size_t)gridDim.y + row) * MAX_SLICES + tid, (uint64_t)0);
     }
     WIDE_MARK(7);
     // The list's first entries are asked for together with its length: what lies behind its end is
@@ -396,7 +369,7 @@ __global__ __launch_bounds__(NT, 4) void k_wide_draw(InlineRows rows_arg, Launch
         // more than the buffers hold (values that tie by the thousand, a row in ascending
         // order): the select that is right for any input, over the whole row
         __syncthreads();
-        select_exhaustive<DT>(a, 0, vocab, a.k, want_lse, cand, min(cfg.dyn_slots, MERGE_CAP), sh);
+        select_exhaustive<DT>(a, 0, cfg.vocab, a.k, want_lse, cand, min(cfg.dyn_slots, MERGE_CAP), sh);
         n = min(sh.n_cand, min(cfg.dyn_slots, MERGE_CAP));
         if (cfg.path_stats != nullptr && tid == 0) {
             atomicAdd(&cfg.path_stats[2], 1u);
@@ -441,7 +414,298 @@ __global__ __launch_bounds__(NT, 4) void k_wide_draw(InlineRows rows_arg, Launch
             atomicAdd(&cfg.path_stats[1], 1u);
         }
     }
-    tail<DT, true>(a, vocab, step, n, sorted, cand, sh, cfg);
+    tail<DT, true>(a, cfg.vocab, step, n, sorted, cand, sh, cfg);
+}
+
+// ---- second launch: the values that reach the bound, then merge, select and tail
+
+template <int DT, bool LSE, bool INLINE>
+__global__ __launch_bounds__(NT, 4) void k_wide_draw(InlineRows rows_arg, LaunchCfg cfg, WideArgs w) {
+    __shared__ Shared sh;
+    __shared__ uint32_t n_mine;
+    constexpr int E = Geo<DT>::E;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, s = blockIdx.x, row = blockIdx.y, S = cfg.slices;
+    if (cfg.served != nullptr && *(const LILY_CONST uint32_t*)(cfg.served + row) != 0u) {
+        return;
+    }
+    WIDE_MARK(5);
+    if (tid == 0) {
+        tail_arrays(sh);
+        n_mine = 0;
+    }
+    RowArgs a;
+    load_row_args(a, wide_table<INLINE>(cfg) + row);
+    apply_selection(a);
+    const uint32_t vocab = cfg.vocab;
+    const uint32_t step = a.step + cfg.step_delta;
+    const bool want_lse = LSE && a.out_logprob != nullptr;
+    const bool pen = (a.flags & F_PEN) != 0;   // (of the kind that only lowers: the host sees to it)
+    // The bound (of the values' worth under the penalties), by every wave for itself; where too many waves had too few
+    // finite lane maxima to name one, the k-th largest of all the lanes' maxima.
+    float bound = bound_of_keys(lane < S ? handed_load(w.slice_keys, (size_t)row * S + lane) : 0ull, a.k, S);
+    if (!(bound > F32_LOWEST)) {   // (the same in every wave)
+        bound = wide_bound_of(w, row, S, a.k, sh);
+    }
+    Geo<DT> g;
+    g.init(a.logits, vocab, s, S);
+    uint64_t* cand = dyn_lds;
+    const uint32_t cap = MERGE_CAP;   // what the slice's own list holds
+    __syncthreads();
+    auto offer = [&](float x, uint32_t id) {
+        if (!(x >= bound)) {
+            return;
+        }
+        if (pen) {
+            x = wide_worth(a, x, id);   // (never more than the raw value: the host sees to it)
+            if (!(x >= bound)) {
+                return;
+            }
+        }
+        const uint32_t at = atomicAdd(&n_mine, 1u);
+        if (at < cap) {
+            cand[at] = composite_of(x / a.temperature, id);
+        }
+    };
+    wide_scan<DT>(g, [&](const u32x4& q, uint32_t c) {
+        if (chunk_max<DT>(q) >= bound) {
+            float v[E];
+            unpack<DT>(q, v);
+#pragma unroll
+            for (int j = 0; j < E; ++j) {
+                offer(v[j], g.id_of(c, j));
+            }
+        }
+    });
+    wide_edges<DT>(a, g, [&](float x, uint32_t id) { offer(x, id); });
+    wide_finish<DT, LSE>(a, cfg, w, sh, n_mine, cand, row, S, step, want_lse, false);
+}
+
+// ---- both in one launch, where a slice is held in registers and all of the launch's workgroups are on the chip
+
+// What the two launches do below, without reading the slice again and without a second launch: each slice leaves its
+// bound where the row's other slices look for it, and forms its sum of exponentials meanwhile.  A slice that
+// does not find them all within WIDE_TRIES looks (another stream's work holds the chip) gives up, and the row is taken by the
+// exhaustive select: every wait ends.
+constexpr uint32_t WIDE_TRIES = 1u << 13, WIDE_HELD_GROUPS = 1024;
+
+template <int DT, bool LSE, bool INLINE>
+__global__ __launch_bounds__(NT, 4) void k_wide_held(InlineRows rows_arg, LaunchCfg cfg, WideArgs w) {
+    __shared__ Shared sh;
+    __shared__ uint32_t n_mine, lost;
+    constexpr int E = Geo<DT>::E, C = (int)STREAM_UNROLL, V = C * E;
+    constexpr uint32_t EMASK = (1u << E) - 1u;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, s = blockIdx.x, row = blockIdx.y, S = cfg.slices;
+    if (cfg.served != nullptr && *(const LILY_CONST uint32_t*)(cfg.served + row) != 0u) {
+        return;
+    }
+    WIDE_MARK(0);
+    if (tid == 0) {
+        tail_arrays(sh);
+        n_mine = 0;
+        lost = 0;
+    }
+    RowArgs a;
+    load_row_args(a, wide_table<INLINE>(cfg) + row);
+    apply_selection(a);
+    const uint32_t step = a.step + cfg.step_delta;
+    const bool want_lse = LSE && a.out_logprob != nullptr;
+    const bool pen = (a.flags & F_PEN) != 0;
+    Geo<DT> g;
+    g.init(a.logits, cfg.vocab, s, S);
+    const uint32_t c_last = max(g.ce, 1u) - 1u;
+    auto chunk_of = [&](int u) -> uint32_t { return g.cb + (uint32_t)u * NT + tid; };
+    auto inside = [&](int u) -> bool { return chunk_of(u) >= g.main_lo && chunk_of(u) < g.main_hi; };
+    u32x4 raw[C];
+#pragma unroll
+    for (int u = 0; u < C; ++u) {
+        raw[u] = gload(reinterpret_cast<const u32x4*>(g.base + (size_t)min(chunk_of(u), c_last) * 16));
+    }
+    // The chunks' bits of the bitmap of listed ids: two bytes hold a chunk's, wherever the row starts (a byte past the
+    // bitmap is the scratch's own).
+    struct Bits16 {
+        uint16_t v;
+    } __attribute__((packed));
+    uint32_t todo = 0;
+    static_assert(V <= 32, "a bit per value");
+    if (pen) {
+        uint32_t listed[C];
+#pragma unroll
+        for (int u = 0; u < C; ++u) {
+            const uint32_t at = min(chunk_of(u), c_last) * (uint32_t)E, id = at < g.pad ? 0u : at - g.pad;
+            listed[u] = ((const LILY_GLOBAL Bits16*)(reinterpret_cast<const char*>(a.touched) + (id >> 3)))->v >> (id & 7u);
+        }
+#pragma unroll
+        for (int u = 0; u < C; ++u) {
+            todo |= (inside(u) ? listed[u] & EMASK : 0u) << (u * E);
+        }
+    }
+    float v[V];
+#pragma unroll
+    for (int u = 0; u < C; ++u) {
+        float x[E];
+        unpack<DT>(raw[u], x);
+#pragma unroll
+        for (int j = 0; j < E; ++j) {
+            v[u * E + j] = inside(u) && x[j] > NEG_INF ? x[j] : NEG_INF;   // (a NaN is worth -inf)
+        }
+    }
+    // The listed ids' true values, one of every chunk at a time with their loads in flight together.
+    while (__ballot(todo != 0u) != 0ull) {
+        uint32_t at[C], count[C];
+        float x[C];
+#pragma unroll
+        for (int u = 0; u < C; ++u) {
+            const uint32_t m = (todo >> (u * E)) & EMASK;
+            at[u] = m != 0u ? (uint32_t)__builtin_ctz(m) : 0xffu;
+            todo &= ~((m & (0u - m)) << (u * E));
+            const uint32_t id = m != 0u ? g.id_of(chunk_of(u), (int)at[u]) : 0u;
+            x[u] = load_logit<DT>(a.logits, id);
+            count[u] = gload(a.counts + id);
+        }
+#pragma unroll
+        for (int u = 0; u < C; ++u) {
+            float t = x[u];
+            if (count[u] > 0u) {
+                t = t > 0.0f ? t / a.repetition : t * a.repetition;
+                t -= a.presence + a.frequency * (float)count[u];
+            }
+            t = t > NEG_INF ? t : NEG_INF;
+#pragma unroll
+            for (int j = 0; j < E; ++j) {
+                v[u * E + j] = at[u] == (uint32_t)j ? t : v[u * E + j];
+            }
+        }
+    }
+    float cm[C], lane_max = NEG_INF;
+#pragma unroll
+    for (int u = 0; u < C; ++u) {
+        cm[u] = v[u * E];
+#pragma unroll
+        for (int j = 1; j < E; ++j) {
+            cm[u] = fmaxf(cm[u], v[u * E + j]);
+        }
+        lane_max = fmaxf(lane_max, cm[u]);
+    }
+    auto true_edge = [&](float x, uint32_t id) -> float { return pen ? wide_worth(a, x, id) : x; };
+    wide_edges<DT>(a, g, [&](float x, uint32_t id) { lane_max = fmaxf(lane_max, true_edge(x, id)); });
+    WIDE_MARK(1);
+    // ---- the slice's keys: 0 stands for those that are not there yet
+    uint64_t* bounds = w.bounds + (size_t)row * MAX_SLICES;
+    const uint64_t own_keys = slice_keys_of(lane_max, a.k, S, sh);
+    if (tid == 0) {
+        store_through(bounds + s, own_keys);
+    }
+    if (want_lse) {
+        LseAcc lse;
+        lse.init();
+#pragma unroll
+        for (int u = 0; u < C; ++u) {
+            if (cm[u] > NEG_INF) {
+                const float safe = lse.rebase(cm[u], a.c2);
+#pragma unroll
+                for (int j = 0; j < E; ++j) {
+                    if (v[u * E + j] > NEG_INF) {
+                        lse.term(v[u * E + j], a.c2, safe);
+                    }
+                }
+            }
+        }
+        wide_edges<DT>(a, g, [&](float x, uint32_t id) {
+            x = true_edge(x, id);
+            if (x > NEG_INF) {
+                lse.add_one(x, a.c2);
+            }
+        });
+        lse_reduce(sh, lse);
+        if (tid == 0) {
+            const size_t slot = (size_t)row * S + s;
+            handed_store(cfg.ws_lse, 2 * slot, sh.lse_mc);
+            handed_store(cfg.ws_lse, 2 * slot + 1, sh.lse_s);
+        }
+    }
+    WIDE_MARK(2);
+    // ---- the row's bound, once all its slices' words are there (a word is the message: nothing else is read for it)
+    uint64_t keys = 0;
+    auto wait_for = [&](const uint64_t* words) {
+        for (uint32_t tries = 0;; ++tries) {
+            keys = lane < S ? load_through(words + lane) : ~0ull;
+            if (__ballot(keys == 0ull) == 0ull) {
+                break;
+            }
+            if (tries == WIDE_TRIES) {
+                if (lane == 0u) {
+                    lost = 1u;
+                }
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+        __syncthreads();
+    };
+    wait_for(bounds);
+    float bound = bound_of_keys(lane < S ? keys : 0ull, a.k, S);
+    if (lost == 0u && !(bound > F32_LOWEST)) {
+        // (the same in all the row's workgroups) Most of the row is -inf: too many waves had no value to name.  The lanes'
+        // maxima change hands, and the bound is the k-th largest of those.
+        handed_store(w.lane_max, ((size_t)row * S + s) * NT + tid, lane_max);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        __syncthreads();
+        uint64_t* handed = bounds + (size_t)gridDim.y * MAX_SLICES;
+        if (tid == 0) {
+            __hip_atomic_store(handed + s, (uint64_t)1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        wait_for(handed);
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        uint32_t T = 0;
+        for (uint32_t t = 0x8000u; t != 0u && lost == 0u; t >>= 1) {
+            if (tid == 0) {
+                sh.hist[0] = 0;
+            }
+            __syncthreads();
+            uint32_t n = 0;
+            for (uint32_t j0 = 0; j0 < S; j0 += 8u) {
+                float x[8];
+#pragma unroll
+                for (uint32_t u = 0; u < 8u; ++u) {
+                    x[u] = handed_load(w.lane_max, ((size_t)row * S + min(j0 + u, S - 1u)) * NT + tid);
+                }
+#pragma unroll
+                for (uint32_t u = 0; u < 8u; ++u) {
+                    const bool reaches = j0 + u < S && x[u] > NEG_INF && (lilym_order_key(x[u]) >> 16) >= (T | t);
+                    n += (uint32_t)__popcll(__ballot(reaches));
+                }
+            }
+            if (lane == 0u) {
+                atomicAdd(&sh.hist[0], n);
+            }
+            __syncthreads();
+            T |= sh.hist[0] >= a.k ? t : 0u;
+            __syncthreads();
+        }
+        bound = T > WIDE_LEAST_KEY ? lilym_key_value(T << 16) : F32_LOWEST;
+    }
+    WIDE_MARK(5);
+    uint64_t* cand = dyn_lds;
+    auto offer = [&](float x, uint32_t id) {
+        if (x >= bound && x > NEG_INF) {
+            const uint32_t at = atomicAdd(&n_mine, 1u);
+            if (at < MERGE_CAP) {
+                cand[at] = composite_of(x / a.temperature, id);
+            }
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < C; ++u) {
+        if (cm[u] >= bound) {
+#pragma unroll
+            for (int j = 0; j < E; ++j) {
+                offer(v[u * E + j], g.id_of(chunk_of(u), j));
+            }
+        }
+    }
+    wide_edges<DT>(a, g, [&](float x, uint32_t id) { offer(true_edge(x, id), id); });
+    __syncthreads();
+    wide_finish<DT, LSE>(a, cfg, w, sh, n_mine, cand, row, S, step, want_lse, lost != 0u);
 }
 
 template <int DT, bool LSE, bool INLINE>
@@ -451,6 +715,10 @@ static hipError_t launch_wide_variant(hipStream_t stream, uint32_t rows, const L
     static const InlineRows none = {};
     const InlineRows& r = inline_rows != nullptr ? *inline_rows : none;
     const size_t dyn2 = (size_t)cfg.dyn_slots * 8;
+    if (w.bounds != nullptr) {
+        hipLaunchKernelGGL((k_wide_held<DT, LSE, INLINE>), grid, block, dyn2, stream, r, cfg, w);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL((k_wide_bound<DT, LSE, INLINE>), grid, block, 0, stream, r, cfg, w);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
@@ -461,16 +729,21 @@ static hipError_t launch_wide_variant(hipStream_t stream, uint32_t rows, const L
 }
 
 hipError_t launch_rows_wide(hipStream_t stream, int dtype, bool lse, uint32_t rows, const LaunchCfg& cfg_in,
-                            const InlineRows* inline_rows, float* lane_max, uint32_t* count) {
+                            const InlineRows* inline_rows, float* lane_max, uint32_t* count, uint64_t* bounds) {
     LaunchCfg cfg = cfg_in;
     // the merging workgroup's candidates, then the tail's arrays behind the first K_CAP of them
     cfg.dyn_slots = MERGE_CAP;
     cfg.cand_cap = MERGE_CAP;
     WideArgs w;
     w.lane_max = Handed<float>{lane_max};
-    w.slice_bound = Handed<float>{lane_max + (size_t)rows * cfg.slices * NT};   // (behind the lanes' maxima)
+    w.slice_keys = Handed<uint64_t>{reinterpret_cast<uint64_t*>(lane_max + (size_t)rows * cfg.slices * NT)};   // (behind the lanes' maxima)
     w.lanes = (uint64_t)cfg.slices * (NT / 2) >= 4ull * cfg.ws_k ? NT / 2 : NT;
     w.count = count;
+    // One launch where every slice is held in registers, wherever its row starts, and the launch's workgroups are all on
+    // the chip at once (four a compute unit: they wait for each other).
+    const uint32_t e = dtype == LILY_BF16 ? 8u : 4u, nch = (cfg.vocab + 2u * (e - 1u)) / e;
+    const bool held = (nch + cfg.slices - 1u) / cfg.slices <= NT * STREAM_UNROLL && (uint64_t)rows * cfg.slices <= WIDE_HELD_GROUPS;
+    w.bounds = held ? bounds : nullptr;
     const bool inl = inline_rows != nullptr;
 #define LILY_WIDE(DT)                                                                               \
     (lse ? (inl ? launch_wide_variant<DT, true, true>(stream, rows, cfg, inline_rows, w)            \

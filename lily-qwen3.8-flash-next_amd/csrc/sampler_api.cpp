@@ -109,6 +109,7 @@ struct lily_sampler {
     // rows that draw among many candidates (rows_wide.hip): null in a view without them
     float* wide_max = nullptr;     // [WIDE_FLOATS] lane maxima, rows x slices x 256
     uint32_t* wide_count = nullptr;  // [WS_ROWS] candidates listed so far, 0 between launches
+    uint64_t* wide_bounds = nullptr; // [2][WS_ROWS][MAX_SLICES] slices' words of a launch under way, 0 between launches
     uint32_t* masked_served = nullptr;   // [WS_ROWS] rows that a launch over masks' words has drawn
     uint32_t ws_rows = WS_ROWS;    // rows that may span several workgroups
     uint32_t ws_slots = WS_SLOTS;  // candidate slots behind ws_cand
@@ -525,16 +526,16 @@ uint32_t wide_slices(const lily_sampler* s, const RowArgs* rows, uint32_t n, int
     uint32_t sl = s->force_slices ? s->force_slices : (2 * TARGET_GROUPS + n - 1) / n;
     const uint32_t e = dtype == LILY_BF16 ? 8 : 4;
     const uint32_t nch = (vocab + 2 * (e - 1)) / e + 1;
-    const uint32_t by_block = (nch + 256u * STREAM_UNROLL - 1) / (256u * STREAM_UNROLL);
+    // (no finer than a block a slice, unless that leaves fewer than four lanes for each of the k)
+    const uint32_t by_block = std::max((nch + 256u * STREAM_UNROLL - 1) / (256u * STREAM_UNROLL), (4u * kmax + 255u) / 256u);
     sl = sl > by_block ? by_block : sl;
     sl = sl > MAX_SLICES ? MAX_SLICES : sl;
     if ((uint64_t)n * MERGE_CAP > s->ws_slots) {   // a row's list of candidates: MERGE_CAP slots
         return 0;
     }
-    const uint64_t by_max = (uint64_t)WIDE_FLOATS / ((uint64_t)n * 257u);   // 256 lane maxima and one value a slice
+    const uint64_t by_max = (uint64_t)WIDE_FLOATS / ((uint64_t)n * 258u);   // 256 lane maxima and a word of keys a slice
     sl = sl > by_max ? (uint32_t)by_max : sl;
-    // the bound is the k-th largest of slices x 256 lane maxima: with twice k of them it is the
-    // median of the lanes' maxima, which about 1.4 k values reach on rows of Gaussian logits
+    // (the bound is one that k of the slices x 256 lane maxima reach)
     if (sl < 2 || (uint64_t)sl * 256u < 2ull * kmax) {
         return 0;
     }
@@ -710,7 +711,7 @@ int launch_part(lily_sampler* s, const LaunchPart& part, const RowArgs* table_de
     }
     if (part.wide) {
         HIP_TRY(launch_rows_wide(s->stream, dtype, part.lse, part.rows, cfg, nullptr, s->wide_max,
-                                 s->wide_count));
+                                 s->wide_count, s->wide_bounds));
         return LILY_OK;
     }
     if (part.masked && served == nullptr) {
@@ -751,7 +752,8 @@ int launch_inline(lily_sampler* s, int dtype, uint32_t vocab, const InlineRows& 
             for (uint32_t i = 0; i < n; ++i) {
                 lse = lse || rows.r[i].out_logprob != nullptr;
             }
-            HIP_TRY(launch_rows_wide(s->stream, dtype, lse, n, cfg, &rows, s->wide_max, s->wide_count));
+            HIP_TRY(launch_rows_wide(s->stream, dtype, lse, n, cfg, &rows, s->wide_max, s->wide_count,
+                                     s->wide_bounds));
             return LILY_OK;
         }
     }
@@ -1166,6 +1168,8 @@ int lily_sampler_create(int device, void* hip_stream, lily_sampler_t** out) {
     if (err == hipSuccess) err = hipMalloc(reinterpret_cast<void**>(&s->wide_count), WS_ROWS * 4);
     if (err == hipSuccess) err = hipMalloc(reinterpret_cast<void**>(&s->masked_served), WS_ROWS * 4);
     if (err == hipSuccess) err = hipMemset(s->wide_count, 0, WS_ROWS * 4);
+    if (err == hipSuccess) err = hipMalloc(reinterpret_cast<void**>(&s->wide_bounds), (size_t)2 * WS_ROWS * MAX_SLICES * 8);
+    if (err == hipSuccess) err = hipMemset(s->wide_bounds, 0, (size_t)2 * WS_ROWS * MAX_SLICES * 8);
     const size_t chain_bytes = (size_t)LILY_MAX_VERIFY_ROWS * CHAIN_CAP * 8 + (LILY_MAX_VERIFY_ROWS + 1) * 4;
     if (err == hipSuccess) err = hipMalloc(reinterpret_cast<void**>(&s->chain_cand), chain_bytes);
     if (err == hipSuccess) err = hipMemset(s->chain_cand, 0, chain_bytes);
@@ -1199,6 +1203,7 @@ void lily_sampler_destroy(lily_sampler_t* s) {
     (void)hipFree(s->ws_ticket);
     (void)hipFree(s->wide_max);
     (void)hipFree(s->wide_count);
+    (void)hipFree(s->wide_bounds);
     (void)hipFree(s->masked_served);
     (void)hipFree(s->chain_cand);
     (void)hipFree(s->table_dev);

@@ -251,6 +251,49 @@ def test_random_launches_of_rows_of_many_candidates(sampler):
     assert went >= 30, went   # (a launch of one or two rows has too few slices for some k)
 
 
+@pytest.mark.parametrize("rows,vocab,bf16", [(1, 32_003, True), (4, 40_001, False), (8, 248_320, False), (26, 151_936, False),
+                                             (27, 151_936, False), (53, 151_937, True), (54, 151_937, True)])
+def test_bounds_over_the_slices(sampler, rows, vocab, bf16):
+    """Rows without top_k either side of the most workgroups that one launch takes (26 and 27 rows in 38
+    slices, 53 and 54 in 19), in slices cut finer than a block, and in the most slices there are: rows of Gaussian
+    logits, which need no exhaustive select; the best 1 100 all in the row's first ids, or spread evenly; all but a contiguous
+    seventh -inf, so that most waves have nothing to name; penalties on the best."""
+    rng = np.random.default_rng(rows + vocab)
+    x = rng.normal(0, 2, (rows, vocab)).astype(np.float32)
+    kw = [dict(temperature=0.8, top_k=0, top_p=0.97, seed=700 + r) for r in range(rows)]
+    checked = sorted({0, rows // 2, rows - 1})
+    fmt = W.to_bf16_bits if bf16 else lambda a: a
+    xs = fmt(x)
+    r, stats = _with_stats(sampler, lambda: run_rows(sampler, xs, kw, [1] * rows, logprobs=True))
+    assert stats[0] == 0 and stats[1] == rows and stats[2] == 0, stats
+    for i in checked:
+        d = O.sample(xs[i], None, o_params(**kw[i]), 1, want_logprob=True)
+        check_row_against_oracle(r, i, d)
+        _check_logprob(r.logprobs[i], d.logprob, i)
+    for i in range(rows):
+        if i % 3 == 0:
+            x[i, :1100] += 9.0
+        elif i % 3 == 1:
+            x[i, :vocab // 3] = -np.inf
+            x[i, vocab // 3 + vocab // 7:] = -np.inf
+        else:
+            x[i, ::vocab // 1100] += 9.0
+    xs = fmt(x)
+    hist = [np.argsort(-x[i])[:300].astype(np.int32) for i in range(rows)]
+    scratch, counts = [], [np.bincount(hh, minlength=vocab).astype(np.uint32) for hh in hist]
+    for hh in hist:
+        sc = LS.SamplerScratch(sampler, vocab)
+        sc.add_history(torch.from_numpy(hh).to(dev()))
+        scratch.append(sc)
+    pkw = [dict(k, repetition_penalty=1.2, presence_penalty=0.5) if i % 2 else k for i, k in enumerate(kw)]
+    r, stats = _with_stats(sampler, lambda: run_rows(sampler, xs, pkw, [2] * rows, scratch=scratch, logprobs=True))
+    assert stats[0] == 0 and stats[1] + stats[2] == rows, stats
+    for i in sorted({*checked, min(1, rows - 1), min(2, rows - 1)}):
+        d = O.sample(xs[i], counts[i], o_params(**pkw[i]), 2, want_logprob=True)
+        check_row_against_oracle(r, i, d)
+        _check_logprob(r.logprobs[i], d.logprob, i)
+
+
 @pytest.mark.parametrize("masked", [False, True], ids=["two-launches", "merged-slices"])
 @pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
 def test_sort_of_many_candidates(sampler, bf16, masked):
