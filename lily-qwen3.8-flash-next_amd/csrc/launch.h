@@ -55,11 +55,16 @@ hipError_t launch_spec_accept(hipStream_t stream, const uint32_t* draws, const u
 // out_f32: the logits are f32 [rows, logits_stride] instead of bf16.  wq.bits 4 / 8: `weight` points
 // at the reference's affine codes (u32 words, weight_stride words a row), wq.scales / wq.biases at
 // bf16 [vocab, d >> wq.group_shift]; f32 logits only.
-// The rows' exponent scales: in device memory, or (p null, at most SCALES_INLINE rows) with the launch itself.
-constexpr uint32_t SCALES_INLINE = 8;
+// The rows' exponent scales: in device memory, or (p null, at most SCALES_INLINE rows) with the launch itself.  A launch that
+// has them with it may also carry something to the device while it runs, for the launches behind it: `pieces` of
+// 16 bytes from src (pinned host memory, mapped into the device) to dst.
+constexpr uint32_t SCALES_INLINE = 128;
 struct RowScales {
     const float* p = nullptr;
     float few[SCALES_INLINE] = {};
+    const void* src = nullptr;
+    void* dst = nullptr;
+    uint32_t pieces = 0;
     RowScales() = default;
     RowScales(const float* from) : p(from) {}
 };

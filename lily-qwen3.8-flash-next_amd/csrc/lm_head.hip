@@ -78,6 +78,7 @@ k_lm_head_bf16(const RowScales scales_arg, const uint16_t* __restrict__ hidden, 
                uint32_t d, uint32_t vocab, void* __restrict__ logits_out, uint64_t logits_stride, float* __restrict__ tile_max,
                float* __restrict__ tile_sum, uint32_t tiles_per_row, uint32_t m_tiles, HeadQuant quant) {
     const float* __restrict__ c2_of_row = scales_of(scales_arg);
+    carry(scales_arg, 0u);
     static_assert(WBITS == 0 || !T::DIRECT, "codes pass through registers");
     constexpr int BM = T::BM, BN = T::BN, BK = T::BK, MI = T::MI, NI = T::NI, ROW_BYTES = T::ROW_BYTES;
     extern __shared__ __align__(16) char lds[];

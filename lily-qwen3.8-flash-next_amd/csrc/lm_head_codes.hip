@@ -94,6 +94,7 @@ k_lm_head_codes(const RowScales scales_arg, const uint16_t* __restrict__ hidden,
                 float* __restrict__ tile_max, float* __restrict__ tile_sum, uint32_t tiles_per_row,
                 const uint16_t* __restrict__ scales, const uint16_t* __restrict__ biases, uint32_t group_shift) {
     const float* __restrict__ c2_of_row = scales_of(scales_arg);
+    carry(scales_arg, gridDim.x - 1u);   // (one with no more tiles than any other)
     constexpr int STEPS = WBITS == 4 ? 2 : 1;          // products over 32 values a wave makes per stage and block
     constexpr uint32_t STAGE_K = 128u * 8u / WBITS;    // values of d in a stage
     constexpr uint32_t WAVE_K = STAGE_K / 4u;          // ... of which a wave multiplies these

@@ -69,6 +69,7 @@ k_lm_head_codes_rows(const RowScales scales_arg, const uint16_t* __restrict__ hi
                      uint32_t m_tiles, const uint16_t* __restrict__ scales, const uint16_t* __restrict__ biases,
                      uint32_t group_shift) {
     const float* __restrict__ c2_of_row = scales_of(scales_arg);
+    carry(scales_arg, 0u);
     constexpr int BM = MI * 32;
     constexpr int STAGE_K = 1024 / WBITS, STEPS = STAGE_K / STEP_K;   // steps of 64 in a stage: 2 or 4
     constexpr int HIDDEN_AHEAD = MI == 4 ? 2 : 4;

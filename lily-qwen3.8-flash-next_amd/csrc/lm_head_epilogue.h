@@ -27,6 +27,18 @@ __device__ __forceinline__ const float* scales_of(const RowScales& c2) {
     return c2.p != nullptr ? c2.p : reinterpret_cast<const float*>(args + offsetof(RowScales, few));
 }
 
+// What the launch carries to the device (RowScales), by workgroup `who`.  (A kernel of its own ahead of the head was a
+// trip across the bus with nothing beside it: 50 rows over 8-bit codes, d = 2560, 127.5 -> 123.7 us a call, 100 bf16 rows
+// 214 -> 211, 16 rows over 8-bit codes of 40 000, d = 2048, 41.0 -> 38.6.)
+__device__ __forceinline__ void carry(const RowScales& c2, uint32_t who) {
+    if (blockIdx.x == who) {
+        const uint4* src = static_cast<const uint4*>(c2.src);
+        for (uint32_t i = threadIdx.x; i < c2.pieces; i += blockDim.x) {
+            static_cast<uint4*>(c2.dst)[i] = src[i];
+        }
+    }
+}
+
 // acc: the sums of a wave's MI x NI products of 32 x 32; four waves, WAVES_M x (4 / WAVES_M), this
 // one at (wm, wn), hold WAVES_M * MI * 32 rows from m0 on by the 128 columns of tile n_tile.  `lds`
 // is free for reuse, (4 / WAVES_M + 2) floats a row; every thread of the workgroup calls.

@@ -2207,16 +2207,33 @@ int rows_with_tiles(lily_sampler* s, const lily_lm_head* h, const lily_rows* b, 
     LaunchPart parts[2];
     const uint32_t n_parts =
         certain < rows ? plan_parts(s, table + certain, rows - certain, (int)b->dtype, b->vocab, parts) : 0u;
-    if (int rc = stage_commit(s, slot, served_off + (size_t)rows * 4)) {
+    const char* dev = reinterpret_cast<const char*>(s->table_dev);
+    const size_t staged = served_off + (size_t)rows * 4;
+    RowScales scales(reinterpret_cast<const float*>(dev + c2_off));
+    // (A producer of this library's own brings what is staged for the draws while it runs; what fits a launch's
+    // arguments goes that way, and is the launch's own when it is replayed.)
+    const bool carried = h != nullptr && round16(staged) > sizeof(PlacedPieces) && rows <= SCALES_INLINE &&
+                         (few_weights.library_rows == 0u || rows < few_weights.library_rows);
+    if (carried) {
+        void* mapped = nullptr;
+        HIP_TRY(hipHostGetDevicePointer(&mapped, s->stage[slot], 0));
+        scales.p = nullptr;
+        std::copy(c2, c2 + rows, scales.few);
+        scales.src = mapped;
+        scales.dst = s->table_dev;
+        scales.pieces = (uint32_t)(round16(staged) / 16u);
+    } else if (int rc = stage_commit(s, slot, staged)) {
         return rc;
     }
-    const char* dev = reinterpret_cast<const char*>(s->table_dev);
     if (h != nullptr) {
         HIP_TRY(launch_lm_head_bf16(s->stream, h->hidden_dev, h->hidden_stride, h->weight_dev,
-                                    h->weight_stride, rows, h->d, b->vocab,
-                                    reinterpret_cast<const float*>(dev + c2_off),
+                                    h->weight_stride, rows, h->d, b->vocab, scales,
                                     const_cast<void*>(b->logits_dev), b->row_stride, h->tile_max_dev,
-                                    h->tile_sum_dev, h->logits_f32 != 0u, HeadWeightsOf(s, h)));
+                                    h->tile_sum_dev, h->logits_f32 != 0u, few_weights));
+    }
+    if (carried) {
+        HIP_TRY(hipEventRecord(s->stage_done[slot], s->stream));
+        s->stage_used[slot] = true;
     }
     uint32_t* served_dev = reinterpret_cast<uint32_t*>(const_cast<char*>(dev) + served_off);
     if (served != 0) {
