@@ -13,6 +13,7 @@
 // admits a third of the vocabulary is left to the launch behind, which streams the row.
 #include "launch.h"
 #include "row_kernel.h"
+#include "sort_sixteen.h"
 
 #if !defined(LILY_DT)
 #error "compile with -DLILY_DT=<lily_dtype>"
@@ -22,11 +23,11 @@ namespace lily {
 
 namespace {
 
-constexpr uint32_t MT = 1024, MWAVE = MT / 64;
+constexpr uint32_t MT = SIXTEEN_THREADS, MWAVE = SIXTEEN_WAVES;
 constexpr uint32_t MASKED_WORDS = MASKED_MAX_VOCAB / 32u, WORDS_PER = MASKED_WORDS / MT;
 constexpr uint32_t MASKED_CAP = 8192;      // values that are sorted
 constexpr uint32_t MASKED_DENSE = 49152;   // ids a mask may admit
-constexpr uint32_t MBINS = 2048;           // of the sort
+constexpr uint32_t MBINS = SIXTEEN_BINS;   // of the sort
 constexpr uint32_t HBINS = 4096;           // of the histograms, 12 bits
 // Dynamic LDS in 64-bit slots: the sorted candidates and the tail's arrays; the sort's bins; the values as they
 // come (the histograms, before there are any); the words that admit anything (bits, number), and where those are
@@ -38,8 +39,7 @@ constexpr uint32_t MASKED_LDS_BYTES = (OFF_PLACED + MASKED_CAP) * 8;
 static_assert(MASKED_WORDS * 6 <= MASKED_CAP * 8 && HBINS * 4 <= MASKED_CAP * 8, "masked rows: LDS layout");
 
 struct MaskedShared {
-    uint32_t wave_u[MWAVE];
-    uint64_t wave_k[MWAVE];
+    SixteenShared six;
     float wave_f[MWAVE];
     double wave_d[MWAVE];
     uint32_t n, bin, above, need;
@@ -47,25 +47,6 @@ struct MaskedShared {
     float bias_delta[STREAM_BIAS_CAP];
     uint32_t biased[MASKED_WORDS / 32];    // bit w: some pair names an id of word w
 };
-
-// The threads' values summed up to and including each, over the whole workgroup; `all`: all of them.
-__device__ __forceinline__ uint32_t scan_all(uint32_t x, MaskedShared& ms, uint32_t& all) {
-    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
-    const uint32_t incl = wave_scan_u32(x);
-    __syncthreads();   // (what the last call left has been read)
-    if (lane == 63u) {
-        ms.wave_u[w] = incl;
-    }
-    __syncthreads();
-    uint32_t before = 0;
-    all = 0;
-    for (uint32_t i = 0; i < MWAVE; ++i) {
-        const uint32_t t = ms.wave_u[i];
-        before += i < w ? t : 0u;
-        all += t;
-    }
-    return before + incl;
-}
 
 template <int DT, bool LSE>
 __device__ __forceinline__ void masked_row(const LILY_CONST RowArgs* src, const LaunchCfg& cfg, Shared& sh, MaskedShared& ms) {
@@ -118,8 +99,8 @@ __device__ __forceinline__ void masked_row(const LILY_CONST RowArgs* src, const 
         admitted += (uint32_t)__popc(bits[i]);
     }
     uint32_t n_words, total;
-    uint32_t place = scan_all(some, ms, n_words) - some;
-    scan_all(admitted, ms, total);
+    uint32_t place = scan_all(some, ms.six, n_words) - some;
+    scan_all(admitted, ms.six, total);
     if (tid < n_bias && ms.bias_id[tid] < vocab) {
         const uint32_t at = ms.bias_id[tid] >> 5;
         atomicOr(&ms.biased[at >> 5], 1u << (at & 31u));
@@ -233,7 +214,7 @@ __device__ __forceinline__ void masked_row(const LILY_CONST RowArgs* src, const 
                 h[i] = hist[HBINS - 1u - (tid * (HBINS / MT) + i)];
                 mine += h[i];
             }
-            uint32_t before = scan_all(mine, ms, whole) - mine;
+            uint32_t before = scan_all(mine, ms.six, whole) - mine;
             if (above + whole <= a.k) {
                 // fewer values than are asked for: all of them
                 break;
@@ -295,129 +276,15 @@ __device__ __forceinline__ void masked_row(const LILY_CONST RowArgs* src, const 
         return;
     }
 
-    // ---- the k best in order: a counting sort (see wg_sort_topk), eight values a thread
+    // ---- the k best in order
     const uint32_t n = min(ms.n, MASKED_CAP), k = min(a.k, n);
     constexpr uint32_t PER = MASKED_CAP / MT;
     uint64_t mine[PER];
-    uint32_t hi = 0u, lo = 0xffffffffu;
 #pragma unroll
     for (uint32_t j = 0; j < PER; ++j) {
         mine[j] = tid + j * MT < n ? mixed[tid + j * MT] : 0ull;
-        const uint32_t key = (uint32_t)(mine[j] >> 32);
-        hi = max(hi, key);
-        lo = mine[j] != 0ull ? min(lo, key) : lo;
     }
-    hi = wave_max_u32(hi);
-    lo = wave_min_u32(lo);
-    if (lane == 0u) {
-        ms.wave_k[w] = ((uint64_t)hi << 32) | lo;
-    }
-#pragma unroll
-    for (uint32_t i = 0; i < MBINS / MT; ++i) {
-        bins[tid + i * MT] = 0u;
-    }
-    __syncthreads();
-    hi = 0u;
-    lo = 0xffffffffu;
-    for (uint32_t i = 0; i < MWAVE; ++i) {
-        hi = max(hi, (uint32_t)(ms.wave_k[i] >> 32));
-        lo = min(lo, (uint32_t)ms.wave_k[i]);
-    }
-    uint32_t longest = 0;
-    if (n != 0u) {
-        const bool crosses = hi >= 0x80000000u && lo < 0x80000000u;
-        const float top = lilym_key_value(hi);
-        const float range = crosses ? top - lilym_key_value(lo) : (float)(hi - lo) + 1.0f;
-        const float scale = (float)MBINS / range * 0.9999f;
-        const bool spread = scale > 0.0f && range < 3.0e38f && scale <= 3.0e38f;
-        auto bin_of = [&](uint64_t c) -> uint32_t {   // never decreases as c does
-            const uint32_t key = (uint32_t)(c >> 32);
-            const float d = crosses ? top - lilym_key_value(key) : (float)(hi - key);
-            return spread ? (uint32_t)fminf(d * scale, (float)(MBINS - 1u)) : 0u;
-        };
-        uint32_t at_of[PER];   // bin, and place in it from bit 16 on
-#pragma unroll
-        for (uint32_t j = 0; j < PER; ++j) {
-            at_of[j] = 0u;
-            if (mine[j] != 0ull) {
-                const uint32_t b = bin_of(mine[j]);
-                at_of[j] = b | (atomicAdd(&bins[b], 1u) << 16);
-            }
-        }
-        __syncthreads();
-        const uint32_t h0 = bins[2u * tid], h1 = bins[2u * tid + 1u];
-        static_assert(MBINS == 2 * MT, "two bins a thread");
-        uint32_t whole;
-        const uint32_t from = scan_all(h0 + h1, ms, whole) - h0 - h1;
-        longest = max(from < k ? h0 : 0u, from + h0 < k ? h1 : 0u);
-        longest = wave_max_u32(longest);
-        __syncthreads();
-        bins[2u * tid] = from;
-        bins[2u * tid + 1u] = from + h0;
-        if (lane == 0u) {
-            ms.wave_u[w] = longest;
-        }
-        __syncthreads();
-        longest = 0;
-        for (uint32_t i = 0; i < MWAVE; ++i) {
-            longest = max(longest, ms.wave_u[i]);
-        }
-        if (longest <= SORT_BIN_MAX) {
-#pragma unroll
-            for (uint32_t j = 0; j < PER; ++j) {
-                if (mine[j] != 0ull) {
-                    placed[bins[at_of[j] & 0xffffu] + (at_of[j] >> 16)] = mine[j];
-                }
-            }
-            __syncthreads();
-            // The few that share a bin are ranked against each other.
-#pragma unroll
-            for (uint32_t j = 0; j < PER; ++j) {
-                if (mine[j] != 0ull) {
-                    const uint32_t b = at_of[j] & 0xffffu, begin = bins[b], end = b + 1u < MBINS ? bins[b + 1u] : n;
-                    if (begin < k) {
-                        uint32_t rank = begin;
-                        for (uint32_t i = begin; i < end; ++i) {
-                            rank += placed[i] > mine[j] ? 1u : 0u;
-                        }
-                        if (rank < k) {
-                            dyn_lds[rank] = mine[j];
-                        }
-                    }
-                }
-            }
-            __syncthreads();
-        } else {
-            // Ties by the hundred, an outlier that stretches the steps: bitonic, all of them.
-            uint32_t p = 128;
-            while (p < n) {
-                p <<= 1;
-            }
-#pragma unroll
-            for (uint32_t j = 0; j < PER; ++j) {
-                placed[tid + j * MT] = mine[j];
-            }
-            __syncthreads();
-            for (uint32_t size = 2; size <= p; size <<= 1) {
-                for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
-                    for (uint32_t i = tid; i < (p >> 1); i += MT) {
-                        const uint32_t pos = (i / stride) * (stride << 1) + (i % stride), partner = pos + stride;
-                        const bool desc = (pos & size) == 0u;
-                        const uint64_t x = placed[pos], y = placed[partner];
-                        if (desc ? x < y : x > y) {
-                            placed[pos] = y;
-                            placed[partner] = x;
-                        }
-                    }
-                    __syncthreads();
-                }
-            }
-            if (tid < k) {
-                dyn_lds[tid] = placed[tid];
-            }
-            __syncthreads();
-        }
-    }
+    sort_by_sixteen(mine, n, k, dyn_lds, bins, placed, ms.six);
     phase(cfg, 6);
     if (tid >= NT) {
         return;   // (the draw is four waves' work: a barrier waits for those that are left)

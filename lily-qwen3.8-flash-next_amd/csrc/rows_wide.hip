@@ -22,6 +22,7 @@
 #endif
 
 #include "row_kernel.h"
+#include "sort_sixteen.h"
 
 namespace lily {
 
@@ -318,12 +319,21 @@ __device__ __forceinline__ float wide_bound_of(const WideArgs& w, uint32_t row, 
     return enough ? lilym_key_value(prefix) : F32_LOWEST;
 }
 
+// Dynamic LDS of sixteen waves, in 64-bit slots: the sorted candidates and the tail's arrays; the sort's bins; a slice's
+// candidates, then the row's by bins.
+constexpr uint32_t SIXTEEN_OFF_BINS = (LILY_SAMPLE_K_CAP * 8 + 3 * LILY_SAMPLE_K_CAP * 4) / 8;
+constexpr uint32_t SIXTEEN_OFF_PLACED = SIXTEEN_OFF_BINS + SIXTEEN_BINS / 2;
+constexpr uint32_t SIXTEEN_LDS_BYTES = (SIXTEEN_OFF_PLACED + MERGE_CAP) * 8;
+
 // From a slice's candidates (n_mine of them in cand) to the row's draw, in the workgroup that arrives last.
 // gave_up: the slice has none because it did not learn the row's bound; the row is then taken
 // by the select that is right for any input.
-template <int DT, bool LSE>
+// Sixteen waves sort, and the first four draw.
+template <int DT, bool LSE, uint32_t THREADS = NT>
 __device__ __forceinline__ void wide_finish(RowArgs& a, const LaunchCfg& cfg, const WideArgs& w, Shared& sh, uint32_t& n_mine,
-                                            uint64_t* cand, uint32_t row, uint32_t S, uint32_t step, bool want_lse, bool gave_up) {
+                                            uint64_t* cand, uint32_t row, uint32_t S, uint32_t step, bool want_lse, bool gave_up,
+                                            SixteenShared* six = nullptr) {
+    constexpr bool SIXTEEN = THREADS == SIXTEEN_THREADS;
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     __syncthreads();
     WIDE_MARK(6);
@@ -337,7 +347,7 @@ __device__ __forceinline__ void wide_finish(RowArgs& a, const LaunchCfg& cfg, co
     __syncthreads();
     const uint32_t base = n_mine;
     if (base + mine <= MERGE_CAP) {
-        for (uint32_t i = tid; i < mine; i += NT) {
+        for (uint32_t i = tid; i < mine; i += THREADS) {
             handed_store(cfg.ws_cand, (size_t)row * MERGE_CAP + base + i, cand[i]);
         }
     }
@@ -352,11 +362,11 @@ __device__ __forceinline__ void wide_finish(RowArgs& a, const LaunchCfg& cfg, co
     WIDE_MARK(7);
     // The list's first entries are asked for together with its length: what lies behind its end is
     // dropped (the slots are the workspace's whatever they hold).
-    constexpr int PER = MERGE_CAP / NT, FIRST = 8;
+    constexpr int PER = MERGE_CAP / THREADS, FIRST = 2048 / THREADS;
     uint64_t mine_c[PER];
 #pragma unroll
     for (int j = 0; j < FIRST; ++j) {
-        mine_c[j] = handed_load(cfg.ws_cand, (size_t)row * MERGE_CAP + tid + (uint32_t)j * NT);
+        mine_c[j] = handed_load(cfg.ws_cand, (size_t)row * MERGE_CAP + tid + (uint32_t)j * THREADS);
     }
     const uint32_t total = load_through(&w.count[row]);
     __syncthreads();   // (everybody has read it)
@@ -369,21 +379,25 @@ __device__ __forceinline__ void wide_finish(RowArgs& a, const LaunchCfg& cfg, co
         // more than the buffers hold (values that tie by the thousand, a row in ascending
         // order): the select that is right for any input, over the whole row
         __syncthreads();
+        if (SIXTEEN && tid >= NT) {
+            return;   // (four waves' work: a barrier waits for those that are left)
+        }
+        cand = dyn_lds;
         select_exhaustive<DT>(a, 0, cfg.vocab, a.k, want_lse, cand, min(cfg.dyn_slots, MERGE_CAP), sh);
         n = min(sh.n_cand, min(cfg.dyn_slots, MERGE_CAP));
         if (cfg.path_stats != nullptr && tid == 0) {
             atomicAdd(&cfg.path_stats[2], 1u);
         }
     } else {
-        if (total > (uint32_t)FIRST * NT) {   // (the same in every thread)
+        if (total > (uint32_t)FIRST * THREADS) {   // (the same in every thread)
 #pragma unroll
             for (int j = FIRST; j < PER; ++j) {
-                mine_c[j] = handed_load(cfg.ws_cand, (size_t)row * MERGE_CAP + tid + (uint32_t)j * NT);
+                mine_c[j] = handed_load(cfg.ws_cand, (size_t)row * MERGE_CAP + tid + (uint32_t)j * THREADS);
             }
         }
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
-            if (tid + (uint32_t)j * NT >= total) {
+            if (tid + (uint32_t)j * THREADS >= total) {
                 mine_c[j] = 0ull;
             }
         }
@@ -405,13 +419,23 @@ __device__ __forceinline__ void wide_finish(RowArgs& a, const LaunchCfg& cfg, co
         }
         __syncthreads();
         WIDE_MARK(13);
-        sorted = wg_sort_topk(cand, mine_c, total, a.k, sh, n);
-        if (!sorted) {
-            n = wg_select_topk(cand, total, a.k, sh);
+        if constexpr (SIXTEEN) {
+            n = min(total, a.k);
+            sort_by_sixteen(mine_c, total, n, dyn_lds, reinterpret_cast<uint32_t*>(dyn_lds + SIXTEEN_OFF_BINS), dyn_lds + SIXTEEN_OFF_PLACED, *six);
+            sorted = true;
+            cand = dyn_lds;
+        } else {
+            sorted = wg_sort_topk(cand, mine_c, total, a.k, sh, n);
+            if (!sorted) {
+                n = wg_select_topk(cand, total, a.k, sh);
+            }
         }
         WIDE_MARK(14);
         if (cfg.path_stats != nullptr && tid == 0) {
             atomicAdd(&cfg.path_stats[1], 1u);
+        }
+        if (SIXTEEN && tid >= NT) {
+            return;
         }
     }
     tail<DT, true>(a, cfg.vocab, step, n, sorted, cand, sh, cfg);
@@ -487,12 +511,19 @@ __global__ __launch_bounds__(NT, 4) void k_wide_draw(InlineRows rows_arg, Launch
 // does not find them all within WIDE_TRIES looks (another stream's work holds the chip) gives up, and the row is taken by the
 // exhaustive select: every wait ends.
 constexpr uint32_t WIDE_TRIES = 1u << 13, WIDE_HELD_GROUPS = 1024;
+// Up to so many workgroups are of sixteen waves each, a piece of 16 bytes a thread, and sort with all of them (1 f32 row of
+// 151 936 23.2 -> 19.8 us, under penalties 24.2 -> 20.5, 4 rows of 32 000 23.1 -> 20.8); launching four times the waves
+// takes that back at 152 (4 rows 24.4 both ways, 13 rows 31.9 -> 35.9).
+constexpr uint32_t WIDE_SIXTEEN_GROUPS = 128;
 
-template <int DT, bool LSE, bool INLINE>
-__global__ __launch_bounds__(NT, 4) void k_wide_held(InlineRows rows_arg, LaunchCfg cfg, WideArgs w) {
+template <int DT, bool LSE, bool INLINE, uint32_t THREADS>
+__global__ __launch_bounds__(THREADS, 4) void k_wide_held(InlineRows rows_arg, LaunchCfg cfg, WideArgs w) {
     __shared__ Shared sh;
     __shared__ uint32_t n_mine, lost;
-    constexpr int E = Geo<DT>::E, C = (int)STREAM_UNROLL, V = C * E;
+    __shared__ float row_bound, wave_m[THREADS / 64];
+    __shared__ double wave_s[THREADS / 64];
+    __shared__ SixteenShared six;
+    constexpr int E = Geo<DT>::E, C = (int)(NT * STREAM_UNROLL / THREADS), V = C * E;
     constexpr uint32_t EMASK = (1u << E) - 1u;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, s = blockIdx.x, row = blockIdx.y, S = cfg.slices;
     if (cfg.served != nullptr && *(const LILY_CONST uint32_t*)(cfg.served + row) != 0u) {
@@ -513,7 +544,7 @@ __global__ __launch_bounds__(NT, 4) void k_wide_held(InlineRows rows_arg, Launch
     Geo<DT> g;
     g.init(a.logits, cfg.vocab, s, S);
     const uint32_t c_last = max(g.ce, 1u) - 1u;
-    auto chunk_of = [&](int u) -> uint32_t { return g.cb + (uint32_t)u * NT + tid; };
+    auto chunk_of = [&](int u) -> uint32_t { return g.cb + (uint32_t)u * THREADS + tid; };
     auto inside = [&](int u) -> bool { return chunk_of(u) >= g.main_lo && chunk_of(u) < g.main_hi; };
     u32x4 raw[C];
 #pragma unroll
@@ -586,8 +617,33 @@ __global__ __launch_bounds__(NT, 4) void k_wide_held(InlineRows rows_arg, Launch
         }
         lane_max = fmaxf(lane_max, cm[u]);
     }
-    auto true_edge = [&](float x, uint32_t id) -> float { return pen ? wide_worth(a, x, id) : x; };
-    wide_edges<DT>(a, g, [&](float x, uint32_t id) { lane_max = fmaxf(lane_max, true_edge(x, id)); });
+    // Ids of partial chunks at the row's ends, one a thread (fewer than 16 at either end).
+    uint32_t edge = 0xffffffffu;
+    float ev = NEG_INF;
+    if (tid < 64u) {
+        edge = g.id_lo + tid < g.edge_lo_end ? g.id_lo + tid : edge;
+    } else if (tid < 128u) {
+        edge = g.edge_hi_begin + tid - 64u < g.id_hi ? g.edge_hi_begin + tid - 64u : edge;
+    }
+    if (edge != 0xffffffffu) {
+        ev = load_logit<DT>(a.logits, edge);
+        ev = pen ? wide_worth(a, ev, edge) : ev;
+        ev = ev > NEG_INF ? ev : NEG_INF;
+        lane_max = fmaxf(lane_max, ev);
+    }
+    if (THREADS != NT) {
+        // (four threads' values are a lane's of the four waves that name keys)
+        float* maxima = reinterpret_cast<float*>(dyn_lds);
+        maxima[tid] = lane_max;
+        __syncthreads();
+        float m = NEG_INF;
+        if (tid < NT) {
+            for (uint32_t i = 0; i < THREADS; i += NT) {
+                m = fmaxf(m, maxima[tid + i]);
+            }
+        }
+        lane_max = m;
+    }
     WIDE_MARK(1);
     // ---- the slice's keys: 0 stands for those that are not there yet
     uint64_t* bounds = w.bounds + (size_t)row * MAX_SLICES;
@@ -610,44 +666,61 @@ __global__ __launch_bounds__(NT, 4) void k_wide_held(InlineRows rows_arg, Launch
                 }
             }
         }
-        wide_edges<DT>(a, g, [&](float x, uint32_t id) {
-            x = true_edge(x, id);
-            if (x > NEG_INF) {
-                lse.add_one(x, a.c2);
+        if (ev > NEG_INF) {
+            lse.add_one(ev, a.c2);
+        }
+        // (as lse_reduce(), whatever the number of waves)
+        const float m_w = wave_max_dpp(lse.mc);
+        const double s_w = wave_sum_d(lse.mc > NEG_INF ? (double)lse.s * exp2((double)lse.mc - (double)m_w) : 0.0);
+        if (lane == 0u) {
+            wave_m[tid >> 6] = m_w;
+            wave_s[tid >> 6] = s_w;
+        }
+        __syncthreads();
+        if (tid < 64u) {
+            const float m_l = lane < THREADS / 64u ? wave_m[lane] : NEG_INF;
+            const float m = wave_max_dpp(m_l);
+            const double all = wave_sum_d(m_l > NEG_INF ? wave_s[lane] * exp2((double)m_l - (double)m) : 0.0);
+            if (lane == 0u) {
+                const size_t slot = (size_t)row * S + s;
+                handed_store(cfg.ws_lse, 2 * slot, (double)m);
+                handed_store(cfg.ws_lse, 2 * slot + 1, all);
             }
-        });
-        lse_reduce(sh, lse);
-        if (tid == 0) {
-            const size_t slot = (size_t)row * S + s;
-            handed_store(cfg.ws_lse, 2 * slot, sh.lse_mc);
-            handed_store(cfg.ws_lse, 2 * slot + 1, sh.lse_s);
         }
     }
     WIDE_MARK(2);
     // ---- the row's bound, once all its slices' words are there (a word is the message: nothing else is read for it)
-    uint64_t keys = 0;
     auto wait_for = [&](const uint64_t* words) {
-        for (uint32_t tries = 0;; ++tries) {
-            keys = lane < S ? load_through(words + lane) : ~0ull;
-            if (__ballot(keys == 0ull) == 0ull) {
-                break;
-            }
-            if (tries == WIDE_TRIES) {
-                if (lane == 0u) {
-                    lost = 1u;
+        if (tid < 64u) {   // (the first wave looks)
+            uint64_t keys = 0;
+            for (uint32_t tries = 0;; ++tries) {
+                keys = lane < S ? load_through(words + lane) : ~0ull;
+                if (__ballot(keys == 0ull) == 0ull) {
+                    break;
                 }
-                break;
+                if (tries == WIDE_TRIES) {
+                    if (lane == 0u) {
+                        lost = 1u;
+                    }
+                    break;
+                }
+                __builtin_amdgcn_s_sleep(1);
             }
-            __builtin_amdgcn_s_sleep(1);
+            const float b = bound_of_keys(lane < S ? keys : 0ull, a.k, S);
+            if (lane == 0u) {
+                row_bound = b;
+            }
         }
         __syncthreads();
     };
     wait_for(bounds);
-    float bound = bound_of_keys(lane < S ? keys : 0ull, a.k, S);
+    float bound = row_bound;
     if (lost == 0u && !(bound > F32_LOWEST)) {
         // (the same in all the row's workgroups) Most of the row is -inf: too many waves had no value to name.  The lanes'
         // maxima change hands, and the bound is the k-th largest of those.
-        handed_store(w.lane_max, ((size_t)row * S + s) * NT + tid, lane_max);
+        if (tid < NT) {
+            handed_store(w.lane_max, ((size_t)row * S + s) * NT + tid, lane_max);
+        }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
         __syncthreads();
         uint64_t* handed = bounds + (size_t)gridDim.y * MAX_SLICES;
@@ -663,7 +736,7 @@ __global__ __launch_bounds__(NT, 4) void k_wide_held(InlineRows rows_arg, Launch
             }
             __syncthreads();
             uint32_t n = 0;
-            for (uint32_t j0 = 0; j0 < S; j0 += 8u) {
+            for (uint32_t j0 = 0; tid < NT && j0 < S; j0 += 8u) {
                 float x[8];
 #pragma unroll
                 for (uint32_t u = 0; u < 8u; ++u) {
@@ -685,7 +758,7 @@ __global__ __launch_bounds__(NT, 4) void k_wide_held(InlineRows rows_arg, Launch
         bound = T > WIDE_LEAST_KEY ? lilym_key_value(T << 16) : F32_LOWEST;
     }
     WIDE_MARK(5);
-    uint64_t* cand = dyn_lds;
+    uint64_t* cand = THREADS == NT ? dyn_lds : dyn_lds + SIXTEEN_OFF_PLACED;
     auto offer = [&](float x, uint32_t id) {
         if (x >= bound && x > NEG_INF) {
             const uint32_t at = atomicAdd(&n_mine, 1u);
@@ -703,9 +776,9 @@ __global__ __launch_bounds__(NT, 4) void k_wide_held(InlineRows rows_arg, Launch
             }
         }
     }
-    wide_edges<DT>(a, g, [&](float x, uint32_t id) { offer(true_edge(x, id), id); });
+    offer(ev, edge);   // (-inf where there is none)
     __syncthreads();
-    wide_finish<DT, LSE>(a, cfg, w, sh, n_mine, cand, row, S, step, want_lse, lost != 0u);
+    wide_finish<DT, LSE, THREADS>(a, cfg, w, sh, n_mine, cand, row, S, step, want_lse, lost != 0u, &six);
 }
 
 template <int DT, bool LSE, bool INLINE>
@@ -716,7 +789,11 @@ static hipError_t launch_wide_variant(hipStream_t stream, uint32_t rows, const L
     const InlineRows& r = inline_rows != nullptr ? *inline_rows : none;
     const size_t dyn2 = (size_t)cfg.dyn_slots * 8;
     if (w.bounds != nullptr) {
-        hipLaunchKernelGGL((k_wide_held<DT, LSE, INLINE>), grid, block, dyn2, stream, r, cfg, w);
+        if (rows * cfg.slices <= WIDE_SIXTEEN_GROUPS) {
+            hipLaunchKernelGGL((k_wide_held<DT, LSE, INLINE, SIXTEEN_THREADS>), grid, dim3(SIXTEEN_THREADS), SIXTEEN_LDS_BYTES, stream, r, cfg, w);
+        } else {
+            hipLaunchKernelGGL((k_wide_held<DT, LSE, INLINE, NT>), grid, block, dyn2, stream, r, cfg, w);
+        }
         return hipGetLastError();
     }
     hipLaunchKernelGGL((k_wide_bound<DT, LSE, INLINE>), grid, block, 0, stream, r, cfg, w);
