@@ -181,7 +181,7 @@ struct LaunchPart {
     bool bitmap_layout = false;
     uint32_t cand_cap = 0;
     bool argmax = false;   // every row is greedy: the kernel that holds nothing else
-    bool wide = false;   // every row draws among many candidates: the two launches of rows_wide.hip
+    bool wide = false;   // every row draws among many candidates: rows_wide.hip
     uint32_t held = 0;   // slices of so many blocks, held in registers (rows_held.hip)
     bool extra = false;  // ... with a mask or a bias list on some row
     bool masked = false; // every row under a mask: a workgroup a row (rows_masked.hip)

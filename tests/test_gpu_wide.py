@@ -1,5 +1,5 @@
 """Rows that draw among many candidates (k > 64; a request without top_k gets the reference's cap
-of 1024, src/kernels/sample.rs:17 and :326-331) through the two launches that spread such a
+of 1024, src/kernels/sample.rs:17 and :326-331) through the launches that spread such a
 row over as many workgroups as a row of few candidates: a bound from the lanes' maxima, then
 the values that reach it.
 
