@@ -539,6 +539,9 @@ __global__ __launch_bounds__(NT, 4) void k_blocks_table(LaunchCfg cfg) {
 
 template <int DT, bool LSE, bool PEN>
 hipError_t launch_blocks(hipStream_t stream, uint32_t rows, const LaunchCfg& cfg) {
+    if (cfg.slices > WAVE_MERGE_LISTS && cfg.slices * cfg.ws_k > WAVE_MERGE_SLOTS) {
+        return hipErrorInvalidValue;   // (more than finish_by_wave() looks at)
+    }
     hipLaunchKernelGGL((k_blocks_table<DT, LSE, PEN>), dim3(cfg.slices, rows), dim3(NT), BLOCKS_LDS_BYTES, stream, cfg);
     return hipGetLastError();
 }

@@ -412,17 +412,20 @@ uint32_t blocks_slices(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint
     if (pen && !s->only_blocks && !(lse && rows <= BLOCKS_GROUPS / 5u)) {
         return 0;
     }
+    const uint32_t e = dtype == LILY_BF16 ? 8 : 4;
+    const uint32_t nch = (vocab + 2 * (e - 1)) / e + 1;
+    uint32_t sl;
     if (rows > BLOCKS_GROUPS / 5u) {
         // (the streaming launches' slices: 280 rows with log-probabilities 43 us in two, 40 in three, without 26.0
         // and 26.5)
-        return choose_slices(s, rows, kmax, vocab, dtype);
+        sl = choose_slices(s, rows, kmax, vocab, dtype);
+    } else {
+        sl = s->force_slices != 0 ? s->force_slices : BLOCKS_GROUPS / rows;
+        const uint32_t by_block = (nch + 256u * STREAM_UNROLL - 1) / (256u * STREAM_UNROLL);   // no finer than a block a slice
+        sl = sl > by_block && s->force_slices == 0 ? by_block : sl;
+        sl = sl > MAX_SLICES ? MAX_SLICES : sl;
     }
-    uint32_t sl = s->force_slices != 0 ? s->force_slices : BLOCKS_GROUPS / rows;
-    const uint32_t e = dtype == LILY_BF16 ? 8 : 4;
-    const uint32_t nch = (vocab + 2 * (e - 1)) / e + 1;
-    const uint32_t by_block = (nch + 256u * STREAM_UNROLL - 1) / (256u * STREAM_UNROLL);   // no finer than a block a slice
-    sl = sl > by_block && s->force_slices == 0 ? by_block : sl;
-    sl = sl > MAX_SLICES ? MAX_SLICES : sl;
+    // (one wave merges a row's slices, whatever their number)
     sl = sl > WAVE_MERGE_LISTS && sl * kmax > HELD_MERGE_SLOTS ? std::max(WAVE_MERGE_LISTS, HELD_MERGE_SLOTS / kmax) : sl;
     const uint64_t by_ws = (uint64_t)s->ws_slots / ((uint64_t)rows * kmax);
     sl = sl > by_ws ? (uint32_t)by_ws : sl;

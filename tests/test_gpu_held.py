@@ -216,3 +216,19 @@ def test_masked_rows_of_many_candidates(monkeypatch, held, bf16, vocab):
         for t in sc:
             t.close()
     s.close()
+
+
+@pytest.mark.parametrize("slices", [40, 64])
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+def test_more_slices_than_a_wave_merges(monkeypatch, bf16, slices):
+    """205 rows a block at a time, k = 64, asked for in more slices than one wave merges (2 048 entries a row):
+    every id of the row can be drawn all the same."""
+    vocab, rows = 131_099, 205
+    rng = np.random.default_rng(slices)
+    x = rng.normal(0, 3, (rows, vocab)).astype(np.float32)
+    x = W.to_bf16_bits(x) if bf16 else x
+    s = _sampler(monkeypatch, "1", slices)
+    kw = [dict(temperature=0.7, top_k=64, top_p=0.97, seed=60 + i) for i in range(rows)]
+    for lp in (False, True):
+        _check(run_rows(s, x, kw, [5] * rows, logprobs=lp, use_plan=True), x, kw, 5, lp)
+    s.close()
