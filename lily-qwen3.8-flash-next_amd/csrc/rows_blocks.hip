@@ -81,7 +81,7 @@ __device__ __forceinline__ bool blocks_row(const LILY_CONST RowArgs* src, const 
         const uint32_t b = min(b_asked, max(nblocks, 1u) - 1u);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            next.raw[u] = gload(reinterpret_cast<const u32x4*>(g.base + (min(chunk_of(b, u), c_last) << 4)));
+            next.raw[u] = gload(reinterpret_cast<const u32x4*>(g.base + (min(chunk_of(b, u), c_last) << 4)));   // (rows are below 4 GiB)
         }
         if (PEN) {
             // (two bytes of the bitmap of listed ids hold a chunk's bits, wherever the row starts)

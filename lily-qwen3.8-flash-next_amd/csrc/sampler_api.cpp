@@ -395,6 +395,9 @@ HeldShape held_shape(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint32
 }
 
 constexpr uint32_t BLOCKS_GROUPS = 1024;
+// Pieces of 16 bytes a row may have there: the kernel counts a row's bytes in 32 bits.  (Longer rows are the exhaustive
+// select's.)
+constexpr uint64_t BLOCKS_MAX_PIECES = 1ull << 28;
 // Workgroups a row where rows without masks and bias lists go a block at a time (rows_blocks.hip); 0: they do not.
 // Up to a fifth of the workgroups that the chip holds at once (four a compute unit) as many as that: workgroups that
 // are not the same number on every compute unit leave some idle (200 rows in 5 slices 53 us, in 3 66), a second
@@ -413,6 +416,9 @@ uint32_t blocks_slices(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint
         return 0;
     }
     const uint32_t e = dtype == LILY_BF16 ? 8 : 4;
+    if (((uint64_t)vocab + 2 * e) / e > BLOCKS_MAX_PIECES) {
+        return 0;
+    }
     const uint32_t nch = (vocab + 2 * (e - 1)) / e + 1;
     uint32_t sl;
     if (rows > BLOCKS_GROUPS / 5u) {

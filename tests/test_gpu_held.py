@@ -232,3 +232,24 @@ def test_more_slices_than_a_wave_merges(monkeypatch, bf16, slices):
     for lp in (False, True):
         _check(run_rows(s, x, kw, [5] * rows, logprobs=lp, use_plan=True), x, kw, 5, lp)
     s.close()
+
+
+def test_row_beyond_four_gibibytes(monkeypatch):
+    """An f32 row of more than 2^30 ids in a plan: its bytes are not counted in 32 bits."""
+    vocab = (1 << 30) + 4099
+    s = _sampler(monkeypatch, "1")
+    x = torch.randn(1, vocab, dtype=torch.float32, device=dev())
+    best = [(1 << 30) + 7, vocab - 1, 5]
+    for at, value in zip(best, (22.0, 21.5, 21.0)):
+        x[0, at] = value
+    out = torch.full((1,), -1, dtype=torch.int32, device=dev())
+    ids = torch.full((1, LS.SAMPLE_K_CAP), -1, dtype=torch.int32, device=dev())
+    torch.cuda.synchronize()
+    plan = s.plan(x, [LS.SamplingParams.greedy(temperature=1.0, top_k=3, top_p=1.0, seed=1)], [0], out, dbg_ids=ids)
+    plan.run(0)
+    s.synchronize()
+    assert ids[0, :3].tolist() == best and out.item() in best
+    plan.close()
+    s.close()
+    del x
+    torch.cuda.empty_cache()
