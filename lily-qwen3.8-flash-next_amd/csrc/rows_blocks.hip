@@ -7,6 +7,12 @@
 // true values, the row's sum takes every value once as it passes, what reaches the bound as it stands is listed
 // with its value, and at the end those that still reach it are ranked; nothing is looked at twice.
 //
+// A block of a dense history (an eighth of the ids and more) lists more than a wave's notes hold: the wave then evaluates
+// them straight from their bits, in a block without a bound once for the bound and once more for the list and the
+// sum.  us a launch, 200 bf16 rows of 151 936, N(0, 2^2), 13 / 25 / 60 % of the ids listed 61 / 77 / 110 (the flat form of
+// select_lowering.h 107 / 136 / 285; given up to the exhaustive select, as such slices once were, 670 to 680), half of the first
+// tenth listed 54 (79).
+//
 // Bound: the vector unit where the row's sum takes most values (200 rows of 248 320 bf16, N(0, 2^2), under penalties
 // 53 us a launch for 99 MB; 76 through the flat form of select_lowering.h, which takes twice the instructions
 // a value and looks at the noted chunks again), the memory where it does not (1 024 rows of 151 936 without
@@ -167,9 +173,18 @@ __device__ __forceinline__ bool blocks_row(const LILY_CONST RowArgs* src, const 
             ref = now;
         }
     };
+    // A listed id's true value, t (NEG_INF in lanes without one), once there is a bound.
+    auto take = [&](float t, uint32_t id) {
+        list(t >= T, t, id);
+        if (LSE && want_lse) {
+            raise(t);
+            const double d = __builtin_fma((double)t, (double)a.c2, -(double)ref);
+            sum += t < T && d > -1000.0 ? pow2_d(d) : 0.0;
+        }
+    };
     // The noted ids, by the wave that noted them, four a lane with all loads in flight.
     auto drain = [&]() {
-        const uint32_t n = min(noted, NOTE_SEG);
+        const uint32_t n = noted;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // (LDS of this wave: in order already)
         __builtin_amdgcn_wave_barrier();
 #pragma unroll 1
@@ -188,17 +203,39 @@ __device__ __forceinline__ bool blocks_row(const LILY_CONST RowArgs* src, const 
                     float t = e0 + (uint32_t)q * 64u + lane < n ? true_value(x[q], count[q]) : NEG_INF;
                     t = t > NEG_INF ? t : NEG_INF;
                     lane_max = fmaxf(lane_max, t);
-                    list(t >= T, t, id[q]);
-                    if (LSE && want_lse) {
-                        raise(t);
-                        const double d = __builtin_fma((double)t, (double)a.c2, -(double)ref);
-                        sum += t < T && d > -1000.0 ? pow2_d(d) : 0.0;
-                    }
+                    take(t, id[q]);
                 }
             }
         }
-        fill = noted > NOTE_SEG ? LIST_SEG + 1u : fill;   // (some were lost: the slice is given up)
         noted = 0u;
+    };
+    // A block's listed ids straight from their bits (E a chunk), where the notes have no room for them; `bounded`: taken,
+    // else looked at for the bound.
+    auto settle = [&](uint32_t b, uint32_t left, bool bounded) {
+#pragma unroll 1
+        while (__ballot(left != 0u) != 0ull) {
+            uint32_t id[4], count[4];
+            float x[4];
+            bool in[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                in[q] = left != 0u;
+                const uint32_t at = in[q] ? (uint32_t)__builtin_ctz(left) : 0u;
+                left &= left - 1u;
+                id[q] = in[q] ? chunk_of(b, (int)(at / (uint32_t)E)) * (uint32_t)E + at % (uint32_t)E - g.pad : 0u;
+                x[q] = load_logit<DT>(a.logits, id[q]);
+                count[q] = gload(a.counts + id[q]);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float t = in[q] ? true_value(x[q], count[q]) : NEG_INF;
+                t = t > NEG_INF ? t : NEG_INF;
+                lane_max = fmaxf(lane_max, t);
+                if (bounded) {
+                    take(t, id[q]);
+                }
+            }
+        }
     };
     // (One copy of the loop's code, each block's registers handed over by moves: three copies, for two blocks on
     // their way, left the instruction cache and were the slower way at every size.)
@@ -251,10 +288,13 @@ __device__ __forceinline__ bool blocks_row(const LILY_CONST RowArgs* src, const 
         // Listed ids leave the chunks whose raw values might matter (their true ones lie no higher, where
         // penalties only lower) and are noted, to be evaluated by the hundred.  In the other chunks, which
         // reach neither the bound nor the cut, they may stay.
+        uint32_t crowd = 0u;
         if (PEN && pen) {
+            const uint32_t noted_before = noted;
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                uint32_t left = raising || cm[u] >= low ? away[u] : 0u;
+                away[u] = raising || cm[u] >= low ? away[u] : 0u;
+                uint32_t left = away[u];
                 uint64_t mask = __ballot(left != 0u);
                 if (mask != 0ull) {
                     cur[u] = chunk_without<DT>(cur[u], left);
@@ -270,6 +310,17 @@ __device__ __forceinline__ bool blocks_row(const LILY_CONST RowArgs* src, const 
                     } while (mask != 0ull);
                 }
             }
+            if (noted > NOTE_SEG) {
+                // (a dense history: the wave goes by the block's bits)
+                noted = noted_before;
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    crowd |= away[u] << (u * E);
+                }
+                if (T == F32_LOWEST) {
+                    settle(b, crowd, false);
+                }
+            }
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -283,6 +334,9 @@ __device__ __forceinline__ bool blocks_row(const LILY_CONST RowArgs* src, const 
         if (PEN) {
             if (pen && (noted > NOTE_SEG / 2u || b + 1u == nblocks)) {
                 drain();
+            }
+            if (__ballot(crowd != 0u) != 0ull) {
+                settle(b, crowd, true);
             }
             if (b + 1u == nblocks) {
                 refresh();

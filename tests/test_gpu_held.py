@@ -253,3 +253,46 @@ def test_row_beyond_four_gibibytes(monkeypatch):
     s.close()
     del x
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+@pytest.mark.parametrize("raising", [False, True], ids=["lowering", "raising"])
+def test_dense_histories_stay_a_block_at_a_time(monkeypatch, bf16, raising):
+    """Rows of which a twentieth to all of the ids are listed, spread evenly or crowded into the first tenth of the
+    vocabulary (where a tokenizer puts what is frequent): no slice is given up to the exhaustive select."""
+    vocab = 131_099
+    shares = [0.05, 0.1, 0.12, 0.13, 0.16, 0.2, 0.24, 0.25, 0.3, 0.4, 0.6, 1.0]
+    crowded = [0.3, 0.6, 0.9, 1.0]   # of the first tenth
+    rows = len(shares) + len(crowded)
+    rng = np.random.default_rng(8)
+    x = rng.normal(0, 2, (rows, vocab)).astype(np.float32)
+    x = W.to_bf16_bits(x) if bf16 else x
+    counts = np.zeros((rows, vocab), dtype=np.uint32)
+    for i, share in enumerate(shares + crowded):
+        n = vocab if i < len(shares) else vocab // 10
+        counts[i, rng.choice(n, int(share * n), replace=False)] = 1
+        counts[i, rng.integers(0, n, 200)] += 1
+    s = _sampler(monkeypatch, "blocks", 5)
+    scratch = []
+    for i in range(rows):
+        t = LS.SamplerScratch(s, vocab)
+        t.add_history(torch.from_numpy(np.repeat(np.arange(vocab, dtype=np.int32), counts[i])).to(dev()))
+        scratch.append(t)
+    stats = torch.zeros(4, dtype=torch.int32, device=dev())
+    pen = (dict(repetition_penalty=0.95, presence_penalty=-0.1, frequency_penalty=0.0625) if raising else
+           dict(repetition_penalty=1.05, presence_penalty=0.25, frequency_penalty=0.125))
+    for k in (20, 64):
+        for lp in (True, False):
+            kw = [dict(temperature=0.8, top_k=k, top_p=0.95, seed=7 + i, **pen) for i in range(rows)]
+            stats.zero_()
+            torch.cuda.synchronize()
+            s.set_path_stats(stats)
+            r = run_rows(s, x, kw, [3] * rows, scratch=scratch, logprobs=lp, use_plan=True)
+            s.set_path_stats(None)
+            _check(r, x, kw, 3, lp, counts)
+            assert stats.cpu().tolist()[:3] == [5 * rows, 0, 0], (k, lp)
+            for i in range(rows):   # (the oracle counted its draw)
+                assert np.array_equal(scratch[i].read_counts().numpy(), counts[i]), i
+    for t in scratch:
+        t.close()
+    s.close()
