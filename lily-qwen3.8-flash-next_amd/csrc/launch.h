@@ -147,8 +147,14 @@ hipError_t launch_rows_masked(hipStream_t stream, int dtype, bool lse, uint32_t 
 // launches (the row's bound, then the values that reach it, merge, select, tail).
 // lane_max [rows][slices][256]; count [rows] and bounds [2][rows][MAX_SLICES], both 0 between launches (bounds: for the
 // one launch that small batches take instead).
+// `looks`: how often a slice of that launch looks for the words of its row's other slices, in either of its waits,
+// before it leaves the row to the exhaustive select.
+struct WideLooks {
+    uint32_t keys = 1u << 13, maxima = 1u << 13;
+};
 hipError_t launch_rows_wide(hipStream_t stream, int dtype, bool lse, uint32_t rows, const LaunchCfg& cfg,
-                            const InlineRows* inline_rows, float* lane_max, uint32_t* count, uint64_t* bounds);
+                            const InlineRows* inline_rows, float* lane_max, uint32_t* count, uint64_t* bounds,
+                            const WideLooks& looks);
 // `bytes` (a multiple of 16) from pinned host memory, mapped into the device at src, to dst.
 hipError_t launch_copy_pieces(hipStream_t stream, const void* src, void* dst, size_t bytes);
 // The same of up to sizeof(PlacedPieces) bytes from any host memory, through the launch's arguments.

@@ -21,6 +21,7 @@
 #define LILY_TAIL_TRACE
 #endif
 
+#include "launch.h"
 #include "row_kernel.h"
 #include "sort_sixteen.h"
 
@@ -44,6 +45,7 @@ struct WideArgs {
     // (0 between launches); null: two launches
     uint64_t* bounds;
     uint32_t* count;      // [rows] candidates the row's slices have left so far (0 between launches)
+    WideLooks looks;
 };
 
 template <bool INLINE>
@@ -508,9 +510,9 @@ __global__ __launch_bounds__(NT, 4) void k_wide_draw(InlineRows rows_arg, Launch
 
 // What the two launches do below, without reading the slice again and without a second launch: each slice leaves its
 // bound where the row's other slices look for it, and forms its sum of exponentials meanwhile.  A slice that
-// does not find them all within WIDE_TRIES looks (another stream's work holds the chip) gives up, and the row is taken by the
+// does not find them all within WideArgs::looks (another stream's work holds the chip) gives up, and the row is taken by the
 // exhaustive select: every wait ends.
-constexpr uint32_t WIDE_TRIES = 1u << 13, WIDE_HELD_GROUPS = 1024;
+constexpr uint32_t WIDE_HELD_GROUPS = 1024;
 // Up to so many workgroups are of sixteen waves each, a piece of 16 bytes a thread, and sort with all of them (1 f32 row of
 // 151 936 23.2 -> 19.8 us, under penalties 24.2 -> 20.5, 4 rows of 32 000 23.1 -> 20.8); launching four times the waves
 // takes that back at 152 (4 rows 24.4 both ways, 13 rows 31.9 -> 35.9).
@@ -690,18 +692,18 @@ __global__ __launch_bounds__(THREADS, 4) void k_wide_held(InlineRows rows_arg, L
     }
     WIDE_MARK(2);
     // ---- the row's bound, once all its slices' words are there (a word is the message: nothing else is read for it)
-    auto wait_for = [&](const uint64_t* words) {
+    auto wait_for = [&](const uint64_t* words, uint32_t looks) {
         if (tid < 64u) {   // (the first wave looks)
             uint64_t keys = 0;
             for (uint32_t tries = 0;; ++tries) {
-                keys = lane < S ? load_through(words + lane) : ~0ull;
-                if (__ballot(keys == 0ull) == 0ull) {
-                    break;
-                }
-                if (tries == WIDE_TRIES) {
+                if (tries == looks) {
                     if (lane == 0u) {
                         lost = 1u;
                     }
+                    break;
+                }
+                keys = lane < S ? load_through(words + lane) : ~0ull;
+                if (__ballot(keys == 0ull) == 0ull) {
                     break;
                 }
                 __builtin_amdgcn_s_sleep(1);
@@ -713,7 +715,7 @@ __global__ __launch_bounds__(THREADS, 4) void k_wide_held(InlineRows rows_arg, L
         }
         __syncthreads();
     };
-    wait_for(bounds);
+    wait_for(bounds, w.looks.keys);
     float bound = row_bound;
     if (lost == 0u && !(bound > F32_LOWEST)) {
         // (the same in all the row's workgroups) Most of the row is -inf: too many waves had no value to name.  The lanes'
@@ -727,7 +729,7 @@ __global__ __launch_bounds__(THREADS, 4) void k_wide_held(InlineRows rows_arg, L
         if (tid == 0) {
             __hip_atomic_store(handed + s, (uint64_t)1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
         }
-        wait_for(handed);
+        wait_for(handed, w.looks.maxima);
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         uint32_t T = 0;
         for (uint32_t t = 0x8000u; t != 0u && lost == 0u; t >>= 1) {
@@ -806,7 +808,8 @@ static hipError_t launch_wide_variant(hipStream_t stream, uint32_t rows, const L
 }
 
 hipError_t launch_rows_wide(hipStream_t stream, int dtype, bool lse, uint32_t rows, const LaunchCfg& cfg_in,
-                            const InlineRows* inline_rows, float* lane_max, uint32_t* count, uint64_t* bounds) {
+                            const InlineRows* inline_rows, float* lane_max, uint32_t* count, uint64_t* bounds,
+                            const WideLooks& looks) {
     LaunchCfg cfg = cfg_in;
     // the merging workgroup's candidates, then the tail's arrays behind the first K_CAP of them
     cfg.dyn_slots = MERGE_CAP;
@@ -816,6 +819,7 @@ hipError_t launch_rows_wide(hipStream_t stream, int dtype, bool lse, uint32_t ro
     w.slice_keys = Handed<uint64_t>{reinterpret_cast<uint64_t*>(lane_max + (size_t)rows * cfg.slices * NT)};   // (behind the lanes' maxima)
     w.lanes = (uint64_t)cfg.slices * (NT / 2) >= 4ull * cfg.ws_k ? NT / 2 : NT;
     w.count = count;
+    w.looks = looks;
     // One launch where every slice is held in registers, wherever its row starts, and the launch's workgroups are all on
     // the chip at once (four a compute unit: they wait for each other).
     const uint32_t e = dtype == LILY_BF16 ? 8u : 4u, nch = (cfg.vocab + 2u * (e - 1u)) / e;

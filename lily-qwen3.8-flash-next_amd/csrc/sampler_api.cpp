@@ -124,6 +124,9 @@ struct lily_sampler {
     uint32_t force_path = 0;
     uint32_t force_slices = 0;
     bool no_wide = false;   // LILY_SAMPLER_WIDE=0: rows of many candidates go the other kernels' way
+    // LILY_SAMPLER_WIDE_LOOKS="keys,maxima,launches": the waits of that many launches of such rows (WideLooks)
+    WideLooks wide_looks;
+    uint32_t wide_looks_launches = 0;
     // LILY_SAMPLER_HELD: "0" = no slices held in registers (rows_held.hip, rows_blocks.hip), "blocks" = every
     // row that can goes a block at a time
     bool no_held = false, only_blocks = false;
@@ -551,6 +554,14 @@ uint32_t wide_slices(const lily_sampler* s, const RowArgs* rows, uint32_t n, int
     return sl;
 }
 
+WideLooks looks_of_launch(lily_sampler* s) {
+    if (s->wide_looks_launches == 0) {
+        return WideLooks();
+    }
+    --s->wide_looks_launches;
+    return s->wide_looks;
+}
+
 // Attaches the phase trace when the launch fits the caller's buffer.
 void attach_trace(const lily_sampler* s, LaunchCfg* cfg, uint32_t rows) {
     if (s->phase_trace != nullptr &&
@@ -720,7 +731,7 @@ int launch_part(lily_sampler* s, const LaunchPart& part, const RowArgs* table_de
     }
     if (part.wide) {
         HIP_TRY(launch_rows_wide(s->stream, dtype, part.lse, part.rows, cfg, nullptr, s->wide_max,
-                                 s->wide_count, s->wide_bounds));
+                                 s->wide_count, s->wide_bounds, looks_of_launch(s)));
         return LILY_OK;
     }
     if (part.masked && served == nullptr) {
@@ -762,7 +773,7 @@ int launch_inline(lily_sampler* s, int dtype, uint32_t vocab, const InlineRows& 
                 lse = lse || rows.r[i].out_logprob != nullptr;
             }
             HIP_TRY(launch_rows_wide(s->stream, dtype, lse, n, cfg, &rows, s->wide_max, s->wide_count,
-                                     s->wide_bounds));
+                                     s->wide_bounds, looks_of_launch(s)));
             return LILY_OK;
         }
     }
@@ -1154,6 +1165,11 @@ int lily_sampler_create(int device, void* hip_stream, lily_sampler_t** out) {
     }
     if (const char* p = std::getenv("LILY_SAMPLER_WIDE")) {
         s->no_wide = std::atoi(p) == 0;
+    }
+    if (const char* p = std::getenv("LILY_SAMPLER_WIDE_LOOKS")) {
+        if (std::sscanf(p, "%u,%u,%u", &s->wide_looks.keys, &s->wide_looks.maxima, &s->wide_looks_launches) != 3) {
+            s->wide_looks_launches = 0;
+        }
     }
     if (const char* p = std::getenv("LILY_SAMPLER_HELD")) {
         s->only_blocks = std::strcmp(p, "blocks") == 0;

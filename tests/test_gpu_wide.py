@@ -294,6 +294,33 @@ def test_bounds_over_the_slices(sampler, rows, vocab, bf16):
         _check_logprob(r.logprobs[i], d.logprob, i)
 
 
+@pytest.mark.parametrize("looks", ["0,8192", "8192,0", "1,1"], ids=["no key", "no maxima", "one look"])
+@pytest.mark.parametrize("rows,bf16", [(2, False), (6, False), (6, True), (20, True)])
+def test_slices_that_stop_waiting_for_each_other(monkeypatch, rows, bf16, looks):
+    """A launch whose slices look for the words of their rows' other slices never, or once, in either wait (the second one
+    belongs to rows with too many waves of -inf), in workgroups of sixteen waves (up to 128 of them) and of four: the rows go to the
+    exhaustive select, and the next launch of the same sampler finds every word as it has to be."""
+    vocab = 151_937
+    rng = np.random.default_rng(rows + bf16)
+    x = rng.normal(0, 2, (rows, vocab)).astype(np.float32)
+    x[1::2, :vocab // 4] = -np.inf
+    x[1::2, vocab // 4 + vocab // 2:] = -np.inf
+    x = W.to_bf16_bits(x) if bf16 else x
+    kw = [dict(temperature=0.8, top_k=0, top_p=0.97, seed=40 + r) for r in range(rows)]
+    monkeypatch.setenv("LILY_SAMPLER_WIDE_LOOKS", looks + ",1")
+    s = LS.Sampler(0)
+    gave_up = {"0,8192": (rows, rows), "8192,0": (rows // 2, rows // 2), "1,1": (0, rows)}[looks]
+    for launch, (least, most) in enumerate((gave_up, (0, 0), (0, 0))):
+        xs = x if launch < 2 else np.roll(x, 1, axis=0)   # (the rows that are half -inf change places with the others)
+        r, stats = _with_stats(s, lambda: run_rows(s, xs, kw, [launch] * rows, logprobs=True, use_plan=rows > 8))
+        assert stats[0] == 0 and stats[1] + stats[2] == rows and least <= stats[2] <= most, (launch, stats)
+        for i in range(rows):
+            d = O.sample(xs[i], None, o_params(**kw[i]), launch, want_logprob=True)
+            check_row_against_oracle(r, i, d)
+            _check_logprob(r.logprobs[i], d.logprob, (launch, i))
+    s.close()
+
+
 @pytest.mark.parametrize("masked", [False, True], ids=["two-launches", "merged-slices"])
 @pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
 def test_sort_of_many_candidates(sampler, bf16, masked):
