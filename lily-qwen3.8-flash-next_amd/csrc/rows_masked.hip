@@ -1,16 +1,23 @@
 // rows_masked.hip - rows under an allow-mask, a workgroup of 1 024 threads a row.  Compiled once per logits
 // type: -DLILY_DT=0|1.
 //
-// A grammar admits some per cent of the vocabulary, in clusters, and such rows name no top_k as a rule: 3 000
+// A grammar admits some per cent of the vocabulary, and such rows name no top_k as a rule: 3 000
 // ids to evaluate, 1 024 of them to sort.  That is a chain of latencies, not work to be spread: cut into
 // four slices of 256 threads each row paid for a hand-over, a second gathering and a sort by one wave a
 // SIMD (64 rows of 151 936 bf16, 2 % admitted: slices done 16 us, ticket 18, sorted 27, drawn 36).  Here
-// sixteen waves list the mask's words that admit anything, evaluate them a word for every 32 lanes (a run of
-// ids is one request), sort in LDS, and the first four waves draw.
+// sixteen waves read the mask, evaluate what it admits, sort in LDS, and the first four waves draw.
 //
-// A mask that admits more ids than the sort holds (8 192) is taken by the same kernel: histograms over the
-// composites' leading bits, every value evaluated anew for each, until what reaches the k-th one's bin fits.  One that
-// admits a third of the vocabulary is left to the launch behind, which streams the row.
+// Ids that lie scattered are listed one by one and evaluated a lane each.  Where they lie in clusters (12 and more to
+// a word that admits any) the words are listed, 32 lanes a word: a run of ids is one request, and nobody lists them.
+// (us a launch, bf16, 151 936 ids, 2 % admitted, by words -> by ids: one by one 1 row 62 -> 23, 64 rows 63 -> 24, in runs of up to 4 / 16
+// ids 41 -> 23 / 28 -> 26, of up to 64 23 -> 26.  Each thread's words lie 1 024 apart, or a cluster would be one
+// thread's to list.)
+//
+// A mask that admits more ids than the sort holds (8 192), in clusters, is taken by the same kernel: histograms over the
+// composites' leading bits, every value evaluated anew for each, until what reaches the k-th one's bin fits.  Others, and
+// those of more words than that pays for, are left to the launch behind, which streams the row (us, this way / left /
+// by that launch alone: 64 rows of 151 936 bf16 in runs of up to 64, 10 % 50 / 74 / 68, 20 % 74 / 91 / 81; all of 49 152 ids
+// 70 / 65 / 59, of 32 000 54 / 61 / 55).
 #include "launch.h"
 #include "row_kernel.h"
 #include "sort_sixteen.h"
@@ -26,12 +33,15 @@ namespace {
 constexpr uint32_t MT = SIXTEEN_THREADS, MWAVE = SIXTEEN_WAVES;
 constexpr uint32_t MASKED_WORDS = MASKED_MAX_VOCAB / 32u, WORDS_PER = MASKED_WORDS / MT;
 constexpr uint32_t MASKED_CAP = 8192;      // values that are sorted
-constexpr uint32_t MASKED_DENSE = 49152;   // ids a mask may admit
+constexpr uint32_t MASKED_CLUSTERED = 12;  // ids a word of a mask in clusters, on average
+// Words that may admit ids where there are more than the sort holds: 0.031 us each, against some 46 us and 0.2 for every
+// 1 000 ids of the row by the launch behind (one row to 64).
+__device__ __forceinline__ uint32_t masked_most_words(uint32_t vocab) { return 800u + vocab / 150u; }
 constexpr uint32_t MBINS = SIXTEEN_BINS;   // of the sort
 constexpr uint32_t HBINS = 4096;           // of the histograms, 12 bits
 // Dynamic LDS in 64-bit slots: the sorted candidates and the tail's arrays; the sort's bins; the values as they
 // come (the histograms, before there are any); the words that admit anything (bits, number), and where those are
-// done with the values by bins.
+// done with the values by bins.  (A list of ids lies where the words would.)
 constexpr uint32_t OFF_BINS = (LILY_SAMPLE_K_CAP * 8 + 3 * LILY_SAMPLE_K_CAP * 4) / 8;
 constexpr uint32_t OFF_MIXED = OFF_BINS + MBINS / 2;
 constexpr uint32_t OFF_PLACED = OFF_MIXED + MASKED_CAP;
@@ -72,12 +82,13 @@ __device__ __forceinline__ void masked_row(const LILY_CONST RowArgs* src, const 
     uint32_t* hist = reinterpret_cast<uint32_t*>(mixed);
     uint32_t* word_bits = reinterpret_cast<uint32_t*>(placed);
     uint16_t* word_at = reinterpret_cast<uint16_t*>(word_bits + MASKED_WORDS);
+    uint32_t* id_list = reinterpret_cast<uint32_t*>(placed);
 
-    // ---- the words that admit anything, in order
+    // ---- what the mask admits: its words, or its ids
     uint32_t bits[WORDS_PER], some = 0, admitted = 0;
 #pragma unroll
     for (uint32_t i = 0; i < WORDS_PER; ++i) {
-        bits[i] = gload(a.allow + min(tid * WORDS_PER + i, words - 1u));
+        bits[i] = gload(a.allow + min(i * MT + tid, words - 1u));
     }
     if (tid == 0) {
         tail_arrays(sh);
@@ -93,29 +104,40 @@ __device__ __forceinline__ void masked_row(const LILY_CONST RowArgs* src, const 
     }
 #pragma unroll
     for (uint32_t i = 0; i < WORDS_PER; ++i) {
-        const uint32_t at = tid * WORDS_PER + i;
+        const uint32_t at = i * MT + tid;
         bits[i] = at < words ? bits[i] & range32_at(0u, vocab, (int64_t)at * 32) : 0u;
         some += bits[i] != 0u ? 1u : 0u;
         admitted += (uint32_t)__popc(bits[i]);
     }
     uint32_t n_words, total;
     uint32_t place = scan_all(some, ms.six, n_words) - some;
-    scan_all(admitted, ms.six, total);
+    const uint32_t id_place = scan_all(admitted, ms.six, total) - admitted;
     if (tid < n_bias && ms.bias_id[tid] < vocab) {
         const uint32_t at = ms.bias_id[tid] >> 5;
         atomicOr(&ms.biased[at >> 5], 1u << (at & 31u));
     }
+    const bool scattered = total < n_words * MASKED_CLUSTERED, listed = scattered && total <= MASKED_CAP;
+    if (listed) {
+        uint32_t to = id_place;
 #pragma unroll
-    for (uint32_t i = 0; i < WORDS_PER; ++i) {
-        if (bits[i] != 0u) {
-            word_bits[place] = bits[i];
-            word_at[place] = (uint16_t)(tid * WORDS_PER + i);
-            ++place;
+        for (uint32_t i = 0; i < WORDS_PER; ++i) {
+            for (uint32_t left = bits[i]; left != 0u; left &= left - 1u) {
+                id_list[to++] = (i * MT + tid) * 32u + (uint32_t)__builtin_ctz(left);
+            }
+        }
+    } else {
+#pragma unroll
+        for (uint32_t i = 0; i < WORDS_PER; ++i) {
+            if (bits[i] != 0u) {
+                word_bits[place] = bits[i];
+                word_at[place] = (uint16_t)(i * MT + tid);
+                ++place;
+            }
         }
     }
     __syncthreads();
-    // Dense masks are better streamed by many workgroups: the launch behind this one takes those rows.
-    const bool served = total <= MASKED_DENSE;
+    // Dense masks are better streamed by many workgroups.
+    const bool served = total <= MASKED_CAP || (!scattered && n_words <= masked_most_words(vocab));
     if (tid == 0) {
         cfg.masked_served[blockIdx.y] = served ? 1u : 0u;
     }
@@ -124,7 +146,21 @@ __device__ __forceinline__ void masked_row(const LILY_CONST RowArgs* src, const 
     }
     phase(cfg, 1);
 
-    // fn(value before the temperature, id, whether there is one) over every admitted id: 32 lanes a word,
+    // An admitted value before the temperature.
+    auto worth = [&](float u, uint32_t id, bool biased, uint32_t count) -> float {
+        if (__ballot(biased) != 0ull) {
+            for (uint32_t j = 0; j < n_bias; ++j) {   // (pairs of one id in the list's order)
+                u = ms.bias_id[j] == id ? u + ms.bias_delta[j] : u;
+            }
+        }
+        if (count > 0u) {
+            u = u > 0.0f ? u / a.repetition : u * a.repetition;
+            u -= a.presence + a.frequency * (float)count;
+        }
+        return u;
+    };
+    auto has_bias = [&](uint32_t word) -> bool { return n_bias != 0u && ((ms.biased[word >> 5] >> (word & 31u)) & 1u) != 0u; };
+    // fn(that value, id, whether there is one) over every admitted id: 32 lanes a word,
     // eight words' loads in flight.
     auto over_admitted = [&](auto&& fn) {
         constexpr uint32_t R = 8;
@@ -138,7 +174,7 @@ __device__ __forceinline__ void masked_row(const LILY_CONST RowArgs* src, const 
                 const uint32_t at = word_at[min(i, n_words - 1u)];
                 in[r] = i < n_words && ((word_bits[min(i, n_words - 1u)] >> (tid & 31u)) & 1u) != 0u;
                 id[r] = min(at * 32u + (tid & 31u), vocab - 1u);
-                biased[r] = n_bias != 0u && ((ms.biased[at >> 5] >> (at & 31u)) & 1u) != 0u;
+                biased[r] = has_bias(at);
                 x[r] = load_logit<DT>(a.logits, id[r]);
                 count[r] = pen ? gload(a.counts + id[r]) : 0u;
             }
@@ -147,24 +183,33 @@ __device__ __forceinline__ void masked_row(const LILY_CONST RowArgs* src, const 
                 if (i0 + r * (MT / 32u) >= n_words) {
                     break;
                 }
-                float u = x[r];
-                if (__ballot(biased[r]) != 0ull) {
-                    for (uint32_t j = 0; j < n_bias; ++j) {   // (pairs of one id in the list's order)
-                        u = ms.bias_id[j] == id[r] ? u + ms.bias_delta[j] : u;
-                    }
-                }
-                if (count[r] > 0u) {
-                    u = u > 0.0f ? u / a.repetition : u * a.repetition;
-                    u -= a.presence + a.frequency * (float)count[r];
-                }
-                fn(u, id[r], in[r]);
+                fn(worth(x[r], id[r], biased[r], count[r]), id[r], in[r]);
             }
+        }
+    };
+    // The same over the listed ids, a lane each, all their loads in flight.
+    auto over_listed = [&](auto&& fn) {
+        constexpr uint32_t R = MASKED_CAP / MT;
+        uint32_t id[R], count[R];
+        float x[R];
+#pragma unroll
+        for (uint32_t r = 0; r < R; ++r) {
+            id[r] = id_list[min(r * MT + tid, total - 1u)];
+            x[r] = load_logit<DT>(a.logits, id[r]);
+            count[r] = pen ? gload(a.counts + id[r]) : 0u;
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < R; ++r) {
+            if (r * MT >= total) {
+                break;
+            }
+            fn(worth(x[r], id[r], has_bias(id[r] >> 5), count[r]), id[r], r * MT + tid < total);
         }
     };
     LseAcc lse;
     lse.init();
-    auto collect = [&](uint64_t least, bool sum) {
-        over_admitted([&](float u, uint32_t id, bool in) {
+    auto collect = [&](auto&& over, uint64_t least, bool sum) {
+        over([&](float u, uint32_t id, bool in) {
             if (sum && in) {
                 lse.add_one(u, a.c2);
             }
@@ -183,8 +228,12 @@ __device__ __forceinline__ void masked_row(const LILY_CONST RowArgs* src, const 
             }
         });
     };
-    if (total <= MASKED_CAP || forced) {
-        collect(0ull, LSE && want_lse);
+    if (listed) {
+        if (total != 0u) {   // (the same in every thread)
+            collect(over_listed, 0ull, LSE && want_lse);
+        }
+    } else if (total <= MASKED_CAP || forced) {
+        collect(over_admitted, 0ull, LSE && want_lse);
     } else {
         // The bin of the k-th composite, twelve bits at a time from the top, until what lies at or above it fits.
         uint64_t prefix = 0ull;
@@ -237,7 +286,7 @@ __device__ __forceinline__ void masked_row(const LILY_CONST RowArgs* src, const 
             }
         }
         __syncthreads();
-        collect(prefix, false);
+        collect(over_admitted, prefix, false);
     }
     phase(cfg, 2);
     if (LSE && want_lse) {

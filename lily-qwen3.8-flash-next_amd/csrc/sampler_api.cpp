@@ -458,11 +458,13 @@ HeldRows held_rows(const RowArgs* rows, uint32_t n) {
 }
 
 constexpr uint32_t MASKED_MAX_ROWS = 256;
-// Whether a launch goes a workgroup a row over the masks' words first (rows_masked.hip): where rows draw among
-// many candidates, and a workgroup a row fills the chip no more than once.  (bf16, 151 936 ids, no top_k, us, before ->
-// now: 2 % admitted 1 row 28.1 -> 24.7, 64 rows 36.3 -> 28.3; a tenth of that 24.8 -> 18.2, 28.5 -> 19.7; ten times as much 71 ->
-// 75, 1 819 -> 86; all of them, which the launch behind takes, 74.7 -> 81.2, 89.9 -> 97.8.  For k <= 64 the
-// streaming selects make less of the difference: 64 rows 21.8 -> 19.8, all ids admitted 32 -> 39.)
+// Whether a launch goes a workgroup a row over the masks first (rows_masked.hip): where rows draw among
+// many candidates, and a workgroup a row fills the chip no more than once.  (bf16, 151 936 ids, no top_k, 1 row / 64, us, the
+// other kernels -> now.  In runs of up to 64 ids: 0.2 % admitted 22.3 / 26.2 -> 15.9 / 16.6, 2 % 26.2 / 33.1 -> 22.7 / 24.8, 10 % 65 / 68
+// -> 48 / 50, 20 % 69 / 81 -> 72 / 74.  One by one: 0.2 % 22.2 / 26.7 -> 15.8 / 16.6, 2 % 25.4 / 29.8 -> 23.0 / 23.7, 5 % 32.3 /
+// 36.9 -> 32.2 / 33.9.  Rows that are left to the launch behind pay for the look at the mask: 10 % one by one 36.7 / 40.6 ->
+// 42.0 / 47.1, all ids 74 / 83 -> 80 / 92.  For k <= 64 the streaming selects make less of the difference: 64 rows
+// 21.8 -> 19.8, all ids admitted 32 -> 39.)
 bool all_masked(const lily_sampler* s, const RowArgs* rows, uint32_t n, uint32_t vocab, uint32_t kmax) {
     if (kmax <= STREAM_K_MAX || n > MASKED_MAX_ROWS || s->masked_served == nullptr || n > s->ws_rows || s->force_path != 0 ||
         s->no_held || (s->force_slices != 0 && !s->only_blocks) || vocab > MASKED_MAX_VOCAB) {

@@ -218,6 +218,36 @@ def test_masked_rows_of_many_candidates(monkeypatch, held, bf16, vocab):
     s.close()
 
 
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+@pytest.mark.parametrize("vocab", [9001, 70_001, 262_144])
+@pytest.mark.parametrize("run", [1, 96], ids=["one by one", "in runs"])
+def test_masks_that_scatter_and_masks_that_cluster(monkeypatch, bf16, vocab, run):
+    """Masks of a few ids, just what the sort holds and one more, twice that, and as many words as the rule for
+    clusters takes and some more; scattered ids and runs; equal values by the thousand, a row of -inf, NaN."""
+    rng = np.random.default_rng(vocab + run)
+    x = _rows(rng, vocab, False)
+    xs = W.to_bf16_bits(x) if bf16 else x
+    words = (vocab + 31) // 32
+    allow = np.zeros((ROWS, words), dtype=np.uint32)
+    most = 32 * (800 + vocab // 150)
+    for i, n in enumerate((3, 8191, 8192, 8193, 16_384, most - 64, most + 64, 1200)):
+        n = min(n, vocab)
+        if run == 1:
+            ids = rng.choice(vocab, n, replace=False)
+        else:
+            starts = np.sort(rng.choice(vocab // run, min(-(-n // run), vocab // run), replace=False)) * run
+            ids = (starts[:, None] + np.arange(run)).ravel()[:n]
+        np.bitwise_or.at(allow[i], ids >> 5, (1 << (ids & 31)).astype(np.uint32))
+    bias = [[(int(i), float(d)) for i, d in zip(rng.integers(0, vocab, 30), rng.choice([-5.0, 5.0, 0.5], 30))]
+            for _ in range(ROWS)]
+    s = _sampler(monkeypatch, "1")
+    for trial, lp in enumerate((True, False)):
+        kw = [dict(temperature=0.8, top_k=0 if trial == 0 else 200, top_p=0.95, seed=9 + i) for i in range(ROWS)]
+        r = run_rows(s, xs, kw, [trial] * ROWS, logprobs=lp, allow=allow, bias=bias, use_plan=trial == 1)
+        _check(r, xs, kw, trial, lp, allow=allow, bias=bias)
+    s.close()
+
+
 @pytest.mark.parametrize("slices", [40, 64])
 @pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
 def test_more_slices_than_a_wave_merges(monkeypatch, bf16, slices):
