@@ -146,6 +146,7 @@ __device__ __forceinline__ uint64_t slice_keys_of(float lane_max, uint32_t k, ui
     return tid != 0u ? 0ull : ((uint64_t)(sh.hist[3] << 16 | sh.hist[2]) << 32) | (sh.hist[1] << 16 | sh.hist[0]);
 }
 // Of the keys that lane l of a wave has of slice l (0 past the last); F32_LOWEST: too many waves had none to name.
+// (A little lower than the keys: values that share the bound's quotient by the temperature rank with it.)
 __device__ __forceinline__ float bound_of_keys(uint64_t keys, uint32_t k, uint32_t S) {
     const uint32_t r = wide_rank(k, S), need = (k + r - 1u) / r;
     uint32_t T = 0;
@@ -159,7 +160,7 @@ __device__ __forceinline__ float bound_of_keys(uint64_t keys, uint32_t k, uint32
         }
         T = n >= need ? t : T;
     }
-    return T > WIDE_LEAST_KEY ? lilym_key_value(T << 16) : F32_LOWEST;
+    return T > WIDE_LEAST_KEY ? lower_by_slack(lilym_key_value(T << 16)) : F32_LOWEST;
 }
 
 // ---- first launch: lane maxima, the slice's sum of exponentials
@@ -318,7 +319,7 @@ __device__ __forceinline__ float wide_bound_of(const WideArgs& w, uint32_t row, 
         }
         __syncthreads();
     }
-    return enough ? lilym_key_value(prefix) : F32_LOWEST;
+    return enough ? lower_by_slack(lilym_key_value(prefix)) : F32_LOWEST;
 }
 
 // Dynamic LDS of sixteen waves, in 64-bit slots: the sorted candidates and the tail's arrays; the sort's bins; a slice's
@@ -757,7 +758,7 @@ __global__ __launch_bounds__(THREADS, 4) void k_wide_held(InlineRows rows_arg, L
             T |= sh.hist[0] >= a.k ? t : 0u;
             __syncthreads();
         }
-        bound = T > WIDE_LEAST_KEY ? lilym_key_value(T << 16) : F32_LOWEST;
+        bound = T > WIDE_LEAST_KEY ? lower_by_slack(lilym_key_value(T << 16)) : F32_LOWEST;
     }
     WIDE_MARK(5);
     uint64_t* cand = THREADS == NT ? dyn_lds : dyn_lds + SIXTEEN_OFF_PLACED;

@@ -321,6 +321,27 @@ def test_slices_that_stop_waiting_for_each_other(monkeypatch, rows, bf16, looks)
     s.close()
 
 
+@pytest.mark.parametrize("rows", [1, 4, 40], ids=["sixteen waves", "one launch", "two launches"])
+def test_values_that_share_a_quotient(sampler, rows):
+    """Thousands of ids at 1.75 and at the float below it, whose quotients by the temperature are the same: the ids decide,
+    whichever value the bound is."""
+    vocab = 151_936
+    rng = np.random.default_rng(rows)
+    value, temperature = np.float32(1.75), np.float32(0.75)
+    below = np.nextafter(value, np.float32(0))
+    assert value / temperature == below / temperature
+    x = rng.random((rows, vocab)).astype(np.float32) * np.float32(0.5)
+    at = np.sort(rng.choice(vocab, 3600, replace=False))
+    x[:, at[::2]], x[:, at[1::2]] = below, value
+    if rows > 1:
+        x[-1, at] = np.where(np.arange(3600) < 1800, below, value)
+    kw = [dict(temperature=0.75, top_k=0, top_p=1.0, seed=8 + r) for r in range(rows)]
+    r, stats = _with_stats(sampler, lambda: run_rows(sampler, x, kw, [3] * rows))
+    assert stats[0] == 0 and stats[1] == rows and stats[2] == 0, stats
+    for i in sorted({0, rows - 1}):
+        check_row_against_oracle(r, i, O.sample(x[i], None, o_params(**kw[i]), 3))
+
+
 @pytest.mark.parametrize("masked", [False, True], ids=["two-launches", "merged-slices"])
 @pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
 def test_sort_of_many_candidates(sampler, bf16, masked):
