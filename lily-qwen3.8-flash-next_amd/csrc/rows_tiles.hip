@@ -320,7 +320,8 @@ __device__ __forceinline__ void tiles_row(const LILY_CONST RowArgs* table, const
             add_summaries(cut);
         }
     }
-    const float bound = lowered(kth);
+    // (values a little below it may share its quotient by the temperature)
+    const float bound = lower_by_slack(lowered(kth));
     const float reach = (want_lse && pen) ? fminf(bound, cut) : bound;   // tiles read
     phase(cfg, 2);
     if (tid == 0) {

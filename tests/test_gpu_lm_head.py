@@ -265,6 +265,34 @@ def test_ties_by_the_thousand_take_the_exhaustive_select(sampler):
     assert stats.cpu().numpy()[2] >= 1
 
 
+@pytest.mark.parametrize("vocab", [20_000, 60_004])
+def test_values_that_share_a_quotient(sampler, vocab):
+    """f32 logits with an id at 1.75 in half of the tiles and one at the float below in the others, whose quotients by
+    the temperature are the same: the ids decide, whichever value the bound is (short rows: the exact one)."""
+    rows, temperature = 3, np.float32(0.75)
+    value = np.float32(1.75)
+    below = np.nextafter(value, np.float32(0))
+    assert value / temperature == below / temperature
+    rng = np.random.default_rng(vocab)
+    x = (rng.random((rows, vocab)) * 0.5).astype(np.float32)
+    tiles = (vocab + TILE - 1) // TILE
+    at = np.arange(tiles) * TILE + 5
+    x[0, at] = np.where(np.arange(tiles) % 2 == 0, below, value)
+    x[1, at] = np.where(np.arange(tiles) < tiles // 2, below, value)
+    g = np.pad(x, ((0, 0), (0, tiles * TILE - vocab)), constant_values=-np.inf).reshape(rows, tiles, TILE)
+    tmax_np = g.max(axis=2).astype(np.float32)
+    c2 = np.float32(1.4426950408889634 / 0.75)
+    tsum_np = np.exp2(g.astype(np.float64) * c2 - (tmax_np * c2).astype(np.float64)[:, :, None]).sum(axis=2)
+    logits, tmax, tsum = (torch.from_numpy(t).to(dev()) for t in (x, tmax_np, tsum_np.astype(np.float32)))
+    params_kw = [dict(temperature=0.75, top_k=40, top_p=1.0, seed=5 + r) for r in range(rows)]
+    params, steps = [ls_params(**kw) for kw in params_kw], [0] * rows
+    ids, lps, cand, counts = _draw_all(
+        sampler, lambda out, lp, di, dc: sampler.sample_rows_tiled(
+            logits, tmax, tsum, params, steps, out, out_logprobs=lp, dbg_ids=di, dbg_counts=dc),
+        logits, params_kw, steps)
+    _check_draws(x, ids, lps, cand, counts, params_kw, steps)
+
+
 def test_rejections(sampler):
     rows, d, vocab = 2, 64, 256
     h = torch.zeros(rows, d, dtype=torch.bfloat16, device=dev())
