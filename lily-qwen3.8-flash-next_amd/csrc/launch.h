@@ -139,7 +139,7 @@ hipError_t launch_rows_held(hipStream_t stream, int dtype, uint32_t blocks, bool
 // The same rows of cfg.table (no mask, no bias list, plain draws) in slices of any length, a block at a time.
 hipError_t launch_rows_blocks(hipStream_t stream, int dtype, bool lse, bool pen, uint32_t rows, const LaunchCfg& cfg);
 // Plain draws under an allow-mask with at most STREAM_BIAS_CAP bias pairs, given inline or as cfg.table: a workgroup a
-// row whatever cfg.slices says, vocabularies up to MASKED_MAX_VOCAB.  cfg.masked_served: which rows it drew.
+// row whatever cfg.slices says, vocabularies up to MASKED_MAX_VOCAB.
 constexpr uint32_t MASKED_MAX_VOCAB = 262144;
 hipError_t launch_rows_masked(hipStream_t stream, int dtype, bool lse, uint32_t rows, const LaunchCfg& cfg,
                               const InlineRows* inline_rows);

@@ -148,8 +148,6 @@ struct LaunchCfg {
     // slice before it, for the merge by one wave (merge_turn_step())
     uint32_t turn_step;
     uint32_t pad_cfg;
-    // rows under a mask, ahead of another launch over the same rows (its `served`): 1 = drawn, 0 = left to that one
-    uint32_t* masked_served;
 };
 
 constexpr uint32_t CHAIN_CAP = LILY_SAMPLE_K_CAP;   // candidates a chained row publishes

@@ -124,16 +124,6 @@ __device__ __forceinline__ bool wide_last(const LaunchCfg& cfg, uint32_t row, ui
     return last_to_arrive(&cfg.ws_ticket[row], S, sh.last, cfg.relaxed_handover != 0u);
 }
 
-// The row's bound.  Each of the row's 4 x S waves names the r-th largest of its lanes' maxima (the leading 16 bits of
-// the order key, by a ballot search); the largest value that ceil(k / r) of the waves name or exceed is then reached
-// by k lanes, so by k values.  r lies a little above the waves' share ceil(k / 4S): where the least of all the waves'
-// share-th values was taken, one poor wave of 244 set the bound (8 f32 rows of 248 320 with k = 1 024: a list
-// beyond MERGE_CAP in every second launch, 1 500 us by the exhaustive select), and a slice of ids that nothing favours did.
-__device__ __forceinline__ uint32_t wide_rank(uint32_t k, uint32_t S) {
-    const uint32_t share = (k + 4u * S - 1u) / (4u * S);
-    return min(share + (share + 7u) / 8u + 1u, 64u);
-}
-constexpr uint32_t WIDE_LEAST_KEY = 0x0080u;   // of F32_LOWEST: what a wave with fewer finite lane maxima names
 // A slice's four keys of 16 bits as one word, never 0, in thread 0 (every thread calls).
 __device__ __forceinline__ uint64_t slice_keys_of(float lane_max, uint32_t k, uint32_t S, Shared& sh) {
     const uint32_t tid = threadIdx.x;
@@ -145,24 +135,6 @@ __device__ __forceinline__ uint64_t slice_keys_of(float lane_max, uint32_t k, ui
     static_assert(NWAVE == 4, "a word of four keys");
     return tid != 0u ? 0ull : ((uint64_t)(sh.hist[3] << 16 | sh.hist[2]) << 32) | (sh.hist[1] << 16 | sh.hist[0]);
 }
-// Of the keys that lane l of a wave has of slice l (0 past the last); F32_LOWEST: too many waves had none to name.
-// (A little lower than the keys: values that share the bound's quotient by the temperature rank with it.)
-__device__ __forceinline__ float bound_of_keys(uint64_t keys, uint32_t k, uint32_t S) {
-    const uint32_t r = wide_rank(k, S), need = (k + r - 1u) / r;
-    uint32_t T = 0;
-#pragma unroll
-    for (int bit = 15; bit >= 0; --bit) {
-        const uint32_t t = T | (1u << bit);
-        uint32_t n = 0;
-#pragma unroll
-        for (int i = 0; i < NWAVE; ++i) {
-            n += (uint32_t)__popcll(__ballot(((uint32_t)(keys >> (16 * i)) & 0xffffu) >= t));
-        }
-        T = n >= need ? t : T;
-    }
-    return T > WIDE_LEAST_KEY ? lower_by_slack(lilym_key_value(T << 16)) : F32_LOWEST;
-}
-
 // ---- first launch: lane maxima, the slice's sum of exponentials
 
 template <int DT, bool LSE, bool INLINE>

@@ -110,7 +110,6 @@ struct lily_sampler {
     float* wide_max = nullptr;     // [WIDE_FLOATS] lane maxima, rows x slices x 256
     uint32_t* wide_count = nullptr;  // [WS_ROWS] candidates listed so far, 0 between launches
     uint64_t* wide_bounds = nullptr; // [2][WS_ROWS][MAX_SLICES] slices' words of a launch under way, 0 between launches
-    uint32_t* masked_served = nullptr;   // [WS_ROWS] rows that a launch over masks' words has drawn
     uint32_t ws_rows = WS_ROWS;    // rows that may span several workgroups
     uint32_t ws_slots = WS_SLOTS;  // candidate slots behind ws_cand
     // Row table of lily_sample_rows batches above INLINE_ROWS.
@@ -458,15 +457,11 @@ HeldRows held_rows(const RowArgs* rows, uint32_t n) {
 }
 
 constexpr uint32_t MASKED_MAX_ROWS = 256;
-// Whether a launch goes a workgroup a row over the masks first (rows_masked.hip): where rows draw among
-// many candidates, and a workgroup a row fills the chip no more than once.  (bf16, 151 936 ids, no top_k, 1 row / 64, us, the
-// other kernels -> now.  In runs of up to 64 ids: 0.2 % admitted 22.3 / 26.2 -> 15.9 / 16.6, 2 % 26.2 / 33.1 -> 22.7 / 24.8, 10 % 65 / 68
-// -> 48 / 50, 20 % 69 / 81 -> 72 / 74.  One by one: 0.2 % 22.2 / 26.7 -> 15.8 / 16.6, 2 % 25.4 / 29.8 -> 23.0 / 23.7, 5 % 32.3 /
-// 36.9 -> 32.2 / 33.9.  Rows that are left to the launch behind pay for the look at the mask: 10 % one by one 36.7 / 40.6 ->
-// 42.0 / 47.1, all ids 74 / 83 -> 80 / 92.  For k <= 64 the streaming selects make less of the difference: 64 rows
-// 21.8 -> 19.8, all ids admitted 32 -> 39.)
+// Whether a launch goes a workgroup a row over the masks (rows_masked.hip, with the figures of both): where rows draw
+// among many candidates, and a workgroup a row fills the chip no more than once.  (For k <= 64 the streaming selects make
+// less of the difference: 64 rows under masks of 2 % 21.8 -> 19.8 us, under masks of all ids 32 -> 39.)
 bool all_masked(const lily_sampler* s, const RowArgs* rows, uint32_t n, uint32_t vocab, uint32_t kmax) {
-    if (kmax <= STREAM_K_MAX || n > MASKED_MAX_ROWS || s->masked_served == nullptr || n > s->ws_rows || s->force_path != 0 ||
+    if (kmax <= STREAM_K_MAX || n > MASKED_MAX_ROWS || s->force_path != 0 ||
         s->no_held || (s->force_slices != 0 && !s->only_blocks) || vocab > MASKED_MAX_VOCAB) {
         return false;
     }
@@ -737,11 +732,8 @@ int launch_part(lily_sampler* s, const LaunchPart& part, const RowArgs* table_de
         return LILY_OK;
     }
     if (part.masked && served == nullptr) {
-        LaunchCfg first = cfg;
-        first.masked_served = s->masked_served;
-        HIP_TRY(launch_rows_masked(s->stream, dtype, part.lse, part.rows, first, nullptr));
-        cfg.served = s->masked_served;
-        cfg.phase_trace = nullptr;
+        HIP_TRY(launch_rows_masked(s->stream, dtype, part.lse, part.rows, cfg, nullptr));
+        return LILY_OK;
     }
     if (part.blocks) {
         HIP_TRY(launch_rows_blocks(s->stream, dtype, part.lse, part.pen, part.rows, cfg));
@@ -815,10 +807,8 @@ int launch_inline(lily_sampler* s, int dtype, uint32_t vocab, const InlineRows& 
     }
     const LaunchShape shp = shape_of(s, rows.r, n, dtype, vocab, slices, kmax);
     if (masked) {
-        cfg.masked_served = s->masked_served;
         HIP_TRY(launch_rows_masked(s->stream, dtype, shp.lse, n, cfg, &rows));
-        cfg.served = s->masked_served;
-        cfg.phase_trace = nullptr;
+        return LILY_OK;
     }
     if (held.blocks != 0) {
         for (uint32_t i = 0; i < n; ++i) {
@@ -1193,7 +1183,6 @@ int lily_sampler_create(int device, void* hip_stream, lily_sampler_t** out) {
     if (err == hipSuccess) err = hipMemset(s->ws_ticket, 0, WS_ROWS * 4);
     if (err == hipSuccess) err = hipMalloc(reinterpret_cast<void**>(&s->wide_max), (size_t)WIDE_FLOATS * 4);
     if (err == hipSuccess) err = hipMalloc(reinterpret_cast<void**>(&s->wide_count), WS_ROWS * 4);
-    if (err == hipSuccess) err = hipMalloc(reinterpret_cast<void**>(&s->masked_served), WS_ROWS * 4);
     if (err == hipSuccess) err = hipMemset(s->wide_count, 0, WS_ROWS * 4);
     if (err == hipSuccess) err = hipMalloc(reinterpret_cast<void**>(&s->wide_bounds), (size_t)2 * WS_ROWS * MAX_SLICES * 8);
     if (err == hipSuccess) err = hipMemset(s->wide_bounds, 0, (size_t)2 * WS_ROWS * MAX_SLICES * 8);
@@ -1231,7 +1220,6 @@ void lily_sampler_destroy(lily_sampler_t* s) {
     (void)hipFree(s->wide_max);
     (void)hipFree(s->wide_count);
     (void)hipFree(s->wide_bounds);
-    (void)hipFree(s->masked_served);
     (void)hipFree(s->chain_cand);
     (void)hipFree(s->table_dev);
     for (uint32_t i = 0; i < STAGE_SLOTS; ++i) {

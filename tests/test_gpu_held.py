@@ -222,29 +222,47 @@ def test_masked_rows_of_many_candidates(monkeypatch, held, bf16, vocab):
 @pytest.mark.parametrize("vocab", [9001, 70_001, 262_144])
 @pytest.mark.parametrize("run", [1, 96], ids=["one by one", "in runs"])
 def test_masks_that_scatter_and_masks_that_cluster(monkeypatch, bf16, vocab, run):
-    """Masks of a few ids, just what the sort holds and one more, twice that, and as many words as the rule for
-    clusters takes and some more; scattered ids and runs; equal values by the thousand, a row of -inf, NaN."""
+    """Masks of a few ids, just what the sort and the list of ids hold and one more, as many words as the rule for
+    clusters takes and some more, all ids; scattered ids and runs, over every kind of row: equal values by the
+    thousand, mostly and wholly -inf, NaN; bias lists, penalties and a forced id."""
     rng = np.random.default_rng(vocab + run)
     x = _rows(rng, vocab, False)
     xs = W.to_bf16_bits(x) if bf16 else x
     words = (vocab + 31) // 32
-    allow = np.zeros((ROWS, words), dtype=np.uint32)
-    most = 32 * (800 + vocab // 150)
-    for i, n in enumerate((3, 8191, 8192, 8193, 16_384, most - 64, most + 64, 1200)):
+    masks = np.zeros((ROWS, words), dtype=np.uint32)
+    most = 32 * (350 + vocab // 170)
+    for i, n in enumerate((3, 8191, 8193, 16_384, 16_385, most - 64, most + 64, vocab)):
         n = min(n, vocab)
-        if run == 1:
+        if run == 1 or n == vocab:
             ids = rng.choice(vocab, n, replace=False)
         else:
             starts = np.sort(rng.choice(vocab // run, min(-(-n // run), vocab // run), replace=False)) * run
             ids = (starts[:, None] + np.arange(run)).ravel()[:n]
-        np.bitwise_or.at(allow[i], ids >> 5, (1 << (ids & 31)).astype(np.uint32))
+        np.bitwise_or.at(masks[i], ids >> 5, (1 << (ids & 31)).astype(np.uint32))
     bias = [[(int(i), float(d)) for i, d in zip(rng.integers(0, vocab, 30), rng.choice([-5.0, 5.0, 0.5], 30))]
             for _ in range(ROWS)]
+    hist = rng.integers(0, vocab, (ROWS, 2000)).astype(np.int32)
+    pen = dict(repetition_penalty=1.2, presence_penalty=0.1, frequency_penalty=0.2)
     s = _sampler(monkeypatch, "1")
-    for trial, lp in enumerate((True, False)):
-        kw = [dict(temperature=0.8, top_k=0 if trial == 0 else 200, top_p=0.95, seed=9 + i) for i in range(ROWS)]
-        r = run_rows(s, xs, kw, [trial] * ROWS, logprobs=lp, allow=allow, bias=bias, use_plan=trial == 1)
-        _check(r, xs, kw, trial, lp, allow=allow, bias=bias)
+    for trial in range(ROWS):
+        lp = trial % 2 == 0
+        allow = np.roll(masks, trial, axis=0)
+        kw = [dict(temperature=0.8, top_k=200 if trial % 4 == 3 else 0, top_p=0.95, seed=9 + i, **(pen if trial % 4 == 2 else {}))
+              for i in range(ROWS)]
+        sc = counts = None
+        if trial % 4 == 2:
+            sc, counts = [], []
+            for i in range(ROWS):
+                t = LS.SamplerScratch(s, vocab)
+                t.add_history(torch.from_numpy(hist[i]).to(dev()))
+                sc.append(t)
+                counts.append(np.bincount(hist[i], minlength=vocab).astype(np.uint32))
+        ext = dict(allow=allow, bias=bias if trial % 3 else [[]] * ROWS,
+                   forced=[i if trial == 4 and i % 2 else None for i in range(ROWS)])
+        r = run_rows(s, xs, kw, [trial] * ROWS, scratch=sc, logprobs=lp, use_plan=trial % 4 == 1, **ext)
+        _check(r, xs, kw, trial, lp, counts, **ext)
+        for t in sc or []:
+            t.close()
     s.close()
 
 
