@@ -8,15 +8,20 @@
 // with its value, and at the end those that still reach it are ranked; nothing is looked at twice.
 //
 // A block of a dense history (an eighth of the ids and more) lists more than a wave's notes hold: the wave then evaluates
-// them straight from their bits, in a block without a bound once for the bound and once more for the list and the
-// sum.  us a launch, 200 bf16 rows of 151 936, N(0, 2^2), 13 / 25 / 60 % of the ids listed 61 / 77 / 110 (the flat form of
+// them straight from their bits, where nothing else gives a bound once for that and once more for the list and the
+// sum.  us a launch, 200 bf16 rows of 151 936, N(0, 2^2), 13 / 25 / 60 % of the ids listed 59 / 72 / 103 (the flat form of
 // select_lowering.h 107 / 136 / 285; given up to the exhaustive select, as such slices once were, 670 to 680), half of the first
-// tenth listed 54 (79).
+// tenth listed 52 (79).
 //
-// Bound: the vector unit where the row's sum takes most values (200 rows of 248 320 bf16, N(0, 2^2), under penalties
-// 53 us a launch for 99 MB; 76 through the flat form of select_lowering.h, which takes twice the instructions
-// a value and looks at the noted chunks again), the memory where it does not (1 024 rows of 151 936 without
-// log-probabilities 56.5 us, 5.5 TB/s; 62 through select_stream.h).
+// Bound: the vector unit where the row's sum takes most values (200 rows of 248 320 bf16, N(0, 2^2), under penalties:
+// 50 us a launch for 99 MB, 25 vector instructions a value, which keep the unit busy two thirds of the time; 74 through
+// the flat form of select_lowering.h, whose scan spends fewer but behind whose scan the noted chunks are looked at again), the memory
+// where it does not (1 000 rows of 151 936, k = 64, without log-probabilities 50 us, 6.1 TB/s; 1 024 rows 62 through
+// select_stream.h).  Rows with a heavy tail, whose sum takes a few chunks, are no faster this way than through
+// select_lowering.h (200 rows of 151 936, 0.5 / 5 / 10 % listed 33.1 / 35.8 / 37.2 us, 32.8 / 34.8 / 36.8 there; 13 % 39, 77 there; 200 rows of
+// 248 320 39.5 / 43.7 / 46.3, 38.1 / 39.3 / 90 there).
+// A chunk with values for the list offers them one by one: a wave-wide test each, most of them for nothing, takes
+// fewer instructions than finding the ones there are (53.0 -> 50.8 us for the 200 rows of 248 320).
 // Tried: listed ids evaluated as their chunks pass (a round trip a block: 82 us for 1 024 rows with a heavy tail,
 // 74 this way), all of them ahead of the blocks (138 us: their gathers read more than the row), three copies
 // of the loop for two blocks on their way (leaves the instruction cache: 3 to 10 % longer).
@@ -287,56 +292,86 @@ __device__ __forceinline__ bool blocks_row(const LILY_CONST RowArgs* src, const 
         }
         // Listed ids leave the chunks whose raw values might matter (their true ones lie no higher, where
         // penalties only lower) and are noted, to be evaluated by the hundred.  In the other chunks, which
-        // reach neither the bound nor the cut, they may stay.
-        uint32_t crowd = 0u;
-        if (PEN && pen) {
-            const uint32_t noted_before = noted;
+        // reach neither the bound nor the cut, they may stay.  The first block's are noted when it has given a bound
+        // (before, all of them were: 200 rows with a heavy tail, 10 % listed, 43.7 -> 40.3 us).
+        const uint32_t noted_before = noted;
+        auto note = [&](int u, uint64_t mask) {
+            uint32_t left = away[u];
+            do {
+                const uint32_t at = noted + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+                if (left != 0u && at < NOTE_SEG) {
+                    notes[at] = chunk_of(b, u) * (uint32_t)E + (uint32_t)__builtin_ctz(left) - g.pad;
+                }
+                noted += (uint32_t)__popcll(mask);
+                left &= left - 1u;
+                mask = __ballot(left != 0u);
+            } while (mask != 0ull);
+        };
+        auto bits = [&]() -> uint32_t {
+            uint32_t all = 0u;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                all |= away[u] << (u * E);
+            }
+            return all;
+        };
+        if (PEN && pen && b != 0u) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 away[u] = raising || cm[u] >= low ? away[u] : 0u;
-                uint32_t left = away[u];
-                uint64_t mask = __ballot(left != 0u);
+                const uint64_t mask = __ballot(away[u] != 0u);
                 if (mask != 0ull) {
-                    cur[u] = chunk_without<DT>(cur[u], left);
+                    cur[u] = chunk_without<DT>(cur[u], away[u]);
                     cm[u] = chunk_max<DT>(cur[u]);
-                    do {
-                        const uint32_t at = noted + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-                        if (left != 0u && at < NOTE_SEG) {
-                            notes[at] = chunk_of(b, u) * (uint32_t)E + (uint32_t)__builtin_ctz(left) - g.pad;
-                        }
-                        noted += (uint32_t)__popcll(mask);
-                        left &= left - 1u;
-                        mask = __ballot(left != 0u);
-                    } while (mask != 0ull);
-                }
-            }
-            if (noted > NOTE_SEG) {
-                // (a dense history: the wave goes by the block's bits)
-                noted = noted_before;
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    crowd |= away[u] << (u * E);
-                }
-                if (T == F32_LOWEST) {
-                    settle(b, crowd, false);
+                    note(u, mask);
                 }
             }
         }
+        if (PEN && pen && b == 0u) {
+            float raw_max[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            block_max = max2_raw(block_max, cm[u]);
-        }
-        lane_max = max2_raw(lane_max, block_max);
-        // (the first block's notes wait for a bound, the last one takes them in)
-        if (b < 4u || (b & 3u) == 3u || (!PEN && b + 1u == nblocks)) {
+            for (int u = 0; u < U; ++u) {
+                raw_max[u] = cm[u];
+                cur[u] = chunk_without<DT>(cur[u], away[u]);
+                cm[u] = chunk_max<DT>(cur[u]);
+                lane_max = max2_raw(lane_max, cm[u]);
+            }
             refresh();
+            if (T == F32_LOWEST) {   // (the same in every thread: what is not listed does not suffice for a bound)
+                settle(b, bits(), false);
+                refresh();
+            }
+            const float low_now = LSE && want_lse ? fminf(T, skip) : T;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                away[u] = raising || raw_max[u] >= low_now ? away[u] : 0u;
+                const uint64_t mask = __ballot(away[u] != 0u);
+                if (mask != 0ull) {
+                    note(u, mask);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                block_max = max2_raw(block_max, cm[u]);
+            }
+            lane_max = max2_raw(lane_max, block_max);
+            // (the last block's comes behind its notes, which it takes in; one a block for four blocks: 400 rows, k = 64, with
+            // log-probabilities 45.4 -> 44.8 us without the third's)
+            if (PEN ? (b < 2u || (b & 3u) == 3u) && b + 1u < nblocks : b < 2u || (b & 3u) == 3u || b + 1u == nblocks) {
+                refresh();
+            }
         }
         if (PEN) {
-            if (pen && (noted > NOTE_SEG / 2u || b + 1u == nblocks)) {
-                drain();
-            }
-            if (__ballot(crowd != 0u) != 0ull) {
-                settle(b, crowd, true);
+            if (pen) {
+                const bool crowd = noted > NOTE_SEG;   // (a dense history: the wave goes by the block's bits)
+                noted = crowd ? noted_before : noted;
+                if (noted > NOTE_SEG / 2u || b + 1u == nblocks) {
+                    drain();
+                }
+                if (crowd) {
+                    settle(b, bits(), true);
+                }
             }
             if (b + 1u == nblocks) {
                 refresh();
@@ -352,24 +387,11 @@ __device__ __forceinline__ bool blocks_row(const LILY_CONST RowArgs* src, const 
             float v[E];
             unpack<DT>(cur[u], v);
             if (some) {
-                uint32_t hits = 0;
 #pragma unroll
                 for (int j = 0; j < E; ++j) {
-                    hits |= v[j] >= T ? 1u << j : 0u;
-                }
-                for (uint32_t left = hits; __ballot(left != 0u) != 0ull; left &= left - 1u) {
-                    const uint32_t j = left != 0u ? (uint32_t)__builtin_ctz(left) : 0u;
-                    float x = v[0];
-#pragma unroll
-                    for (int q = 1; q < E; ++q) {
-                        x = j == (uint32_t)q ? v[q] : x;
-                    }
-                    list(left != 0u, x, chunk_of(b, u) * (uint32_t)E + j - g.pad);
-                }
-                if (LSE) {
-#pragma unroll
-                    for (int j = 0; j < E; ++j) {
-                        v[j] = ((hits >> j) & 1u) != 0u ? NEG_INF : v[j];   // (their terms are formed with the list's)
+                    list(v[j] >= T, v[j], chunk_of(b, u) * (uint32_t)E + (uint32_t)j - g.pad);
+                    if (LSE) {
+                        v[j] = v[j] >= T ? NEG_INF : v[j];   // (their terms are formed with the list's)
                     }
                 }
             }
