@@ -364,7 +364,10 @@ struct HeldShape {
 };
 // Workgroups of a launch: as many as the chip holds at once (four a compute unit with one block, three with two).
 // Rows under penalties without log-probabilities stay below that (bf16, 151 936 ids, streamed -> held: 40 rows
-// in 19 slices 21.9 -> 21.9 us, 50 rows 22.3 -> 23.2, 60 rows in 10 slices of two blocks 23.8 -> 25.6).
+// in 19 slices 21.9 -> 21.9 us, 50 rows 22.3 -> 23.2), and bf16 slices of two blocks are not for rows under penalties: every
+// listed id is looked up there (without log-probabilities 60 rows in 10 slices 23.8 -> 25.6; with them a block at a time -> held, 130
+// rows of 60 000, N(0, 2^2), 0.5 / 5 / 10 % of the ids listed 23.8 / 27.4 / 29.1 -> 21.8 / 27.7 / 31.3, with a heavy tail 21.5 / 22.6 /
+// 23.3 -> 21.9 / 27.8 / 31.5, where the kernels before took 22.4 / 23.1 / 26.1).
 constexpr uint32_t HELD_MAX_GROUPS[3] = {0, 1024, 768};
 // Rows with masks too, and in slices of two blocks up to a workgroup a compute unit (2 % admitted: 30 rows, k = 50,
 // 21.8 -> 19.6, 64 rows in slices of two blocks 21.8 -> 27.3; 16 f32 rows of 248 320, k = 64, 23.6 -> 24.0 in two).
@@ -387,7 +390,7 @@ HeldShape held_shape(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint32
         if (extra && (uint64_t)rows * sl > HELD_MAX_GROUPS_EXTRA[blocks]) {
             continue;
         }
-        if (pen && !lse && ((uint64_t)rows * sl > HELD_MAX_GROUPS_LISTED || (blocks == 2 && dtype == LILY_BF16))) {
+        if (pen && ((!lse && (uint64_t)rows * sl > HELD_MAX_GROUPS_LISTED) || (blocks == 2 && dtype == LILY_BF16))) {
             continue;
         }
         out.blocks = blocks;
@@ -405,10 +408,10 @@ constexpr uint64_t BLOCKS_MAX_PIECES = 1ull << 28;
 // are not the same number on every compute unit leave some idle (200 rows in 5 slices 53 us, in 3 66), a second
 // generation costs more than the slices save.
 //
-// Which launches: bf16 rows of 151 936, us, before -> a block at a time.  Without penalties all of them (with
-// log-probabilities 100 rows 35.0 -> 23.8, 1 024 77.5 -> 70.2; without 19.2 -> 16.6, 62.0 -> 56.6).  Under penalties
-// those with log-probabilities up to a fifth of the chip's workgroups: flat rows of 248 320 59.0 -> 39.6 at 100, 75.7 ->
-// 53.1 at 200, rows with a heavy tail 33.4 -> 31.7 and 40.3 -> 39.6, but at 280 rows 89.5 -> 72.2 and 40.5 -> 44.9.
+// Which launches: bf16 rows of 151 936, us, before -> a block at a time.  Without penalties all of them (k = 64, with
+// log-probabilities 100 rows 35.0 -> 23.5, 1 000 77 -> 64; without 19.2 -> 15.5, 62 -> 50).  Under penalties
+// those with log-probabilities up to a fifth of the chip's workgroups: flat rows of 248 320 63.8 -> 42 at 80, 74 ->
+// 51 at 200, rows with a heavy tail 31 -> 32 and 38 -> 39.5; at 280 rows, when a flat one took 72 (89.5), such rows took 44.9 (40.5).
 // Without log-probabilities the streaming kernel's coarse map is the cheaper look at listed ids (80 rows 23.5 -> 25.3).
 uint32_t blocks_slices(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint32_t vocab, int dtype, bool pen, bool lse) {
     if (s->force_path != 0 || s->no_held || kmax > STREAM_K_MAX) {
@@ -432,6 +435,11 @@ uint32_t blocks_slices(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint
         const uint32_t by_block = (nch + 256u * STREAM_UNROLL - 1) / (256u * STREAM_UNROLL);   // no finer than a block a slice
         sl = sl > by_block && s->force_slices == 0 ? by_block : sl;
         sl = sl > MAX_SLICES ? MAX_SLICES : sl;
+        if (s->force_slices == 0) {
+            // (as many as that many blocks a slice need: 130 rows of 60 000 in 7 slices were a block and a 25th each)
+            const uint32_t blocks = (by_block + sl - 1) / sl;
+            sl = (by_block + blocks - 1) / blocks;
+        }
     }
     // (one wave merges a row's slices, whatever their number)
     sl = sl > WAVE_MERGE_LISTS && sl * kmax > HELD_MERGE_SLOTS ? std::max(WAVE_MERGE_LISTS, HELD_MERGE_SLOTS / kmax) : sl;
