@@ -45,10 +45,9 @@ __device__ __forceinline__ f32x4 product(const w32x4& a, const w32x4& b, const f
 
 // Words from one column's scales and biases to the next's: one more than there are groups (an even
 // number: an odd distance spreads the 16 columns a product reads at once over the banks without a
-// computed turn), unless just that word costs a workgroup its place (92 groups: two a compute unit;
-// 252: one; 16 columns then lie 28 or 60 banks apart, which are different ones too).
+// computed turn).  Two workgroups a compute unit up to 94 groups, with and without that word.
 __host__ __device__ constexpr uint32_t scale_pitch(uint32_t groups) {
-    return groups == 92u || groups >= GROUPS_MAX ? groups : groups + 1u;
+    return groups + 1u;
 }
 // Bytes of LDS a launch needs: the stages, then every scale and bias of the tile's 128 columns (the partial
 // sums take their place at a tile's end, while the next one's are in registers), the reductions.
@@ -57,7 +56,7 @@ inline uint32_t codes_lds_bytes(uint32_t groups) {
     return (uint32_t)RING_BYTES + (sz > (uint32_t)PART_BYTES ? sz : (uint32_t)PART_BYTES) + (uint32_t)RED_BYTES;
 }
 
-static_assert(RING_BYTES + LILY_TILE_COLS * GROUPS_MAX * 4 + RED_BYTES <= CU_LDS_BYTES, "the scales' place");
+static_assert(RING_BYTES + LILY_TILE_COLS * scale_pitch(GROUPS_MAX) * 4 + RED_BYTES <= CU_LDS_BYTES, "the scales' place");
 
 }  // namespace
 
