@@ -400,3 +400,38 @@ def test_sort_with_more_empty_places_than_candidates(sampler, bf16):
     r = run_rows(sampler, x, kw, [0] * 3, allow=allow)
     for i in range(3):
         check_row_against_oracle(r, i, O.sample(x[i], None, o_params(**kw[i]), 0, allow=allow[i]))
+
+
+@pytest.mark.parametrize("masked", [False, True], ids=["one launch", "masked"])
+@pytest.mark.parametrize("n", [1200, 3000, 8200])
+def test_sort_by_sixteen_waves(sampler, n, masked):
+    """The sort of sixteen waves on values around zero: outliers on both sides, infinities, values near zero with one
+    outlier (they share a bin, which is sorted by exchanges with what precedes it), 300 equal ones ahead of the rest, behind the
+    best and across the k-th, all equal.  `masked`: so many allowed ids; else about as many as reach the row's
+    bound, of a launch over one row."""
+    rng = np.random.default_rng(n)
+    vocab = 151_936
+    some = rng.choice(vocab, n, replace=False)
+    x = np.full((8, vocab), -np.inf, dtype=np.float32)
+    x[:, some] = rng.normal(0, 1, (8, n))
+    x[0, some[:6]] = 300, -300, 80, 2.0e38, -2.0e38, -80
+    x[1, some[:2]] = np.inf, 50
+    x[2, some] *= 1.0e-4
+    x[2, some[0]] = 0.9
+    order = some[np.argsort(-x[3, some])]
+    x[3, order[:300]] = 5.0
+    x[4, some[np.argsort(-x[4, some])][100:400]] = 1.0e-3
+    x[5, some[np.argsort(-x[5, some])][900:1200]] = 0.0
+    x[6, some] = 1.0
+    x[7, some] = rng.standard_t(2, n) * 4
+    allow = np.zeros((8, (vocab + 31) // 32), dtype=np.uint32)
+    np.bitwise_or.at(allow, (slice(None), some >> 5), (1 << (some & 31)).astype(np.uint32))
+    for trial, k in enumerate((0, 300)):
+        kw = [dict(temperature=1.0, top_k=k, top_p=0.99, seed=700 + i) for i in range(8)]
+        whole = run_rows(sampler, x, kw, [trial] * 8, allow=allow) if masked else None
+        for i in range(8):
+            d = O.sample(x[i], None, o_params(**kw[i]), trial, allow=allow[i] if masked else None)
+            if masked:
+                check_row_against_oracle(whole, i, d)
+            else:
+                check_row_against_oracle(run_rows(sampler, x[i:i + 1], kw[i:i + 1], [trial]), 0, d)
