@@ -58,20 +58,28 @@ __device__ __forceinline__ const LILY_CONST RowArgs* wide_table(const LaunchCfg&
 }
 
 // One pass over the slice's chunks, four loads in flight per thread, every load unconditional
-// (a chunk number past the slice is replaced by the slice's last; `use` says whether it counts).
-template <int DT, class F>
-__device__ __forceinline__ void wide_scan(const Geo<DT>& g, F&& per_chunk) {
+// (a chunk number past the slice is replaced by the slice's last).  before(): called once the first loads are on their
+// way; true = what it did had no registers for them, they are made again.
+template <int DT, class B, class F>
+__device__ __forceinline__ void wide_scan(const Geo<DT>& g, B&& before, F&& per_chunk) {
     const uint32_t tid = threadIdx.x;
     if (g.main_hi <= g.main_lo) {
+        before();
         return;
     }
-    for (uint32_t c0 = g.main_lo; c0 < g.main_hi; c0 += 4u * NT) {
-        u32x4 q[4];
+    u32x4 q[4];
+    auto fetch = [&](uint32_t c0) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const uint32_t c = min(c0 + (uint32_t)u * NT + tid, g.main_hi - 1u);
             q[u] = gload(reinterpret_cast<const u32x4*>(g.base + (size_t)c * 16));
         }
+    };
+    fetch(g.main_lo);
+    if (before()) {
+        fetch(g.main_lo);
+    }
+    for (uint32_t c0 = g.main_lo;;) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const uint32_t c = c0 + (uint32_t)u * NT + tid;
@@ -79,6 +87,11 @@ __device__ __forceinline__ void wide_scan(const Geo<DT>& g, F&& per_chunk) {
                 per_chunk(q[u], c);
             }
         }
+        c0 += 4u * NT;
+        if (c0 >= g.main_hi) {
+            break;
+        }
+        fetch(c0);
     }
 }
 
@@ -156,7 +169,7 @@ __global__ __launch_bounds__(NT, 4) void k_wide_bound(InlineRows rows_arg, Launc
     float lane_max = NEG_INF;
     LseAcc lse;
     lse.init();
-    wide_scan<DT>(g, [&](const u32x4& q, uint32_t c) {
+    wide_scan<DT>(g, []() { return false; }, [&](const u32x4& q, uint32_t c) {
         float v[E];
         unpack<DT>(q, v);
         float m;
@@ -305,8 +318,8 @@ constexpr uint32_t SIXTEEN_LDS_BYTES = (SIXTEEN_OFF_PLACED + MERGE_CAP) * 8;
 // by the select that is right for any input.
 // Sixteen waves sort, and the first four draw.
 template <int DT, bool LSE, uint32_t THREADS = NT>
-__device__ __forceinline__ void wide_finish(RowArgs& a, const LaunchCfg& cfg, const WideArgs& w, Shared& sh, uint32_t& n_mine,
-                                            uint64_t* cand, uint32_t row, uint32_t S, uint32_t step, bool want_lse, bool gave_up,
+__device__ __forceinline__ void wide_finish(const LILY_CONST RowArgs* src, const LaunchCfg& cfg, const WideArgs& w, Shared& sh,
+                                            uint32_t& n_mine, uint64_t* cand, uint32_t row, uint32_t S, bool gave_up,
                                             SixteenShared* six = nullptr) {
     constexpr bool SIXTEEN = THREADS == SIXTEEN_THREADS;
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
@@ -344,6 +357,10 @@ __device__ __forceinline__ void wide_finish(RowArgs& a, const LaunchCfg& cfg, co
         mine_c[j] = handed_load(cfg.ws_cand, (size_t)row * MERGE_CAP + tid + (uint32_t)j * THREADS);
     }
     const uint32_t total = load_through(&w.count[row]);
+    RowArgs a;
+    read_again(a, src);
+    const uint32_t step = a.step + cfg.step_delta;
+    const bool want_lse = LSE && a.out_logprob != nullptr;
     __syncthreads();   // (everybody has read it)
     if (tid == 0) {
         store_through(&w.count[row], 0u);
@@ -422,6 +439,7 @@ template <int DT, bool LSE, bool INLINE>
 __global__ __launch_bounds__(NT, 4) void k_wide_draw(InlineRows rows_arg, LaunchCfg cfg, WideArgs w) {
     __shared__ Shared sh;
     __shared__ uint32_t n_mine;
+    __shared__ float row_bound;
     constexpr int E = Geo<DT>::E;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, s = blockIdx.x, row = blockIdx.y, S = cfg.slices;
     if (cfg.served != nullptr && *(const LILY_CONST uint32_t*)(cfg.served + row) != 0u) {
@@ -436,20 +454,28 @@ __global__ __launch_bounds__(NT, 4) void k_wide_draw(InlineRows rows_arg, Launch
     load_row_args(a, wide_table<INLINE>(cfg) + row);
     apply_selection(a);
     const uint32_t vocab = cfg.vocab;
-    const uint32_t step = a.step + cfg.step_delta;
-    const bool want_lse = LSE && a.out_logprob != nullptr;
     const bool pen = (a.flags & F_PEN) != 0;   // (of the kind that only lowers: the host sees to it)
-    // The bound (of the values' worth under the penalties), by every wave for itself; where too many waves had too few
-    // finite lane maxima to name one, the k-th largest of all the lanes' maxima.
-    float bound = bound_of_keys(lane < S ? handed_load(w.slice_keys, (size_t)row * S + lane) : 0ull, a.k, S);
-    if (!(bound > F32_LOWEST)) {   // (the same in every wave)
-        bound = wide_bound_of(w, row, S, a.k, sh);
-    }
     Geo<DT> g;
     g.init(a.logits, vocab, s, S);
     uint64_t* cand = dyn_lds;
     const uint32_t cap = MERGE_CAP;   // what the slice's own list holds
-    __syncthreads();
+    const uint64_t keys = lane < S ? handed_load(w.slice_keys, (size_t)row * S + lane) : 0ull;
+    float bound = F32_LOWEST;
+    auto find_bound = [&]() -> bool {
+        if (tid < 64u) {
+            const float b = bound_of_keys(keys, a.k, S);
+            if (lane == 0u) {
+                row_bound = b;
+            }
+        }
+        __syncthreads();
+        bound = row_bound;
+        const bool none = !(bound > F32_LOWEST);   // (the same in every wave)
+        if (none) {
+            bound = wide_bound_of(w, row, S, a.k, sh);
+        }
+        return none;
+    };
     auto offer = [&](float x, uint32_t id) {
         if (!(x >= bound)) {
             return;
@@ -465,7 +491,7 @@ __global__ __launch_bounds__(NT, 4) void k_wide_draw(InlineRows rows_arg, Launch
             cand[at] = composite_of(x / a.temperature, id);
         }
     };
-    wide_scan<DT>(g, [&](const u32x4& q, uint32_t c) {
+    wide_scan<DT>(g, find_bound, [&](const u32x4& q, uint32_t c) {
         if (chunk_max<DT>(q) >= bound) {
             float v[E];
             unpack<DT>(q, v);
@@ -476,7 +502,7 @@ __global__ __launch_bounds__(NT, 4) void k_wide_draw(InlineRows rows_arg, Launch
         }
     });
     wide_edges<DT>(a, g, [&](float x, uint32_t id) { offer(x, id); });
-    wide_finish<DT, LSE>(a, cfg, w, sh, n_mine, cand, row, S, step, want_lse, false);
+    wide_finish<DT, LSE>(wide_table<INLINE>(cfg) + row, cfg, w, sh, n_mine, cand, row, S, false);
 }
 
 // ---- both in one launch, where a slice is held in registers and all of the launch's workgroups are on the chip
@@ -513,7 +539,6 @@ __global__ __launch_bounds__(THREADS, 4) void k_wide_held(InlineRows rows_arg, L
     RowArgs a;
     load_row_args(a, wide_table<INLINE>(cfg) + row);
     apply_selection(a);
-    const uint32_t step = a.step + cfg.step_delta;
     const bool want_lse = LSE && a.out_logprob != nullptr;
     const bool pen = (a.flags & F_PEN) != 0;
     Geo<DT> g;
@@ -753,7 +778,7 @@ __global__ __launch_bounds__(THREADS, 4) void k_wide_held(InlineRows rows_arg, L
     }
     offer(ev, edge);   // (-inf where there is none)
     __syncthreads();
-    wide_finish<DT, LSE, THREADS>(a, cfg, w, sh, n_mine, cand, row, S, step, want_lse, lost != 0u, &six);
+    wide_finish<DT, LSE, THREADS>(wide_table<INLINE>(cfg) + row, cfg, w, sh, n_mine, cand, row, S, lost != 0u, &six);
 }
 
 template <int DT, bool LSE, bool INLINE>

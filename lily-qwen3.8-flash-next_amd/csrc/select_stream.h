@@ -107,9 +107,20 @@ constexpr uint32_t WIDE_LEAST_KEY = 0x0080u;   // of F32_LOWEST: what a wave wit
 // (A little lower than the keys: values that share the bound's quotient by the temperature rank with it.)
 __device__ __forceinline__ float bound_of_keys(uint64_t keys, uint32_t k, uint32_t S) {
     const uint32_t r = wide_rank(k, S), need = (k + r - 1u) / r;
-    uint32_t T = 0;
+    // (the waves' keys differ in their last bits only, as a rule)
+    uint32_t hi = 0u, lo = 0xffffu;
 #pragma unroll
-    for (int bit = 15; bit >= 0; --bit) {
+    for (int i = 0; i < NWAVE; ++i) {
+        const uint32_t key = (uint32_t)(keys >> (16 * i)) & 0xffffu;
+        hi = max(hi, key);
+        lo = key != 0u ? min(lo, key) : lo;
+    }
+    hi = wave_max_u32(hi);
+    lo = wave_min_u32(lo);
+    const int bits = hi != lo ? 32 - __builtin_clz(hi ^ lo) : 0;
+    uint32_t T = hi >> bits << bits;
+#pragma unroll 1
+    for (int bit = bits - 1; bit >= 0; --bit) {
         const uint32_t t = T | (1u << bit);
         uint32_t n = 0;
 #pragma unroll
