@@ -517,6 +517,7 @@ void fill_cfg(const lily_sampler* s, LaunchCfg* cfg, uint32_t rows, uint32_t voc
 // the device) without mask or bias list, penalties none or of the kind that only lowers (the
 // second launch passes over chunks whose raw values stay below the bound), some row with
 // k > STREAM_K_MAX, and at least two workgroups a row.  0 = no.
+constexpr uint32_t WIDE_FINE_GROUPS = 512;
 uint32_t wide_slices(const lily_sampler* s, const RowArgs* rows, uint32_t n, int dtype, uint32_t vocab) {
     if (s->wide_max == nullptr || s->no_wide || s->force_path != 0 || n > s->ws_rows) {
         return 0;
@@ -543,8 +544,12 @@ uint32_t wide_slices(const lily_sampler* s, const RowArgs* rows, uint32_t n, int
     uint32_t sl = s->force_slices ? s->force_slices : (2 * TARGET_GROUPS + n - 1) / n;
     const uint32_t e = dtype == LILY_BF16 ? 8 : 4;
     const uint32_t nch = (vocab + 2 * (e - 1)) / e + 1;
-    // (no finer than a block a slice, unless that leaves fewer than four lanes for each of the k)
-    const uint32_t by_block = std::max((nch + 256u * STREAM_UNROLL - 1) / (256u * STREAM_UNROLL), (4u * kmax + 255u) / 256u);
+    // (no finer than a block a slice, unless that leaves fewer than two lanes for each of the k - four, up to two
+    // workgroups a compute unit: f32 rows of 32 003, no top_k, in 16 slices and in 8, 4 rows 22.1 and 22.5 us, 16 rows 26.3 and 33.5,
+    // 40 rows 28.8 and 26.3, 64 rows 33.6 and 27.6; 64 bf16 rows of 49 152 44.5 and 34.7)
+    const uint32_t by_four = (4u * kmax + 255u) / 256u;
+    const uint32_t by_lanes = (uint64_t)n * by_four <= WIDE_FINE_GROUPS ? by_four : (2u * kmax + 255u) / 256u;
+    const uint32_t by_block = std::max((nch + 256u * STREAM_UNROLL - 1) / (256u * STREAM_UNROLL), by_lanes);
     sl = sl > by_block ? by_block : sl;
     sl = sl > MAX_SLICES ? MAX_SLICES : sl;
     if ((uint64_t)n * MERGE_CAP > s->ws_slots) {   // a row's list of candidates: MERGE_CAP slots

@@ -294,6 +294,14 @@ def test_bounds_over_the_slices(sampler, rows, vocab, bf16):
         _check_logprob(r.logprobs[i], d.logprob, i)
 
 
+@pytest.mark.parametrize("rows,vocab,bf16", [(32, 32_003, True), (33, 32_003, True), (64, 32_003, False), (70, 66_585, True), (40, 9_001, False),
+                                             (128, 66_585, True)])
+def test_bounds_over_fewer_slices(sampler, rows, vocab, bf16):
+    """The same where short rows are cut for four lanes to each of the k (512 workgroups) and for two, in one launch
+    and, past 1 024 workgroups, in two."""
+    test_bounds_over_the_slices(sampler, rows, vocab, bf16)
+
+
 @pytest.mark.parametrize("looks", ["0,8192", "8192,0", "1,1"], ids=["no key", "no maxima", "one look"])
 @pytest.mark.parametrize("rows,bf16", [(2, False), (6, False), (6, True), (20, True)])
 def test_slices_that_stop_waiting_for_each_other(monkeypatch, rows, bf16, looks):
