@@ -357,6 +357,26 @@ uint32_t choose_slices(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint
     return sl < 1 ? 1 : sl;
 }
 
+// Whether every row of a launch is a draw that the kernels of rows_held.hip and rows_blocks.hip take, and what some row has
+// of a mask, a mask or a bias list, penalties, a log-probability.
+struct HeldRows {
+    bool all = true, masked = false, extra = false, pen = false, lse = false;
+    void add(const RowArgs& row) {
+        all = all && row.mode != MODE_ARGMAX && (row.flags & F_STREAM) != 0;
+        masked = masked || row.allow != nullptr;
+        extra = extra || row.allow != nullptr || row.n_bias != 0;
+        pen = pen || (row.flags & F_PEN) != 0;
+        lse = lse || row.out_logprob != nullptr;
+    }
+};
+HeldRows held_rows(const RowArgs* rows, uint32_t n) {
+    HeldRows h;
+    for (uint32_t i = 0; i < n && h.all; ++i) {
+        h.add(rows[i]);
+    }
+    return h;
+}
+
 // Rows of few candidates whose slices a workgroup can hold in registers (rows_held.hip): how many blocks
 // of 256 x STREAM_UNROLL pieces of 16 bytes a slice then has, and how many slices a row.  blocks 0: not this way.
 struct HeldShape {
@@ -372,7 +392,11 @@ constexpr uint32_t HELD_MAX_GROUPS[3] = {0, 1024, 768};
 // Rows with masks too, and in slices of two blocks up to a workgroup a compute unit (2 % admitted: 30 rows, k = 50,
 // 21.8 -> 19.6, 64 rows in slices of two blocks 21.8 -> 27.3; 16 f32 rows of 248 320, k = 64, 23.6 -> 24.0 in two).
 constexpr uint32_t HELD_MAX_GROUPS_LISTED = 768, HELD_MAX_GROUPS_EXTRA[3] = {0, 600, 256};
-HeldShape held_shape(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint32_t vocab, int dtype, bool pen, bool lse, bool extra) {
+// ... and, where one slice does not do, in at least so many, as long as those fit: most of what a mask admits reaches
+// the bound of a slice that has few of them, and is ranked there (bf16, 2 % admitted, k = 50, 16 rows of 9 001 in two slices and in nine
+// 21.0 and 18.6, of 20 000 in three 20.9 and 17.4, of 32 003 in four 23.7 and 20.1; streamed 19.9, 22.7 and 21.7; 5 000 in one 15.6 and 16.3).
+constexpr uint32_t HELD_MASKED_SLICES = 9;
+HeldShape held_shape(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint32_t vocab, int dtype, const HeldRows& is) {
     HeldShape out;
     if (s->force_path != 0 || s->no_held || s->only_blocks || kmax > STREAM_K_MAX || rows > s->ws_rows) {
         return out;
@@ -381,16 +405,19 @@ HeldShape held_shape(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint32
     const uint32_t nch = (vocab + 2 * (e - 1)) / e + 1;   // wherever the row starts
     for (uint32_t blocks = 1; blocks <= 2 && out.blocks == 0; ++blocks) {
         const uint32_t per = blocks * 256u * STREAM_UNROLL, least = (nch + per - 1) / per;
-        const uint32_t sl = s->force_slices > least ? s->force_slices : least;
+        uint32_t sl = s->force_slices > least ? s->force_slices : least;
+        if (is.masked && blocks == 1 && least > 1 && s->force_slices == 0) {
+            sl = std::max(sl, std::min(HELD_MASKED_SLICES, HELD_MAX_GROUPS_EXTRA[1] / rows));
+        }
         if (sl > MAX_SLICES || (s->force_slices != 0 && s->force_slices < least) ||
             (sl > WAVE_MERGE_LISTS && sl * kmax > HELD_MERGE_SLOTS) ||
             (uint64_t)rows * sl * kmax > s->ws_slots || (uint64_t)rows * sl > HELD_MAX_GROUPS[blocks]) {
             continue;
         }
-        if (extra && (uint64_t)rows * sl > HELD_MAX_GROUPS_EXTRA[blocks]) {
+        if (is.extra && (uint64_t)rows * sl > HELD_MAX_GROUPS_EXTRA[blocks]) {
             continue;
         }
-        if (pen && ((!lse && (uint64_t)rows * sl > HELD_MAX_GROUPS_LISTED) || (blocks == 2 && dtype == LILY_BF16))) {
+        if (is.pen && ((!is.lse && (uint64_t)rows * sl > HELD_MAX_GROUPS_LISTED) || (blocks == 2 && dtype == LILY_BF16))) {
             continue;
         }
         out.blocks = blocks;
@@ -446,22 +473,6 @@ uint32_t blocks_slices(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint
     const uint64_t by_ws = (uint64_t)s->ws_slots / ((uint64_t)rows * kmax);
     sl = sl > by_ws ? (uint32_t)by_ws : sl;
     return sl < 1 ? 1 : sl;
-}
-
-// Whether every row of a launch is a draw that those kernels take, and what some row has of a mask or a bias
-// list, penalties, a log-probability.
-struct HeldRows {
-    bool all = true, extra = false, pen = false, lse = false;
-};
-HeldRows held_rows(const RowArgs* rows, uint32_t n) {
-    HeldRows h;
-    for (uint32_t i = 0; i < n && h.all; ++i) {
-        h.all = rows[i].mode != MODE_ARGMAX && (rows[i].flags & F_STREAM) != 0;
-        h.extra = h.extra || rows[i].allow != nullptr || rows[i].n_bias != 0;
-        h.pen = h.pen || (rows[i].flags & F_PEN) != 0;
-        h.lse = h.lse || rows[i].out_logprob != nullptr;
-    }
-    return h;
 }
 
 constexpr uint32_t MASKED_MAX_ROWS = 256;
@@ -682,7 +693,7 @@ uint32_t plan_parts(const lily_sampler* s, RowArgs* table, uint32_t rows, int dt
     // (a launch that holds its slices takes both kinds alike)
     const HeldRows whole = held_rows(table, rows);
     const bool together =
-        whole.all && held_shape(s, rows, max_k(table, rows), vocab, dtype, whole.pen, whole.lse, whole.extra).blocks != 0;
+        whole.all && held_shape(s, rows, max_k(table, rows), vocab, dtype, whole).blocks != 0;
     const bool split = !together && heavy != 0 && rows - heavy >= SPLIT_MIN_LIGHT;
     if (split) {
         std::stable_partition(table, table + rows,
@@ -705,7 +716,7 @@ uint32_t plan_parts(const lily_sampler* s, RowArgs* table, uint32_t rows, int dt
         part.extra = is.extra;
         part.pen = is.pen;
         if (is.all) {
-            const HeldShape held = held_shape(s, part.rows, part.ws_k, vocab, dtype, is.pen, is.lse, is.extra);
+            const HeldShape held = held_shape(s, part.rows, part.ws_k, vocab, dtype, is);
             const uint32_t blocks = held.blocks == 0 && !is.extra && part.rows <= s->ws_rows
                                         ? blocks_slices(s, part.rows, part.ws_k, vocab, dtype, is.pen, is.lse) : 0u;
             part.held = held.blocks;
@@ -786,7 +797,7 @@ int launch_inline(lily_sampler* s, int dtype, uint32_t vocab, const InlineRows& 
     }
     const HeldRows is = held_rows(rows.r, n);
     const HeldShape held =
-        !chained && is.all ? held_shape(s, n, kmax, vocab, dtype, is.pen, is.lse, is.extra) : HeldShape();
+        !chained && is.all ? held_shape(s, n, kmax, vocab, dtype, is) : HeldShape();
     const bool masked = !chained && !verify && all_masked(s, rows.r, n, vocab, kmax);
     const uint32_t slices = held.blocks != 0 ? held.slices : choose_slices(s, n, kmax, vocab, dtype);
     fill_cfg(s, &cfg, n, vocab, slices, kmax, 0, nullptr);
@@ -1264,7 +1275,7 @@ uint32_t lily_sampler_slices_for(const lily_sampler_t* s, uint32_t rows, uint32_
     if (s == nullptr || rows == 0) {
         return 0;
     }
-    const HeldShape held = held_shape(s, rows, k ? k : 1, vocab, (int)dtype, false, false, false);
+    const HeldShape held = held_shape(s, rows, k ? k : 1, vocab, (int)dtype, HeldRows());
     const uint32_t blocks = blocks_slices(s, rows, k ? k : 1, vocab, (int)dtype, false, false);
     return held.blocks != 0 ? held.slices : blocks != 0 ? blocks : choose_slices(s, rows, k ? k : 1, vocab, (int)dtype);
 }
@@ -2128,7 +2139,8 @@ int rows_with_tiles(lily_sampler* s, const lily_lm_head* h, const lily_rows* b, 
     // Rows under penalties whose slices can be held in registers are drawn from their logits at once (masks: most
     // rows are drawn from a few tiles): the launch that would stand behind the draws from summaries anyway is no slower for drawing them
     // all (4 rows under penalties 17 us, 23 with the summaries first; 24 rows 27 and 31).
-    bool held = true, behind_pen = false, behind_lse = false, behind_extra = false;
+    bool held = true;
+    HeldRows rows_behind;
     uint32_t behind = 0, behind_k = 1;
     for (uint32_t r = 0; r < rows; ++r) {
         const RowArgs& row = packed[r];
@@ -2136,16 +2148,13 @@ int rows_with_tiles(lily_sampler* s, const lily_lm_head* h, const lily_rows* b, 
         const bool pen = serve && row.mode != MODE_ARGMAX && ((row.flags & F_PEN) != 0 || row.allow != nullptr);
         group_of[r] = !serve ? 2 : (pen ? 1 : 0);
         if (group_of[r] != 0) {
-            const HeldRows is = held_rows(&row, 1);
-            held = held && is.all && (!serve || row.allow == nullptr);
-            behind_pen = behind_pen || is.pen;
-            behind_lse = behind_lse || is.lse;
-            behind_extra = behind_extra || is.extra;
+            rows_behind.add(row);
+            held = held && rows_behind.all && (!serve || row.allow == nullptr);
             behind += 1;
             behind_k = row.k > behind_k ? row.k : behind_k;
         }
     }
-    held = held && behind != 0 && held_shape(s, behind, behind_k, b->vocab, (int)b->dtype, behind_pen, behind_lse, behind_extra).blocks != 0;
+    held = held && behind != 0 && held_shape(s, behind, behind_k, b->vocab, (int)b->dtype, rows_behind).blocks != 0;
     auto scale_of_row = [&](uint32_t r) { return std::isfinite(packed[r].c2) ? packed[r].c2 : 0.0f; };
     // Few rows, none of which the summaries may decline: everything travels with the launches (carried to the
     // device by a kernel of its own the descriptors cost 2.8 of the 223 us of four rows over bf16 weights).

@@ -344,3 +344,40 @@ def test_dense_histories_stay_a_block_at_a_time(monkeypatch, bf16, raising):
     for t in scratch:
         t.close()
     s.close()
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+@pytest.mark.parametrize("rows,vocab", [(3, 4099), (3, 8205), (20, 9001), (70, 20_000), (100, 32_003), (299, 9001), (301, 9001)])
+def test_masked_rows_in_more_slices(monkeypatch, bf16, rows, vocab):
+    """Masks over rows a little longer than a block, in as many slices as are asked for of such rows, as the launch has room
+    for, and in two; the first of the masks admits nothing, the next ones one id, all ids, the last eight; one row draws a forced id."""
+    rng = np.random.default_rng(rows + vocab)
+    x = rng.normal(0, 3, (rows, vocab)).astype(np.float32)
+    x[1] = 1.5
+    allow = np.stack([W.allow_mask(rng, vocab, frac=0.02) for _ in range(rows)])
+    allow[0] = 0
+    allow[1] = 0
+    allow[1, vocab // 64] = 1
+    allow[2] = 0xffffffff
+    if vocab % 32:
+        allow[2, -1] = (1 << vocab % 32) - 1
+    if rows > 3:
+        allow[3] = 0
+        for i in range(vocab - 8, vocab):
+            allow[3, i >> 5] |= np.uint32(1 << (i & 31))
+    xs = W.to_bf16_bits(x) if bf16 else x
+    kw = [dict(temperature=0.8, top_k=(50, 64, 3, 20)[i % 4], top_p=0.95, seed=40 + i) for i in range(rows)]
+    forced = [i if i == rows // 2 and i > 3 else None for i in range(rows)]
+    s = _sampler(monkeypatch, "1")
+    for lp in (False, True):
+        r = run_rows(s, xs, kw, [2] * rows, allow=allow, forced=forced, logprobs=lp)
+        some = sorted({*range(min(6, rows)), rows // 2, rows - 1})
+        for i in some:
+            if forced[i] is not None:
+                assert r.ids[i] == forced[i]
+                continue
+            d = O.sample(xs[i], None, o_params(**kw[i]), 2, allow=allow[i], want_logprob=lp)
+            check_row_against_oracle(r, i, d)
+            if lp and np.isfinite(d.logprob):
+                assert abs(r.logprobs[i] - d.logprob) <= 1e-5 * max(1.0, abs(d.logprob)), (i, r.logprobs[i], d.logprob)
+    s.close()
