@@ -13,6 +13,11 @@
 // select_lowering.h 107 / 136 / 285; given up to the exhaustive select, as such slices once were, 670 to 680), half of the first
 // tenth listed 52 (79).
 //
+// Clusters of likely ids fill some waves and leave others what lies behind; the bound is the poorest wave's, and all of a
+// cluster reaches it.  A wave whose list might run over goes on behind a bound of its own, from its chunks and its list, which
+// it makes short.  (600 bf16 rows of 151 936, k = 20, 1 000 neighbours 9 above the rest: 54 us, the streaming select 49;
+// 2 480 when such slices were given up.  3 000 inside the row: 49, 43 and 2 480.  For rows without clusters the look costs 0.3 to 0.6 us.)
+//
 // Bound: the vector unit where the row's sum takes most values (200 rows of 248 320 bf16, N(0, 2^2), under penalties:
 // 50 us a launch for 99 MB, 25 vector instructions a value, which keep the unit busy two thirds of the time; 74 through
 // the flat form of select_lowering.h, whose scan spends fewer but behind whose scan the noted chunks are looked at again), the memory
@@ -38,7 +43,7 @@ namespace lily {
 
 namespace {
 
-constexpr uint32_t LIST_SEG = 512;                   // values a wave lists over its slice
+constexpr uint32_t LIST_SEG = 640;                   // values a wave lists: 64 chunks', and 64 candidates with their ties
 constexpr uint32_t LIST_CAP = LIST_SEG * NWAVE;
 constexpr uint32_t FINAL_CAP = 512;                  // ... of which so many reach the last bound
 constexpr uint32_t NOTE_SEG = 512;                   // listed ids a wave notes before it evaluates them
@@ -130,7 +135,7 @@ __device__ __forceinline__ bool blocks_row(const LILY_CONST RowArgs* src, const 
     // A term below 2^-21 / vocab of the largest one cannot move the row's sum by more than 2^-21 of it.
     const float lse_cut = (log2f((float)vocab) + 21.0f) * (a.temperature * 0.6931471805599453f);
     float lane_max = ev;        // of true values
-    float T = F32_LOWEST;       // the bound, the same in every thread
+    float T = F32_LOWEST;       // the bound, the same in every thread of a wave
     float skip = NEG_INF;       // chunks at or below it are left out of the sum
     float ref = F32_LOWEST;     // the wave's reference: terms are 2^(x * c2 - ref)
     double sum = 0.0;
@@ -180,11 +185,70 @@ __device__ __forceinline__ bool blocks_row(const LILY_CONST RowArgs* src, const 
     };
     // A listed id's true value, t (NEG_INF in lanes without one), once there is a bound.
     auto take = [&](float t, uint32_t id) {
-        list(t >= T, t, id);
+        const bool in = t >= T;
+        list(in, t, id);
         if (LSE && want_lse) {
             raise(t);
             const double d = __builtin_fma((double)t, (double)a.c2, -(double)ref);
-            sum += t < T && d > -1000.0 ? pow2_d(d) : 0.0;
+            sum += !in && d > -1000.0 ? pow2_d(d) : 0.0;
+        }
+    };
+    // The wave's list made short: the k-th largest value on it is a bound (this wave's from here on, a little below it as
+    // ever), what does not reach it goes into the sum.  (Ties stay; with too many of them the list overflows.)
+    // (It is rare, and read from LDS over and over: what it would hold in registers the blocks need.)
+    auto compact = [&]() {
+        const uint32_t n = min(fill, LIST_SEG);
+        uint32_t found = 0u;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // (LDS of this wave: in order already)
+        __builtin_amdgcn_wave_barrier();
+        const uint32_t* values = reinterpret_cast<const uint32_t*>(pairs + w * LIST_SEG) + 1;   // (the upper halves)
+        auto key_of = [&](uint32_t i0) -> uint32_t {   // 0 past the last
+            const uint32_t key = lilym_order_key(lilym_bits_f32(values[2u * min(i0 + lane, LIST_SEG - 1u)]));
+            return i0 + lane < n ? key : 0u;
+        };
+        uint32_t hi = 0u, lo = 0xffffffffu;
+#pragma unroll 5
+        for (uint32_t i0 = 0; i0 < LIST_SEG; i0 += 64u) {
+            const uint32_t key = key_of(i0);
+            hi = max(hi, key);
+            lo = key != 0u ? min(lo, key) : lo;
+        }
+        hi = wave_max_u32(hi);
+        lo = wave_min_u32(lo);
+        if (n < a.k) {
+            return;
+        }
+        // (from the first bit in which the values differ to where just k reach)
+        const int bits = hi != lo ? 32 - __builtin_clz(hi ^ lo) : 0;
+        found = bits < 32 ? hi >> bits << bits : 0u;
+#pragma unroll 1
+        for (int bit = bits - 1; bit >= 0; --bit) {
+            const uint32_t at = found | (1u << bit);
+            uint32_t reach = 0;
+#pragma unroll 5
+            for (uint32_t i0 = 0; i0 < LIST_SEG; i0 += 64u) {
+                reach += (uint32_t)__popcll(__ballot(key_of(i0) >= at));
+            }
+            found = reach >= a.k ? at : found;
+            if (reach == a.k) {
+                break;
+            }
+        }
+        T = fmaxf(T, lower_by_slack(lilym_key_value(found)));
+        fill = 0u;
+#pragma unroll 1
+        for (uint32_t i0 = 0; i0 < n; i0 += 64u) {   // (what stays moves to places that have been read)
+            const uint64_t p = pairs[w * LIST_SEG + min(i0 + lane, n - 1u)];
+            __builtin_amdgcn_wave_barrier();
+            const float x = lilym_bits_f32((uint32_t)(p >> 32));
+            const bool there = i0 + lane < n, stays = there && x >= T;
+            list(stays, x, (uint32_t)p);
+            __builtin_amdgcn_wave_barrier();
+            if (LSE && want_lse) {
+                raise(there && !stays ? x : NEG_INF);
+                const double d = __builtin_fma((double)x, (double)a.c2, -(double)ref);
+                sum += there && !stays && d > -1000.0 ? pow2_d(d) : 0.0;
+            }
         }
     };
     // The noted ids, by the wave that noted them, four a lane with all loads in flight.
@@ -194,6 +258,9 @@ __device__ __forceinline__ bool blocks_row(const LILY_CONST RowArgs* src, const 
         __builtin_amdgcn_wave_barrier();
 #pragma unroll 1
         for (uint32_t e0 = 0; e0 < n; e0 += 256u) {
+            if (fill > LIST_SEG - 256u && fill <= LIST_SEG) {
+                compact();
+            }
             uint32_t id[4], count[4];
             float x[4];
 #pragma unroll
@@ -219,6 +286,9 @@ __device__ __forceinline__ bool blocks_row(const LILY_CONST RowArgs* src, const 
     auto settle = [&](uint32_t b, uint32_t left, bool bounded) {
 #pragma unroll 1
         while (__ballot(left != 0u) != 0ull) {
+            if (bounded && fill > LIST_SEG - 256u && fill <= LIST_SEG) {
+                compact();
+            }
             uint32_t id[4], count[4];
             float x[4];
             bool in[4];
@@ -337,7 +407,7 @@ __device__ __forceinline__ bool blocks_row(const LILY_CONST RowArgs* src, const 
                 lane_max = max2_raw(lane_max, cm[u]);
             }
             refresh();
-            if (T == F32_LOWEST) {   // (the same in every thread: what is not listed does not suffice for a bound)
+            if (T == F32_LOWEST) {   // (the same in every thread as yet: what is not listed does not suffice for a bound)
                 settle(b, bits(), false);
                 refresh();
             }
@@ -377,9 +447,40 @@ __device__ __forceinline__ bool blocks_row(const LILY_CONST RowArgs* src, const 
                 refresh();
             }
         }
+        // Values that might not all find a place: a cluster of likely ids, of which the other waves have few, whose
+        // bounds are the least.  Behind the k-th largest of the block's chunks no more than k have any, and a list of k is there.
+        uint64_t reaches[U];
+        uint32_t reaching = 0;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const bool some = __ballot(cm[u] >= T) != 0ull;
+            reaches[u] = __ballot(cm[u] >= T);
+            reaching += (uint32_t)__popcll(reaches[u]);
+        }
+        if (fill + (uint32_t)E * reaching > LIST_SEG && fill <= LIST_SEG) {
+            uint32_t key[U], found = 0u;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                key[u] = cm[u] > NEG_INF ? lilym_order_key(cm[u]) >> 16 : 0u;
+            }
+#pragma unroll 1
+            for (uint32_t bit = 0x8000u; bit != 0u; bit >>= 1) {
+                uint32_t reach = 0;
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    reach += (uint32_t)__popcll(__ballot(key[u] >= (found | bit)));
+                }
+                found = reach >= a.k ? found | bit : found;
+            }
+            T = found != 0u ? fmaxf(T, lower_by_slack(lilym_key_value(found << 16))) : T;
+            compact();
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                reaches[u] = __ballot(cm[u] >= T);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool some = reaches[u] != 0ull;
             const bool summed = LSE && want_lse && __ballot(cm[u] > skip) != 0ull;
             if (!some && !summed) {
                 continue;
@@ -422,6 +523,19 @@ __device__ __forceinline__ bool blocks_row(const LILY_CONST RowArgs* src, const 
     if (nblocks == 0u) {
         refresh();
     }
+    if (fill > FINAL_CAP / NWAVE && fill <= LIST_SEG) {
+        // (what all waves list is to be ranked in one piece)
+        uint32_t reach = 0;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        for (uint32_t i0 = 0; i0 < fill; i0 += 64u) {
+            const float x = lilym_bits_f32((uint32_t)(pairs[w * LIST_SEG + min(i0 + lane, fill - 1u)] >> 32));
+            reach += (uint32_t)__popcll(__ballot(i0 + lane < fill && x >= T));
+        }
+        if (reach > FINAL_CAP / NWAVE) {
+            compact();
+        }
+    }
     if (__ballot(edge != 0xffffffffu) != 0ull) {
         list(ev >= T && ev > NEG_INF, ev, edge);
         if (LSE && want_lse) {
@@ -441,6 +555,7 @@ __device__ __forceinline__ bool blocks_row(const LILY_CONST RowArgs* src, const 
     }
     if (lane == 0u) {
         sh.qfill[w] = fill;
+        sh.bound[parity][w] = T;
     }
     if (tid == 0u) {
         sh.n_fc = 0u;
@@ -459,6 +574,7 @@ __device__ __forceinline__ bool blocks_row(const LILY_CONST RowArgs* src, const 
         total += sh.qfill[i];
         ends[i] = total;
         overflow = overflow || sh.qfill[i] > LIST_SEG;
+        T = fmaxf(T, sh.bound[parity][i]);   // (any wave's)
     }
     double mc = 0.0, rest = 0.0;   // the reference of the slice's sum, and the sum of what was not listed
     if (LSE && want_lse) {

@@ -7,7 +7,10 @@
 // Here each thread keeps its 16 to 64 values, turns the few that bias list, mask or penalties touch
 // into their true ones where they lie, and from there on every row is a plain one: the bound is one of
 // true values, what reaches it is listed once, and nothing can fail but the list's place (ties by
-// the thousand), where the exhaustive select takes over.
+// the thousand), where the exhaustive select takes over.  Ids that are admitted, or likely, in clusters
+// fill some waves and leave others nothing: the bound then comes from the chunks of 16 bytes (64 bf16 rows of 50 257, k = 50,
+// 30 % admitted in runs of 128: 27 us, 85 streamed; 4 rows under penalties, 1 000 neighbours 9 above the rest, 18.5 and 90.
+// With the waves' bounds alone such slices were given up: 333 and 98).
 #include <type_traits>
 
 #include "launch.h"
@@ -27,7 +30,7 @@ constexpr uint32_t HELD_CAP = HELD_SEG * NWAVE;
 // and the tail begin at the front again.
 constexpr uint32_t HELD_LDS_BYTES = LILY_SAMPLE_K_CAP * 8 + 3 * LILY_SAMPLE_K_CAP * 4;
 static_assert(HELD_MERGE_SLOTS == WAVE_MERGE_SLOTS, "held rows: what one wave merges");
-static_assert(HELD_LDS_BYTES >= (HELD_CAP + 64 + 128 + 64) * 8 && HELD_LDS_BYTES >= WAVE_MERGE_SLOTS * 8, "held rows: LDS layout");
+static_assert(HELD_LDS_BYTES >= (HELD_CAP + 64 + NT + NT / 4) * 8 && HELD_LDS_BYTES >= WAVE_MERGE_SLOTS * 8, "held rows: LDS layout");
 
 // Workgroups a compute unit shall hold: by the registers that the values take.
 template <int DT, int NB>
@@ -253,19 +256,60 @@ __device__ __forceinline__ bool held_row(const LILY_CONST RowArgs* src, const La
         T = fminf(T, sh.bound[0][i]);
         top = fmaxf(top, sh.wmax[0][i]);
     }
-    if (T == F32_LOWEST) {
-        // (Masks: a wave with fewer values than its share.  Any wave's k-th largest lane maximum is a bound too.)
-        const uint32_t Pk = wave_kth_key16(lane_max > NEG_INF ? (lilym_order_key(lane_max) >> 16) : 0u, a.k);
-        if (lane == 0u) {
-            sh.bound[1][w] = Pk != 0u ? lilym_key_value(Pk << 16) : F32_LOWEST;
+    // The k-th largest of the chunks' largest values, of all the waves' (which all call) or of this one's; F32_LOWEST where
+    // fewer than k have one.
+    auto chunks_bound = [&](bool all) -> float {
+        uint32_t key[C], found = 0;
+#pragma unroll
+        for (int u = 0; u < C; ++u) {
+            key[u] = cm[u] > NEG_INF ? lilym_order_key(cm[u]) >> 16 : 0u;
         }
-        __syncthreads();
-        for (int i = 0; i < NWAVE; ++i) {
-            T = fmaxf(T, sh.bound[1][i]);
+        // (the first look: whether k have any)
+#pragma unroll 1
+        for (int bit = 16; bit >= 0; --bit) {
+            const uint32_t at = bit == 16 ? 1u : found | (1u << bit);
+            uint32_t reach = 0;
+#pragma unroll
+            for (int u = 0; u < C; ++u) {
+                reach += (uint32_t)__popcll(__ballot(key[u] >= at));
+            }
+            if (all) {
+                uint32_t* counts = sh.hist + (bit & 1) * NWAVE;   // (a barrier lies between a place's readers and its next writer)
+                if (lane == 0u) {
+                    counts[w] = reach;
+                }
+                __syncthreads();
+                reach = counts[0];
+                for (int i = 1; i < NWAVE; ++i) {
+                    reach += counts[i];
+                }
+            }
+            if (bit == 16) {
+                if (reach < a.k) {
+                    break;
+                }
+            } else {
+                found = reach >= a.k ? at : found;
+            }
         }
+        return found != 0u ? lilym_key_value(found << 16) : F32_LOWEST;
+    };
+    if (T == F32_LOWEST && !forced) {
+        // Masks, rows that are mostly -inf: a wave with fewer values than its share.
+        T = chunks_bound(true);
     }
     // (values a little below the bound may share its quotient by the temperature)
     T = forced ? __builtin_huge_valf() : lower_by_slack(T);
+    // Where the bound of the poorest wave lets clusters through whole: the k-th largest of a wave's own chunks is a bound too,
+    // which k of them reach, ties aside, and that much has its place.
+    uint32_t reaching = 0;
+#pragma unroll
+    for (int u = 0; u < C; ++u) {
+        reaching += (uint32_t)__popcll(__ballot(cm[u] >= T));
+    }
+    if (reaching > 64u) {
+        T = fmaxf(T, lower_by_slack(chunks_bound(false)));   // (this wave's from here on)
+    }
     phase(cfg, 2);
 
     // ---- what reaches it is listed, the rest goes into the sum
@@ -384,15 +428,16 @@ __device__ __forceinline__ bool held_row(const LILY_CONST RowArgs* src, const La
                 listed_sum = wave_sum_d(lane < n ? term(x) : 0.0);
             }
         }
-    } else if (!overflow && n <= 128u) {
-        // Up to two waves' worth (k from 40 on): two threads an entry, each counts what it has ahead of
-        // it in one half of the list, sixteen at a time.
-        const uint32_t entry = tid & 127u, half = tid >> 7;
+    } else if (!overflow && n <= NT) {
+        // Up to four waves' worth (k from 40 on, masks): up to two waves' two threads an entry, each counts what it has ahead
+        // of it in one half of the list, sixteen at a time; else a thread an entry.
+        const bool two = n <= NT / 2u;
+        const uint32_t entry = two ? tid & (NT / 2u - 1u) : tid, half = two ? tid / (NT / 2u) : 0u;
         const uint64_t p = entry < n ? pair_at(entry) : 0ull;
         const float x = lilym_bits_f32((uint32_t)(p >> 32));
         const uint64_t mine = entry < n ? composite_of(x / a.temperature, (uint32_t)p) : 0ull;
-        uint64_t* all = ranked + 64;   // [128], then each entry's count in the upper half
-        uint32_t* upper = reinterpret_cast<uint32_t*>(all + 128);
+        uint64_t* all = ranked + 64;   // [NT], then each entry's count in the upper half
+        uint32_t* upper = reinterpret_cast<uint32_t*>(all + NT);
         if (half == 0u) {
             all[entry] = mine;
         }
@@ -407,7 +452,8 @@ __device__ __forceinline__ bool held_row(const LILY_CONST RowArgs* src, const La
         }
         __syncthreads();
         uint32_t ahead = 0;
-        for (uint32_t i = half * 64u; i < min(n, half * 64u + 64u); i += 16u) {
+        const uint32_t to = two ? min(n, half * 64u + 64u) : n;
+        for (uint32_t i = half * 64u; i < to; i += 16u) {
             uint64_t other[16];
 #pragma unroll
             for (int q = 0; q < 16; ++q) {
@@ -423,7 +469,7 @@ __device__ __forceinline__ bool held_row(const LILY_CONST RowArgs* src, const La
         }
         __syncthreads();
         if (half == 0u && mine != 0ull) {
-            ahead += upper[entry];
+            ahead += two ? upper[entry] : 0u;
             if (ahead < 64u) {
                 ranked[ahead] = mine;
             }

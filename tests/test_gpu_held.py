@@ -381,3 +381,82 @@ def test_masked_rows_in_more_slices(monkeypatch, bf16, rows, vocab):
             if lp and np.isfinite(d.logprob):
                 assert abs(r.logprobs[i] - d.logprob) <= 1e-5 * max(1.0, abs(d.logprob)), (i, r.logprobs[i], d.logprob)
     s.close()
+
+
+CLUSTERS = ((0, 40, 9.0), (1000, 300, 9.0), (0, 1000, 30.0), (9000, 3000, 9.0), (700, 12_000, 5.0))
+
+
+def _with_stats(s, fn):
+    stats = torch.zeros(4, dtype=torch.int32, device=dev())
+    s.set_path_stats(stats)
+    try:
+        out = fn()
+    finally:
+        s.synchronize()
+        s.set_path_stats(None)
+    return out, stats.cpu().numpy()
+
+
+@pytest.mark.parametrize("held", ["1", "blocks"], ids=["held", "blocks"])
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+@pytest.mark.parametrize("pen", [False, True], ids=["plain", "penalties"])
+def test_clusters_of_likely_ids(monkeypatch, held, bf16, pen):
+    """Neighbouring ids that lead by far, some forty up to twelve thousand of them, at the row's start and inside: some waves
+    of a slice hold nothing else, others none, and all of the cluster reaches the bound of those.  No slice is
+    given up for it.  With penalties on ids of the clusters, log-probabilities and more slices than a block needs; rows that rise
+    and fall all along are drawn rightly too, whichever way."""
+    vocab = 50_021
+    rng = np.random.default_rng(77)
+    x = rng.normal(0, 2, (len(CLUSTERS) + 2, vocab)).astype(np.float32)
+    for i, (at, n, lift) in enumerate(CLUSTERS):
+        x[i, at:at + n] += lift
+    x[-2].sort()
+    x[-1] = -np.sort(-x[-1])
+    xs = W.to_bf16_bits(x) if bf16 else x
+    rows = len(x)
+    more = dict(repetition_penalty=1.1, presence_penalty=0.2, frequency_penalty=0.1) if pen else {}
+    for slices in (0, 3, 16):
+        s = _sampler(monkeypatch, held, slices)
+        for k, lp in ((64, True), (20, False), (50, True)):
+            kw = [dict(temperature=0.9, top_k=k, top_p=0.99, seed=60 + i, **more) for i in range(rows)]
+            hist = rng.integers(0, 4000, (rows, 1500)).astype(np.int32)
+            for n in (rows, len(CLUSTERS)):
+                sc = counts = None
+                if pen:
+                    sc, counts = [], [np.bincount(hist[i], minlength=vocab).astype(np.uint32) for i in range(n)]
+                    for i in range(n):
+                        t = LS.SamplerScratch(s, vocab)
+                        t.add_history(torch.from_numpy(hist[i]).to(dev()))
+                        sc.append(t)
+                # (the blocks' way takes resident batches only)
+                r, stats = _with_stats(s, lambda: run_rows(s, xs[:n], kw[:n], [3] * n, scratch=sc, logprobs=lp, use_plan=True))
+                _check(r, xs[:n], kw[:n], 3, lp, counts)
+                assert n == rows or stats[2] == 0, (slices, k, stats)
+                for t in sc or []:
+                    t.close()
+        s.close()
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+@pytest.mark.parametrize("vocab", [20_011, 50_257])
+def test_masks_in_clusters(monkeypatch, bf16, vocab):
+    """Masks of runs of 16 to 1 000 ids, 5 to 60 % of them admitted: waves of a slice with hundreds of values beside waves with none.
+    No slice is given up for it."""
+    rng = np.random.default_rng(vocab)
+    rows = 12
+    x = rng.normal(0, 2, (rows, vocab)).astype(np.float32)
+    allow = np.zeros((rows, (vocab + 31) // 32), dtype=np.uint32)
+    for i in range(rows):
+        run, frac = (16, 64, 250, 1000)[i % 4], (0.05, 0.2, 0.6)[i % 3]
+        on = np.repeat(rng.random(vocab // run + 1) < frac, run)[:vocab]
+        ids = np.nonzero(on)[0]
+        np.bitwise_or.at(allow[i], ids >> 5, (1 << (ids & 31)).astype(np.uint32))
+    xs = W.to_bf16_bits(x) if bf16 else x
+    for slices in (0, 13):
+        s = _sampler(monkeypatch, "1", slices)
+        for k in (20, 50, 64):
+            kw = [dict(temperature=0.8, top_k=k, top_p=0.95, seed=80 + i) for i in range(rows)]
+            r, stats = _with_stats(s, lambda: run_rows(s, xs, kw, [5] * rows, allow=allow, logprobs=True))
+            _check(r, xs, kw, 5, True, allow=allow)
+            assert stats[2] == 0, (slices, k, stats)
+        s.close()
