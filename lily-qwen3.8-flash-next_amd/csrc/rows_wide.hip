@@ -60,7 +60,7 @@ __device__ __forceinline__ const LILY_CONST RowArgs* wide_table(const LaunchCfg&
 // One pass over the slice's chunks, four loads in flight per thread, every load unconditional
 // (a chunk number past the slice is replaced by the slice's last).  before(): called once the first loads are on their
 // way; true = what it did had no registers for them, they are made again.
-template <int DT, class B, class F>
+template <int DT, uint32_t THREADS = NT, class B, class F>
 __device__ __forceinline__ void wide_scan(const Geo<DT>& g, B&& before, F&& per_chunk) {
     const uint32_t tid = threadIdx.x;
     if (g.main_hi <= g.main_lo) {
@@ -71,7 +71,7 @@ __device__ __forceinline__ void wide_scan(const Geo<DT>& g, B&& before, F&& per_
     auto fetch = [&](uint32_t c0) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            const uint32_t c = min(c0 + (uint32_t)u * NT + tid, g.main_hi - 1u);
+            const uint32_t c = min(c0 + (uint32_t)u * THREADS + tid, g.main_hi - 1u);
             q[u] = gload(reinterpret_cast<const u32x4*>(g.base + (size_t)c * 16));
         }
     };
@@ -82,12 +82,12 @@ __device__ __forceinline__ void wide_scan(const Geo<DT>& g, B&& before, F&& per_
     for (uint32_t c0 = g.main_lo;;) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            const uint32_t c = c0 + (uint32_t)u * NT + tid;
+            const uint32_t c = c0 + (uint32_t)u * THREADS + tid;
             if (c < g.main_hi) {
                 per_chunk(q[u], c);
             }
         }
-        c0 += 4u * NT;
+        c0 += 4u * THREADS;
         if (c0 >= g.main_hi) {
             break;
         }
@@ -121,12 +121,12 @@ __device__ __forceinline__ uint32_t wide_bits(const uint32_t* words, uint32_t id
 }
 
 // The ids of the partial 16-byte chunks at the slice's ends, one by one.
-template <int DT, class F>
+template <int DT, uint32_t THREADS = NT, class F>
 __device__ __forceinline__ void wide_edges(const RowArgs& a, const Geo<DT>& g, F&& per_id) {
     for (int side = 0; side < 2; ++side) {
         const uint32_t lo = side == 0 ? g.id_lo : g.edge_hi_begin;
         const uint32_t hi = side == 0 ? g.edge_lo_end : g.id_hi;
-        for (uint32_t id = lo + threadIdx.x; id < hi; id += NT) {
+        for (uint32_t id = lo + threadIdx.x; id < hi; id += THREADS) {
             per_id(load_logit<DT>(a.logits, id), id);
         }
     }
@@ -313,21 +313,127 @@ constexpr uint32_t SIXTEEN_OFF_BINS = (LILY_SAMPLE_K_CAP * 8 + 3 * LILY_SAMPLE_K
 constexpr uint32_t SIXTEEN_OFF_PLACED = SIXTEEN_OFF_BINS + SIXTEEN_BINS / 2;
 constexpr uint32_t SIXTEEN_LDS_BYTES = (SIXTEEN_OFF_PLACED + MERGE_CAP) * 8;
 
+// The row's best where more of its values reach the bound than the list holds (a cluster of likely ids, ties by the
+// thousand, no bound): MERGE_CAP at most of them to cand, the k best among them, in any order, by one workgroup.  Histograms of the composites'
+// leading bits, twelve more each time (sixteen composites at most share all but the last four bits), until what lies at or above
+// the k-th one's bin fits.  (4 bf16 rows of 248 320 under penalties, 6 000 neighbours 9 above the rest, 113 us; by the
+// exhaustive select, which looks at every id nine times, 3 850.  4 rows of 50 257, 3 000 neighbours, 50 and 573.)
+template <int DT, uint32_t THREADS>
+__device__ __forceinline__ uint32_t wide_collect(const RowArgs& a, uint32_t vocab, float bound, uint64_t* cand, SixteenShared& six,
+                                                 uint32_t& count) {
+    constexpr int E = Geo<DT>::E;
+    constexpr uint32_t BINS = 4096, OWN = BINS / THREADS;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
+    const bool pen = (a.flags & F_PEN) != 0;   // (of the kind that only lowers: the host sees to it)
+    uint32_t* hist = reinterpret_cast<uint32_t*>(cand);
+    static_assert(BINS * 4u <= MERGE_CAP * 8u, "the histogram lies where the entries will");
+    Geo<DT> g;
+    g.init(a.logits, vocab, 0u, 1u);
+    // fn(composite) of every id whose value reaches the bound
+    auto over = [&](auto&& fn) {
+        auto one = [&](float x, uint32_t id) {
+            if (x >= bound) {
+                x = pen ? wide_worth(a, x, id) : x;   // (never more than the raw value)
+                if (x >= bound) {
+                    fn(composite_of(x / a.temperature, id));
+                }
+            }
+        };
+        wide_scan<DT, THREADS>(g, []() { return false; }, [&](const u32x4& q, uint32_t c) {
+            if (chunk_max<DT>(q) >= bound) {
+                float v[E];
+                unpack<DT>(q, v);
+#pragma unroll
+                for (int j = 0; j < E; ++j) {
+                    one(v[j], g.id_of(c, j));
+                }
+            }
+        });
+        wide_edges<DT, THREADS>(a, g, one);
+    };
+    uint64_t prefix = 0ull;
+    uint32_t above = 0;   // composites above everything under the prefix
+    for (int shift = 52; shift >= 4; shift -= 12) {
+        __syncthreads();
+        for (uint32_t i = tid; i < BINS; i += THREADS) {
+            hist[i] = 0u;
+        }
+        __syncthreads();
+        const uint64_t under = shift == 52 ? 0ull : ~0ull << (shift + 12);
+        over([&](uint64_t c) {
+            if ((c & under) == prefix) {
+                atomicAdd(&hist[(uint32_t)(c >> shift) & (BINS - 1u)], 1u);
+            }
+        });
+        __syncthreads();
+        // from the top: thread t holds bins BINS - OWN (t + 1) .. + OWN - 1
+        uint32_t h[OWN], mine = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < OWN; ++i) {
+            h[i] = hist[BINS - 1u - (tid * OWN + i)];
+            mine += h[i];
+        }
+        const uint32_t incl = wave_scan_u32(mine);
+        if (lane == 63u) {
+            six.wave_u[w] = incl;
+        }
+        __syncthreads();
+        uint32_t before = incl - mine, whole = 0;
+        for (uint32_t i = 0; i < THREADS / 64u; ++i) {
+            before += i < w ? six.wave_u[i] : 0u;
+            whole += six.wave_u[i];
+        }
+        if (above + whole <= MERGE_CAP) {
+            break;   // (all that lies under the prefix)
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < OWN; ++i) {
+            if (above + before < a.k && above + before + h[i] >= a.k) {
+                six.wave_k[0] = ((uint64_t)(BINS - 1u - (tid * OWN + i)) << 32) | (above + before);
+                count = above + before + h[i];
+            }
+            before += h[i];
+        }
+        __syncthreads();
+        prefix |= (six.wave_k[0] >> 32) << shift;
+        above = (uint32_t)six.wave_k[0];
+        if (count <= MERGE_CAP) {
+            break;
+        }
+    }
+    __syncthreads();
+    if (tid == 0) {
+        count = 0;
+    }
+    __syncthreads();
+    over([&](uint64_t c) {
+        if (c >= prefix) {
+            const uint32_t at = atomicAdd(&count, 1u);
+            if (at < MERGE_CAP) {
+                cand[at] = c;
+            }
+        }
+    });
+    __syncthreads();
+    return min(count, MERGE_CAP);
+}
+
 // From a slice's candidates (n_mine of them in cand) to the row's draw, in the workgroup that arrives last.
-// gave_up: the slice has none because it did not learn the row's bound; the row is then taken
-// by the select that is right for any input.
+// bound: the row's; gave_up: the slice has none because it did not learn it, and looks at the whole row
+// should it finish it.  HELD: of k_wide_held (the second launch of two, which are many rows, keeps the exhaustive select: with
+// wide_collect() in it 128 f32 rows of 131 072 take 59 to 62 us instead of 54).
 // Sixteen waves sort, and the first four draw.
-template <int DT, bool LSE, uint32_t THREADS = NT>
+template <int DT, bool LSE, uint32_t THREADS, bool HELD>
 __device__ __forceinline__ void wide_finish(const LILY_CONST RowArgs* src, const LaunchCfg& cfg, const WideArgs& w, Shared& sh,
-                                            uint32_t& n_mine, uint64_t* cand, uint32_t row, uint32_t S, bool gave_up,
-                                            SixteenShared* six = nullptr) {
+                                            uint32_t& n_mine, uint64_t* cand, uint32_t row, uint32_t S, float bound, bool gave_up,
+                                            SixteenShared& six) {
     constexpr bool SIXTEEN = THREADS == SIXTEEN_THREADS;
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     __syncthreads();
     WIDE_MARK(6);
     // The slice's candidates go behind those the row's other slices have left (any order: the
     // select does not care).  A row whose list would pass MERGE_CAP is counted on and not
-    // written: the last workgroup sees the count and takes the exhaustive select.
+    // written: the last workgroup sees the count and collects them itself.
     const uint32_t mine = gave_up ? MERGE_CAP + 1u : n_mine;
     if (tid == 0) {
         n_mine = __hip_atomic_fetch_add(&w.count[row], mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -365,31 +471,35 @@ __device__ __forceinline__ void wide_finish(const LILY_CONST RowArgs* src, const
     if (tid == 0) {
         store_through(&w.count[row], 0u);
     }
-    uint32_t n;
-    bool sorted = false;
-    if (total > MERGE_CAP) {
-        // more than the buffers hold (values that tie by the thousand, a row in ascending
-        // order): the select that is right for any input, over the whole row
-        __syncthreads();
-        if (SIXTEEN && tid >= NT) {
-            return;   // (four waves' work: a barrier waits for those that are left)
-        }
+    uint32_t n = 0, found = total;
+    bool sorted = false, exhausted = false;
+    if (SIXTEEN) {
         cand = dyn_lds;
-        select_exhaustive<DT>(a, 0, cfg.vocab, a.k, want_lse, cand, min(cfg.dyn_slots, MERGE_CAP), sh);
-        n = min(sh.n_cand, min(cfg.dyn_slots, MERGE_CAP));
-        if (cfg.path_stats != nullptr && tid == 0) {
-            atomicAdd(&cfg.path_stats[2], 1u);
-        }
-    } else {
-        if (total > (uint32_t)FIRST * THREADS) {   // (the same in every thread)
+    }
+    if (total > MERGE_CAP) {   // (the same in every thread)
+        if constexpr (HELD) {
+            found = wide_collect<DT, THREADS>(a, cfg.vocab, gave_up ? F32_LOWEST : bound, cand, six, n_mine);
 #pragma unroll
-            for (int j = FIRST; j < PER; ++j) {
-                mine_c[j] = handed_load(cfg.ws_cand, (size_t)row * MERGE_CAP + tid + (uint32_t)j * THREADS);
+            for (int j = 0; j < PER; ++j) {
+                mine_c[j] = cand[tid + (uint32_t)j * THREADS];
             }
+        } else {
+            __syncthreads();
+            select_exhaustive<DT>(a, 0, cfg.vocab, a.k, want_lse, cand, min(cfg.dyn_slots, MERGE_CAP), sh);
+            n = min(sh.n_cand, min(cfg.dyn_slots, MERGE_CAP));
+            exhausted = true;
         }
+        __syncthreads();
+    } else if (total > (uint32_t)FIRST * THREADS) {
+#pragma unroll
+        for (int j = FIRST; j < PER; ++j) {
+            mine_c[j] = handed_load(cfg.ws_cand, (size_t)row * MERGE_CAP + tid + (uint32_t)j * THREADS);
+        }
+    }
+    if (!exhausted) {
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
-            if (tid + (uint32_t)j * THREADS >= total) {
+            if (tid + (uint32_t)j * THREADS >= found) {
                 mine_c[j] = 0ull;
             }
         }
@@ -412,23 +522,22 @@ __device__ __forceinline__ void wide_finish(const LILY_CONST RowArgs* src, const
         __syncthreads();
         WIDE_MARK(13);
         if constexpr (SIXTEEN) {
-            n = min(total, a.k);
-            sort_by_sixteen(mine_c, total, n, dyn_lds, reinterpret_cast<uint32_t*>(dyn_lds + SIXTEEN_OFF_BINS), dyn_lds + SIXTEEN_OFF_PLACED, *six);
+            n = min(found, a.k);
+            sort_by_sixteen(mine_c, found, n, dyn_lds, reinterpret_cast<uint32_t*>(dyn_lds + SIXTEEN_OFF_BINS), dyn_lds + SIXTEEN_OFF_PLACED, six);
             sorted = true;
-            cand = dyn_lds;
         } else {
-            sorted = wg_sort_topk(cand, mine_c, total, a.k, sh, n);
+            sorted = wg_sort_topk(cand, mine_c, found, a.k, sh, n);
             if (!sorted) {
-                n = wg_select_topk(cand, total, a.k, sh);
+                n = wg_select_topk(cand, found, a.k, sh);
             }
         }
-        WIDE_MARK(14);
-        if (cfg.path_stats != nullptr && tid == 0) {
-            atomicAdd(&cfg.path_stats[1], 1u);
-        }
-        if (SIXTEEN && tid >= NT) {
-            return;
-        }
+    }
+    WIDE_MARK(14);
+    if (cfg.path_stats != nullptr && tid == 0) {
+        atomicAdd(&cfg.path_stats[total > MERGE_CAP ? 2 : 1], 1u);
+    }
+    if (SIXTEEN && tid >= NT) {
+        return;   // (the draw is four waves' work: a barrier waits for those that are left)
     }
     tail<DT, true>(a, cfg.vocab, step, n, sorted, cand, sh, cfg);
 }
@@ -440,6 +549,7 @@ __global__ __launch_bounds__(NT, 4) void k_wide_draw(InlineRows rows_arg, Launch
     __shared__ Shared sh;
     __shared__ uint32_t n_mine;
     __shared__ float row_bound;
+    __shared__ SixteenShared none;   // (four waves: not used)
     constexpr int E = Geo<DT>::E;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, s = blockIdx.x, row = blockIdx.y, S = cfg.slices;
     if (cfg.served != nullptr && *(const LILY_CONST uint32_t*)(cfg.served + row) != 0u) {
@@ -502,7 +612,7 @@ __global__ __launch_bounds__(NT, 4) void k_wide_draw(InlineRows rows_arg, Launch
         }
     });
     wide_edges<DT>(a, g, [&](float x, uint32_t id) { offer(x, id); });
-    wide_finish<DT, LSE>(wide_table<INLINE>(cfg) + row, cfg, w, sh, n_mine, cand, row, S, false);
+    wide_finish<DT, LSE, NT, false>(wide_table<INLINE>(cfg) + row, cfg, w, sh, n_mine, cand, row, S, F32_LOWEST, false, none);
 }
 
 // ---- both in one launch, where a slice is held in registers and all of the launch's workgroups are on the chip
@@ -778,7 +888,7 @@ __global__ __launch_bounds__(THREADS, 4) void k_wide_held(InlineRows rows_arg, L
     }
     offer(ev, edge);   // (-inf where there is none)
     __syncthreads();
-    wide_finish<DT, LSE, THREADS>(wide_table<INLINE>(cfg) + row, cfg, w, sh, n_mine, cand, row, S, lost != 0u, &six);
+    wide_finish<DT, LSE, THREADS, true>(wide_table<INLINE>(cfg) + row, cfg, w, sh, n_mine, cand, row, S, bound, lost != 0u, six);
 }
 
 template <int DT, bool LSE, bool INLINE>

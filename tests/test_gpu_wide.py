@@ -443,3 +443,47 @@ def test_sort_by_sixteen_waves(sampler, n, masked):
                 check_row_against_oracle(whole, i, d)
             else:
                 check_row_against_oracle(run_rows(sampler, x[i:i + 1], kw[i:i + 1], [trial]), 0, d)
+
+
+@pytest.mark.parametrize("rows,vocab,bf16", [(1, 50_257, True), (2, 60_001, False), (6, 50_257, True), (6, 151_936, False), (60, 151_936, True)])
+@pytest.mark.parametrize("pen", [False, True], ids=["plain", "penalties"])
+def test_clusters_of_many_candidates(sampler, rows, vocab, bf16, pen):
+    """More values at the row's bound than its list holds, by sixteen waves, by four, behind one launch and two: clusters of neighbours
+    that lead by far, one value everywhere, all but a few of one value, rows that fall all along; k of 1 024, 700 and 65."""
+    rng = np.random.default_rng(rows + vocab)
+    x = rng.normal(0, 2, (rows, vocab)).astype(np.float32)
+    kinds = 6
+    for i in range(rows):
+        kind = (i + (0 if rows > 1 else 1)) % kinds
+        if kind == 0:
+            x[i, 300:6300] += 9.0
+        elif kind == 1:
+            x[i, vocab // 2:vocab // 2 + 9000] += 9.0
+        elif kind == 2:
+            x[i, :] = 1.5
+        elif kind == 3:
+            x[i, 7:] = -2.0
+        elif kind == 4:
+            x[i] = -np.sort(-x[i])
+        else:
+            x[i, 100:100 + vocab // 3] += 5.0
+    xs = W.to_bf16_bits(x) if bf16 else x
+    more = dict(repetition_penalty=1.1, presence_penalty=0.25, frequency_penalty=0.125) if pen else {}
+    for trial, k in enumerate((0, 700, 65)):
+        kw = [dict(temperature=0.75, top_k=k, top_p=0.99, seed=900 + i, **more) for i in range(rows)]
+        hist = rng.integers(0, 8000, (rows, 600)).astype(np.int32)
+        scratch = None
+        if pen:
+            scratch = []
+            for i in range(rows):
+                sc = LS.SamplerScratch(sampler, vocab)
+                sc.add_history(torch.from_numpy(hist[i]).to(dev()))
+                scratch.append(sc)
+        r = run_rows(sampler, xs, kw, [trial] * rows, scratch=scratch, logprobs=True, use_plan=trial == 1)
+        for i in range(min(rows, 2 * kinds)):
+            counts = np.bincount(hist[i], minlength=vocab).astype(np.uint32) if pen else None
+            d = O.sample(xs[i], counts, o_params(**kw[i]), trial, want_logprob=True)
+            check_row_against_oracle(r, i, d)
+            _check_logprob(r.logprobs[i], d.logprob, (k, i))
+        for sc in scratch or []:
+            sc.close()
