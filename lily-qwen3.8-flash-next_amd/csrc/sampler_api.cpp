@@ -475,12 +475,14 @@ uint32_t blocks_slices(const lily_sampler* s, uint32_t rows, uint32_t kmax, uint
     return sl < 1 ? 1 : sl;
 }
 
-constexpr uint32_t MASKED_MAX_ROWS = 256;
+constexpr uint32_t MASKED_MAX_ROWS = 256, MASKED_MIN_K = 512;
 // Whether a launch goes a workgroup a row over the masks (rows_masked.hip, with the figures of both): where rows draw
-// among many candidates, and a workgroup a row fills the chip no more than once.  (For k <= 64 the streaming selects make
-// less of the difference: 64 rows under masks of 2 % 21.8 -> 19.8 us, under masks of all ids 32 -> 39.)
+// among many candidates, and a workgroup a row fills the chip no more than once.  (For fewer candidates several slices a row
+// look at an open mask's values sooner than one workgroup, and what is open the host does not know.  One row of 151 936 bf16, slices /
+// one workgroup: k = 100 under a mask of 2 % 26 / 19 us, 10 % 28 / 37, 30 % 36 / 57, open 40 / 62; k = 400 30 / 21, 34 / 44, 54 / 62, 55 / 67;
+// k = 700 31 / 23, 39 / 48, 66 / 58, 69 / 66.)
 bool all_masked(const lily_sampler* s, const RowArgs* rows, uint32_t n, uint32_t vocab, uint32_t kmax) {
-    if (kmax <= STREAM_K_MAX || n > MASKED_MAX_ROWS || s->force_path != 0 ||
+    if (kmax < MASKED_MIN_K || n > MASKED_MAX_ROWS || s->force_path != 0 ||
         s->no_held || (s->force_slices != 0 && !s->only_blocks) || vocab > MASKED_MAX_VOCAB) {
         return false;
     }
