@@ -460,3 +460,31 @@ def test_masks_in_clusters(monkeypatch, bf16, vocab):
             _check(r, xs, kw, 5, True, allow=allow)
             assert stats[2] == 0, (slices, k, stats)
         s.close()
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+@pytest.mark.parametrize("share", [1.0, 0.06, -0.3], ids=["open", "one by one", "in runs"])
+def test_masked_sums_of_small_terms(monkeypatch, bf16, share):
+    """One id carries the row, the others add a 50th in terms of 2^-24 to 2^-22 of it, near half a step of its sum in f32: as a sum of f32
+    values in order the log-probability is off by 1e-5; every term's own error is below 2^-21 of it, so that 1e-7 holds
+    with the result's own rounding (of the rest's 0.02 and of the result, below 2e-8 each)."""
+    vocab = 248_320
+    rng = np.random.default_rng(11)
+    x = rng.normal(0, 0.01, (4, vocab)).astype(np.float32)
+    lead = 1234
+    x[:, lead] = 15.5, 16.0, 16.5, 17.0
+    on = rng.random(vocab) < share if share > 0 else np.repeat(rng.random(vocab // 64) < -share, 64)
+    on[lead] = True
+    x[:, lead] += np.float32(np.log(on.sum() / vocab))
+    ids = np.nonzero(on)[0]
+    allow = np.zeros((4, (vocab + 31) // 32), dtype=np.uint32)
+    np.bitwise_or.at(allow, (slice(None), ids >> 5), (1 << (ids & 31)).astype(np.uint32))
+    xs = W.to_bf16_bits(x) if bf16 else x
+    kw = [dict(temperature=1.0, top_k=0, top_p=0.5, seed=i) for i in range(4)]
+    s = _sampler(monkeypatch, "1")
+    r = run_rows(s, xs, kw, [0] * 4, allow=allow, logprobs=True)
+    for i in range(4):
+        d = O.sample(xs[i], None, o_params(**kw[i]), 0, allow=allow[i], want_logprob=True)
+        check_row_against_oracle(r, i, d)
+        assert d.chosen == lead and abs(r.logprobs[i] - d.logprob) <= 1e-7, (i, r.logprobs[i], d.logprob)
+    s.close()
