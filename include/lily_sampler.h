@@ -149,7 +149,7 @@ int lily_sampler_set_phase_trace(lily_sampler_t* s, uint64_t* trace_dev, uint64_
  * (sparse or bitmap), [2] for the exhaustive select; [3] collects a bit per reason the streaming
  * select gave a slice up.  A row of k > 64 that the way for rows of many candidates
  * draws (plain rows without mask or bias list, penalties none or lowering) adds 1 to [1], or to
- * [2], once, whatever the number of its workgroups; so does one that is drawn by a workgroup of its
+ * [2] where more of its values reached its bound than its list holds, once, whatever the number of its workgroups; so does one that is drawn by a workgroup of its
  * own under a mask.  NULL stops. */
 int lily_sampler_set_path_stats(lily_sampler_t* s, uint32_t* stats_dev);
 /* Measurement aid with no counterpart in the reference: one launch that only reads `rows` rows of
@@ -160,7 +160,8 @@ int lily_sampler_set_path_stats(lily_sampler_t* s, uint32_t* stats_dev);
  * row_bytes and stride_bytes multiples of 16. */
 int lily_probe_read(lily_sampler_t* s, const void* base_dev, uint32_t rows, uint64_t row_bytes,
                     uint64_t stride_bytes, uint32_t* out_dev);
-/* Workgroups per row the next launch of `rows` rows with candidate count k would use. */
+/* Workgroups per row of a launch of `rows` plain rows with candidate count k, from a resident batch: without penalties,
+ * masks, bias lists and log-probabilities, which may give another number. */
 uint32_t lily_sampler_slices_for(const lily_sampler_t* s, uint32_t rows, uint32_t k, uint32_t vocab,
                                  lily_dtype dtype);
 
