@@ -527,12 +527,12 @@ void fill_cfg(const lily_sampler* s, LaunchCfg* cfg, uint32_t rows, uint32_t voc
     cfg->list_cap = SPECIAL_LIST_CAP;
 }
 
+constexpr uint32_t WIDE_FINE_GROUPS = 512;
 // Whether a launch over `rows` goes the way of rows that draw among many candidates, and over how
 // many workgroups a row then: every row a plain draw (not forced, given as it is or selected on
 // the device) without mask or bias list, penalties none or of the kind that only lowers (the
 // second launch passes over chunks whose raw values stay below the bound), some row with
 // k > STREAM_K_MAX, and at least two workgroups a row.  0 = no.
-constexpr uint32_t WIDE_FINE_GROUPS = 512;
 uint32_t wide_slices(const lily_sampler* s, const RowArgs* rows, uint32_t n, int dtype, uint32_t vocab) {
     if (s->wide_max == nullptr || s->no_wide || s->force_path != 0 || n > s->ws_rows) {
         return 0;
